@@ -12,14 +12,19 @@ void set_status(int s);
 int init_device(int device);
 int dw_noalloc_setup(int device);  // looks up the fixed partial-sum array of the current device
 
+struct StageBlock;  // pinned host memory and device memory of one size, from a pool (ptl_runtime.hip)
+
 // Maps caller pointers to device pointers.  Device pointers pass through;
 // host pointers get a device buffer from a pool kept between calls, filled
 // before the kernels run (copy_in) and copied back by finish() (copy_out).
 // finish() synchronises only when something was staged.
+// Small host tensors share one pinned block: the CPU copies them into it as they are mapped, failed() - which every
+// caller asks after its mappings and before its launches - enqueues one kernel that fetches all of them, and finish()
+// one that writes all results back.
 class Stager {
    public:
     // device_only: host pointers are rejected instead of staged (callers that may not allocate)
-    explicit Stager(bool device_only = false) : device_only_(device_only) {}
+    explicit Stager(bool device_only = false) : root_(scope()), device_only_(device_only) {}
     ~Stager();
     Stager(const Stager &) = delete;
     Stager &operator=(const Stager &) = delete;
@@ -36,11 +41,15 @@ class Stager {
     T *inout(T *p, size_t n) {
         return static_cast<T *>(map(p, n * sizeof(T), true, true));
     }
-    bool failed() const { return failed_; }
+    bool failed();  // enqueues the copies that are pending
     bool rejected() const { return rejected_; }  // failed because of the arguments, not because of HIP
     int finish(int rc);
     // Gives the staging buffers back without copying anything out (the kernels they were mapped for did not run).
     void discard();
+
+    // The Stager that those made on this thread from now on share (NULL: each its own): a call made of several steps
+    // fetches every host tensor once and waits once, at the end.  A step that fails still returns nothing.
+    static Stager *&scope();
 
    private:
     struct Item {
@@ -49,9 +58,19 @@ class Stager {
         size_t bytes;
         bool copy_out;
         bool copied_in;
+        bool in_block;   // dev lies in block_
+        bool pending;    // in the pinned half of the block, to be fetched
     };
     void *map(const void *p, size_t bytes, bool copy_in, bool copy_out);
+    bool launch_block_copy(bool in);
+    void release();
+    void keep_outputs(bool keep);
     std::vector<Item> items_;
+    Stager *root_;
+    std::vector<size_t> marked_;  // items of root_ that this step is the first to write
+    StageBlock *block_ = nullptr;
+    size_t block_used_ = 0;
+    bool pending_ = false;
     bool failed_ = false;
     bool finished_ = false;
     bool device_only_ = false;

@@ -7,6 +7,9 @@
 extern "C" {
 #endif
 void ptl_internal_set_status(int status);
+/* The steps of one call between these two share the device copies of its host tensors. */
+void ptl_internal_stage_begin(void);
+int ptl_internal_stage_end(int rc);
 /* mat[N x M] += bias broadcast: per_row = 0 adds bias[j] to column j,
  * per_row = 1 adds bias[i] to row i (mm_bias_add_transposed,
  * lib/sources/pulp_train_utils_fp32.c:1286). */

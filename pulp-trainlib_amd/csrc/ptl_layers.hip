@@ -693,9 +693,10 @@ static int conv2d_bw(const Args *a, int ns, const char *fn) {
             }
         }
     }
+    ptl_internal_stage_begin();  // (host tensors: fetched once for both steps)
     int rc = wg ? conv2d_wg<T>(a, ns, fn) : 0;
     if (rc == 0 && ig) rc = conv2d_ig<T>(a, ns, fn);
-    return rc;
+    return ptl_internal_stage_end(rc);
 }
 
 template <typename T, typename Args>

@@ -27,12 +27,14 @@ void pulp_conv2d_fp32_bw_input_grads_cl(void *p) { ptl_internal_set_status(ptl_c
 void pulp_conv2d_fp32_bw_cl(void *p) {
     struct Conv2D_args *a = (struct Conv2D_args *)p;
     int rc = 0;
-    if (a && a->skip_wg_grad == 0) rc = ptl_conv2d_fp32_wg_batched(a, 1);
-    if (a && a->skip_in_grad == 0) {
+    ptl_internal_stage_begin();
+    if (a && a->skip_wg_grad == 0) rc = ptl_conv2d_fp32_bw_batched(a, 1);
+    /* (the weight gradient wants strides that divide the extent, the input gradient alone does not) */
+    if (a && a->skip_in_grad == 0 && (rc != 0 || a->skip_wg_grad != 0)) {
         int r2 = ptl_conv2d_fp32_ig_batched(a, 1);
         if (rc == 0) rc = r2;
     }
-    ptl_internal_set_status(a ? rc : 1);
+    ptl_internal_set_status(ptl_internal_stage_end(a ? rc : 1));
 }
 
 void pulp_conv2d_fp16_fw_cl(void *p) { ptl_internal_set_status(ptl_conv2d_fp16_fw_batched(p, 1)); }
@@ -42,12 +44,14 @@ void pulp_conv2d_fp16_bw_input_grads_cl(void *p) { ptl_internal_set_status(ptl_c
 void pulp_conv2d_fp16_bw_cl(void *p) {
     struct Conv2D_args_fp16 *a = (struct Conv2D_args_fp16 *)p;
     int rc = 0;
-    if (a && a->skip_wg_grad == 0) rc = ptl_conv2d_fp16_wg_batched(a, 1);
-    if (a && a->skip_in_grad == 0) {
+    ptl_internal_stage_begin();
+    if (a && a->skip_wg_grad == 0) rc = ptl_conv2d_fp16_bw_batched(a, 1);
+    /* (the weight gradient wants strides that divide the extent, the input gradient alone does not) */
+    if (a && a->skip_in_grad == 0 && (rc != 0 || a->skip_wg_grad != 0)) {
         int r2 = ptl_conv2d_fp16_ig_batched(a, 1);
         if (rc == 0) rc = r2;
     }
-    ptl_internal_set_status(a ? rc : 1);
+    ptl_internal_set_status(ptl_internal_stage_end(a ? rc : 1));
 }
 
 /* ---- Pointwise (lib/sources/pulp_conv_pw_fp32.c, pulp_conv_pw_fp16.c) ------ */
@@ -59,12 +63,13 @@ void pulp_conv_pw_fp32_bw_input_grads_cl(void *p) { ptl_internal_set_status(ptl_
 void pulp_conv_pw_fp32_bw_cl(void *p) {
     struct PointWise_Conv_args *a = (struct PointWise_Conv_args *)p;
     int rc = 0;
+    ptl_internal_stage_begin();
     if (a && a->skip_wg_grad == 0) rc = ptl_conv_pw_fp32_wg_batched(a, 1);
     if (a && a->skip_in_grad == 0) {
         int r2 = ptl_conv_pw_fp32_ig_batched(a, 1);
         if (rc == 0) rc = r2;
     }
-    ptl_internal_set_status(a ? rc : 1);
+    ptl_internal_set_status(ptl_internal_stage_end(a ? rc : 1));
 }
 
 void pulp_conv_pw_fp16_fw_cl(void *p) { ptl_internal_set_status(ptl_conv_pw_fp16_fw_batched(p, 1)); }
@@ -74,12 +79,13 @@ void pulp_conv_pw_fp16_bw_input_grads_cl(void *p) { ptl_internal_set_status(ptl_
 void pulp_conv_pw_fp16_bw_cl(void *p) {
     struct PointWise_Conv_args_fp16 *a = (struct PointWise_Conv_args_fp16 *)p;
     int rc = 0;
+    ptl_internal_stage_begin();
     if (a && a->skip_wg_grad == 0) rc = ptl_conv_pw_fp16_wg_batched(a, 1);
     if (a && a->skip_in_grad == 0) {
         int r2 = ptl_conv_pw_fp16_ig_batched(a, 1);
         if (rc == 0) rc = r2;
     }
-    ptl_internal_set_status(a ? rc : 1);
+    ptl_internal_set_status(ptl_internal_stage_end(a ? rc : 1));
 }
 
 /* ---- Depthwise (lib/sources/pulp_conv_dw_fp32.c, pulp_conv_dw_fp16.c) ------ */
@@ -91,12 +97,13 @@ void pulp_conv_dw_fp32_bw_input_grads_cl(void *p) { ptl_internal_set_status(ptl_
 void pulp_conv_dw_fp32_bw_cl(void *p) {
     struct DepthWise_Conv_args *a = (struct DepthWise_Conv_args *)p;
     int rc = 0;
+    ptl_internal_stage_begin();
     if (a && a->skip_wg_grad == 0) rc = ptl_conv_dw_fp32_wg_batched(a, 1);
     if (a && a->skip_in_grad == 0) {
         int r2 = ptl_conv_dw_fp32_ig_batched(a, 1);
         if (rc == 0) rc = r2;
     }
-    ptl_internal_set_status(a ? rc : 1);
+    ptl_internal_set_status(ptl_internal_stage_end(a ? rc : 1));
 }
 
 void pulp_conv_dw_fp16_fw_cl(void *p) { ptl_internal_set_status(ptl_conv_dw_fp16_fw_batched(p, 1)); }
@@ -106,12 +113,13 @@ void pulp_conv_dw_fp16_bw_input_grads_cl(void *p) { ptl_internal_set_status(ptl_
 void pulp_conv_dw_fp16_bw_cl(void *p) {
     struct DepthWise_Conv_args_fp16 *a = (struct DepthWise_Conv_args_fp16 *)p;
     int rc = 0;
+    ptl_internal_stage_begin();
     if (a && a->skip_wg_grad == 0) rc = ptl_conv_dw_fp16_wg_batched(a, 1);
     if (a && a->skip_in_grad == 0) {
         int r2 = ptl_conv_dw_fp16_ig_batched(a, 1);
         if (rc == 0) rc = r2;
     }
-    ptl_internal_set_status(a ? rc : 1);
+    ptl_internal_set_status(ptl_internal_stage_end(a ? rc : 1));
 }
 
 /* The kernels the depthwise layer forks (lib/sources/pulp_conv_naive_fp32.c:29,
@@ -196,12 +204,13 @@ void pulp_linear_fp32_bw_input_grads_cl(void *p) { ptl_internal_set_status(ptl_l
 void pulp_linear_fp32_bw_cl(void *p) {
     struct Linear_args *a = (struct Linear_args *)p;
     int rc = 0;
+    ptl_internal_stage_begin();
     if (a && a->skip_wg_grad == 0) rc = ptl_linear_fp32_wg_batched(a, 1);
     if (a && a->skip_in_grad == 0) {
         int r2 = ptl_linear_fp32_ig_batched(a, 1);
         if (rc == 0) rc = r2;
     }
-    ptl_internal_set_status(a ? rc : 1);
+    ptl_internal_set_status(ptl_internal_stage_end(a ? rc : 1));
 }
 
 void pulp_linear_fp16_fw_cl(void *p) { ptl_internal_set_status(ptl_linear_fp16_fw_batched(p, 1)); }
@@ -211,12 +220,13 @@ void pulp_linear_fp16_bw_input_grads_cl(void *p) { ptl_internal_set_status(ptl_l
 void pulp_linear_fp16_bw_cl(void *p) {
     struct Linear_args_fp16 *a = (struct Linear_args_fp16 *)p;
     int rc = 0;
+    ptl_internal_stage_begin();
     if (a && a->skip_wg_grad == 0) rc = ptl_linear_fp16_wg_batched(a, 1);
     if (a && a->skip_in_grad == 0) {
         int r2 = ptl_linear_fp16_ig_batched(a, 1);
         if (rc == 0) rc = r2;
     }
-    ptl_internal_set_status(a ? rc : 1);
+    ptl_internal_set_status(ptl_internal_stage_end(a ? rc : 1));
 }
 
 /* ---- mm family and mm_manager ------------------------------------------------- */

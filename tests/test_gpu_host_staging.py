@@ -1,0 +1,59 @@
+"""Host tensors: calls on them give the bits of the same calls on device tensors, whatever mix of small tensors (which
+travel together through one pinned block) and large ones (a copy each) a call has."""
+import numpy as np
+import pytest
+import torch
+
+import helpers as hp
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+# (a byte-odd tensor; below, at and above the largest tensor of a block: 1 MiB; more than a block of 4 MiB in all)
+@pytest.mark.parametrize("dt,n_in,n_out", [("fp16", 3, 5), ("fp32", 33, 65), ("fp32", 512, 512), ("fp32", 513, 512),
+                                           ("fp16", 1000, 900)])
+@pytest.mark.parametrize("skip", [(0, 0), (1, 0), (0, 1)])
+def test_linear_on_host_arrays_matches_device(pkg, gpu, dt, n_in, n_out, skip):
+    nd = hp.np_dtype(dt)
+    x, w, dy = (hp.uniform(5 + i, s, dtype=nd) for i, s in enumerate(((n_in,), (n_out, n_in), (n_out,))))
+    res = []
+    for place in (lambda a: a.copy(), lambda a: torch.from_numpy(a).to(DEV)):
+        t = [place(a) for a in (x, np.full(n_in, 3, nd), w, np.full((n_out, n_in), 3, nd), np.zeros(n_out, nd), dy)]
+        a, keep = hp.linear_args(pkg, *t, n_in, n_out)
+        a.skip_wg_grad, a.skip_in_grad = skip
+        pkg.call("pulp_linear_%s_fw_cl" % dt, a)
+        pkg.call("pulp_linear_%s_bw_cl" % dt, a)
+        assert gpu.ptl_sync() == 0
+        res.append([v if isinstance(v, np.ndarray) else v.cpu().numpy() for v in t])
+    for h, d in zip(*res):
+        assert np.array_equal(h, d)
+
+
+def test_a_call_with_more_host_tensors_than_one_copy_kernel_takes(pkg, gpu):
+    nd, opts, keep, ref = np.float32, [], [], []
+    for i in range(45):  # 90 tensors, the last ones beyond the block
+        n = 40000 if i > 12 else 7 + i
+        w, dw = hp.uniform(i, (n,), dtype=nd), hp.uniform(100 + i, (n,), dtype=nd)
+        ref.append(w - np.float32(0.5) * dw)
+        o, kp = hp.optim_args(pkg, "fp32", w, dw, None, None, 0.5, 0.0)
+        opts.append(o)
+        keep.append((kp, w))
+    table = (type(opts[0]) * len(opts))(*opts)
+    assert gpu.ptl_gradient_descent_fp32_multi(table, len(opts)) == 0, gpu.ptl_last_error().decode()
+    for (_, w), r in zip(keep, ref):
+        assert np.allclose(w, r, rtol=0, atol=1e-6)
+
+
+def test_a_rejected_step_returns_nothing_and_the_other_still_runs(pkg, gpu):
+    """A stride that does not divide the extent: the weight gradient rejects it, the input gradient does not."""
+    Ci, Co, H, K, s = 4, 8, 10, 3, 2
+    Ho = hp.conv_out(H, K, 1, 1, s)
+    x, w, dy = (hp.uniform(9 + i, sh) for i, sh in enumerate(((Ci, H, H), (Co, Ci, K, K), (Co, Ho, Ho))))
+    dx, dw = np.full_like(x, 3), np.full_like(w, 3)
+    a, keep = hp.conv2d_args(pkg, x, dx, w, dw, np.zeros_like(dy), dy, Ci, H, H, Co, K, K, Ho, Ho, (1, 1, 1, 1), (s, s))
+    with pytest.raises(RuntimeError):
+        pkg.call("pulp_conv2d_fp32_bw_cl", a)
+    ref = torch.nn.grad.conv2d_input((1, Ci, H, H), torch.from_numpy(w).double(), torch.from_numpy(dy).double()[None],
+                                     stride=s, padding=1)[0]
+    assert np.all(dw == 3) and hp.rel_l2(dx, ref.numpy()) <= 1e-4
