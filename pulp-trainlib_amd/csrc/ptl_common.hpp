@@ -57,6 +57,7 @@ struct GemmArgs {
     const void *B;
     void *C;       // output tensor (written through `c` when splits == 1)
     float *ws;     // split-K partial sums, [splits][N][M] fp32
+    const void *bias;  // added per m where the product is stored (not by the register-staged kernel)
     OperandMap a;  // rows = n index
     OperandMap b;  // rows = m index
     OutMap c;
@@ -162,11 +163,19 @@ int gemm_async(GemmArgs &g);
 // tile shape, else one after the other.
 template <typename T>
 int gemm_pair(const GemmArgs &g0, const GemmArgs &g1);
+// The one launch alone: -1 when the products do not share one.
+template <typename T>
+int gemm_pair_lean(const GemmArgs &g0, const GemmArgs &g1);
+// Weight, input and (where db is given) bias gradient of a dense layer in one launch: on one sample; on a batch.
+template <typename T>
+int linear_one_bw(const T *x, const T *W, const T *dy, T *dW, T *dx, T *db, int in, int out);
+template <typename T>
+int linear_bw_ragged(const T *X, const T *W, const T *dY, T *dW, T *dX, T *db, int ns, int in, int out);
 template <typename T>
 int gemm_async_pair(GemmArgs &g0, GemmArgs &g1);
 
-// GEMV / outer-product kernels for products with a unit dimension.
+// GEMV / outer-product kernels for products with a unit dimension.  `bias` (per column) is added where it is given.
 template <typename T>
-int mm_dispatch(const T *A, const T *B, T *C, int N, int M, int K, int trans_B);
+int mm_dispatch(const T *A, const T *B, T *C, int N, int M, int K, int trans_B, const T *bias = nullptr);
 
 }  // namespace ptl

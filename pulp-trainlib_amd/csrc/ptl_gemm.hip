@@ -17,6 +17,8 @@
 //   * optional split-K: grid.y slices k, fp32 partials go to a workspace and a
 //     second kernel sums them in a fixed order (deterministic).
 #include "ptl_common.hpp"
+#include "ptl_ragged.hpp"
+#include "ptl_gemm_async.hpp"
 
 namespace ptl {
 
@@ -347,7 +349,7 @@ __global__ __launch_bounds__(256) void gemm_kernel(const GemmArgs g) {
 // and many splits the kernel lives on memory-level parallelism.
 template <typename T>
 __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float *__restrict__ ws, T *__restrict__ C,
-                                                            OutMap c, int N, int M, int splits) {
+                                                            OutMap c, int N, int M, int splits, const T *__restrict__ bias) {
     __shared__ float part[4][64];
     const size_t total = (size_t)N * M;
     const int o = threadIdx.x & 63, sg = threadIdx.x >> 6;
@@ -373,7 +375,20 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float *__restr
     int on, om, h, w;
     axis_decode(c.n, n, on, h, w);
     axis_decode(c.m, m, om, h, w);
+    if (bias) s += (float)bias[m];
     C[on + om] = (T)s;
+}
+
+// The bias of a product that the register-staged kernel has stored.
+template <typename T>
+__global__ __launch_bounds__(256) void bias_map_kernel(T *__restrict__ C, OutMap c, int N, int M, const T *__restrict__ bias) {
+    const size_t idx = (size_t)blockIdx.x * 256 + threadIdx.x;
+    if (idx >= (size_t)N * M) return;
+    const int n = (int)(idx / M), m = (int)(idx % M);
+    int on, om, h, w;
+    axis_decode(c.n, n, on, h, w);
+    axis_decode(c.m, m, om, h, w);
+    C[on + om] = (T)((float)C[on + om] + (float)bias[m]);
 }
 
 // ---------------------------------------------------------------------------
@@ -476,6 +491,64 @@ static int launch_staged(GemmArgs &g) {
     return hip_ok(hipGetLastError(), "gemm launch") ? 0 : 2;
 }
 
+// The product as the kernel for any size and alignment takes it: both operands matrices that are contiguous along k or
+// along their rows, k a single axis or runs of one (sample, pixel), the rows of one operand likewise.  -1: not such a
+// product.
+template <typename T>
+static int gemm_ragged(const GemmArgs &gin) {
+    constexpr long long ES = (long long)sizeof(T);
+    GemmArgs g = gin;
+    bool swapped = false;
+    auto two = [](const AxisMap &a) { return !axis_is_single(a); };
+    // the operand whose rows have two digits, and the one along which the output is contiguous, go second
+    if (two(g.a.row) || (!two(g.b.row) && g.c.m.o0 != 1 && g.c.n.o0 == 1)) {
+        GemmArgs t = g;
+        t.A = g.B; t.B = g.A; t.a = g.b; t.b = g.a; t.N = g.M; t.M = g.N; t.c.n = g.c.m; t.c.m = g.c.n;
+        g = t;
+        swapped = true;
+    }
+    auto simple = [](const AxisMap &a) { return axis_is_single(a) || (a.d1 >= (1 << 30) && a.n % a.d0 == 0); };
+    if (!simple(g.a.k) || !simple(g.b.k) || !axis_is_single(g.a.row) || !simple(g.b.row) || !simple(g.c.m) || !axis_is_single(g.c.n)) return -1;
+    if (!no_coords(g.a.row) || !no_coords(g.a.k) || !no_coords(g.b.row) || !no_coords(g.b.k) || g.taps > 1) return -1;
+    if (two(g.a.k) != two(g.b.k) || (two(g.a.k) && g.a.k.d0 != g.b.k.d0) || two(g.b.row) != two(g.c.m) ||
+        (two(g.b.row) && g.b.row.d0 != g.c.m.d0) || g.c.n.ob || g.c.m.ob)
+        return -1;
+    RagArgs r = {};
+    RagProd &p = r.p[0];
+    r.count = 1;
+    p.N = g.N;
+    p.M = g.M;
+    p.K = two(g.a.k) ? g.a.k.d0 : g.K;
+    p.runs = g.K / p.K;
+    p.m_in = two(g.b.row) ? g.b.row.d0 : g.M;
+    p.outer = g.M / p.m_in;
+    auto operand = [&](const OperandMap &o, const void *base, int rows, RagOp &q) {
+        const AxisMap &row = o.row, &k = o.k;
+        const int in = axis_is_single(row) ? rows : row.d0;
+        if (row.ob < 0 || k.ob < 0 || row.o0 <= 0 || k.o0 <= 0 || row.o1 < 0 || k.o1 < 0) return -1;
+        if (k.o0 != 1 && row.o0 != 1) return -1;
+        if ((long long)row.o0 * ES >= (1ll << 24) || (long long)k.o0 * ES >= (1ll << 24)) return -1;  // (128 rows in 32 bits)
+        q.p = reinterpret_cast<const char *>(base) + (row.ob + (long long)k.ob) * ES;
+        q.rows = in;
+        q.row_b = (unsigned)(row.o0 * ES);
+        q.k_b = (unsigned)(k.o0 * ES);
+        q.run_b = p.runs > 1 ? (long long)k.o1 * ES : 0;
+        q.outer_b = in < rows ? (long long)row.o1 * ES : 0;
+        // (a piece must fit into the contiguous run it is read from)
+        constexpr int VEC = 16 / (int)sizeof(T);
+        const bool kc = k.o0 == 1 && p.K >= VEC, rc = row.o0 == 1 && in >= VEC;
+        return kc && (!rc || p.K >= in) ? (int)RAG_KC : rc ? (int)RAG_RC : -1;
+    };
+    const int am = operand(g.a, g.A, g.N, p.a), bm = operand(g.b, g.B, g.M, p.b);
+    if (am < 0 || bm < 0 || (p.outer > 1 && bm != RAG_RC)) return -1;
+    p.bias = g.bias;
+    p.bias_n = swapped;
+    p.C = g.C;
+    p.cn = rag_axis(g.N, g.c.n.o0);
+    p.cm = two(g.c.m) ? rag_axis2(g.c.m.d0, g.c.m.o0, g.c.m.o1) : rag_axis(g.M, g.c.m.o0);
+    return ragged<T>(r, am, bm, am, bm);
+}
+
 template <typename T>
 int gemm(const GemmArgs &gin) {
     if (!ensure_init()) return 2;
@@ -487,23 +560,39 @@ int gemm(const GemmArgs &gin) {
     g.b.mode = choose_mode<T>(g.b, g.B, g.M, g.K);
 
     int rc = -1;
-    if (st.gemm_path != 1) rc = gemm_async<T>(g);
+    if (st.gemm_path != 1) {
+        // whole slabs of aligned rows: the look-up-free kernel; other matrices: the one for any size and alignment;
+        // index maps with coordinates: the gathering kernel
+        constexpr int SK = 128 / (int)sizeof(T);
+        const bool lean_runs = g.a.mode == FILL_VEC_K && g.b.mode == FILL_VEC_K && !axis_is_single(g.a.k) && g.a.k.d0 == g.b.k.d0 &&
+                               g.a.k.d0 % SK == 0;
+        if (!lean_runs && !(plain_operand<T>(g.a, SK, g.K) && plain_operand<T>(g.b, SK, g.K))) {
+            rc = gemm_ragged<T>(g);
+            if (rc >= 0) return rc;
+        }
+        rc = gemm_async<T>(g);
+    }
     if (rc > 0) return rc;
     if (rc < 0) {
         rc = launch_staged<T>(g);
         if (rc) return rc;
+        if (g.bias && g.splits == 1) {
+            hipLaunchKernelGGL((bias_map_kernel<T>), dim3((unsigned)(((size_t)g.N * g.M + 255) / 256)), dim3(256), 0, st.stream,
+                               reinterpret_cast<T *>(g.C), g.c, g.N, g.M, reinterpret_cast<const T *>(g.bias));
+            if (!hip_ok(hipGetLastError(), "bias add launch")) return 2;
+        }
     }
     if (g.splits > 1) {
         size_t total = (size_t)g.N * g.M;
         hipLaunchKernelGGL((splitk_reduce_kernel<T>), dim3((unsigned)((total + 63) / 64)), dim3(256), 0,
-                           st.stream, g.ws, reinterpret_cast<T *>(g.C), g.c, g.N, g.M, g.splits);
+                           st.stream, g.ws, reinterpret_cast<T *>(g.C), g.c, g.N, g.M, g.splits, reinterpret_cast<const T *>(g.bias));
         if (!hip_ok(hipGetLastError(), "split-k reduce launch")) return 2;
     }
     return 0;
 }
 
 template <typename T>
-int gemm_pair(const GemmArgs &g0in, const GemmArgs &g1in) {
+int gemm_pair_lean(const GemmArgs &g0in, const GemmArgs &g1in) {
     if (!ensure_init()) return 2;
     GemmArgs g0 = g0in, g1 = g1in;
     if (state().gemm_path == 0 && g0.N > 0 && g0.M > 0 && g0.K > 0 && g1.N > 0 && g1.M > 0 && g1.K > 0) {
@@ -514,9 +603,59 @@ int gemm_pair(const GemmArgs &g0in, const GemmArgs &g1in) {
         int rc = gemm_async_pair<T>(g0, g1);
         if (rc >= 0) return rc;
     }
-    int rc = gemm<T>(g0in);
+    return -1;
+}
+
+template <typename T>
+int gemm_pair(const GemmArgs &g0in, const GemmArgs &g1in) {
+    int rc = gemm_pair_lean<T>(g0in, g1in);
+    if (rc >= 0) return rc;
+    rc = gemm<T>(g0in);
     return rc ? rc : gemm<T>(g1in);
 }
+template int gemm_pair_lean<float>(const GemmArgs &, const GemmArgs &);
+template int gemm_pair_lean<half_t>(const GemmArgs &, const GemmArgs &);
+
+// dW[o][i] = sum_b dY[b][o] X[b][i] and dX[b][i] = sum_o dY[b][o] W[o][i] and
+// the bias gradient db[o] = sum_b dY[b][o] (null: none) as one launch of the kernel for any size and alignment; -1 when a
+// row is shorter than its 16-byte pieces.
+template <typename T>
+int linear_bw_ragged(const T *X, const T *W, const T *dY, T *dW, T *dX, T *db, int ns, int in, int out) {
+    constexpr int VEC = 16 / (int)sizeof(T), ES = (int)sizeof(T);
+    if (in < VEC || out < VEC || in >= (1 << 22) || out >= (1 << 22)) return -1;
+    auto matrix = [](const T *p, int rows, int row_stride, int k_stride) {
+        RagOp q = {};
+        q.p = reinterpret_cast<const char *>(p);
+        q.rows = rows;
+        q.row_b = (unsigned)row_stride * ES;
+        q.k_b = (unsigned)k_stride * ES;
+        return q;
+    };
+    RagArgs r = {};
+    r.count = 2;
+    RagProd &w = r.p[0], &x = r.p[1];
+    w.a = matrix(dY, out, 1, out);
+    w.b = matrix(X, in, 1, in);
+    w.C = dW;
+    w.N = out;
+    w.M = w.m_in = in;
+    w.K = ns;
+    w.row_sum = db;
+    w.cn = rag_axis(out, in);
+    w.cm = rag_axis(in, 1);
+    x.a = matrix(dY, ns, out, 1);
+    x.b = matrix(W, in, 1, in);
+    x.C = dX;
+    x.N = ns;
+    x.M = x.m_in = in;
+    x.K = out;
+    x.cn = rag_axis(ns, in);
+    x.cm = rag_axis(in, 1);
+    w.runs = x.runs = w.outer = x.outer = 1;
+    return ragged<T>(r, RAG_RC, RAG_RC, RAG_KC, RAG_RC);
+}
+template int linear_bw_ragged<float>(const float *, const float *, const float *, float *, float *, float *, int, int, int);
+template int linear_bw_ragged<half_t>(const half_t *, const half_t *, const half_t *, half_t *, half_t *, half_t *, int, int, int);
 
 template int gemm_pair<float>(const GemmArgs &, const GemmArgs &);
 template int gemm_pair<half_t>(const GemmArgs &, const GemmArgs &);
@@ -524,243 +663,189 @@ template int gemm<float>(const GemmArgs &);
 template int gemm<half_t>(const GemmArgs &);
 
 // ---------------------------------------------------------------------------
-// Products with a unit dimension (Linear at batch 1): bandwidth-bound kernels.
+// Products with a unit dimension (Linear at batch 1): bound by the launch below about 1 MB (2.5 us of host time each),
+// by memory above.  All of them read and write 16-byte pieces at any element alignment; the last piece of a row is the
+// one that ends with it (columns it shares with the piece before are worked out twice, with the same result), rows
+// shorter than a piece go element by element (V = 1).
 // ---------------------------------------------------------------------------
+constexpr int GV_NT = 1024;
 
-// y[r] = sum_k Mx[r*K + k] * x[k]; one wave per row.
-template <typename T>
-__global__ __launch_bounds__(256) void gemv_rowdot_kernel(const T *__restrict__ Mx, const T *__restrict__ x,
-                                                          T *__restrict__ y, int R, int K, int vec_ok) {
-    constexpr int VEC = Traits<T>::VEC;
-    int row = blockIdx.x * 4 + (threadIdx.x >> 6);
-    int lane = threadIdx.x & 63;
+template <typename T, int V>
+struct GvPiece {
+    T e[V];
+};
+template <typename T, int V>
+__device__ inline GvPiece<T, V> gv_load(const T *p) {
+    GvPiece<T, V> v;
+    __builtin_memcpy(&v, p, sizeof(v));
+    return v;
+}
+
+// y[r] = sum_k Mx[r*K + k] * x[k] (+ bias[r]); one wave per row.
+template <typename T, int V>
+__global__ __launch_bounds__(256) void gemv_rowdot_kernel(const T *__restrict__ Mx, const T *__restrict__ x, T *__restrict__ y,
+                                                          const T *__restrict__ bias, int R, int K) {
+    const int row = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
     if (row >= R) return;
     const T *p = Mx + (size_t)row * K;
     float s = 0.f;
-    if (vec_ok) {
-        for (int k = lane * VEC; k < K; k += 64 * VEC) {
-            Stage<T> a, b;
-            a.v[0] = *reinterpret_cast<const uint4 *>(p + k);
-            b.v[0] = *reinterpret_cast<const uint4 *>(x + k);
+    const int whole = K / V * V;
+    for (int k = lane * V; k < whole; k += 64 * V) {
+        const GvPiece<T, V> a = gv_load<T, V>(p + k), b = gv_load<T, V>(x + k);
 #pragma unroll
-            for (int i = 0; i < VEC; ++i) s += (float)a.e[i] * (float)b.e[i];
-        }
-    } else {
-        for (int k = lane; k < K; k += 64) s += (float)p[k] * (float)x[k];
+        for (int i = 0; i < V; ++i) s += (float)a.e[i] * (float)b.e[i];
     }
+    if (whole + lane < K) s += (float)p[whole + lane] * (float)x[whole + lane];
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) s += __shfl_down(s, o, 64);
-    if (lane == 0) y[row] = (T)s;
+    if (lane == 0) y[row] = (T)(bias ? s + (float)bias[row] : s);
 }
 
-// part[z][m] = sum_{k in slice z} x[k] * Mx[k*M + m]
-template <typename T>
-__global__ __launch_bounds__(256) void gemv_coldot_kernel(const T *__restrict__ x, const T *__restrict__ Mx,
-                                                          float *__restrict__ part, int K, int M, int kchunk) {
-    int m = blockIdx.x * 256 + threadIdx.x;
-    if (m >= M) return;
-    int k0 = blockIdx.y * kchunk;
-    int k1 = min(K, k0 + kchunk);
-    float s = 0.f;
-    for (int k = k0; k < k1; ++k) s += (float)x[k] * (float)Mx[(size_t)k * M + m];
-    part[(size_t)blockIdx.y * M + m] = s;
-}
-
-// Same product with 16-byte loads: a workgroup owns CV*VEC consecutive columns and a
-// slice of k; thread (kl, cv) sums rows k0+kl, k0+kl+32, ... of column vector cv, the
-// 32 row-lanes are then folded through LDS.
-template <typename T>
-__global__ __launch_bounds__(256) void gemv_coldot_vec_kernel(const T *__restrict__ x, const T *__restrict__ Mx,
-                                                              float *__restrict__ part, int K, int M, int kchunk) {
-    constexpr int VEC = Traits<T>::VEC, CV = 8, KL = 256 / CV;
+// y[m] = sum_k x[k] * Mx[k*M + m] for the four pieces of columns of workgroup `block`: thread (kl, cv) sums rows kl,
+// kl + 256, ... of piece cv with four loads in flight, the rows meet in LDS (first eight, then the rest).
+template <typename T, int V>
+__device__ inline void gemv_coldot_block(const T *__restrict__ x, const T *__restrict__ Mx, T *__restrict__ y, int K, int M,
+                                         int block, float *red) {
+    constexpr int CV = 4, KL = GV_NT / CV, U = 4;
     const int cv = threadIdx.x % CV, kl = threadIdx.x / CV;
-    const int col = (blockIdx.x * CV + cv) * VEC;
-    const int k0 = blockIdx.y * kchunk, k1 = min(K, k0 + kchunk);
-    float acc[VEC];
+    const int want = (block * CV + cv) * V, col = want + V <= M ? want : M - V;
+    float acc[V];
 #pragma unroll
-    for (int i = 0; i < VEC; ++i) acc[i] = 0.f;
-    if (col < M) {
-        for (int k = k0 + kl; k < k1; k += KL) {
-            Stage<T> v;
-            v.v[0] = *reinterpret_cast<const uint4 *>(Mx + (size_t)k * M + col);
-            float xv = (float)x[k];
+    for (int i = 0; i < V; ++i) acc[i] = 0.f;
+    const T *p = Mx + col;
+    if (want < M) {
+        for (int k = kl; k < K; k += U * KL) {
+            GvPiece<T, V> v[U];
+            float xv[U];
 #pragma unroll
-            for (int i = 0; i < VEC; ++i) acc[i] += xv * (float)v.e[i];
-        }
-    }
-    __shared__ float red[KL][CV * VEC + 1];
-#pragma unroll
-    for (int i = 0; i < VEC; ++i) red[kl][cv * VEC + i] = acc[i];
-    __syncthreads();
-    if (threadIdx.x < CV * VEC) {
-        float s = 0.f;
-#pragma unroll 8
-        for (int r = 0; r < KL; ++r) s += red[r][threadIdx.x];
-        int c = blockIdx.x * CV * VEC + threadIdx.x;
-        if (c < M) part[(size_t)blockIdx.y * M + c] = s;
-    }
-}
-
-// The same product in ONE launch for moderate K: a workgroup owns 4*VEC consecutive columns and
-// ALL rows; thread (kl, cv) sums rows kl, kl+64, ... of column vector cv with eight loads in
-// flight, the 64 row-lanes are folded through LDS.  (A cross-workgroup "last arriver adds the
-// partials" variant was tried: the device-scope fences it needs write back the whole L2 per
-// workgroup and made it twice as slow as two launches.)
-template <typename T>
-__global__ __launch_bounds__(256) void gemv_coldot_whole_kernel(const T *__restrict__ x, const T *__restrict__ Mx,
-                                                                T *__restrict__ y, int K, int M) {
-    constexpr int VEC = Traits<T>::VEC, CV = 4, KL = 256 / CV;
-    const int cv = threadIdx.x % CV, kl = threadIdx.x / CV;
-    const int col = (blockIdx.x * CV + cv) * VEC;
-    float acc[VEC];
-#pragma unroll
-    for (int i = 0; i < VEC; ++i) acc[i] = 0.f;
-    if (col < M) {
-        const T *p = Mx + col;
-        int k = kl;
-        for (; k + 7 * KL < K; k += 8 * KL) {
-            Stage<T> v[8];
-            float xv[8];
-#pragma unroll
-            for (int u = 0; u < 8; ++u) {
-                v[u].v[0] = *reinterpret_cast<const uint4 *>(p + (size_t)(k + u * KL) * M);
-                xv[u] = (float)x[k + u * KL];
+            for (int u = 0; u < U; ++u) {  // (rows beyond the end: the last one, times zero)
+                const int kk = k + u * KL < K ? k + u * KL : K - 1;
+                v[u] = gv_load<T, V>(p + (size_t)kk * M);
+                xv[u] = (float)x[kk];
             }
 #pragma unroll
-            for (int u = 0; u < 8; ++u)
+            for (int u = 0; u < U; ++u) {
+                if (k + u * KL >= K) break;
 #pragma unroll
-                for (int i = 0; i < VEC; ++i) acc[i] += xv[u] * (float)v[u].e[i];
-        }
-        for (; k < K; k += KL) {
-            Stage<T> v;
-            v.v[0] = *reinterpret_cast<const uint4 *>(p + (size_t)k * M);
-            const float xv = (float)x[k];
-#pragma unroll
-            for (int i = 0; i < VEC; ++i) acc[i] += xv * (float)v.e[i];
+                for (int i = 0; i < V; ++i) acc[i] += xv[u] * (float)v[u].e[i];
+            }
         }
     }
-    __shared__ float red[KL][CV * VEC + 1];
+    // lanes of a wave that share a piece are CV apart
 #pragma unroll
-    for (int i = 0; i < VEC; ++i) red[kl][cv * VEC + i] = acc[i];
+    for (int i = 0; i < V; ++i)
+#pragma unroll
+        for (int o = 32; o >= CV; o >>= 1) acc[i] += __shfl_xor(acc[i], o, 64);
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    if (lane < CV) {
+#pragma unroll
+        for (int i = 0; i < V; ++i) red[wave * (CV * V) + lane * V + i] = acc[i];
+    }
     __syncthreads();
-    if (threadIdx.x < CV * VEC) {
+    if ((int)threadIdx.x < CV * V) {
+        const int c = threadIdx.x / V, first = (block * CV + c) * V, at = first + V <= M ? first : M - V;
         float s = 0.f;
-#pragma unroll 8
-        for (int r = 0; r < KL; ++r) s += red[r][threadIdx.x];
-        const int c = blockIdx.x * CV * VEC + threadIdx.x;
-        if (c < M) y[c] = (T)s;
+#pragma unroll
+        for (int w = 0; w < GV_NT / 64; ++w) s += red[w * (CV * V) + threadIdx.x];
+        if (first < M) y[at + threadIdx.x % V] = (T)s;
     }
 }
 
-template <typename T>
-__global__ __launch_bounds__(256) void colsum_reduce_kernel(const float *__restrict__ part, T *__restrict__ y,
-                                                            int M, int splits) {
-    int m = blockIdx.x * 256 + threadIdx.x;
-    if (m >= M) return;
-    float s = 0.f;
-    for (int z = 0; z < splits; ++z) s += part[(size_t)z * M + m];
-    y[m] = (T)s;
+template <typename T, int V>
+__global__ __launch_bounds__(GV_NT) void gemv_coldot_kernel(const T *__restrict__ x, const T *__restrict__ Mx, T *__restrict__ y,
+                                                            int K, int M) {
+    __shared__ float red[GV_NT / 64 * 4 * V];
+    gemv_coldot_block<T, V>(x, Mx, y, K, M, blockIdx.x, red);
 }
 
-// C[n*M + m] = a[n] * b[m]
-template <typename T>
-__global__ __launch_bounds__(256) void outer_kernel(const T *__restrict__ a, const T *__restrict__ b,
-                                                    T *__restrict__ C, int N, int M) {
-    size_t idx = (size_t)blockIdx.x * 256 + threadIdx.x;
-    size_t total = (size_t)N * M;
-    if (idx >= total) return;
-    int n = (int)(idx / M), m = (int)(idx % M);
-    C[idx] = (T)((float)a[n] * (float)b[m]);
-}
-
-// Same with 16-byte stores (M a multiple of the vector, b and C 16-byte aligned): a thread owns VEC
-// consecutive columns of four consecutive rows.
-template <typename T>
-__global__ __launch_bounds__(256) void outer_vec_kernel(const T *__restrict__ a, const T *__restrict__ b,
-                                                        T *__restrict__ C, int N, int M) {
-    constexpr int VEC = Traits<T>::VEC;
-    const int mv = M / VEC;
-    const size_t idx = (size_t)blockIdx.x * 256 + threadIdx.x;
-    const size_t total = (size_t)((N + 3) / 4) * mv;
-    if (idx >= total) return;
-    const int n0 = (int)(idx / mv) * 4, m = (int)(idx % mv) * VEC;
-    Stage<T> bv, out;
-    bv.v[0] = *reinterpret_cast<const uint4 *>(b + m);
+// C[n*M + m] = a[n] * b[m]: unit `i` is a piece of columns of four consecutive rows; the first piece of a row also copies
+// a[n] to `copy` where that is wanted (the bias gradient of one sample).
+template <typename T, int V>
+__device__ inline void outer_unit(const T *__restrict__ a, const T *__restrict__ b, T *__restrict__ C, T *__restrict__ copy,
+                                  int N, int M, RagDiv per_row, unsigned i) {
+    const unsigned q = per_row.m ? __umulhi(i, per_row.m) >> per_row.s : i;
+    const int n0 = (int)q * 4, want = (int)(i - q * per_row.d) * V;
+    if (n0 >= N) return;
+    const int m = want + V <= M ? want : M - V;
+    const GvPiece<T, V> bv = gv_load<T, V>(b + m);
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
         if (n0 + r >= N) break;
-        const float av = (float)a[n0 + r];
+        const T an = a[n0 + r];
+        const float av = (float)an;
+        GvPiece<T, V> out;
 #pragma unroll
-        for (int i = 0; i < VEC; ++i) out.e[i] = (T)(av * (float)bv.e[i]);
-        *reinterpret_cast<uint4 *>(C + (size_t)(n0 + r) * M + m) = out.v[0];
+        for (int e = 0; e < V; ++e) out.e[e] = (T)(av * (float)bv.e[e]);
+        __builtin_memcpy(C + (size_t)(n0 + r) * M + m, &out, sizeof(out));
+        if (copy && want == 0) copy[n0 + r] = an;
     }
 }
 
+template <typename T, int V>
+__global__ __launch_bounds__(GV_NT) void outer_kernel(const T *__restrict__ a, const T *__restrict__ b, T *__restrict__ C, int N,
+                                                      int M, RagDiv per_row) {
+    outer_unit<T, V>(a, b, C, nullptr, N, M, per_row, blockIdx.x * GV_NT + threadIdx.x);
+}
+
+// Both gradients of a dense layer on one sample in one launch (1024 x 1024 in fp32: 5.9 us as two launches, bound by the
+// host; 3.3 as one): the first `cols` workgroups sum columns for dX, the rest write dW (and db = dY).
+template <typename T, int V>
+__global__ __launch_bounds__(GV_NT) void linear_one_bw_kernel(const T *__restrict__ x, const T *__restrict__ W,
+                                                              const T *__restrict__ dy, T *__restrict__ dW, T *__restrict__ dx,
+                                                              T *__restrict__ db, int in, int out, RagDiv per_row, int cols) {
+    __shared__ float red[GV_NT / 64 * 4 * V];
+    if ((int)blockIdx.x < cols)
+        gemv_coldot_block<T, V>(dy, W, dx, out, in, blockIdx.x, red);
+    else
+        outer_unit<T, V>(dy, x, dW, db, out, in, per_row, (blockIdx.x - cols) * GV_NT + threadIdx.x);
+}
+
+static unsigned outer_blocks(int N, int M, int V) {
+    return (unsigned)(((size_t)((N + 3) / 4) * ((M + V - 1) / V) + GV_NT - 1) / GV_NT);
+}
+
+template <typename T, int V>
+static int linear_one_bw_v(const T *x, const T *W, const T *dy, T *dW, T *dx, T *db, int in, int out) {
+    const int cols = (in + 4 * V - 1) / (4 * V);
+    hipLaunchKernelGGL((linear_one_bw_kernel<T, V>), dim3(cols + outer_blocks(out, in, V)), dim3(GV_NT), 0, state().stream, x, W,
+                       dy, dW, dx, db, in, out, rag_div((in + V - 1) / V), cols);
+    return hip_ok(hipGetLastError(), "linear backward launch") ? 0 : 2;
+}
 template <typename T>
-static int gemv_rowdot(const T *Mx, const T *x, T *y, int R, int K) {
+int linear_one_bw(const T *x, const T *W, const T *dy, T *dW, T *dx, T *db, int in, int out) {
     constexpr int VEC = Traits<T>::VEC;
-    State &st = state();
-    int vec_ok = (K % VEC == 0) && (reinterpret_cast<uintptr_t>(Mx) % 16 == 0) &&
-                 (reinterpret_cast<uintptr_t>(x) % 16 == 0);
-    hipLaunchKernelGGL((gemv_rowdot_kernel<T>), dim3((R + 3) / 4), dim3(256), 0, st.stream, Mx, x, y, R, K,
-                       vec_ok);
+    return in >= VEC ? linear_one_bw_v<T, VEC>(x, W, dy, dW, dx, db, in, out) : linear_one_bw_v<T, 1>(x, W, dy, dW, dx, db, in, out);
+}
+template int linear_one_bw<float>(const float *, const float *, const float *, float *, float *, float *, int, int);
+template int linear_one_bw<half_t>(const half_t *, const half_t *, const half_t *, half_t *, half_t *, half_t *, int, int);
+
+template <typename T>
+static int gemv_rowdot(const T *Mx, const T *x, T *y, const T *bias, int R, int K) {
+    hipLaunchKernelGGL((gemv_rowdot_kernel<T, Traits<T>::VEC>), dim3((R + 3) / 4), dim3(256), 0, state().stream, Mx, x, y, bias, R, K);
     return hip_ok(hipGetLastError(), "gemv launch") ? 0 : 2;
 }
 
 template <typename T>
-int mm_dispatch(const T *A, const T *B, T *C, int N, int M, int K, int trans_B) {
+int mm_dispatch(const T *A, const T *B, T *C, int N, int M, int K, int trans_B, const T *bias) {
     if (!ensure_init()) return 2;
     if (N <= 0 || M <= 0 || K <= 0) return 0;  // K == 0 leaves C untouched, as mm() does
     State &st = state();
-    if (K == 1) {
-        size_t total = (size_t)N * M;
-        constexpr int VO = Traits<T>::VEC;
-        if (M % VO == 0 && reinterpret_cast<uintptr_t>(B) % 16 == 0 && reinterpret_cast<uintptr_t>(C) % 16 == 0) {
-            size_t units = (size_t)((N + 3) / 4) * (M / VO);
-            hipLaunchKernelGGL((outer_vec_kernel<T>), dim3((unsigned)((units + 255) / 256)), dim3(256), 0, st.stream,
-                               A, B, C, N, M);
-            return hip_ok(hipGetLastError(), "outer launch") ? 0 : 2;
-        }
-        hipLaunchKernelGGL((outer_kernel<T>), dim3((unsigned)((total + 255) / 256)), dim3(256), 0, st.stream, A,
-                           B, C, N, M);
+    constexpr int VEC = Traits<T>::VEC;
+    if (K == 1 && !bias) {
+        if (M >= VEC)
+            hipLaunchKernelGGL((outer_kernel<T, VEC>), dim3(outer_blocks(N, M, VEC)), dim3(GV_NT), 0, st.stream, A, B, C, N, M,
+                               rag_div((M + VEC - 1) / VEC));
+        else
+            hipLaunchKernelGGL((outer_kernel<T, 1>), dim3(outer_blocks(N, M, 1)), dim3(GV_NT), 0, st.stream, A, B, C, N, M, rag_div(M));
         return hip_ok(hipGetLastError(), "outer launch") ? 0 : 2;
     }
-    if (M == 1) return gemv_rowdot<T>(A, B, C, N, K);  // B is K x 1 or 1 x K: the same vector
-    if (N == 1 && trans_B) return gemv_rowdot<T>(B, A, C, M, K);
-    constexpr int VECW = Traits<T>::VEC;
-    if (N == 1 && M % VECW == 0 && reinterpret_cast<uintptr_t>(B) % 16 == 0) {
-        const int colblk = 8 * VECW;
-        int blocks_m = (M + colblk - 1) / colblk;
-        int splits = (2 * st.num_cu + blocks_m - 1) / blocks_m;
-        if (splits > (K + 31) / 32) splits = (K + 31) / 32;
-        if (splits < 1) splits = 1;
-        int kchunk = (K + splits - 1) / splits;
-        splits = (K + kchunk - 1) / kchunk;
-        float *part = workspace((size_t)splits * M * sizeof(float));
-        if (!part) return 2;
-        if (K <= 4096) {  // one launch: each workgroup sums whole columns
-            hipLaunchKernelGGL((gemv_coldot_whole_kernel<T>), dim3((M + 4 * VECW - 1) / (4 * VECW)), dim3(256), 0,
-                               st.stream, A, B, C, K, M);
-            return hip_ok(hipGetLastError(), "gemv launch") ? 0 : 2;
-        }
-        hipLaunchKernelGGL((gemv_coldot_vec_kernel<T>), dim3(blocks_m, splits), dim3(256), 0, st.stream, A, B, part,
-                           K, M, kchunk);
-        hipLaunchKernelGGL((colsum_reduce_kernel<T>), dim3((M + 255) / 256), dim3(256), 0, st.stream, part, C, M,
-                           splits);
-        return hip_ok(hipGetLastError(), "gemv launch") ? 0 : 2;
-    }
-    if (N == 1) {
-        int splits = (st.num_cu * 256 + M - 1) / M;  // about one thread-column per lane of the chip
-        if (splits > K / 8) splits = K / 8;
-        if (splits < 1) splits = 1;
-        int kchunk = (K + splits - 1) / splits;
-        splits = (K + kchunk - 1) / kchunk;
-        float *part = workspace((size_t)splits * M * sizeof(float));
-        if (!part) return 2;
-        hipLaunchKernelGGL((gemv_coldot_kernel<T>), dim3((M + 255) / 256, splits), dim3(256), 0, st.stream, A,
-                           B, part, K, M, kchunk);
-        hipLaunchKernelGGL((colsum_reduce_kernel<T>), dim3((M + 255) / 256), dim3(256), 0, st.stream, part, C, M,
-                           splits);
+    if (M == 1 && !bias) return gemv_rowdot<T>(A, B, C, nullptr, N, K);  // B is K x 1 or 1 x K: the same vector
+    if (N == 1 && trans_B) return gemv_rowdot<T>(B, A, C, bias, M, K);
+    if (N == 1 && !bias) {
+        if (M >= VEC)
+            hipLaunchKernelGGL((gemv_coldot_kernel<T, VEC>), dim3((M + 4 * VEC - 1) / (4 * VEC)), dim3(GV_NT), 0, st.stream, A, B, C, K, M);
+        else
+            hipLaunchKernelGGL((gemv_coldot_kernel<T, 1>), dim3((M + 3) / 4), dim3(GV_NT), 0, st.stream, A, B, C, K, M);
         return hip_ok(hipGetLastError(), "gemv launch") ? 0 : 2;
     }
     GemmArgs g = {};
@@ -783,10 +868,11 @@ int mm_dispatch(const T *A, const T *B, T *C, int N, int M, int K, int trans_B) 
     g.b.HL = g.b.WL = 1;
     g.c.n = axis_plain(N, M);
     g.c.m = axis_plain(M, 1);
+    g.bias = bias;
     return gemm<T>(g);
 }
 
-template int mm_dispatch<float>(const float *, const float *, float *, int, int, int, int);
-template int mm_dispatch<half_t>(const half_t *, const half_t *, half_t *, int, int, int, int);
+template int mm_dispatch<float>(const float *, const float *, float *, int, int, int, int, const float *);
+template int mm_dispatch<half_t>(const half_t *, const half_t *, half_t *, int, int, int, int, const half_t *);
 
 }  // namespace ptl

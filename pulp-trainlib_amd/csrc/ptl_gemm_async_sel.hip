@@ -102,7 +102,7 @@ int gemm_async(GemmArgs &g) {
             return (few == 64 || few % 128 == 0) && few <= 256 && many % 64 == 0 &&
                    (long)(many / 64) * ((few + 127) / 128) >= 4L * st.num_cu;
         };
-        if (g.splits == 1 && g.taps <= 1 && g.K % SK == 0 && g.K <= 4 * SK && (streams(g.N, g.M) || streams(g.M, g.N))) {
+        if (g.splits == 1 && g.taps <= 1 && !g.bias && g.K % SK == 0 && g.K <= 4 * SK && (streams(g.N, g.M) || streams(g.M, g.N))) {
             GemmArgs gs = g;
             if (!streams(g.N, g.M)) {
                 gs.A = g.B;

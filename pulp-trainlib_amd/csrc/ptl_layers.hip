@@ -56,36 +56,140 @@ __global__ __launch_bounds__(256) void zero_kernel(T *__restrict__ dst, size_t n
     }
 }
 
-// out[b][c][pix] += bias[c] (CHW) or out[b][pix][c] += bias[c] (HWC)
+// out[b][c][pix] += bias[c] (CHW) or out[b][pix][c] += bias[c] (HWC: inner = 1): a thread adds to one 16-byte piece, the
+// elements of which start at channel and position of the first and walk on (element by element and with a 64-bit
+// division each it took 16 us for 7.6 M elements in fp16, 4.9 this way).
 template <typename T>
-__global__ __launch_bounds__(256) void bias_add_kernel(T *__restrict__ out, const T *__restrict__ bias, size_t total,
-                                                       int C, int inner) {
-    size_t idx = (size_t)blockIdx.x * 256 + threadIdx.x;
-    if (idx >= total) return;
-    int c = (int)((idx / inner) % C);
-    out[idx] = (T)((float)out[idx] + (float)bias[c]);
+__global__ __launch_bounds__(256) void bias_add_kernel(T *__restrict__ out, const T *__restrict__ bias, unsigned total,
+                                                       unsigned C, unsigned inner) {
+    constexpr unsigned V = 16 / sizeof(T);
+    const unsigned i0 = (blockIdx.x * 256 + threadIdx.x) * V;
+    if (i0 >= total) return;
+    unsigned q = i0 / inner, p = i0 - q * inner, c = q % C;
+    T v[V];
+    const bool whole = i0 + V <= total;
+    if (whole) __builtin_memcpy(v, out + i0, 16);
+#pragma unroll
+    for (unsigned e = 0; e < V; ++e) {
+        if (whole) v[e] = (T)((float)v[e] + (float)bias[c]);
+        else if (i0 + e < total) out[i0 + e] = (T)((float)out[i0 + e] + (float)bias[c]);
+        if (++p == inner) {
+            p = 0;
+            c = c + 1 == C ? 0 : c + 1;
+        }
+    }
+    if (whole) __builtin_memcpy(out + i0, v, 16);
 }
 
-// bias_diff[c] = sum over samples and pixels of dY; one workgroup per channel.
+// part[s][c] = sum of dY over the positions of share s: channel-major tensors give a workgroup a channel and a share of
+// its (sample, position) axis, read in 16-byte pieces inside each sample.
 template <typename T>
-__global__ __launch_bounds__(256) void bias_grad_kernel(const T *__restrict__ dy, T *__restrict__ db, int ns, int C,
-                                                        int pix, int hwc) {
-    int c = blockIdx.x;
+__global__ __launch_bounds__(256) void bias_grad_kernel(const T *__restrict__ dy, float *__restrict__ part, T *__restrict__ db,
+                                                        int ns, int C, int pix, int per_share) {
+    constexpr int V = 16 / (int)sizeof(T);
+    const int c = blockIdx.x, b0 = blockIdx.y * per_share, b1 = min(ns, b0 + per_share);
+    const int pieces = (pix + V - 1) / V;  // per sample
     float s = 0.f;
-    size_t n = (size_t)ns * pix;
-    for (size_t i = threadIdx.x; i < n; i += 256) {
-        size_t b = i / pix, p = i % pix;
-        size_t off = hwc ? ((b * pix + p) * C + c) : ((b * C + c) * pix + p);
-        s += (float)dy[off];
+    for (int i = threadIdx.x; i < (b1 - b0) * pieces; i += 256) {
+        const int b = i / pieces, p = (i - b * pieces) * V;
+        const T *src = dy + ((size_t)(b0 + b) * C + c) * pix + p;
+        if (p + V <= pix) {
+            T v[V];
+            __builtin_memcpy(v, src, 16);
+#pragma unroll
+            for (int e = 0; e < V; ++e) s += (float)v[e];
+        } else {
+            for (int e = 0; p + e < pix; ++e) s += (float)src[e];
+        }
     }
-    __shared__ float red[256];
-    red[threadIdx.x] = s;
+    __shared__ float red[4];
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) s += __shfl_down(s, o, 64);
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = s;
     __syncthreads();
-    for (int o = 128; o > 0; o >>= 1) {
-        if ((int)threadIdx.x < o) red[threadIdx.x] += red[threadIdx.x + o];
-        __syncthreads();
+    if (threadIdx.x == 0) {
+        s = red[0] + red[1] + red[2] + red[3];
+        if (gridDim.y == 1) db[c] = (T)s;
+        else part[(size_t)blockIdx.y * C + c] = s;
     }
-    if (threadIdx.x == 0) db[c] = (T)red[0];
+}
+
+// The same for tensors with the channels innermost (and for batches of vectors): a workgroup owns 64 channels and a share
+// of the rows, four rows at a time with four loads in flight.
+template <typename T>
+__global__ __launch_bounds__(256) void bias_grad_rows_kernel(const T *__restrict__ dy, float *__restrict__ part, T *__restrict__ db,
+                                                             int rows, int C, int per_share) {
+    const int o = threadIdx.x & 63, w = threadIdx.x >> 6, c = blockIdx.x * 64 + o;
+    const int r0 = blockIdx.y * per_share, r1 = min(rows, r0 + per_share);
+    float s = 0.f;
+    if (c < C) {
+        int r = r0 + w;
+        for (; r + 12 < r1; r += 16) {
+            float v[4];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) v[u] = (float)dy[(size_t)(r + 4 * u) * C + c];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) s += v[u];
+        }
+        for (; r < r1; r += 4) s += (float)dy[(size_t)r * C + c];
+    }
+    __shared__ float red[4][64];
+    red[w][o] = s;
+    __syncthreads();
+    if (w == 0 && c < C) {
+        s = red[0][o] + red[1][o] + red[2][o] + red[3][o];
+        if (gridDim.y == 1) db[c] = (T)s;
+        else part[(size_t)blockIdx.y * C + c] = s;
+    }
+}
+
+template <typename T>
+__global__ __launch_bounds__(256) void bias_grad_sum_kernel(const float *__restrict__ part, T *__restrict__ db, int C, int shares) {
+    const int o = threadIdx.x & 63, w = threadIdx.x >> 6, c = blockIdx.x * 64 + o;
+    float s = 0.f;
+    if (c < C)
+        for (int z = w; z < shares; z += 4) s += part[(size_t)z * C + c];
+    __shared__ float red[4][64];
+    red[w][o] = s;
+    __syncthreads();
+    if (w == 0 && c < C) db[c] = (T)(red[0][o] + red[1][o] + red[2][o] + red[3][o]);
+}
+
+// db[c] = sum of dY over samples and positions: one launch where the channels alone fill the chip or little is to be read,
+// else shares of it and their sum (45 channels of 27 753 positions in fp32: 37.6 us with one workgroup per channel and a
+// 64-bit division per element, 8.5 this way).
+template <typename T>
+static int bias_grad(const T *dy, T *db, int ns, int C, int pix, int hwc) {
+    State &st = state();
+    const bool by_rows = hwc || pix == 1;
+    const long long rows = (long long)ns * pix, units = by_rows ? rows : ns, wide = by_rows ? (C + 63) / 64 : C;
+    // a share is worth a launch only if it shortens the walk of a workgroup by a good deal
+    const long long walk = by_rows ? rows / 16 : rows / (256 * (16 / (long long)sizeof(T)));
+    long long shares = 1;
+    if (walk > 32) shares = (2ll * st.num_cu + wide - 1) / wide;
+    if (shares > units) shares = units;
+    if (shares > (walk + 7) / 8) shares = (walk + 7) / 8;
+    if (shares < 1) shares = 1;
+    const long long per = (units + shares - 1) / shares;
+    shares = (units + per - 1) / per;
+    float *part = nullptr;
+    if (shares > 1 && !(part = workspace((size_t)shares * C * sizeof(float)))) return 2;
+    if (by_rows)
+        hipLaunchKernelGGL((bias_grad_rows_kernel<T>), dim3((unsigned)wide, (unsigned)shares), dim3(256), 0, st.stream, dy, part, db,
+                           (int)rows, C, (int)per);
+    else
+        hipLaunchKernelGGL((bias_grad_kernel<T>), dim3(C, (unsigned)shares), dim3(256), 0, st.stream, dy, part, db, ns, C, pix, (int)per);
+    if (shares > 1)
+        hipLaunchKernelGGL((bias_grad_sum_kernel<T>), dim3((C + 63) / 64), dim3(256), 0, st.stream, part, db, C, (int)shares);
+    return hip_ok(hipGetLastError(), "bias grad launch") ? 0 : 2;
+}
+
+// (the piece index of a tensor below 2^31 elements fits 32 bits)
+template <typename T>
+static void launch_bias_add(T *out, const T *bias, size_t total, int C, int inner) {
+    constexpr size_t V = 16 / sizeof(T);
+    hipLaunchKernelGGL((bias_add_kernel<T>), dim3((unsigned)((total + 256 * V - 1) / (256 * V))), dim3(256), 0, state().stream, out,
+                       bias, (unsigned)total, (unsigned)C, (unsigned)inner);
 }
 
 static inline unsigned blocks_for(size_t n) { return (unsigned)((n + 255) / 256); }
@@ -312,8 +416,7 @@ static int conv2d_fw(const Args *a, int ns, const char *fn) {
     q.C = Y;
     if (rc < 0) rc = gemm<T>(q);
     if (rc == 0 && bias) {
-        hipLaunchKernelGGL((bias_add_kernel<T>), dim3(blocks_for(out_n)), dim3(256), 0, state().stream, Y, bias,
-                           out_n, g.Co, g.hwc ? 1 : P);
+        launch_bias_add<T>(Y, bias, out_n, g.Co, g.hwc ? 1 : P);
         if (!hip_ok(hipGetLastError(), "bias add launch")) rc = 2;
     }
     return sg.finish(rc);
@@ -399,11 +502,7 @@ static int conv2d_wg(const Args *a, int ns, const char *fn) {
     q.c.n = axis_plain(g.Co, K);
     q.c.m = axis_plain(K, 1);
     if (rc < 0) rc = gemm<T>(q);
-    if (rc == 0 && db) {
-        hipLaunchKernelGGL((bias_grad_kernel<T>), dim3(g.Co), dim3(256), 0, state().stream, dY, db, ns, g.Co, P,
-                           g.hwc);
-        if (!hip_ok(hipGetLastError(), "bias grad launch")) rc = 2;
-    }
+    if (rc == 0 && db) rc = bias_grad<T>(dY, db, ns, g.Co, P, g.hwc);
     return sg.finish(rc);
 }
 
@@ -807,14 +906,6 @@ static int pw_step(const Args *a, int ns, int step, const char *fn) {
 // W is [out][in] row-major (lib/sources/pulp_linear_fp32.c:39-46); sample b of
 // the input/output blobs is a vector of blob->dim elements.
 
-template <typename T>
-__global__ __launch_bounds__(256) void rowvec_add_kernel(T *__restrict__ y, const T *__restrict__ b, size_t total,
-                                                         int dim) {
-    size_t idx = (size_t)blockIdx.x * 256 + threadIdx.x;
-    if (idx >= total) return;
-    y[idx] = (T)((float)y[idx] + (float)b[idx % dim]);
-}
-
 template <typename T, typename Args>
 static int linear_step(const Args *a, int ns, int step, const char *fn) {
     if (!a || !a->input || !a->coeff || !a->output) {
@@ -847,16 +938,7 @@ static int linear_step(const Args *a, int ns, int step, const char *fn) {
         T *Y = sg.out(reinterpret_cast<T *>(a->output->data), (size_t)ns * out);
         const T *bias = use_bias ? sg.in(reinterpret_cast<const T *>(a->bias->data), (size_t)out) : nullptr;
         if (sg.failed()) return 2;
-        if (ns == 1)
-            rc = mm_dispatch<T>(Wt, X, Y, out, 1, in, 0);
-        else
-            rc = mm_dispatch<T>(X, Wt, Y, ns, out, in, 1);  // Y[b][o] = X[b][:] . W[o][:]
-        if (rc == 0 && bias) {
-            size_t total = (size_t)ns * out;
-            hipLaunchKernelGGL((rowvec_add_kernel<T>), dim3(blocks_for(total)), dim3(256), 0, state().stream, Y,
-                               bias, total, out);
-            if (!hip_ok(hipGetLastError(), "bias add launch")) rc = 2;
-        }
+        rc = mm_dispatch<T>(X, Wt, Y, ns, out, in, 1, bias);  // Y[b][o] = X[b][:] . W[o][:] + bias[o]
     } else if (step == STEP_BW_BOTH) {
         // weight and input gradient of a batch in one launch
         const T *X = sg.in(reinterpret_cast<const T *>(a->input->data), (size_t)ns * in);
@@ -866,6 +948,7 @@ static int linear_step(const Args *a, int ns, int step, const char *fn) {
         T *dX = sg.out(reinterpret_cast<T *>(a->input->diff), (size_t)ns * in);
         T *db = use_bias ? sg.out(reinterpret_cast<T *>(a->bias->diff), (size_t)out) : nullptr;
         if (sg.failed()) return 2;
+        if (ns == 1) return sg.finish(linear_one_bw<T>(X, Wt, dY, dW, dX, db, in, out));
         GemmArgs q = {}, r = {};
         q.A = dY;  // dW[o][i] = sum_b dY[b][o] * X[b][i]
         q.B = X;
@@ -893,12 +976,18 @@ static int linear_step(const Args *a, int ns, int step, const char *fn) {
         r.a.HL = r.a.WL = r.b.HL = r.b.WL = 1;
         r.c.n = axis_plain(ns, in);
         r.c.m = axis_plain(in, 1);
-        rc = gemm_pair<T>(q, r);
-        if (rc == 0 && db) {
-            hipLaunchKernelGGL((bias_grad_kernel<T>), dim3(out), dim3(256), 0, state().stream, dY, db, ns, out, 1,
-                               1);
-            if (!hip_ok(hipGetLastError(), "bias grad launch")) rc = 2;
+        // Whole slabs of aligned rows: the look-up-free pair.  Other layers, and small ones with a bias (whose gradient
+        // would be a launch of its own: 2.5-4 us against the 1-2 us that the pair is faster), take the kernel for any
+        // size up to the work at which the look-up-free kernels' larger tiles make up for two launches.
+        const double flops = 4.0 * ns * in * out;
+        rc = -1;
+        if (!db || flops > 4e9) rc = gemm_pair_lean<T>(q, r);
+        if (rc < 0 && state().gemm_path == 0 && flops <= (sizeof(T) == 2 ? 3e10 : 1e10)) {
+            rc = linear_bw_ragged<T>(X, Wt, dY, dW, dX, db, ns, in, out);
+            if (rc >= 0) return sg.finish(rc);
         }
+        if (rc < 0) rc = gemm_pair<T>(q, r);
+        if (rc == 0 && db) rc = bias_grad<T>(dY, db, ns, out, 1, 1);
     } else if (step == STEP_WGT_GRAD) {
         const T *X = sg.in(reinterpret_cast<const T *>(a->input->data), (size_t)ns * in);
         const T *dY = sg.in(reinterpret_cast<const T *>(a->output->diff), (size_t)ns * out);
@@ -924,11 +1013,7 @@ static int linear_step(const Args *a, int ns, int step, const char *fn) {
             q.c.m = axis_plain(in, 1);
             rc = gemm<T>(q);
         }
-        if (rc == 0 && db) {  // db[o] = sum_b dY[b][o]
-            hipLaunchKernelGGL((bias_grad_kernel<T>), dim3(out), dim3(256), 0, state().stream, dY, db, ns, out, 1,
-                               1);
-            if (!hip_ok(hipGetLastError(), "bias grad launch")) rc = 2;
-        }
+        if (rc == 0 && db) rc = bias_grad<T>(dY, db, ns, out, 1, 1);  // db[o] = sum_b dY[b][o]
     } else {
         const T *Wt = sg.in(reinterpret_cast<const T *>(a->coeff->data), (size_t)out * in);
         const T *dY = sg.in(reinterpret_cast<const T *>(a->output->diff), (size_t)ns * out);
@@ -952,8 +1037,7 @@ static int bias_add_mat(T *mat, const T *bias, int N, int M, int per_row) {
     T *m = sg.inout(mat, total);
     const T *b = sg.in(bias, (size_t)(per_row ? N : M));
     if (sg.failed()) return 2;
-    hipLaunchKernelGGL((bias_add_kernel<T>), dim3(blocks_for(total)), dim3(256), 0, state().stream, m, b, total,
-                       per_row ? N : M, per_row ? M : 1);
+    launch_bias_add<T>(m, b, total, per_row ? N : M, per_row ? M : 1);
     return sg.finish(hip_ok(hipGetLastError(), "bias add launch") ? 0 : 2);
 }
 
@@ -969,8 +1053,7 @@ static int rowsum_mat(const T *mat, T *out, int N, int K) {
     const T *m = sg.in(mat, (size_t)N * K);
     T *o = sg.out(out, (size_t)N);
     if (sg.failed()) return 2;
-    hipLaunchKernelGGL((bias_grad_kernel<T>), dim3(N), dim3(256), 0, state().stream, m, o, 1, N, K, 0);
-    return sg.finish(hip_ok(hipGetLastError(), "row sum launch") ? 0 : 2);
+    return sg.finish(bias_grad<T>(m, o, 1, N, K, 0));
 }
 
 template <typename T, typename Args>
@@ -1282,26 +1365,18 @@ int ptl_linear_fp16_wg_batched(const struct Linear_args_fp16 *a, int ns) {
     return ptl::linear_step<half_t>(a, ns, STEP_WGT_GRAD, "pulp_linear_fp16_bw_param_grads_cl");
 }
 int ptl_linear_fp32_bw_batched(const struct Linear_args *a, int ns) {
-    if (a && (a->skip_wg_grad || a->skip_in_grad || ns == 1)) {  // one of the two, or one sample: the single steps
+    if (a && (a->skip_wg_grad || a->skip_in_grad)) {  // one of the two
         int rc = a->skip_wg_grad ? 0 : ptl::linear_step<float>(a, ns, STEP_WGT_GRAD, "pulp_linear_fp32_bw_cl");
         if (rc == 0 && !a->skip_in_grad) rc = ptl::linear_step<float>(a, ns, STEP_IN_GRAD, "pulp_linear_fp32_bw_cl");
         return rc;
     }
-    if (ns == 1) {
-        int rc = ptl::linear_step<float>(a, 1, STEP_WGT_GRAD, "pulp_linear_fp32_bw_cl");
-        return rc ? rc : ptl::linear_step<float>(a, 1, STEP_IN_GRAD, "pulp_linear_fp32_bw_cl");
-    }
     return ptl::linear_step<float>(a, ns, STEP_BW_BOTH, "pulp_linear_fp32_bw_cl");
 }
 int ptl_linear_fp16_bw_batched(const struct Linear_args_fp16 *a, int ns) {
-    if (a && (a->skip_wg_grad || a->skip_in_grad || ns == 1)) {  // one of the two, or one sample: the single steps
+    if (a && (a->skip_wg_grad || a->skip_in_grad)) {  // one of the two
         int rc = a->skip_wg_grad ? 0 : ptl::linear_step<half_t>(a, ns, STEP_WGT_GRAD, "pulp_linear_fp16_bw_cl");
         if (rc == 0 && !a->skip_in_grad) rc = ptl::linear_step<half_t>(a, ns, STEP_IN_GRAD, "pulp_linear_fp16_bw_cl");
         return rc;
-    }
-    if (ns == 1) {
-        int rc = ptl::linear_step<half_t>(a, 1, STEP_WGT_GRAD, "pulp_linear_fp16_bw_cl");
-        return rc ? rc : ptl::linear_step<half_t>(a, 1, STEP_IN_GRAD, "pulp_linear_fp16_bw_cl");
     }
     return ptl::linear_step<half_t>(a, ns, STEP_BW_BOTH, "pulp_linear_fp16_bw_cl");
 }

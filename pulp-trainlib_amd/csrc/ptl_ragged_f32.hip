@@ -1,0 +1,6 @@
+// MFMA product for tensors of any size and alignment, fp32 operands.
+#include "ptl_ragged.inc"
+
+namespace ptl {
+template int ragged<float>(RagArgs &, int, int, int, int);
+}  // namespace ptl

@@ -204,13 +204,8 @@ void pulp_linear_fp32_bw_input_grads_cl(void *p) { ptl_internal_set_status(ptl_l
 void pulp_linear_fp32_bw_cl(void *p) {
     struct Linear_args *a = (struct Linear_args *)p;
     int rc = 0;
-    ptl_internal_stage_begin();
-    if (a && a->skip_wg_grad == 0) rc = ptl_linear_fp32_wg_batched(a, 1);
-    if (a && a->skip_in_grad == 0) {
-        int r2 = ptl_linear_fp32_ig_batched(a, 1);
-        if (rc == 0) rc = r2;
-    }
-    ptl_internal_set_status(ptl_internal_stage_end(a ? rc : 1));
+    if (a && !(a->skip_wg_grad && a->skip_in_grad)) rc = ptl_linear_fp32_bw_batched(a, 1);
+    ptl_internal_set_status(a ? rc : 1);
 }
 
 void pulp_linear_fp16_fw_cl(void *p) { ptl_internal_set_status(ptl_linear_fp16_fw_batched(p, 1)); }
@@ -220,13 +215,8 @@ void pulp_linear_fp16_bw_input_grads_cl(void *p) { ptl_internal_set_status(ptl_l
 void pulp_linear_fp16_bw_cl(void *p) {
     struct Linear_args_fp16 *a = (struct Linear_args_fp16 *)p;
     int rc = 0;
-    ptl_internal_stage_begin();
-    if (a && a->skip_wg_grad == 0) rc = ptl_linear_fp16_wg_batched(a, 1);
-    if (a && a->skip_in_grad == 0) {
-        int r2 = ptl_linear_fp16_ig_batched(a, 1);
-        if (rc == 0) rc = r2;
-    }
-    ptl_internal_set_status(ptl_internal_stage_end(a ? rc : 1));
+    if (a && !(a->skip_wg_grad && a->skip_in_grad)) rc = ptl_linear_fp16_bw_batched(a, 1);
+    ptl_internal_set_status(a ? rc : 1);
 }
 
 /* ---- mm family and mm_manager ------------------------------------------------- */
