@@ -229,4 +229,12 @@ int conv_taps_wg(const ConvTileDesc &d, const void *X, const void *dY, void *dW)
 template <typename T>
 int conv_tile_wg(const ConvTileDesc &d, const void *X, const void *dY, void *dW);
 
+// The layer as products with implicit patch matrices, any geometry (ptl_conv_any.hip); d describes the forward layer, dense
+// tensors in either layout.  Null: bias, or in the backward call any of dW, dX, db (db only together with dW).  -1 when the
+// layer does not fit.
+template <typename T>
+int conv_any_fw(const ConvTileDesc &d, const void *X, const void *Wt, const void *bias, void *Y);
+template <typename T>
+int conv_any_bw(const ConvTileDesc &d, const void *X, const void *dY, const void *Wt, void *dW, void *dX, void *db);
+
 }  // namespace ptl

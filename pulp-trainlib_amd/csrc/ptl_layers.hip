@@ -282,6 +282,44 @@ static int conv_geom(const Args *a, ConvGeom &g, const char *fn, bool need_divis
     return 0;
 }
 
+static ConvTileDesc forward_desc(const ConvGeom &g, int ns) {
+    ConvTileDesc d = {};
+    d.in_hwc = g.hwc ? 1 : 0;
+    d.batch = ns; d.Cin = g.Ci; d.Hin = g.H; d.Win = g.W;
+    d.Cout = g.Co; d.Ho = g.Ho; d.Wo = g.Wo;
+    d.KH = g.Hk; d.KW = g.Wk; d.sh = g.sh; d.sw = g.sw;
+    d.padU = g.Up; d.padD = g.Dp; d.padL = g.Lp; d.padR = g.Rp;
+    d.x_sb = (long long)g.Ci * g.H * g.W; d.x_sc = (long long)g.H * g.W; d.x_sy = g.W;
+    return d;
+}
+
+// Whether the products with patch matrices (ptl_conv_any.hip) go before the kernels for small problems (raw tiles of one
+// image, the gathering product): by the multiplications of a step, counted by how full its tiles are.  Measured on 300
+// layers from 1 x 3 -> 8 channels on 7 x 7 to 200 x 500 -> 500 on 64 x 64; below these lines they are 10-30 % behind (their
+// launches cost 2-3 us more: addresses of patches before the first load), above 1.1 to 6 times as fast.  Strides: the other
+// route of the input gradient runs over a zero-stuffed tensor.  Channel-minor layers whose channels are no whole pieces have
+// their filters re-laid first, as all have for the input gradient (not worth it for a handful of pixels).  A bias is a launch
+// of its own on the other routes.
+template <typename T>
+static bool any_pays(const ConvGeom &g, int ns, int steps, bool bias) {
+    if (state().gemm_path == 7) return true;
+    if (state().gemm_path != 0) return false;
+    constexpr int VEC = 16 / (int)sizeof(T);
+    auto fill = [](double n, int unit) { return n / ((long long)((n + unit - 1) / unit) * unit); };
+    const int K = g.Ci * g.Hk * g.Wk;
+    const bool strided = g.sh > 1 || g.sw > 1, odd = g.hwc && g.Ci % VEC != 0, half = sizeof(T) == 2;
+    double mflop = 2e-6 * ns * g.Co * g.Ho * g.Wo * K * fill(g.Co, 32) * fill(K, 64);
+    if (g.hwc) mflop *= fill(g.Ci, VEC);
+    if (bias) mflop *= steps == 1 ? 4 : 1.5;
+    if (steps == 1) {
+        if (half && !g.hwc && !strided && g.Co <= 16) return false;  // (the raw tiles: 31 against 42 us for 38 -> 16 on 50 x 37)
+        return mflop >= (g.hwc ? (odd ? (half ? 200 : 600) : half ? 5 : 60) : half ? 240 : 5);
+    }
+    if (steps == 2) return mflop >= (g.hwc ? (half ? 20 : 300) : strided ? 200 : 300);
+    if ((long long)ns * g.H * g.W < 256 && (long long)g.Co * K > (1 << 18)) return false;
+    return mflop >= (strided ? 15 : half ? (g.hwc ? 240 : 300) : g.hwc ? 1500 : 320);
+}
+
 // Patch axis over output pixels (sample, ho, wo) and over kernel taps.
 static AxisMap pix_axis(const ConvGeom &g, int ns) {
     AxisMap a = {};
@@ -359,27 +397,23 @@ static int conv2d_fw(const Args *a, int ns, const char *fn) {
     state().last_conv_direct = 0;
     state().last_conv_resident = 0;
     if (state().gemm_path != 1) {
-        ConvTileDesc d = {};
-        d.batch = ns; d.Cin = g.Ci; d.Hin = g.H; d.Win = g.W;
-        d.Cout = g.Co; d.Ho = g.Ho; d.Wo = g.Wo;
-        d.KH = g.Hk; d.KW = g.Wk; d.sh = g.sh; d.sw = g.sw;
-        d.padU = g.Up; d.padD = g.Dp; d.padL = g.Lp; d.padR = g.Rp;
-        d.x_sb = (long long)g.Ci * g.H * g.W; d.x_sc = (long long)g.H * g.W; d.x_sy = g.W;
+        ConvTileDesc d = forward_desc(g, ns);
         OutMap c;
         if (!g.hwc) {
             d.w_base = 0; d.w_sm = K; d.w_sc = g.Hk * g.Wk; d.w_sy = g.Wk; d.w_sx = 1;
             c.n = axis_two(ns * P, P, g.Co * P, 1);
             c.m = axis_plain(g.Co, P);
         } else {  // X[b][h][w][ci], W[co][hk][wk][ci], Y[b][pix][co]
-            d.in_hwc = 1;
             d.w_base = 0; d.w_sm = K; d.w_sc = 1; d.w_sy = g.Wk * g.Ci; d.w_sx = g.Ci;
             c.n = axis_plain(ns * P, g.Co);
             c.m = axis_plain(g.Co, 1);
         }
+        if (state().gemm_path == 7 && (rc = conv_any_fw<T>(d, X, Wt, bias, Y)) >= 0) return sg.finish(rc);
         if (!g.hwc) rc = conv_small<T>(d, X, Wt, Y);
         // (a normalisation to apply on the way in is the small-layer kernel's business alone: nothing was launched)
         if (rc == CONV_PRE_REFUSED || conv_small_pre_pending()) return CONV_PRE_REFUSED;
         if (rc < 0) rc = conv_taps<T>(d, X, Wt, Y, c);
+        if (rc < 0 && any_pays<T>(g, ns, 1, bias != nullptr) && (rc = conv_any_fw<T>(d, X, Wt, bias, Y)) >= 0) return sg.finish(rc);
         if (rc < 0) rc = conv_tile<T>(d, X, Wt, Y, c);
         if (rc > 0) return sg.finish(rc);
         if (rc == 0) state().last_conv_direct = 1;
@@ -452,21 +486,17 @@ static int conv2d_wg(const Args *a, int ns, const char *fn) {
     state().last_conv_direct = 0;
     state().last_conv_resident = 0;
     if (state().gemm_path != 1) {
-        ConvTileDesc d = {};
-        d.in_hwc = g.hwc ? 1 : 0;
-        d.batch = ns; d.Cin = g.Ci; d.Hin = g.H; d.Win = g.W;
-        d.Cout = g.Co; d.Ho = g.Ho; d.Wo = g.Wo;
-        d.KH = g.Hk; d.KW = g.Wk; d.sh = g.sh; d.sw = g.sw;
-        d.padU = g.Up; d.padD = g.Dp; d.padL = g.Lp; d.padR = g.Rp;
-        d.x_sb = (long long)g.Ci * g.H * g.W; d.x_sc = (long long)g.H * g.W; d.x_sy = g.W;
+        const ConvTileDesc d = forward_desc(g, ns);
         // the kernel with resident channel-blocked tiles where it is preferred; else the resident output tile kernel,
         // else (or on request) the sum over taps.  From 256 channels on either side and 16384 output pixels the sum
         // over taps goes before the output tile kernel (measured: 81 against 91 us for 256 -> 256 on 14x14 at batch
         // 128, 455 against 533 us on 28x28 at batch 256; at batch 8 the output tile kernel takes 26 against 34 us)
+        if (state().gemm_path == 7 && (rc = conv_any_bw<T>(d, X, dY, nullptr, dW, nullptr, db)) >= 0) return sg.finish(rc);
         const bool taps_first = d.Cin >= 128 && d.Cout >= 128 && (d.Cin >= 256 || d.Cout >= 256) &&
                                 (long long)ns * g.Ho * g.Wo >= 16384;
         if (g.hwc) {  // channel-minor tensors: the sum over taps from 64 channels on, else the gathering GEMM below
-            rc = conv_taps_wg<T>(d, X, dY, dW);
+            if (!any_pays<T>(g, ns, 2, db != nullptr) || (sizeof(T) == 2 && conv_halo_wg_hwc_fits(d, X, dY) && conv_halo_wg_hwc_preferred(d)))
+                rc = conv_taps_wg<T>(d, X, dY, dW);
         } else if ((rc = conv_small_wg<T>(d, X, dY, dW,
                                            static_cast<const void *>(dW) == static_cast<const void *>(a->coeff->diff))) >= 0) {
             // (small 3x3 layers: one launch for the partial sums over sample ranges, one to add them)
@@ -477,6 +507,7 @@ static int conv2d_wg(const Args *a, int ns, const char *fn) {
             if (rc < 0) rc = conv_tile_wg<T>(d, X, dY, dW);
             if (rc < 0 && state().gemm_path != 3) rc = conv_taps_wg<T>(d, X, dY, dW);
         }
+        if (rc < 0 && any_pays<T>(g, ns, 2, db != nullptr) && (rc = conv_any_bw<T>(d, X, dY, nullptr, dW, nullptr, db)) >= 0) return sg.finish(rc);
         if (rc > 0) return sg.finish(rc);
         if (rc == 0) state().last_conv_direct = 1;
     }
@@ -579,6 +610,16 @@ static int conv2d_ig(const Args *a, int ns, const char *fn) {
         return sg.finish(gemm<T>(q));
     }
 
+    if (state().gemm_path == 7) {
+        ConvTileDesc d = {};
+        d.in_hwc = g.hwc ? 1 : 0;
+        d.batch = ns; d.Cin = g.Ci; d.Hin = g.H; d.Win = g.W;
+        d.Cout = g.Co; d.Ho = g.Ho; d.Wo = g.Wo;
+        d.KH = g.Hk; d.KW = g.Wk; d.sh = g.sh; d.sw = g.sw;
+        d.padU = g.Up; d.padD = g.Dp; d.padL = g.Lp; d.padR = g.Rp;
+        const int rc = conv_any_bw<T>(d, nullptr, dY, Wt, nullptr, dX, nullptr);
+        if (rc >= 0) return sg.finish(rc);
+    }
     // Small stride-2 layers (3x3 or 1x1): the small-layer kernel stuffs the zeros while it fills its LDS tile.
     if (!g.hwc && g.sh == 2 && g.sw == 2 && g.Hk == g.Wk && (g.Hk == 3 || g.Hk == 1)) {
         ConvTileDesc d = {};
@@ -593,6 +634,11 @@ static int conv2d_ig(const Args *a, int ns, const char *fn) {
         state().last_conv_resident = 0;
         const int rc = conv_small<T>(d, dY, Wt, dX);
         if (rc == 0) state().last_conv_direct = 1;
+        if (rc >= 0) return sg.finish(rc);
+    }
+
+    if ((g.sh != 1 || g.sw != 1) && any_pays<T>(g, ns, 4, false)) {
+        const int rc = conv_any_bw<T>(forward_desc(g, ns), nullptr, dY, Wt, nullptr, dX, nullptr);
         if (rc >= 0) return sg.finish(rc);
     }
 
@@ -643,6 +689,9 @@ static int conv2d_ig(const Args *a, int ns, const char *fn) {
         // (the zero-stuffed gradient of a strided layer lives in the scratch buffer the tap route would reuse)
         int rc = !g.hwc ? conv_small<T>(d, dY, Wt, dX) : -1;
         if (rc < 0 && g.sh == 1 && g.sw == 1) rc = conv_taps<T>(d, dY, Wt, dX, c);
+        if (rc < 0 && g.sh == 1 && g.sw == 1 && any_pays<T>(g, ns, 4, false) &&
+            (rc = conv_any_bw<T>(forward_desc(g, ns), nullptr, dY, Wt, nullptr, dX, nullptr)) >= 0)
+            return sg.finish(rc);
         if (rc < 0) rc = conv_tile<T>(d, dY, Wt, dX, c);
         if (rc == 0) state().last_conv_direct = 1;
         if (rc >= 0) return sg.finish(rc);
@@ -790,6 +839,36 @@ static int conv2d_bw(const Args *a, int ns, const char *fn) {
                 // to the caller; the two single-step calls below are the only writers
                 sg.discard();
             }
+        }
+    }
+    // Both gradients as products with patch matrices, except where one of them has a kernel of its own that is ahead: the
+    // resident-tile kernels, and the raw-tile weight gradient of large unit-stride 3x3 and 1x1 layers (26 us against 48 for
+    // 128 -> 32 channels on 22 x 32 at batch 94).
+    if (wg && ig && ns >= 1 && a->input && a->coeff && a->output && (a->USE_BIASES != 1 || a->bias)) {
+        ConvGeom g;
+        if (int rc = conv_geom(a, g, fn, true)) return rc;
+        if (!ensure_init()) return 2;
+        const int P = g.Ho * g.Wo, K = g.Ci * g.Hk * g.Wk;
+        const size_t in_n = (size_t)ns * g.Ci * g.H * g.W, out_n = (size_t)ns * g.Co * P;
+        const ConvTileDesc d = forward_desc(g, ns);
+        const bool unit = g.sh == 1 && g.sw == 1, scatter = K == g.Ci && !unit;
+        const bool own_wg = unit && sizeof(T) == 2 && !g.hwc && g.Hk <= 3 && 2e-9 * ns * g.Co * P * K >= 1;
+        const bool resident = sizeof(T) == 2 && g.hwc && conv_halo_wg_hwc_fits(d, nullptr, nullptr) && conv_halo_wg_hwc_preferred(d);
+        const bool forced = state().gemm_path == 7;
+        if ((forced || (!own_wg && !resident && !scatter)) && fits_int(in_n) && fits_int(out_n) && any_pays<T>(g, ns, 6, a->USE_BIASES == 1)) {
+            Stager sg;
+            const T *X = sg.in(reinterpret_cast<const T *>(a->input->data), in_n);
+            const T *dY = sg.in(reinterpret_cast<const T *>(a->output->diff), out_n);
+            const T *Wt = sg.in(reinterpret_cast<const T *>(a->coeff->data), (size_t)g.Co * K);
+            T *dW = sg.out(reinterpret_cast<T *>(a->coeff->diff), (size_t)g.Co * K);
+            T *dX = sg.out(reinterpret_cast<T *>(a->input->diff), in_n);
+            T *db = a->USE_BIASES == 1 ? sg.out(reinterpret_cast<T *>(a->bias->diff), (size_t)g.Co) : nullptr;
+            if (sg.failed()) return sg.rejected() ? 1 : 2;
+            state().last_conv_direct = 0;
+            state().last_conv_resident = 0;
+            const int rc = conv_any_bw<T>(d, X, dY, Wt, dW, dX, db);
+            if (rc >= 0) return sg.finish(rc);
+            sg.discard();
         }
     }
     ptl_internal_stage_begin();  // (host tensors: fetched once for both steps)

@@ -19,24 +19,39 @@ inline RagDiv rag_div(long long dv) {
     return r;
 }
 
-// How the 16-byte chunks of an operand are found.  KC and RC: a matrix whose rows (KC) or whose k columns (RC) are
-// contiguous.  GK and GR: an implicit patch matrix over a channel-minor or channel-blocked tensor, whose chunks are VEC
-// channels of one tap at one pixel - with pixels as the rows (GK) or as the contraction index (GR).
-enum RagMode : int { RAG_KC = 0, RAG_RC = 1, RAG_GK = 2, RAG_GR = 3 };
+// How an operand's tile is filled.  KC and RC: 16-byte pieces of a matrix whose rows (KC) or whose k columns (RC) are
+// contiguous.  The others are implicit patch matrices (RagGeo): XK and XR gather a channel-major tensor element by element,
+// neighbouring lanes at neighbouring pixels, with pixels as the rows and (channel, tap) as k (XK) or the other way round
+// (XR); GK and GR read channel-minor tensors in pieces of VEC channels of one tap at one pixel, with pixels as the rows
+// and (tap, piece) as k (GK) or the other way round (GR).
+enum RagMode : int { RAG_KC = 0, RAG_RC = 1, RAG_GK = 2, RAG_GR = 3, RAG_XK = 4, RAG_XR = 5 };
 
 struct RagOp {
-    const char *p;     // first element
-    int rows;          // extent along the output
+    const char *p;     // first element (XK, XR: see RagGeo)
+    int rows;          // extent along the output (GR: taps x pieces x VEC)
     unsigned row_b;    // KC: bytes from row to row
     unsigned k_b;      // RC: bytes from k to k
-    long long run_b;   // bytes from one run of k to the next
+    long long run_b;   // bytes from one run of k to the next (KC, RC)
     long long outer_b; // RC: bytes between the outer digits of the rows
-    // GK, GR: pixel = (b, y, x) -> bytes, chunk = (tap row, tap column, channel chunk) -> bytes
-    RagDiv d_x, d_y;         // extents of x and y
-    unsigned px, py, pb;
-    RagDiv d_cb, d_kw;       // channel chunks per tap, taps per row
-    unsigned tc, tx, ty;
-    int chunks;              // taps x channel chunks
+};
+
+// An implicit patch matrix: pixel q = (b, qy, qx), tap t = (jy, jx), element at row qy*sy + y0 + ty*jy and column
+// qx*sx + x0 + tx*jx of channel c of image b, zero outside of the H x W image.  ty = tx = 1 for a forward pass, -1 for the
+// input gradient.  Offsets are unsigned: the tensor pointer is moved back by what the smallest of them would lack.
+constexpr int RAG_TAPS = 25;          // one validity bit per tap and for the seven taps after the last of a channel
+constexpr int RAG_TAB = RAG_TAPS + 7;
+struct RagGeo {
+    RagDiv d_x, d_y;        // extents of qx and qy
+    unsigned pb, py, px;    // bytes per step of b, qy, qx
+    int y0, x0, sy, sx, ty, tx, H, W;
+    RagDiv d_t, d_kw;       // taps, taps per row
+    RagDiv d_cb;            // GK, GR: pieces per tap
+    unsigned every_row, every_channel, all_taps;  // bit 0 of every row of taps, of every channel's taps (GK: bit 0); the taps
+    unsigned plane;         // XK, XR: bytes from channel to channel
+    unsigned size;          // XK, XR: bytes from the moved pointer to the end of the tensor
+    unsigned cut;           // GK, GR: bytes that the last piece of a tap lacks
+    const char *zeros;      // GK, GR: 16 zero bytes
+    int tab[RAG_TAB];       // bytes of tap t; XK, XR: of entry j = tap j % taps of channel j / taps
 };
 
 // Output axis: index -> (q2, q1, q0) with the radices of d1 and d0 -> elements.  q0 below `lim` only.
@@ -52,28 +67,79 @@ struct RagProd {
     RagOp a, b;        // C(n, m) = sum over runs and k of a(n, k) * b(m, k)
     void *C;
     RagAxis cn, cm;
-    int N, M, K;       // K: k per run (GR: pixels, GK: 128-byte slabs of chunks are counted from b.chunks)
-    int runs;          // runs of K (KC / RC operands)
+    int N, M, K;       // K: k per run (GK: pieces)
+    int runs;          // runs of K (with a patch matrix: run r is image r)
     int outer, m_in;   // RC second operand: M = outer x m_in, tiles stay inside one outer digit (outer == 1: m_in == M)
     const void *bias;  // added per n (bias_n) or per m
     int bias_n;
-    void *row_sum;     // sum over k of a(n, k), as an extra column of ones in b (RC / GR second operand)
+    void *row_sum;     // sum over k of a(n, k), as an extra column of ones in b (RC, GR, XR)
     // set by the launcher
     float *ws;         // partial sums [split][N][pitch]
     int pitch, splits, slabs_per_split;
     int tiles_n, tiles_m, tiles_in;  // tiles along n, along m, along m inside one outer digit
 };
 
-constexpr int RAG_MAX = 5;
+constexpr int RAG_MAX = 2;
 struct RagArgs {
     RagProd p[RAG_MAX];
     int first[RAG_MAX + 1];  // first workgroup of each product
     int count;
 };
 
+struct RagSums {  // the products whose contraction was split
+    RagProd p[4];
+    int first[5];
+    int count;
+};
+
 // The products in one launch (plus one for their partial sums where the contraction is split).  The first product has
-// the modes (a0, b0), the others (a1, b1).  0 = launched, -1 = no such combination of modes, 2 = a HIP failure.
+// the modes (a0, b0), the other (a1, b1).  0 = launched, -1 = no such combination of modes, 2 = a HIP failure.
 template <typename T>
 int ragged(RagArgs &r, int a0, int b0, int a1, int b1);
+
+// Filters re-laid for a product: dst[row][k], k = (outer, tap, inner), from src at row*row_s + outer*outer_s + inner*inner_s
+// + tap_at + jy*tap_y + jx*tap_x; inner values from `lim` on are zeros.  All in elements.
+struct RagRelay {
+    void *dst;
+    int rows, outer, taps, inner, lim, kw;
+    int row_s, outer_s, inner_s, tap_at, tap_y, tap_x;
+    RagDiv by_k, by_inner, by_taps, by_kw;  // set by the launcher
+};
+
+// A channel-major tensor re-laid channel-minor: dst[b][pixel][cp] from src[b][channel][pixel], zeros from channel c on; cp is
+// a whole number of 16-byte pieces.
+struct RagTurn {
+    const void *src;
+    void *dst;
+    int batch, c, cp, pix;
+};
+
+// Products with patch matrices: N of them, one or the phases of a strided input gradient (up to four).
+constexpr int RAG_CONV_MAX = 4;
+template <int N>
+struct RagConvOf {
+    RagProd p[N];
+    int first[N + 1];
+    int count;
+    RagGeo geo[N];          // of each product's patch matrix
+    RagGeo geo_a;           // of a first operand that is gathered too (XR; one product)
+    const void *relay_src;  // blocks behind the last product re-lay filters for a later product
+    RagRelay relay[RAG_CONV_MAX];
+    int relays, relay_first[RAG_CONV_MAX + 1];
+};
+typedef RagConvOf<RAG_CONV_MAX> RagConvArgs;
+// The tiles and splits that ragged_conv() would choose for the products (of which sizes and runs count), and the clocks of
+// 2.4 GHz that this would take.
+struct RagPlan {
+    int shape, splits;
+    double clocks;
+};
+template <typename T>
+RagPlan ragged_conv_plan(const RagProd *p, int count, int a, int b);
+template <typename T>
+int ragged_conv(RagConvArgs &r, int a, int b, const RagPlan &plan);
+// The re-laying alone, filters of r and tensors (n <= 2).
+template <typename T>
+int ragged_relay(RagConvArgs &r, const RagTurn *turn, int n);
 
 }  // namespace ptl
