@@ -176,11 +176,11 @@ static const AnyPlan &any_plan(const ConvTileDesc &d, int steps) {
             a.clocks += a.ig.clocks;
         }
         // a launch for the layouts, and the bytes it moves (clocks fitted like those of the tiles)
-        if (turn || (d.in_hwc && steps == ANY_FW && any_padded(d.Cin, ES) != d.Cin) || steps == ANY_IG) a.clocks += 11500;
+        if (turn || (d.in_hwc && steps == ANY_FW && any_padded(d.Cin, ES) != d.Cin) || steps == ANY_IG) a.clocks += 12500;
         if (turn) {
             const double x = steps == ANY_IG ? 0 : (double)d.batch * d.Hin * d.Win * (d.Cin + any_padded(d.Cin, ES)) * ES;
             const double y = steps == ANY_FW ? 0 : (double)d.batch * d.Ho * d.Wo * (d.Cout + any_padded(d.Cout, ES)) * ES;
-            a.clocks += (x + y) / 1350;
+            a.clocks += (x + y) / (ES == 2 ? 1500 : 2000);
         }
         if (turn == 0 || a.clocks < best.clocks) best = a;
     }

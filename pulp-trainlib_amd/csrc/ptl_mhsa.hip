@@ -21,6 +21,7 @@
 #include "ptl_gemm_async.inc"
 #include "ptl_host.hpp"
 #include "ptl_internal.h"
+#include "ptl_ragged.hpp"
 #include "ptl_structs.h"
 
 namespace ptl {
@@ -51,15 +52,31 @@ static float q_rsqrt_host(float number) {
     return y * (1.5f - (x2 * y * y));
 }
 
+// Reductions over the wave in registers (shifts inside rows of 16 lanes, then from row to row; the last lane has the
+// result): a chain of six shuffles through LDS took most of the softmax phase.
+template <int CTRL>
+__device__ inline float dpp_from(float v, float otherwise) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(__builtin_bit_cast(int, otherwise), __builtin_bit_cast(int, v), CTRL, 0xf, 0xf, false));
+}
+__device__ inline float last_lane(float v) { return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), 63)); }
 __device__ inline float wave_max(float v) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o));
-    return v;
+    v = fmaxf(v, dpp_from<0x111>(v, -FLT_MAX));  // row_shr 1, 2, 4, 8
+    v = fmaxf(v, dpp_from<0x112>(v, -FLT_MAX));
+    v = fmaxf(v, dpp_from<0x114>(v, -FLT_MAX));
+    v = fmaxf(v, dpp_from<0x118>(v, -FLT_MAX));
+    v = fmaxf(v, dpp_from<0x142>(v, -FLT_MAX));  // row_bcast 15, 31
+    v = fmaxf(v, dpp_from<0x143>(v, -FLT_MAX));
+    return last_lane(v);
 }
 __device__ inline float wave_sum(float v) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
-    return v;
+    v += dpp_from<0x111>(v, 0.f);
+    v += dpp_from<0x112>(v, 0.f);
+    v += dpp_from<0x114>(v, 0.f);
+    v += dpp_from<0x118>(v, 0.f);
+    // (a broadcast reaches rows that have their part already: rows 1 and 3, then 2 and 3, take it)
+    v += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x142, 0xa, 0xf, false));
+    v += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x143, 0xc, 0xf, false));
+    return last_lane(v);
 }
 
 // S[r][c] = scale * sum_d R[d][r0 + r] * Cm[d][c] for 32 rows r and every column c < L, into the LDS tile
@@ -440,7 +457,7 @@ struct AttnArgs {
     const float *rs;         // row sums of dP.P [ns][heads][L]    (backward II)
     float *o0, *o1, *o2;     // kernel outputs (see each kernel)
     const float *zero;       // 256 zero bytes: source of elements that do not exist
-    int L, H, heads, F, LP;
+    int L, H, heads, F, LP, ns;
     float scale;
 };
 
@@ -609,106 +626,141 @@ __global__ __launch_bounds__(ATT_NT) void attn_bw_key_kernel(AttnArgs a) {
 }
 
 // ---------------------------------------------------------------------------------------------------------
-// Resident variants for sequences of at most 200 tokens and head sizes of 33..64 (ViT geometry): everything a
-// workgroup needs comes in by LDS-DMA in one volley at its start (a single trip to memory instead of one per
-// phase), and all fragments are read from LDS.  Sixteen waves per workgroup (one workgroup per CU: the panels
-// take 150 KB), so that every SIMD has four waves to choose from while some wait (measured 3 % faster than eight).
-constexpr int RS_NW = 16;           // waves
-constexpr int RS_NT = RS_NW * 64;   // threads
-constexpr int RS_RPW = 32 / RS_NW;  // score rows per wave
-constexpr int RS_KS = RS_NW / 2;    // contraction ranges of the token-contracting products
-constexpr int RS_LC = 224;  // key columns covered: 7 blocks of 32
-constexpr int RS_KD = 200;  // contraction depth over tokens (25 groups of 8)
-constexpr int RS_KP = 232;  // pitch of a [d][token] panel read with lanes along tokens (4 rows apart = 32 banks)
-constexpr int RS_VP = 204;  // pitch of a [d][token] panel read as 16-byte fragments along tokens
-constexpr int RS_SP = 228;  // pitch of the [32][token] score tile (16-byte fragments along tokens)
-constexpr int RS_FW_FLOATS = 64 * 32 + 64 * RS_KP + 64 * RS_VP + 32 * RS_SP;
-constexpr int RS_KEY_FLOATS = 2 * 64 * RS_VP + 2 * RS_KD * 32 + RS_KD;
-static_assert(RS_NW * 32 * ATT_RP <= 64 * 32 + 64 * RS_KP, "parked accumulators fit the first two panels");
+// Sequences of at most 256 tokens and heads of at most 64 (HB = 1: 32): the score tile of 32 queries and the one operand
+// that a product needs along its other axis are in LDS, everything else goes from global memory to the matrix cores'
+// registers (lanes along the tokens: whole lines), since no other wave of the workgroup needs it.  78 KB for 197 tokens,
+// so that two workgroups share a CU and one's loads hide behind the other's products; with all three operands resident
+// (150 KB, one workgroup of 16 waves) the phases followed one another: 37 / 37 / 41 us for 32 x 3 heads of 64 and 197
+// tokens, 29 / 28 / 30 this way, of which the products take 7 / 9 / 7 at the matrix rate.
+constexpr int SQ_NW = 8;           // waves
+constexpr int SQ_NT = SQ_NW * 64;  // threads
+constexpr int SQ_RPW = 32 / SQ_NW; // score rows per wave
+constexpr int SQ_L = 256;          // tokens
+// Pitch of the [d][token] and [row][token] tiles: whole groups of eight and an odd number of 16-byte units, so that
+// 16-byte fragments along the tokens meet different banks.
+__host__ __device__ constexpr int sq_pitch(int L) { return (L + 7) / 8 * 8 + 4; }
+template <int HB>
+constexpr size_t sq_lds(int L, bool key) {
+    const size_t tiles = (size_t)(32 * HB + (key ? 1 : 32)) * sq_pitch(L), parked = (size_t)SQ_NW * 32 * ATT_RP;
+    return (tiles > parked ? tiles : parked) * sizeof(float);
+}
 
-// S[r][c] = scale * sum_d Rs[d][r] * Cs[d][c]: Rs is [64][32], Cs [64][RS_KP], both in LDS; one 32-column
-// block per wave.
-__device__ inline void scores_resident(const float *Rs, const float *Cs, int CB, float scale, float *S, int wave,
-                                       int l32, int half) {
-    for (int cb = wave; cb < CB; cb += RS_NW) {
+// Workgroups go to the eight XCDs in turn, each with an L2 of its own: all tiles of a head take ids of the same XCD, so that
+// its operands come from memory once and not once per tile.  False: no head for this workgroup.
+struct SqPlace {
+    int tile, h, b, part;
+};
+__device__ inline bool sq_place(const AttnArgs &a, int parts, SqPlace &p) {
+    const unsigned tiles = (unsigned)(a.L + 31) / 32u * (unsigned)parts, j = blockIdx.x >> 3, group = j / tiles, t = j - group * tiles;
+    const unsigned head = group * 8u + (blockIdx.x & 7u);
+    if (head >= (unsigned)(a.heads * a.ns)) return false;
+    p.b = (int)(head / (unsigned)a.heads);
+    p.h = (int)(head - (unsigned)p.b * a.heads);
+    p.tile = (int)(t / (unsigned)parts);
+    p.part = (int)(t % (unsigned)parts);
+    return true;
+}
+
+// S[r][c] = scale * sum_d R[d][r0 + r] * C[d][c] for c < L, zero up to the next group of eight; R and C are [H][L] in
+// global memory.  One block of 32 columns per wave.
+// then(): what is asked for behind the operands.
+template <int HB, typename Then>
+__device__ inline void sq_scores(const float *__restrict__ R, const float *__restrict__ C, int L, int H, int r0, float scale,
+                                 float *S, int wave, int l32, int half, Then then) {
+    constexpr int STEPS = 16 * HB;
+    const int pitch = sq_pitch(L), blocks = (L + 31) >> 5;
+    const unsigned r = (unsigned)min(r0 + l32, L - 1);
+    if (wave >= blocks) then();
+    static_assert(SQ_L / 32 <= SQ_NW, "a block per wave");
+    if (wave < blocks) {
+        const int c = wave * 32 + l32;
+        const unsigned cc = (unsigned)min(c, L - 1);
         mh_f32x16 acc = {0};
+        float af[STEPS], bf[STEPS];
 #pragma unroll
-        for (int g = 0; g < 8; ++g) {
-            const int d4 = g * 8 + half * 4;
-            float4 x, y;
-            x.x = Rs[d4 * 32 + l32];
-            x.y = Rs[(d4 + 1) * 32 + l32];
-            x.z = Rs[(d4 + 2) * 32 + l32];
-            x.w = Rs[(d4 + 3) * 32 + l32];
-            const float *cp = Cs + d4 * RS_KP + cb * 32 + l32;
-            y.x = cp[0];
-            y.y = cp[RS_KP];
-            y.z = cp[2 * RS_KP];
-            y.w = cp[3 * RS_KP];
-            mfma4(acc, x, y);
+        for (int s = 0; s < STEPS; ++s) {
+            const unsigned row = (unsigned)(min(2 * s + half, H - 1) * L);
+            af[s] = R[row + r];
+            bf[s] = C[row + cc];
         }
+        __builtin_amdgcn_sched_barrier(0);  // (all of them in flight before the first is waited for)
+        then();
 #pragma unroll
-        for (int v = 0; v < 16; ++v) S[(8 * (v / 4) + 4 * half + (v % 4)) * RS_SP + cb * 32 + l32] = acc[v] * scale;
+        for (int s = 0; s < STEPS; ++s) {
+            const bool in = 2 * s + half < H;  // (beyond the head: zeros)
+            acc = __builtin_amdgcn_mfma_f32_32x32x2f32(in ? af[s] : 0.f, in ? bf[s] : 0.f, acc, 0, 0, 0);
+        }
+        if (c < pitch - 4) {
+#pragma unroll
+            for (int v = 0; v < 16; ++v) S[(8 * (v / 4) + 4 * half + (v % 4)) * pitch + c] = c < L ? acc[v] * scale : 0.f;
+        }
     }
 }
 
-// Parked partial tiles of the RS_KS contraction ranges -> out[d][x0 + x] (d < H, x0 + x < L).
-__device__ inline void mix_store(const float *red, int L, int H, int x0, float *__restrict__ out, int tid) {
-    for (int idx = tid; idx < 64 * 32; idx += RS_NT) {
+// Parked partial tiles of the contraction ranges -> out[d][x0 + x] (d < H, x0 + x < L).
+template <int HB>
+__device__ inline void sq_store(const mh_f32x16 &acc, float *red, int L, int H, int x0, float *__restrict__ out, int tid, int wave,
+                                int l32, int half) {
+    __syncthreads();  // (the tiles have been read)
+#pragma unroll
+    for (int v = 0; v < 16; ++v) red[(wave * 32 + 8 * (v / 4) + 4 * half + (v % 4)) * ATT_RP + l32] = acc[v];
+    __syncthreads();
+    for (int idx = tid; idx < 32 * HB * 32; idx += SQ_NT) {
         const int d = idx >> 5, xx = idx & 31;
         float s = 0.f;
 #pragma unroll
-        for (int k2 = 0; k2 < RS_KS; ++k2) s += red[((2 * k2 + (d >> 5)) * 32 + (d & 31)) * ATT_RP + xx];
+        for (int k = 0; k < SQ_NW / HB; ++k) s += red[((HB * k + (d >> 5)) * 32 + (d & 31)) * ATT_RP + xx];
         if (d < H && x0 + xx < L) out[(size_t)d * L + x0 + xx] = s;
     }
 }
 
-// out[d][r0 + r] = sum_c Vs[d][c] * S[r][c] (d < H): Vs [64][RS_VP] and S [32][RS_SP] in LDS, S zero beyond L.
-// Waves: (block of 32 d) x (range of the contraction); the ranges meet in `red`.
-__device__ inline void mix_resident(const float *Vs, const float *S, int L, int H, int r0, float *__restrict__ out,
-                                    float *red, int tid, int wave, int l32, int half) {
-    const int db = wave & 1, ks = wave >> 1;
-    const int ngroups = (L + 7) >> 3, per = (ngroups + RS_KS - 1) / RS_KS;
-    const int g_end = min(ngroups, (ks + 1) * per);
+// out[d][r0 + r] = sum_c V[d][c] * S[r][c]: V and S in LDS, both zero beyond L.  Waves: (block of 32 d) x (range of c).
+template <int HB>
+__device__ inline void sq_mix(const float *Vs, const float *S, int L, int H, int r0, float *__restrict__ out, float *red, int tid,
+                              int wave, int l32, int half) {
+    constexpr int KS = SQ_NW / HB;
+    const int pitch = sq_pitch(L), db = wave % HB, ks = wave / HB;
+    const int groups = (L + 7) >> 3, per = (groups + KS - 1) / KS, end = min(groups, (ks + 1) * per);
     mh_f32x16 acc = {0};
-    for (int g = ks * per; g < g_end; ++g) {
+    for (int g = ks * per; g < end; ++g) {
         const int k4 = g * 8 + half * 4;
-        mfma4(acc, *reinterpret_cast<const float4 *>(Vs + (db * 32 + l32) * RS_VP + k4),
-              *reinterpret_cast<const float4 *>(S + l32 * RS_SP + k4));
+        mfma4(acc, *reinterpret_cast<const float4 *>(Vs + (db * 32 + l32) * pitch + k4),
+              *reinterpret_cast<const float4 *>(S + l32 * pitch + k4));
     }
-#pragma unroll
-    for (int v = 0; v < 16; ++v) red[(wave * 32 + 8 * (v / 4) + 4 * half + (v % 4)) * ATT_RP + l32] = acc[v];
-    __syncthreads();
-    mix_store(red, L, H, r0, out, tid);
+    sq_store<HB>(acc, red, L, H, r0, out, tid, wave, l32, half);
 }
 
-__global__ __launch_bounds__(RS_NT) void attn_fw_res_kernel(AttnArgs a) {
+// Rows of V ([H][L], zeros beyond either) on their way into LDS; complete after sq_arrived() and a barrier.
+template <int HB>
+__device__ inline TileEdge sq_fetch(const float *g, int L, int H, float *lds, const float *zero, int tid, int wave, int lane) {
+    const int cols = (L + 7) / 8 * 8;
+    tile_dma<SQ_NW>(g, L, 32 * HB, cols, H, L, lds, sq_pitch(L), zero, wave, lane);
+    return tile_edge_load(g, L, 32 * HB, cols, H, L, lds, sq_pitch(L), tid);
+}
+
+template <int HB>
+__global__ __launch_bounds__(SQ_NT, 4) void attn_fw_res_kernel(AttnArgs a) {
     extern __shared__ __attribute__((aligned(16))) float att_lds[];
-    float *Qs = att_lds, *Ks = Qs + 64 * 32, *Vs = Ks + 64 * RS_KP, *S = Vs + 64 * RS_VP, *red = att_lds;
-    const int r0 = blockIdx.x * 32, h = blockIdx.y, b = blockIdx.z, L = a.L;
+    SqPlace at;
+    if (!sq_place(a, 1, at)) return;
+    const int r0 = at.tile * 32, h = at.h, b = at.b, L = a.L, pitch = sq_pitch(L);
+    float *S = att_lds, *Vs = S + 32 * pitch;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int l32 = lane & 31, half = lane >> 5;
     const size_t hoff = ((size_t)b * a.F + (size_t)h * a.H) * L;
-    tile_dma<RS_NW>(a.q + hoff + r0, L, 64, 32, a.H, L - r0, Qs, 32, a.zero, wave, lane);
-    tile_dma<RS_NW>(a.k + hoff, L, 64, RS_LC, a.H, L, Ks, RS_KP, a.zero, wave, lane);
-    tile_dma<RS_NW>(a.v + hoff, L, 64, RS_KD, a.H, L, Vs, RS_VP, a.zero, wave, lane);
-    const TileEdge e0 = tile_edge_load(a.q + hoff + r0, L, 64, 32, a.H, L - r0, Qs, 32, tid);
-    const TileEdge e1 = tile_edge_load(a.k + hoff, L, 64, RS_LC, a.H, L, Ks, RS_KP, tid);
-    const TileEdge e2 = tile_edge_load(a.v + hoff, L, 64, RS_KD, a.H, L, Vs, RS_VP, tid);
-    tile_edge_store(e0);
-    tile_edge_store(e1);
-    tile_edge_store(e2);
+    TileEdge edge;
+    sq_scores<HB>(a.q + hoff, a.k + hoff, L, a.H, r0, a.scale, S, wave, l32, half,
+                  [&] { edge = sq_fetch<HB>(a.v + hoff, L, a.H, Vs, a.zero, tid, wave, lane); });
+    tile_edge_store(edge);
     wait_vmcnt<0>();
-    __syncthreads();
-    scores_resident(Qs, Ks, (L + 31) >> 5, a.scale, S, wave, l32, half);
     __syncthreads();
     // softmax of this wave's rows over the keys (lib/sources/pulp_act_fp32.c:187-225): max, approximate
     // exponential of the difference, sum, division; the rows' reductions run side by side
     float *P = a.o0 + ((size_t)b * a.heads + h) * L * L;
-    float sv[RS_RPW][4], mx[RS_RPW], sum[RS_RPW];
+    float sv[SQ_RPW][4], mx[SQ_RPW], sum[SQ_RPW];
 #pragma unroll
-    for (int i = 0; i < RS_RPW; ++i) {
-        const float *srow = S + (wave * RS_RPW + i) * RS_SP;
+    for (int i = 0; i < SQ_RPW; ++i) {
+        const float *srow = S + (wave * SQ_RPW + i) * pitch;
         mx[i] = -FLT_MAX;
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
@@ -718,11 +770,9 @@ __global__ __launch_bounds__(RS_NT) void attn_fw_res_kernel(AttnArgs a) {
         }
     }
 #pragma unroll
-    for (int o = 32; o > 0; o >>= 1)
+    for (int i = 0; i < SQ_RPW; ++i) mx[i] = wave_max(mx[i]);
 #pragma unroll
-        for (int i = 0; i < RS_RPW; ++i) mx[i] = fmaxf(mx[i], __shfl_xor(mx[i], o));
-#pragma unroll
-    for (int i = 0; i < RS_RPW; ++i) {
+    for (int i = 0; i < SQ_RPW; ++i) {
         sum[i] = 0.f;
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
@@ -732,65 +782,59 @@ __global__ __launch_bounds__(RS_NT) void attn_fw_res_kernel(AttnArgs a) {
         }
     }
 #pragma unroll
-    for (int o = 32; o > 0; o >>= 1)
+    for (int i = 0; i < SQ_RPW; ++i) sum[i] = wave_sum(sum[i]);
 #pragma unroll
-        for (int i = 0; i < RS_RPW; ++i) sum[i] += __shfl_xor(sum[i], o);
-#pragma unroll
-    for (int i = 0; i < RS_RPW; ++i) {
-        const int row = wave * RS_RPW + i;
-        float *srow = S + row * RS_SP;
+    for (int i = 0; i < SQ_RPW; ++i) {
+        const int row = wave * SQ_RPW + i;
+        float *srow = S + row * pitch;
         const bool live = r0 + row < L;
         const float inv = 1.0f / sum[i];  // one division per row; the products differ from quotients by an ulp at most
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
             const int c = lane + 64 * j;
-            if (c < RS_LC) {
-                const float pv = c < L ? sv[i][j] * inv : 0.f;
+            if (c < L) {
+                const float pv = sv[i][j] * inv;
                 srow[c] = pv;
-                if (live && c < L) P[(size_t)(r0 + row) * L + c] = pv;
+                if (live) P[(size_t)(r0 + row) * L + c] = pv;
             }
         }
     }
     __syncthreads();
-    mix_resident(Vs, S, L, a.H, r0, a.o1 + hoff, red, tid, wave, l32, half);
+    sq_mix<HB>(Vs, S, L, a.H, r0, a.o1 + hoff, att_lds, tid, wave, l32, half);
 }
 
-__global__ __launch_bounds__(RS_NT) void attn_bw_query_res_kernel(AttnArgs a) {
+template <int HB>
+__global__ __launch_bounds__(SQ_NT, 4) void attn_bw_query_res_kernel(AttnArgs a) {
     extern __shared__ __attribute__((aligned(16))) float att_lds[];
-    float *Qs = att_lds, *Ks = Qs + 64 * 32, *Vs = Ks + 64 * RS_KP, *S = Vs + 64 * RS_VP, *red = att_lds;
-    const int r0 = blockIdx.x * 32, h = blockIdx.y, b = blockIdx.z, L = a.L;
+    SqPlace at;
+    if (!sq_place(a, 1, at)) return;
+    const int r0 = at.tile * 32, h = at.h, b = at.b, L = a.L, pitch = sq_pitch(L);
+    float *S = att_lds, *Ks = S + 32 * pitch;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int l32 = lane & 31, half = lane >> 5;
     const size_t hoff = ((size_t)b * a.F + (size_t)h * a.H) * L;
     const size_t poff = ((size_t)b * a.heads + h) * L * L;
-    tile_dma<RS_NW>(a.da + hoff + r0, L, 64, 32, a.H, L - r0, Qs, 32, a.zero, wave, lane);
-    tile_dma<RS_NW>(a.v + hoff, L, 64, RS_LC, a.H, L, Ks, RS_KP, a.zero, wave, lane);
-    tile_dma<RS_NW>(a.k + hoff, L, 64, RS_KD, a.H, L, Vs, RS_VP, a.zero, wave, lane);
-    const TileEdge e0 = tile_edge_load(a.da + hoff + r0, L, 64, 32, a.H, L - r0, Qs, 32, tid);
-    const TileEdge e1 = tile_edge_load(a.v + hoff, L, 64, RS_LC, a.H, L, Ks, RS_KP, tid);
-    const TileEdge e2 = tile_edge_load(a.k + hoff, L, 64, RS_KD, a.H, L, Vs, RS_VP, tid);
-    // this wave's probability rows ride along in registers
-    float pr[RS_RPW][4];
+    // dP[query][key] = sum_d dA[d][query] v[d][key]   (lib/sources/pulp_mhsa_fp32.c:958-1060)
+    TileEdge edge;
+    float pr[SQ_RPW][4];  // this wave's probability rows
+    sq_scores<HB>(a.da + hoff, a.v + hoff, L, a.H, r0, 1.0f, S, wave, l32, half, [&] {
+        edge = sq_fetch<HB>(a.k + hoff, L, a.H, Ks, a.zero, tid, wave, lane);
+    });
 #pragma unroll
-    for (int i = 0; i < RS_RPW; ++i)
+    for (int i = 0; i < SQ_RPW; ++i)
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
-            const int row = r0 + wave * RS_RPW + i, c = lane + 64 * j;
+            const int row = r0 + wave * SQ_RPW + i, c = lane + 64 * j;
             pr[i][j] = (row < L && c < L) ? a.p[poff + (size_t)row * L + c] : 0.f;
         }
-    tile_edge_store(e0);
-    tile_edge_store(e1);
-    tile_edge_store(e2);
+    tile_edge_store(edge);
     wait_vmcnt<0>();
     __syncthreads();
-    // dP[query][key] = sum_d dA[d][query] v[d][key]   (lib/sources/pulp_mhsa_fp32.c:958-1060)
-    scores_resident(Qs, Ks, (L + 31) >> 5, 1.0f, S, wave, l32, half);
-    __syncthreads();
     // softmax backward (lib/sources/pulp_act_fp32.c:335-390) and the scaling (:1176-1183)
-    float gv[RS_RPW][4], sum[RS_RPW];
+    float gv[SQ_RPW][4], sum[SQ_RPW];
 #pragma unroll
-    for (int i = 0; i < RS_RPW; ++i) {
-        const float *srow = S + (wave * RS_RPW + i) * RS_SP;
+    for (int i = 0; i < SQ_RPW; ++i) {
+        const float *srow = S + (wave * SQ_RPW + i) * pitch;
         sum[i] = 0.f;
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
@@ -800,89 +844,84 @@ __global__ __launch_bounds__(RS_NT) void attn_bw_query_res_kernel(AttnArgs a) {
         }
     }
 #pragma unroll
-    for (int o = 32; o > 0; o >>= 1)
+    for (int i = 0; i < SQ_RPW; ++i) sum[i] = wave_sum(sum[i]);
 #pragma unroll
-        for (int i = 0; i < RS_RPW; ++i) sum[i] += __shfl_xor(sum[i], o);
-#pragma unroll
-    for (int i = 0; i < RS_RPW; ++i) {
-        const int row = wave * RS_RPW + i;
-        float *srow = S + row * RS_SP;
+    for (int i = 0; i < SQ_RPW; ++i) {
+        const int row = wave * SQ_RPW + i;
+        float *srow = S + row * pitch;
         const bool live = r0 + row < L;
         float *dprow = a.o0 + poff + (size_t)(r0 + row) * L;
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
             const int c = lane + 64 * j;
-            if (c < RS_LC) {
-                if (live && c < L) dprow[c] = gv[i][j];
-                srow[c] = c < L ? ((gv[i][j] - sum[i]) * pr[i][j]) * a.scale : 0.f;
+            if (c < L) {
+                if (live) dprow[c] = gv[i][j];
+                srow[c] = ((gv[i][j] - sum[i]) * pr[i][j]) * a.scale;
             }
         }
         if (live && lane == 0) a.o2[((size_t)b * a.heads + h) * L + r0 + row] = sum[i];
     }
     __syncthreads();
     // dq[d][query] = sum_key k[d][key] dS[query][key]   (:1342-1360)
-    mix_resident(Vs, S, L, a.H, r0, a.o1 + hoff, red, tid, wave, l32, half);
+    sq_mix<HB>(Ks, S, L, a.H, r0, a.o1 + hoff, att_lds, tid, wave, l32, half);
 }
 
-// Key side: tile of 32 keys; dA and q ([d][query], 16-byte fragments along the queries) and the key columns
-// of P and dP ([query][32 keys]) are resident; dS replaces dP in place before the products.
+// Key side, a tile of 32 keys: one workgroup forms dv, one dk.  dA (q) is resident as [d][query], the key
+// columns of P (and dP) go straight to registers, 128 bytes of a query per half wave.
 //   dv[d][key] = sum_query dA[d][query] P[query][key]                         (:884-902)
 //   dk[d][key] = sum_query q[d][query] dS[query][key], dS = (dP - rs) P scale  (:1244-1330)
-__global__ __launch_bounds__(RS_NT) void attn_bw_key_res_kernel(AttnArgs a) {
-    extern __shared__ __attribute__((aligned(16))) float att_lds[];
-    float *dAs = att_lds, *Qs = dAs + 64 * RS_VP, *Pp = Qs + 64 * RS_VP, *Gp = Pp + RS_KD * 32, *rsl = Gp + RS_KD * 32;
-    float *red = att_lds;
-    const int c0 = blockIdx.x * 32, h = blockIdx.y, b = blockIdx.z, L = a.L, H = a.H;
+template <int HB, bool DK>
+__device__ inline void sq_key(const AttnArgs &a, const SqPlace &at, float *lds) {
+    constexpr int KS = SQ_NW / HB, STEP = 4;
+    const int c0 = at.tile * 32, L = a.L, H = a.H, pitch = sq_pitch(L);
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int l32 = lane & 31, half = lane >> 5;
-    const size_t hoff = ((size_t)b * a.F + (size_t)h * H) * L;
-    const size_t poff = ((size_t)b * a.heads + h) * L * L;
-    tile_dma<RS_NW>(a.da + hoff, L, 64, RS_KD, H, L, dAs, RS_VP, a.zero, wave, lane);
-    tile_dma<RS_NW>(a.q + hoff, L, 64, RS_KD, H, L, Qs, RS_VP, a.zero, wave, lane);
-    tile_dma<RS_NW>(a.p + poff + c0, L, RS_KD, 32, L, L - c0, Pp, 32, a.zero, wave, lane);
-    tile_dma<RS_NW>(a.dp + poff + c0, L, RS_KD, 32, L, L - c0, Gp, 32, a.zero, wave, lane);
-    const TileEdge e0 = tile_edge_load(a.da + hoff, L, 64, RS_KD, H, L, dAs, RS_VP, tid);
-    const TileEdge e1 = tile_edge_load(a.q + hoff, L, 64, RS_KD, H, L, Qs, RS_VP, tid);
-    const TileEdge e2 = tile_edge_load(a.p + poff + c0, L, RS_KD, 32, L, L - c0, Pp, 32, tid);
-    const TileEdge e3 = tile_edge_load(a.dp + poff + c0, L, RS_KD, 32, L, L - c0, Gp, 32, tid);
-    const float rsv = (tid < RS_KD && tid < L) ? a.rs[((size_t)b * a.heads + h) * L + tid] : 0.f;
-    tile_edge_store(e0);
-    tile_edge_store(e1);
-    tile_edge_store(e2);
-    tile_edge_store(e3);
-    if (tid < RS_KD) rsl[tid] = rsv;
+    const size_t hoff = ((size_t)at.b * a.F + (size_t)at.h * H) * L, row0 = (size_t)at.b * a.heads + at.h;
+    const float *P = a.p + row0 * L * L, *G = a.dp + row0 * L * L;
+    const TileEdge edge = sq_fetch<HB>((DK ? a.q : a.da) + hoff, L, H, lds, a.zero, tid, wave, lane);
+    float *rsl = lds + 32 * HB * pitch;  // (zeros up to the next group of eight)
+    if (DK && tid < pitch) rsl[tid] = tid < L ? a.rs[row0 * L + tid] : 0.f;
+    const int db = wave % HB, ks = wave / HB;
+    const unsigned c = (unsigned)min(c0 + l32, L - 1);
+    const int groups = (L + 7) >> 3, per = (groups + KS - 1) / KS, g0 = ks * per, end = min(groups, g0 + per);
+    tile_edge_store(edge);
     wait_vmcnt<0>();
     __syncthreads();
-    for (int idx = tid; idx < RS_KD * 32; idx += RS_NT) Gp[idx] = ((Gp[idx] - rsl[idx >> 5]) * Pp[idx]) * a.scale;
-    __syncthreads();
-    const int db = wave & 1, ks = wave >> 1;
-    const int ngroups = (L + 7) >> 3, per = (ngroups + RS_KS - 1) / RS_KS;
-    const int g_end = min(ngroups, (ks + 1) * per);
-    mh_f32x16 accv = {0}, acck = {0};
-    for (int g = ks * per; g < g_end; ++g) {
-        const int k4 = g * 8 + half * 4;
-        float4 pb, sb;
-        pb.x = Pp[k4 * 32 + l32];
-        pb.y = Pp[(k4 + 1) * 32 + l32];
-        pb.z = Pp[(k4 + 2) * 32 + l32];
-        pb.w = Pp[(k4 + 3) * 32 + l32];
-        sb.x = Gp[k4 * 32 + l32];
-        sb.y = Gp[(k4 + 1) * 32 + l32];
-        sb.z = Gp[(k4 + 2) * 32 + l32];
-        sb.w = Gp[(k4 + 3) * 32 + l32];
-        mfma4(accv, *reinterpret_cast<const float4 *>(dAs + (db * 32 + l32) * RS_VP + k4), pb);
-        mfma4(acck, *reinterpret_cast<const float4 *>(Qs + (db * 32 + l32) * RS_VP + k4), sb);
-    }
-    float *outs[2] = {a.o0 + hoff, a.o1 + hoff};
+    mh_f32x16 acc = {0};
+    for (int g = g0; g < end; g += STEP) {
+        float p[STEP][4], q[STEP][4];  // of the four queries of a group that this half holds
 #pragma unroll
-    for (int which = 0; which < 2; ++which) {
-        __syncthreads();
+        for (int u = 0; u < STEP; ++u)
 #pragma unroll
-        for (int v = 0; v < 16; ++v)
-            red[(wave * 32 + 8 * (v / 4) + 4 * half + (v % 4)) * ATT_RP + l32] = which ? acck[v] : accv[v];
-        __syncthreads();
-        mix_store(red, L, H, c0, outs[which], tid);
+            for (int j = 0; j < 4; ++j) {
+                const unsigned o = (unsigned)(min(min(g + u, end - 1) * 8 + half * 4 + j, L - 1) * L) + c;
+                p[u][j] = P[o];
+                if (DK) q[u][j] = G[o];
+            }
+        __builtin_amdgcn_sched_barrier(0);  // (all of them in flight before the first is waited for)
+#pragma unroll
+        for (int u = 0; u < STEP; ++u) {
+            if (g + u >= end) break;
+            const int k4 = (g + u) * 8 + half * 4;
+            float o[4];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                o[j] = DK ? ((q[u][j] - rsl[k4 + j]) * p[u][j]) * a.scale : p[u][j];
+                if (k4 + j >= L) o[j] = 0.f;
+            }
+            mfma4(acc, *reinterpret_cast<const float4 *>(lds + (db * 32 + l32) * pitch + k4), make_float4(o[0], o[1], o[2], o[3]));
+        }
     }
+    sq_store<HB>(acc, lds, L, H, c0, (DK ? a.o1 : a.o0) + hoff, tid, wave, l32, half);
+}
+
+template <int HB>
+__global__ __launch_bounds__(SQ_NT, 4) void attn_bw_key_res_kernel(AttnArgs a) {
+    extern __shared__ __attribute__((aligned(16))) float att_lds[];
+    SqPlace at;
+    if (!sq_place(a, 2, at)) return;
+    if (at.part == 1) sq_key<HB, true>(a, at, att_lds);
+    else sq_key<HB, false>(a, at, att_lds);
 }
 
 // Row softmax over H rows of W (one wave per row).
@@ -974,24 +1013,32 @@ static int launch_attn(int which, AttnArgs &a, int ns) {
     return hip_ok(hipGetLastError(), "attention launch") ? 0 : 2;
 }
 
+template <int HB>
+static int launch_attn_res(int which, AttnArgs &a, int ns) {
+    void (*kern)(AttnArgs) = which == 0 ? attn_fw_res_kernel<HB> : which == 1 ? attn_bw_query_res_kernel<HB> : attn_bw_key_res_kernel<HB>;
+    static bool attr_set[3] = {false, false, false};
+    if (!attr_set[which]) {
+        if (!hip_ok(hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                        (int)sq_lds<HB>(SQ_L, which == 2)),
+                    "hipFuncSetAttribute"))
+            return 2;
+        attr_set[which] = true;
+    }
+    a.ns = ns;
+    const long long blocks = ((long long)ns * a.heads + 7) / 8 * 8 * ((a.L + 31) / 32) * (which == 2 ? 2 : 1);
+    if (blocks >= (1ll << 31)) {
+        set_error("attention: too many heads");
+        return 1;
+    }
+    hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(SQ_NT), sq_lds<HB>(a.L, which == 2), state().stream, a);
+    return hip_ok(hipGetLastError(), "attention launch") ? 0 : 2;
+}
+
 static int launch_attn_any(int which, AttnArgs &a, int ns) {
-    if (a.L <= RS_KD && a.H > 32 && a.H <= 64) {
+    if (a.L <= SQ_L && a.H <= 64) {
         a.zero = static_cast<const float *>(state().zeros);
         if (!a.zero) return 2;
-        void (*kern)(AttnArgs) =
-            which == 0 ? attn_fw_res_kernel : which == 1 ? attn_bw_query_res_kernel : attn_bw_key_res_kernel;
-        const size_t lds = (size_t)(which == 2 ? RS_KEY_FLOATS : RS_FW_FLOATS) * sizeof(float);
-        static bool attr_set[3] = {false, false, false};
-        if (!attr_set[which]) {
-            if (!hip_ok(hipFuncSetAttribute(reinterpret_cast<const void *>(kern),
-                                            hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024),
-                        "hipFuncSetAttribute"))
-                return 2;
-            attr_set[which] = true;
-        }
-        dim3 grid((a.L + 31) / 32, a.heads, ns);
-        hipLaunchKernelGGL(kern, grid, dim3(RS_NT), lds, state().stream, a);
-        return hip_ok(hipGetLastError(), "attention launch") ? 0 : 2;
+        return a.H <= 32 ? launch_attn_res<1>(which, a, ns) : launch_attn_res<2>(which, a, ns);
     }
     if (a.H <= 32) return launch_attn<32>(which, a, ns);
     if (a.H <= 64) return launch_attn<64>(which, a, ns);
@@ -1183,6 +1230,59 @@ static PanelArgs acts_times_acts(int N, int M, int L, int ns) {
     return p;
 }
 
+// The same products for the kernel of any size and alignment: out[b][N x L] = W(N x K) . act[b][K x L] (tiles stay inside a
+// sample), W with rows of K or, transposed, columns of N; and out[N x M] = sum over samples and tokens.  Activations are
+// formed in one tile shape with the contraction whole, so that a sample's do not depend on the batch it is in.
+static RagOp rag_matrix(const float *p, int rows, int row_stride, int k_stride, long long run = 0, long long outer = 0) {
+    RagOp o = {};
+    o.p = reinterpret_cast<const char *>(p);
+    o.rows = rows;
+    o.row_b = (unsigned)row_stride * 4u;
+    o.k_b = (unsigned)k_stride * 4u;
+    o.run_b = run * 4;
+    o.outer_b = outer * 4;
+    return o;
+}
+static RagProd rag_weights_times_acts(const float *W, bool transposed, const float *act, float *out, int N, int K, int L, int ns) {
+    RagProd p = {};
+    p.a = transposed ? rag_matrix(W, N, 1, N) : rag_matrix(W, N, K, 1);
+    p.b = rag_matrix(act, L, 1, L, 0, (long long)K * L);
+    p.C = out;
+    p.N = N;
+    p.M = ns * L;
+    p.m_in = L;
+    p.outer = ns;
+    p.K = K;
+    p.runs = 1;
+    p.cn = rag_axis(N, L);
+    p.cm = rag_axis2(L, 1, N * L);
+    p.whole_k = 1;
+    return p;
+}
+static RagProd rag_acts_times_acts(const float *A, const float *B, float *out, int N, int M, int L, int ns) {
+    RagProd p = {};
+    p.a = rag_matrix(A, N, L, 1, (long long)N * L);
+    p.b = rag_matrix(B, M, L, 1, (long long)M * L);
+    p.C = out;
+    p.N = N;
+    p.M = p.m_in = M;
+    p.outer = 1;
+    p.K = L;
+    p.runs = ns;
+    p.cn = rag_axis(N, M);
+    p.cm = rag_axis(M, 1);
+    return p;
+}
+// (small tiles with all waves on the contraction up to 128 tokens: 92 -> 65 us for 7 x 19 tokens, 125 -> 96 for 8 x 64)
+static int rag_tile_of(int L) { return L <= 128 ? 32 : 64; }
+// Rows and runs of k hold whole pieces (the panels take what has shorter ones, and what paths 6 and 7 ask of them).  Against
+// the panels: 83 -> 65 us for 7 x 6 heads of 48 and 19 tokens, 507 -> 430 for 46 x 6 and 192, 123 -> 96 for 8 x 8 of 64 and 64
+// tokens, 227 -> 208 for 32 x 3 of 64 and 197, all forward + backward; equal for single samples.
+static bool rag_takes(const MhsaDims &m) {
+    const int path = state().gemm_path;
+    return path != 6 && path != 7 && m.L >= 4 && m.E >= 4 && m.F >= 4 && m.L < (1 << 20) && m.E < (1 << 20) && m.F < (1 << 20);
+}
+
 static bool mhsa_fits(const MhsaDims &m, int ns) {
     const size_t lim = (size_t)1 << 31;
     return (size_t)ns * m.E * m.L < lim && (size_t)ns * m.F * m.L < lim && (size_t)ns * m.heads * m.L * m.L < lim &&
@@ -1218,7 +1318,18 @@ static int mhsa_fw(const Mhsa_args *a, int ns, const char *fn) {
     float *Y = sg.out(a->output->data, xe);
     if (sg.failed()) return 2;
     int rc = 0;
-    {
+    const bool rag = rag_takes(m);
+    if (rag) {
+        RagArgs r = {};
+        r.shape = rag_tile_of(L);
+        r.count = 3;
+        for (int j = 0; j < 3; ++j) {
+            r.p[j] = rag_weights_times_acts(W[j], true, X, QKV[j], F, E, L, ns);
+            r.p[j].bias = bias[j];
+            r.p[j].bias_n = 1;
+        }
+        rc = ragged<float>(r, RAG_RC, RAG_RC, RAG_RC, RAG_RC);
+    } else {
         // q/k/v[F x L] = W^T . X + bias in one launch (weights stored E x F: lib/sources/pulp_mhsa_fp32.c:70-325)
         PanelArgs p = weights_times_acts(F, E, L, ns, 1, F);
         p.nout = 3;
@@ -1245,7 +1356,13 @@ static int mhsa_fw(const Mhsa_args *a, int ns, const char *fn) {
         t.scale = q_rsqrt_host((float)m.H);
         rc = launch_attn_any(0, t, ns);
     }
-    if (rc == 0) {
+    if (rc == 0 && rag) {
+        RagArgs r = {};
+        r.shape = rag_tile_of(L);
+        r.count = 1;
+        r.p[0] = rag_weights_times_acts(Wo, false, att, Y, E, F, L, ns);
+        rc = ragged<float>(r, RAG_KC, RAG_RC, RAG_KC, RAG_RC);
+    } else if (rc == 0) {
         // output[E x L] = Wout[E x F] . attention_map (:599-609)
         PanelArgs p = weights_times_acts(E, F, L, ns, F, 1);
         p.A[0] = Wo;
@@ -1297,7 +1414,14 @@ static int mhsa_bw(const Mhsa_args *a, int ns, const char *fn) {
     // dWout[E x F] = sum over samples of dY . att^T (:742-760) and datt[F x L] = Wout^T . dY (:816-834), one launch;
     // the sample groups of dWout are added up at the end, together with those of the input weights' gradients
     PanelArgs pwo = acts_times_acts(E, F, L, ns);
-    {
+    const bool rag = rag_takes(m);
+    if (rag) {  // (dWout comes with the other weights' gradients)
+        RagArgs r = {};
+        r.shape = rag_tile_of(L);
+        r.count = 1;
+        r.p[0] = rag_weights_times_acts(Wo, true, dY, datt, F, E, L, ns);
+        rc = ragged<float>(r, RAG_RC, RAG_RC, RAG_RC, RAG_RC);
+    } else {
         pwo.A[0] = dY;
         pwo.B[0] = att;
         pwo.C[0] = dWo;
@@ -1333,7 +1457,22 @@ static int mhsa_bw(const Mhsa_args *a, int ns, const char *fn) {
         t.o2 = nullptr;
         rc = launch_attn_any(2, t, ns);
     }
-    if (rc == 0) {
+    if (rc == 0 && rag) {
+        RagArgs r = {};
+        r.shape = rag_tile_of(L);
+        r.count = 5;
+        RagProd &x = r.p[0];
+        x = rag_weights_times_acts(W[0], false, dQKV[0], dX, E, F, L, ns);
+        x.runs = 3;
+        x.add = 1;
+        for (int j = 0; j < 2; ++j) {
+            r.hop_a[j] = reinterpret_cast<const char *>(W[j + 1]) - reinterpret_cast<const char *>(W[j]);
+            r.hop_b[j] = reinterpret_cast<const char *>(dQKV[j + 1]) - reinterpret_cast<const char *>(dQKV[j]);
+        }
+        for (int j = 0; j < 3; ++j) r.p[1 + j] = rag_acts_times_acts(dQKV[j], X, dW[j], F, E, L, ns);
+        r.p[4] = rag_acts_times_acts(dY, att, dWo, E, F, L, ns);
+        rc = ragged<float>(r, RAG_KC, RAG_RC, RAG_KC, RAG_KC);
+    } else if (rc == 0) {
         // dW_{q,k,v}[F x E] = sum over samples of d{q,k,v} . X^T (:1425-1560) and
         // dX[E x L] += W_q . dq + W_k . dk + W_v . dv (:1589-1745), one launch
         PanelArgs p = acts_times_acts(F, E, L, ns);

@@ -72,6 +72,8 @@ struct RagProd {
     int outer, m_in;   // RC second operand: M = outer x m_in, tiles stay inside one outer digit (outer == 1: m_in == M)
     const void *bias;  // added per n (bias_n) or per m
     int bias_n;
+    int whole_k;       // the contraction is not split
+    int add;           // C keeps what it holds, the product is added to it
     void *row_sum;     // sum over k of a(n, k), as an extra column of ones in b (RC, GR, XR)
     // set by the launcher
     float *ws;         // partial sums [split][N][pitch]
@@ -79,21 +81,25 @@ struct RagProd {
     int tiles_n, tiles_m, tiles_in;  // tiles along n, along m, along m inside one outer digit
 };
 
-constexpr int RAG_MAX = 2;
+constexpr int RAG_MAX = 5;
 struct RagArgs {
     RagProd p[RAG_MAX];
     int first[RAG_MAX + 1];  // first workgroup of each product
     int count;
+    int shape;  // 32, 64: that tile, whatever it costs (sums in the same order at every size); 0: the cheapest
+    // of the first product of (KC, RC) before (KC, KC) only: up to three runs of k lie anywhere, run r + 1 hop_a[r],
+    // hop_b[r] bytes behind run r (its run_b is not used)
+    long long hop_a[2], hop_b[2];
 };
 
 struct RagSums {  // the products whose contraction was split
-    RagProd p[4];
-    int first[5];
+    RagProd p[5];
+    int first[6];
     int count;
 };
 
 // The products in one launch (plus one for their partial sums where the contraction is split).  The first product has
-// the modes (a0, b0), the other (a1, b1).  0 = launched, -1 = no such combination of modes, 2 = a HIP failure.
+// the modes (a0, b0), the others (a1, b1).  0 = launched, -1 = no such combination of modes, 2 = a HIP failure.
 template <typename T>
 int ragged(RagArgs &r, int a0, int b0, int a1, int b1);
 
@@ -128,10 +134,10 @@ struct RagConvOf {
     int relays, relay_first[RAG_CONV_MAX + 1];
 };
 typedef RagConvOf<RAG_CONV_MAX> RagConvArgs;
-// The tiles and splits that ragged_conv() would choose for the products (of which sizes and runs count), and the clocks of
+// The tiles and slabs per workgroup that ragged_conv() would choose for the products (of which sizes and runs count), and the clocks of
 // 2.4 GHz that this would take.
 struct RagPlan {
-    int shape, splits;
+    int shape, per_wg;
     double clocks;
 };
 template <typename T>
