@@ -1239,7 +1239,10 @@ __global__ __launch_bounds__(256) void patch_kernel(const T *__restrict__ src, T
 // is read in as few instructions as the layout allows: WIDE (rows of the tensor start on 16-byte boundaries) takes
 // the aligned 16-byte pieces that cover the window - the window then starts up to a piece early, `shift` elements
 // that the offsets table skips - and otherwise one element per lane, one wave per window row.
-
+// The writes bound it (a 3x3 filter writes nine elements per one read), and whole chunks serve rows of any length and
+// start: the last chunk of a row piece ends with the piece, the channels are split into equal pieces whatever their
+// number.  154 channels of 60 x 253 in fp16, 3 x 3: 47.6 us, 106.6 one element at a time;
+// 186 channels of 212 x 154 in fp32: 110 us, before 258.
 template <typename T, bool WIDE>
 __global__ __launch_bounds__(256) void patch_rows_kernel(const T *__restrict__ src, T *__restrict__ buf, PatchGeom g, int R,
                                                          int CB, int LW, unsigned m_pk, unsigned m_wk, unsigned m_hk) {
@@ -1248,10 +1251,11 @@ __global__ __launch_bounds__(256) void patch_rows_kernel(const T *__restrict__ s
     typedef const T __attribute__((address_space(1))) *GlobalT;
     typedef const PatchPiece __attribute__((address_space(1))) *GlobalPiece;
     extern __shared__ __attribute__((aligned(16))) char smem[];
-    const int PK = g.Hk * g.Wk, Q = g.C * PK, nq = CB * PK;
-    unsigned short *offs = reinterpret_cast<unsigned short *>(smem);                    // [nq], nq a multiple of VEC
-    T *lds = reinterpret_cast<T *>(smem + (((size_t)nq * 2 + 15) & ~(size_t)15));      // [CB * Hk][LW], one spare slot
     const int wp0 = blockIdx.x * R, hp = blockIdx.y, c0 = blockIdx.z * CB;
+    CB = min(CB, g.C - c0);
+    const int PK = g.Hk * g.Wk, Q = g.C * PK, nq = CB * PK;  // (at least a chunk)
+    unsigned short *offs = reinterpret_cast<unsigned short *>(smem);                    // [nq]
+    T *lds = reinterpret_cast<T *>(smem + (((size_t)nq * 2 + 15) & ~(size_t)15));      // [CB * Hk][LW], one spare slot
     const int nr = min(R, g.Wp - wp0);
     const int w_first = wp0 * g.w_mul + g.w_add, h_first = hp * g.h_mul + g.h_add;
     const int w_start = WIDE ? (w_first & ~(VEC - 1)) : w_first, shift = w_first - w_start;  // (& rounds down below 0 too)
@@ -1308,12 +1312,17 @@ __global__ __launch_bounds__(256) void patch_rows_kernel(const T *__restrict__ s
     __syncthreads();
     // a thread keeps one chunk position of the buffer rows (its table entries stay in registers) and walks down the
     // positions; a row piece longer than the workgroup takes several sweeps
-    const int cpr = nq / VEC;  // chunks of this workgroup per buffer row
+    // (a row piece that is no whole number of chunks: its last chunk ends with it and repeats values of the one before)
+    const int cpr = (nq + VEC - 1) / VEC;  // chunks of this workgroup per buffer row
     const int span = min(cpr, 256), pstep = 256 / span, p0 = threadIdx.x / span;
     T *base = buf + ((size_t)hp * g.Wp + wp0) * Q + (size_t)c0 * PK;
     for (int qc = threadIdx.x - p0 * span; qc < cpr && p0 < pstep; qc += span) {
         int o[VEC];
-        if (VEC == 8) {
+        const int q0 = min(qc * VEC, nq - VEC);
+        if (q0 != qc * VEC) {
+#pragma unroll
+            for (int e = 0; e < VEC; ++e) o[e] = offs[q0 + e];
+        } else if (VEC == 8) {
             const uint4 t4 = *reinterpret_cast<const uint4 *>(offs + qc * 8);
             o[0] = t4.x & 0xffffu; o[1] = t4.x >> 16; o[2] = t4.y & 0xffffu; o[3] = t4.y >> 16;
             o[4 % VEC] = t4.z & 0xffffu; o[5 % VEC] = t4.z >> 16; o[6 % VEC] = t4.w & 0xffffu; o[7 % VEC] = t4.w >> 16;
@@ -1322,15 +1331,12 @@ __global__ __launch_bounds__(256) void patch_rows_kernel(const T *__restrict__ s
             o[0] = t2.x & 0xffffu; o[1] = t2.x >> 16; o[2] = t2.y & 0xffffu; o[3] = t2.y >> 16;
         }
         const T *win = lds + p0 * g.w_mul;
-        T *dst = base + (size_t)p0 * Q + qc * VEC;
+        T *dst = base + (size_t)p0 * Q + q0;
         for (int p_l = p0; p_l < nr; p_l += pstep) {
-            union {
-                uint4 u;
-                T e[VEC];
-            } v;
+            T v[VEC];
 #pragma unroll
-            for (int e = 0; e < VEC; ++e) v.e[e] = win[o[e]];
-            *reinterpret_cast<uint4 *>(dst) = v.u;
+            for (int e = 0; e < VEC; ++e) v[e] = win[o[e]];
+            memcpy(dst, v, 16);  // (wherever the row starts)
             win += pstep * g.w_mul;
             dst += (size_t)pstep * Q;
         }
@@ -1485,7 +1491,7 @@ static int patch_rows(const T *src, T *buf, const PatchGeom &g) {
     if (g.hwc || g.col_major) return -1;
     const int PK = g.Hk * g.Wk;
     const long long Q = (long long)g.C * PK;
-    if (reinterpret_cast<uintptr_t>(buf) % 16 || (Q * ES) % 16 || g.Wp < 16 || Q >= 65536 || g.Hp >= 65536 || g.Wk > 32 ||
+    if (g.Wp < 16 || Q < VEC || Q >= 65536 || g.Hp >= 65536 || g.Wk > 32 ||
         g.w_mul > 8 || (long long)(g.C + 64) * g.Hs * g.Ws >= ((long long)1 << 31))  // (32-bit element offsets, with slack)
         return -1;
     // rows of the tensor that start on 16-byte boundaries are read as aligned 16-byte pieces
@@ -1505,16 +1511,18 @@ static int patch_rows(const T *src, T *buf, const PatchGeom &g) {
     LW = ES == 2 ? (((LW + 1) & ~1) | 2) : (LW | 1);
     // (table of column offsets, window, one spare slot)
     auto bytes = [&](int cb) { return (((size_t)cb * PK * 2 + 15) & ~(size_t)15) + (size_t)cb * g.Hk * LW * ES + 16; };
-    int CB = g.C;
-    while (bytes(CB) > 40 * 1024 && CB % 2 == 0) CB /= 2;
-    // whole buffer rows per workgroup (one contiguous run of R x Q elements) unless that leaves CUs idle; a
-    // workgroup's piece of a buffer row stays a few cache lines long
+    // Whole buffer rows per workgroup (one contiguous run of R x Q elements) unless their window is too large for LDS or
+    // that leaves CUs idle; a workgroup's piece of a buffer row stays a few cache lines long.
+    int nz = 1;
+    auto channels = [&](int z) { return (g.C + z - 1) / z; };
+    while (bytes(channels(nz)) > 40 * 1024 && channels(nz) > 1) nz *= 2;
     const long long per_z = (long long)((g.Wp + R - 1) / R) * g.Hp;
-    while (per_z * (g.C / CB) < 2LL * state().num_cu && CB % 2 == 0 && (CB / 2) * PK * ES >= 256 && ((CB / 2) * PK) % VEC == 0)
-        CB /= 2;
-    if (bytes(CB) > 64 * 1024 || (CB * PK) % VEC || CB * g.Hk * LW >= 65536 || g.C / CB >= 65536) return -1;
+    while (per_z * nz < 2LL * state().num_cu && channels(2 * nz) * PK * ES >= 256) nz *= 2;
+    const int CB = channels(nz), last = g.C - (g.C + CB - 1) / CB * CB + CB;  // channels of the last piece
+    nz = (g.C + CB - 1) / CB;
+    if (bytes(CB) > 64 * 1024 || last * PK < VEC || CB * g.Hk * LW >= 65536 || nz >= 65536) return -1;
     auto magic = [](unsigned d) { return (unsigned)((((unsigned long long)1 << 32) + d - 1) / d); };
-    dim3 grid((g.Wp + R - 1) / R, g.Hp, g.C / CB);
+    dim3 grid((g.Wp + R - 1) / R, g.Hp, nz);
     if (wide)
         hipLaunchKernelGGL((patch_rows_kernel<T, true>), grid, dim3(256), bytes(CB), state().stream, src, buf, g, R, CB, LW,
                            magic(PK), magic(g.Wk), magic(g.Hk));
@@ -1812,55 +1820,43 @@ struct Transp2D {
     long long in_rs, out_rs, in_bs, out_bs, in_base, out_base;
 };
 
+// 64 x 64 tiles through LDS, 16 bytes per access on both sides wherever the rows start (a wave's eight rows of 128 bytes
+// need no alignment for that); what is left of a row behind its last whole piece moves element by element.  Memory
+// bounds it: over matrices of odd sizes 1.3x the rate of moving each element by itself, aligned ones as before.
+typedef unsigned TranspPiece __attribute__((ext_vector_type(4), aligned(1)));
 template <typename T>
 __global__ __launch_bounds__(256) void transpose2d_kernel(const T *__restrict__ in, T *__restrict__ out, Transp2D g) {
-    __shared__ T tile[64][65];
-    in += g.in_base + (long long)blockIdx.z * g.in_bs;
-    out += g.out_base + (long long)blockIdx.z * g.out_bs;
-    int j0 = blockIdx.x * 64, i0 = blockIdx.y * 64;
-    int tx = threadIdx.x & 63, ty = threadIdx.x >> 6;
-    for (int r = ty; r < 64; r += 4) {
-        int i = i0 + r, j = j0 + tx;
-        if (i < g.N && j < g.M) tile[r][tx] = in[(long long)i * g.in_rs + j];
-    }
-    __syncthreads();
-    for (int r = ty; r < 64; r += 4) {
-        int j = j0 + r, i = i0 + tx;
-        if (i < g.N && j < g.M) out[(long long)j * g.out_rs + i] = tile[tx][r];
-    }
-}
-
-// The same with 16-byte global accesses on both sides (rows, row strides, bases and pointers multiples of 16
-// bytes).  The tile is kept as dwords with a pitch of 33 (fp16: two columns per dword) or 65 (fp32), so the
-// column walk of the second phase is conflict free; a thread gathers the VEC elements of its output chunk from
-// VEC tile rows and stores them at once.
-template <typename T>
-__global__ __launch_bounds__(256) void transpose2d_vec_kernel(const T *__restrict__ in, T *__restrict__ out, Transp2D g) {
     constexpr int VEC = 16 / (int)sizeof(T), CH = 64 / VEC;  // chunks per tile row
     constexpr int PITCH = sizeof(T) == 2 ? 66 : 65;          // elements
     __shared__ __attribute__((aligned(16))) T tile[64 * PITCH];
     in += g.in_base + (long long)blockIdx.z * g.in_bs;
     out += g.out_base + (long long)blockIdx.z * g.out_bs;
     const int j0 = blockIdx.x * 64, i0 = blockIdx.y * 64;
+    union Piece {
+        TranspPiece u;
+        T e[VEC];
+        unsigned d[4];
+    };
 #pragma unroll
     for (int it = 0; it < 64 * CH / 256; ++it) {
         const int item = it * 256 + threadIdx.x, r = item / CH, c = item % CH;
         const int i = i0 + r, j = j0 + c * VEC;
-        if (i < g.N && j < g.M) {  // (M is a multiple of VEC: a chunk is inside or outside)
-            union {
-                uint4 u;
-                T e[VEC];
-                unsigned d[4];
-            } v;
-            v.u = *reinterpret_cast<const uint4 *>(in + (long long)i * g.in_rs + j);
-            if (sizeof(T) == 2) {
-                unsigned *row = reinterpret_cast<unsigned *>(tile + r * PITCH + c * VEC);  // 4-byte aligned
+        if (i >= g.N || j >= g.M) continue;
+        Piece v;
+        const T *src = in + (long long)i * g.in_rs + j;
+        if (j + VEC <= g.M) {
+            v.u = *reinterpret_cast<const TranspPiece *>(src);
+        } else {
 #pragma unroll
-                for (int k = 0; k < 4; ++k) row[k] = v.d[k];
-            } else {
+            for (int k = 0; k < VEC; ++k) v.e[k] = j + k < g.M ? src[k] : (T)0;
+        }
+        if (sizeof(T) == 2) {
+            unsigned *row = reinterpret_cast<unsigned *>(tile + r * PITCH + c * VEC);  // 4-byte aligned
 #pragma unroll
-                for (int k = 0; k < VEC; ++k) tile[r * PITCH + c * VEC + k] = v.e[k];
-            }
+            for (int k = 0; k < 4; ++k) row[k] = v.d[k];
+        } else {
+#pragma unroll
+            for (int k = 0; k < VEC; ++k) tile[r * PITCH + c * VEC + k] = v.e[k];
         }
     }
     __syncthreads();
@@ -1868,14 +1864,17 @@ __global__ __launch_bounds__(256) void transpose2d_vec_kernel(const T *__restric
     for (int it = 0; it < 64 * CH / 256; ++it) {
         const int item = it * 256 + threadIdx.x, r = item / CH, c = item % CH;  // output row j0 + r, rows i0 + c*VEC ..
         const int j = j0 + r, i = i0 + c * VEC;
-        if (j < g.M && i < g.N) {
-            union {
-                uint4 u;
-                T e[VEC];
-            } v;
+        if (j >= g.M || i >= g.N) continue;
+        Piece v;
 #pragma unroll
-            for (int k = 0; k < VEC; ++k) v.e[k] = tile[(c * VEC + k) * PITCH + r];
-            *reinterpret_cast<uint4 *>(out + (long long)j * g.out_rs + i) = v.u;
+        for (int k = 0; k < VEC; ++k) v.e[k] = tile[(c * VEC + k) * PITCH + r];
+        T *dst = out + (long long)j * g.out_rs + i;
+        if (i + VEC <= g.N) {
+            *reinterpret_cast<TranspPiece *>(dst) = v.u;
+        } else {
+#pragma unroll
+            for (int k = 0; k < VEC; ++k)
+                if (i + k < g.N) dst[k] = v.e[k];
         }
     }
 }
@@ -1883,16 +1882,9 @@ __global__ __launch_bounds__(256) void transpose2d_vec_kernel(const T *__restric
 template <typename T>
 static int transpose2d_strided(const T *in, T *out, int N, int M, long long in_rs, long long out_rs, int batch,
                                long long in_bs, long long out_bs, long long in_base, long long out_base) {
-    constexpr int VEC = 16 / (int)sizeof(T);
-    Transp2D g = {N, M, in_rs, out_rs, in_bs, out_bs, in_base, out_base};
-    dim3 grid((M + 63) / 64, (N + 63) / 64, batch);
-    auto mult = [](long long v) { return v % VEC == 0; };
-    const bool vec = mult(N) && mult(M) && mult(in_rs) && mult(out_rs) && mult(in_bs) && mult(out_bs) && mult(in_base) &&
-                     mult(out_base) && reinterpret_cast<uintptr_t>(in) % 16 == 0 && reinterpret_cast<uintptr_t>(out) % 16 == 0;
-    if (vec)
-        hipLaunchKernelGGL((transpose2d_vec_kernel<T>), grid, dim3(256), 0, state().stream, in, out, g);
-    else
-        hipLaunchKernelGGL((transpose2d_kernel<T>), grid, dim3(256), 0, state().stream, in, out, g);
+    const Transp2D g = {N, M, in_rs, out_rs, in_bs, out_bs, in_base, out_base};
+    const dim3 grid((M + 63) / 64, (N + 63) / 64, batch);
+    hipLaunchKernelGGL((transpose2d_kernel<T>), grid, dim3(256), 0, state().stream, in, out, g);
     return hip_ok(hipGetLastError(), "transpose launch") ? 0 : 2;
 }
 
@@ -1902,6 +1894,7 @@ static int transpose2d_dev(const T *in, T *out, int N, int M) {
 }
 
 constexpr int MAX_ND = 8;
+
 struct NdPerm {
     int nd;
     int out_dim[MAX_ND];    // extent of output axis i
