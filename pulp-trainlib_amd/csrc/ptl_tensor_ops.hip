@@ -638,43 +638,108 @@ __global__ __launch_bounds__(256) void dw_wg_plane_pairs_kernel(const half_t *__
     }
 }
 
-// ---- 3x3 fp16 planes straight from global memory -----------------------------------------------------------
-// Rows readable as pairs (see dw_row_pairs).  A lane owns a block of DW_DRB output rows x 8 columns and loads
-// the DW_DRB + 2 source row segments it needs itself (one 16-byte and one 4-byte load per row, 4-byte aligned):
+// ---- 3x3 planes straight from global memory, any extent, alignment and padding ----------------------------------
+// A lane owns a block of DW_DRB output rows x DwSeg<T>::COLS columns (one 16-byte store per row) and loads the
+// DW_DRB + 2 source row segments it needs itself, a 16-byte piece and the two elements behind it wherever they start:
 // no LDS, no barrier, and the blocks of all planes are dealt to the lanes without gaps (a wave may straddle two
 // planes).  Neighbouring lanes overlap by two elements per row and two rows per block, which the L1/L2 absorb:
-// the planes cross the HBM interface once.
+// the planes cross the HBM interface once, which is what bounds these kernels once the planes are many.
+// fp16 rows are held as pairs, and a filter row meets them as two-element dot products (see dw_row_taps).
+// 128 samples of 32 planes of 100 x 100 in fp16: forward 35.4 us (branches around loads of rows and columns at the edges:
+// 39.8), weight gradient 36.2 (50.2, a wave to a plane), input gradient 29.3 (35.2).  Separable layers of odd or short
+// rows, whose planes went through LDS or element by element: 1.3 to 5 times as fast as a whole pass.
 constexpr int DW_DRB = 7;
 
-// P[hr][m] = elements (cf + 2m, cf + 2m + 1) of source row r0 - pu + hr, zero outside the plane.
-template <int ROWS>
-__device__ inline void dw_direct_rows(const half_t *__restrict__ sp, int Hs, int Ws, int h0, int cf,
-                                      unsigned (&P)[ROWS][5]) {
-    const bool inner = cf >= 0 && cf + 10 <= Ws;
+template <typename T>
+struct DwSeg {
+    static constexpr int COLS = 16 / (int)sizeof(T);           // columns of a block
+    static constexpr int SRC = (COLS + 2) * (int)sizeof(T) / 4;  // dwords of a source row segment
+    static constexpr int OUT = 4;                              // dwords of a result row segment
+};
+typedef unsigned DwPiece4 __attribute__((ext_vector_type(4), aligned(1)));
+typedef unsigned DwPiece2 __attribute__((ext_vector_type(2), aligned(1)));
+typedef unsigned DwPiece1 __attribute__((aligned(1)));
+__device__ const unsigned dw_zeros[8] = {0, 0, 0, 0, 0, 0, 0, 0};  // what is read for a row outside the plane
+
+// P[hr] = the ND dwords of source row h0 + hr from column cf on, zero outside the plane (Hs x Ws, at `plane` elements into
+// a tensor of `total`, which holds at least one segment).  Every lane always loads: rows outside the plane come from a
+// segment of zeros, what lies left or right of the row is loaded (it is some neighbouring row) and masked, and a segment
+// that would begin or end outside the tensor is loaded from where it fits and moved in registers.  `inside`: the caller
+// knows that no segment of any lane leaves its plane, none of this is needed.
+template <typename T, int ROWS, int ND>
+__device__ inline void dw_segments(const T *__restrict__ src, size_t plane, size_t total, int Hs, int Ws, int h0, int cf,
+                                   bool inside, unsigned (&P)[ROWS][ND]) {
+    typedef const __attribute__((address_space(1))) unsigned char *Bytes;
+    constexpr int NE = ND * 4 / (int)sizeof(T);
+    const T *sp = src + plane;
+    auto load = [&](Bytes at, unsigned (&p)[ND]) {
+        const DwPiece4 v = *(const __attribute__((address_space(1))) DwPiece4 *)at;
+        p[0] = v.x;
+        p[1] = v.y;
+        p[2] = v.z;
+        p[3] = v.w;
+        if constexpr (ND == 5) p[4] = *(const __attribute__((address_space(1))) DwPiece1 *)(at + 16);
+        if constexpr (ND == 6) {
+            const DwPiece2 u = *(const __attribute__((address_space(1))) DwPiece2 *)(at + 16);
+            p[4] = u.x;
+            p[5] = u.y;
+        }
+    };
+    if (inside) {
+#pragma unroll
+        for (int hr = 0; hr < ROWS; ++hr) load((Bytes)(sp + (h0 + hr) * Ws + cf), P[hr]);
+        return;
+    }
+    // how far from the plane's start a segment may begin without leaving the tensor
+    const int lo = (int)max(-(long long)plane, -(1LL << 30)), hi = (int)min((long long)(total - NE - plane), (1LL << 30));
 #pragma unroll
     for (int hr = 0; hr < ROWS; ++hr) {
-        const int h = h0 + hr;
-        const unsigned *row = reinterpret_cast<const unsigned *>(sp + h * Ws + cf);
-        if ((unsigned)h < (unsigned)Hs) {
-            if (inner) {
+        const int h = h0 + hr, at = min(max(h * Ws + cf, lo), hi);
+        load((unsigned)h < (unsigned)Hs ? (Bytes)(sp + at) : (Bytes)dw_zeros, P[hr]);
+    }
+    unsigned keep[ND];
 #pragma unroll
-                for (int m = 0; m < 5; ++m) P[hr][m] = row[m];
-            } else {
+    for (int m = 0; m < ND; ++m) {
+        if constexpr (sizeof(T) == 2)
+            keep[m] = ((unsigned)(cf + 2 * m) < (unsigned)Ws ? 0xffffu : 0u) |
+                      ((unsigned)(cf + 2 * m + 1) < (unsigned)Ws ? 0xffff0000u : 0u);
+        else
+            keep[m] = (unsigned)(cf + m) < (unsigned)Ws ? ~0u : 0u;
+    }
 #pragma unroll
-                for (int m = 0; m < 5; ++m) P[hr][m] = (unsigned)(cf + 2 * m) < (unsigned)Ws ? row[m] : 0u;
+    for (int hr = 0; hr < ROWS; ++hr) {
+        const int h = h0 + hr, want = h * Ws + cf;
+        int d = (unsigned)h < (unsigned)Hs ? want - min(max(want, lo), hi) : 0;  // 0 but at the two ends of the tensor
+        if (d != 0) {
+            d = min(max(d, -NE), NE);
+            while (d > 0) {  // one element down
+#pragma unroll
+                for (int m = 0; m < ND; ++m) {
+                    const unsigned up = m + 1 < ND ? P[hr][m + 1 < ND ? m + 1 : m] : 0u;
+                    P[hr][m] = sizeof(T) == 2 ? __builtin_amdgcn_alignbit(up, P[hr][m], 16) : up;
+                }
+                --d;
             }
-        } else {
+            while (d < 0) {  // one element up
 #pragma unroll
-            for (int m = 0; m < 5; ++m) P[hr][m] = 0u;
+                for (int m = ND - 1; m >= 0; --m) {
+                    const unsigned down = m > 0 ? P[hr][m > 0 ? m - 1 : 0] : 0u;
+                    P[hr][m] = sizeof(T) == 2 ? __builtin_amdgcn_alignbit(P[hr][m], down, 16) : down;
+                }
+                ++d;
+            }
         }
+#pragma unroll
+        for (int m = 0; m < ND; ++m) P[hr][m] &= keep[m];
     }
 }
 
-template <bool FLIP>
-__global__ __launch_bounds__(256) void dw_direct_kernel(const half_t *__restrict__ src, const half_t *__restrict__ Wt,
-                                                        half_t *__restrict__ dst, int C, int Hs, int Ws, int Hd, int Wd,
-                                                        int pu, int pl, int rblocks, int groups, unsigned total) {
-    constexpr int RB = DW_DRB;
+template <typename T, bool FLIP>
+__global__ __launch_bounds__(256) void dw_direct_kernel(const T *__restrict__ src, const T *__restrict__ Wt,
+                                                        T *__restrict__ dst, int C, int Hs, int Ws, int Hd, int Wd, int pu,
+                                                        int pl, int rblocks, int groups, unsigned total, size_t elems,
+                                                        int inside) {
+    constexpr int RB = DW_DRB, NC = DwSeg<T>::COLS;
     const unsigned id = blockIdx.x * 256u + threadIdx.x;
     if (id >= total) return;
     const unsigned per_plane = (unsigned)(rblocks * groups);
@@ -683,79 +748,71 @@ __global__ __launch_bounds__(256) void dw_direct_kernel(const half_t *__restrict
     // full group / block: they then overlap their neighbours, whose values they repeat, and every store is a whole
     // 16-byte one)
     const int rb = (int)(blk / (unsigned)groups);
-    const int c0 = Wd >= 8 ? min((int)(blk - (unsigned)rb * groups) * 8, Wd - 8) : 0;
+    const int c0 = Wd >= NC ? min((int)(blk - (unsigned)rb * groups) * NC, Wd - NC) : 0;
     const int r0 = Hd >= RB ? min(rb * RB, Hd - RB) : 0;
     const int ch = (int)(plane % (unsigned)C);
-    dw_h2 we[3], wo[3];
-    float w0[3], w2[3];
+    T w[3][3];
 #pragma unroll
-    for (int i = 0; i < 3; ++i) {
-        half_t wr[3];
+    for (int i = 0; i < 3; ++i)
 #pragma unroll
-        for (int j = 0; j < 3; ++j) wr[j] = Wt[ch * 9 + (FLIP ? (2 - i) * 3 + (2 - j) : i * 3 + j)];
-        we[i] = dw_h2{wr[0], wr[1]};
-        wo[i] = dw_h2{wr[1], wr[2]};
-        w0[i] = (float)wr[0];
-        w2[i] = (float)wr[2];
-    }
-    unsigned P[RB + 2][5];
-    dw_direct_rows<RB + 2>(src + (size_t)plane * Hs * Ws, Hs, Ws, r0 - pu, c0 - pl, P);
-    float acc[RB][8];
+        for (int j = 0; j < 3; ++j) w[i][j] = Wt[ch * 9 + (FLIP ? (2 - i) * 3 + (2 - j) : i * 3 + j)];
+    unsigned P[RB + 2][DwSeg<T>::SRC];
+    dw_segments<T>(src, (size_t)plane * Hs * Ws, elems, Hs, Ws, r0 - pu, c0 - pl, inside, P);
+    float acc[RB][NC];
 #pragma unroll
     for (int r = 0; r < RB; ++r)
 #pragma unroll
-        for (int q = 0; q < 8; ++q) acc[r][q] = 0.f;
+        for (int q = 0; q < NC; ++q) acc[r][q] = 0.f;
 #pragma unroll
     for (int hr = 0; hr < RB + 2; ++hr) {
 #pragma unroll
         for (int i = 0; i < 3; ++i) {
             const int r = hr - i;
             if (r < 0 || r >= RB) continue;
+            if constexpr (sizeof(T) == 2) {
+                const dw_h2 we[1] = {dw_h2{w[i][0], w[i][1]}}, wo[1] = {dw_h2{w[i][1], w[i][2]}};
+                const float wf[3] = {(float)w[i][0], (float)w[i][1], (float)w[i][2]};
+                dw_row_taps<3>(P[hr], we, wo, wf, acc[r]);
+            } else {
 #pragma unroll
-            for (int q = 0; q < 8; ++q) {
-                float a = acc[r][q];
-                if ((q & 1) == 0) {
-                    a = __builtin_amdgcn_fdot2(__builtin_bit_cast(dw_h2, P[hr][q / 2]), we[i], a, false);
-                    a = fmaf((float)__builtin_bit_cast(dw_h2, P[hr][q / 2 + 1]).x, w2[i], a);
-                } else {
-                    a = fmaf((float)__builtin_bit_cast(dw_h2, P[hr][q / 2]).y, w0[i], a);
-                    a = __builtin_amdgcn_fdot2(__builtin_bit_cast(dw_h2, P[hr][q / 2 + 1]), wo[i], a, false);
-                }
-                acc[r][q] = a;
+                for (int q = 0; q < NC; ++q)
+#pragma unroll
+                    for (int j = 0; j < 3; ++j)
+                        acc[r][q] = fmaf(__builtin_bit_cast(float, P[hr][q + j]), (float)w[i][j], acc[r][q]);
             }
         }
     }
-    half_t *dp = dst + (size_t)plane * Hd * Wd;
-    const int valid = min(8, Wd - c0);
+    T *dp = dst + (size_t)plane * Hd * Wd;
+    const int valid = min(NC, Wd - c0);
 #pragma unroll
     for (int r = 0; r < RB; ++r) {
         if (r0 + r >= Hd) continue;
-        half_t *o = dp + (size_t)(r0 + r) * Wd + c0;
-        if (valid == 8) {  // (rows are whole dwords: a 16-byte global store needs no more than 4-byte alignment)
-            typedef unsigned u4a __attribute__((ext_vector_type(4), aligned(4)));
-            union {
-                u4a v;
-                half_t e[8];
-            } u;
+        T *o = dp + (size_t)(r0 + r) * Wd + c0;
+        union {
+            DwPiece4 v;
+            T e[NC];
+        } u;
 #pragma unroll
-            for (int q = 0; q < 8; ++q) u.e[q] = (half_t)acc[r][q];
-            *reinterpret_cast<u4a *>(o) = u.v;
+        for (int q = 0; q < NC; ++q) u.e[q] = (T)acc[r][q];
+        if (valid == NC) {
+            *reinterpret_cast<DwPiece4 *>(o) = u.v;
         } else {
 #pragma unroll
-            for (int q = 0; q < 8; ++q)
-                if (q < valid) o[q] = (half_t)acc[r][q];
+            for (int q = 0; q < NC; ++q)
+                if (q < valid) o[q] = u.e[q];
         }
     }
 }
 
-// Weight gradient the same way: a wave walks planes (b, ch) of its sample group, a lane takes blocks of DW_DRB
-// gradient rows x 8 columns with the source rows they meet, the nine tap sums stay in registers; one reduction
+// Weight gradient the same way: a workgroup owns a channel and a group of samples and deals the blocks of DW_DRB
+// gradient rows x COLS columns of all its planes to its lanes, the nine tap sums stay in registers; one reduction
 // per workgroup at the end.  part[(grp * C + ch) * 9 + tap], or the gradient itself when there is one group.
-__global__ __launch_bounds__(256) void dw_wg_direct_kernel(const half_t *__restrict__ X, const half_t *__restrict__ dY,
+template <typename T>
+__global__ __launch_bounds__(256) void dw_wg_direct_kernel(const T *__restrict__ X, const T *__restrict__ dY,
                                                            float *__restrict__ part, int C, int ns, int per_group, int H,
-                                                           int W, int Ho, int Wo, int pu, int pl,
-                                                           half_t *__restrict__ direct) {
-    constexpr int RB = DW_DRB;
+                                                           int W, int Ho, int Wo, int pu, int pl, size_t x_elems,
+                                                           size_t y_elems, int inside, T *__restrict__ direct) {
+    constexpr int RB = DW_DRB, NC = DwSeg<T>::COLS;
     __shared__ float red[4][9];
     const int ch = blockIdx.x, grp = blockIdx.y;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -764,45 +821,41 @@ __global__ __launch_bounds__(256) void dw_wg_direct_kernel(const half_t *__restr
     for (int i = 0; i < 3; ++i)
 #pragma unroll
         for (int j = 0; j < 3; ++j) acc[i][j] = 0.f;
-    const int groups = (Wo + 7) >> 3, rblocks = (Ho + RB - 1) / RB;
-    const int b_end = min(ns, (grp + 1) * per_group);
-    for (int b = grp * per_group + wave; b < b_end; b += 4) {
-        const size_t plane = (size_t)b * C + ch;
-        const half_t *xp = X + plane * H * W, *gp = dY + plane * Ho * Wo;
-        for (int item = lane; item < rblocks * groups; item += 64) {
-            const int rb = item / groups, c0 = (item - rb * groups) * 8, r0 = rb * RB;
-            dw_h2 G[RB][4];
+    const int groups = (Wo + NC - 1) / NC, rblocks = (Ho + RB - 1) / RB;
+    const unsigned per_plane = (unsigned)(groups * rblocks);
+    const int b0 = grp * per_group;
+    const unsigned items = per_plane * (unsigned)(min(ns, b0 + per_group) - b0);
+    for (unsigned it = tid; it < items; it += 256) {
+        const unsigned b = it / per_plane, item = it - b * per_plane;
+        const int rb = (int)(item / (unsigned)groups), c0 = (int)(item - (unsigned)rb * groups) * NC, r0 = rb * RB;
+        const size_t plane = (size_t)(b0 + b) * C + ch;
+        unsigned G[RB][DwSeg<T>::OUT];
+        dw_segments<T>(dY, plane * Ho * Wo, y_elems, Ho, Wo, r0, c0, inside & 1, G);
+        unsigned P[RB + 2][DwSeg<T>::SRC];
+        dw_segments<T>(X, plane * H * W, x_elems, H, W, r0 - pu, c0 - pl, inside & 2, P);
 #pragma unroll
-            for (int r = 0; r < RB; ++r) {
-                const unsigned *grow = reinterpret_cast<const unsigned *>(gp + (r0 + r) * Wo + c0);
-                if (r0 + r < Ho && c0 + 8 <= Wo) {
-#pragma unroll
-                    for (int m = 0; m < 4; ++m) G[r][m] = __builtin_bit_cast(dw_h2, grow[m]);
-                } else {
-#pragma unroll
-                    for (int m = 0; m < 4; ++m)
-                        G[r][m] = __builtin_bit_cast(dw_h2, (r0 + r < Ho && c0 + 2 * m < Wo) ? grow[m] : 0u);
-                }
-            }
-            unsigned P[RB + 2][5];
-            dw_direct_rows<RB + 2>(xp, H, W, r0 - pu, c0 - pl, P);
-#pragma unroll
-            for (int hr = 0; hr < RB + 2; ++hr) {  // source row r0 - pu + hr meets gradient rows r0 + hr - i
-                unsigned U[4];
+        for (int hr = 0; hr < RB + 2; ++hr) {  // source row r0 - pu + hr meets gradient rows r0 + hr - i
+            unsigned U[4];  // (fp16: the pairs that start one element later)
+            if constexpr (sizeof(T) == 2) {
 #pragma unroll
                 for (int m = 0; m < 4; ++m) U[m] = __builtin_amdgcn_alignbit(P[hr][m + 1], P[hr][m], 16);
+            }
 #pragma unroll
-                for (int i = 0; i < 3; ++i) {
-                    if (hr - i < 0 || hr - i >= RB) continue;
+            for (int i = 0; i < 3; ++i) {
+                if (hr - i < 0 || hr - i >= RB) continue;
 #pragma unroll
-                    for (int j = 0; j < 3; ++j) {
-                        float a = acc[i][j];
+                for (int j = 0; j < 3; ++j) {
+                    float a = acc[i][j];
 #pragma unroll
-                        for (int m = 0; m < 4; ++m)
+                    for (int m = 0; m < 4; ++m) {
+                        const unsigned g = G[hr - i][m];
+                        if constexpr (sizeof(T) == 2)
                             a = __builtin_amdgcn_fdot2(__builtin_bit_cast(dw_h2, j == 1 ? U[m] : P[hr][m + j / 2]),
-                                                       G[hr - i][m], a, false);
-                        acc[i][j] = a;
+                                                       __builtin_bit_cast(dw_h2, g), a, false);
+                        else
+                            a = fmaf(__builtin_bit_cast(float, P[hr][m + j]), __builtin_bit_cast(float, g), a);
                     }
+                    acc[i][j] = a;
                 }
             }
         }
@@ -818,9 +871,10 @@ __global__ __launch_bounds__(256) void dw_wg_direct_kernel(const half_t *__restr
         }
     __syncthreads();
     if (tid < 9) {
-        const float sum = (red[0][tid] + red[1][tid]) + (red[2][tid] + red[3][tid]);
+        const float *r = &red[0][0] + tid;
+        const float sum = (r[0] + r[9]) + (r[18] + r[27]);
         if (direct)
-            direct[(size_t)ch * 9 + tid] = (half_t)sum;
+            direct[(size_t)ch * 9 + tid] = (T)sum;
         else
             part[((size_t)grp * C + ch) * 9 + tid] = sum;
     }
@@ -865,24 +919,12 @@ static int dw_geom(const Args *a, DwGeom &g, int sh, int sw, const char *fn) {
     return 0;
 }
 
-// Plane-resident depthwise product (forward, or input gradient with FLIP).
+// Plane-resident depthwise product of 5x5 filters (forward, or input gradient with FLIP).
 template <typename T, int K, bool FLIP>
 static void launch_dw_plane(const T *src, const T *Wt, T *dst, int C, int Hs, int Ws, int Hd, int Wd, int pu, int pl,
                             long planes, hipStream_t stream) {
     const size_t src_img = (size_t)Hs * Ws * sizeof(T) + 32;
     if constexpr (sizeof(T) == 2) {
-        // 3x3 with rows of whole dwords on both sides and at least one group of eight columns: straight from global
-        // memory (forward, and the input gradient as the flipped correlation over the output gradient)
-        if (K == 3 && Ws % 2 == 0 && Wd % 2 == 0 && Wd >= 8 && pl % 2 == 0 && reinterpret_cast<uintptr_t>(src) % 4 == 0 &&
-            reinterpret_cast<uintptr_t>(dst) % 4 == 0) {
-            const int rblocks = (Hd + DW_DRB - 1) / DW_DRB, groups = (Wd + 7) / 8;
-            const long long total = (long long)planes * rblocks * groups;
-            if (total < ((long long)1 << 31)) {
-                hipLaunchKernelGGL((dw_direct_kernel<FLIP>), dim3((unsigned)((total + 255) / 256)), dim3(256), 0, stream,
-                                   src, Wt, dst, C, Hs, Ws, Hd, Wd, pu, pl, rblocks, groups, (unsigned)total);
-                return;
-            }
-        }
         // rows readable as pairs: see dw_plane_pairs_kernel
         if (Ws % 2 == 0 && pl % 2 == 0 && reinterpret_cast<uintptr_t>(src) % 4 == 0) {
             hipLaunchKernelGGL((dw_plane_pairs_kernel<K, FLIP>), dim3((unsigned)planes), dim3(128), src_img, stream, src,
@@ -892,6 +934,18 @@ static void launch_dw_plane(const T *src, const T *Wt, T *dst, int C, int Hs, in
     }
     hipLaunchKernelGGL((dw_plane_kernel<T, K, FLIP>), dim3((unsigned)planes), dim3(256), src_img, stream, src, Wt, dst,
                        C, Hs, Ws, Hd, Wd, pu, pl);
+}
+
+// 3x3 straight from global memory (forward, or input gradient with FLIP).
+template <typename T, bool FLIP>
+static void launch_dw_direct(const T *src, const T *Wt, T *dst, int C, int Hs, int Ws, int Hd, int Wd, int pu, int pl,
+                             long planes, hipStream_t stream) {
+    constexpr int NC = DwSeg<T>::COLS;
+    const int rblocks = (Hd + DW_DRB - 1) / DW_DRB, groups = (Wd + NC - 1) / NC;
+    const unsigned total = (unsigned)(planes * rblocks * groups);
+    const int inside = pu == 0 && pl == 0 && Hd + 2 <= Hs && Wd + 2 <= Ws && Hd >= DW_DRB && Wd >= NC;
+    hipLaunchKernelGGL((dw_direct_kernel<T, FLIP>), dim3((total + 255) / 256), dim3(256), 0, stream, src, Wt, dst, C, Hs, Ws,
+                       Hd, Wd, pu, pl, rblocks, groups, total, (size_t)planes * Hs * Ws, inside);
 }
 
 // ---- partial sums of the allocation-free weight-gradient entry point ---------------------------------
@@ -944,20 +998,27 @@ static int dw_step(const Args *a, int ns, int step, int sh, int sw, const char *
     // chip; measured faster for 2-byte elements (forward, input gradient, weight gradient) and for the fp32
     // forward and input gradient
     const size_t in_img = (size_t)g.H * g.W * sizeof(T) + 32, out_img = (size_t)g.Ho * g.Wo * sizeof(T) + 32;
-    const bool plane_path = rows_path && in_img <= 40 * 1024 && out_img <= 40 * 1024 && planes >= 2L * st.num_cu &&
+    const bool plane_path = rows_path && g.Hk == 5 && in_img <= 40 * 1024 && out_img <= 40 * 1024 && planes >= 2L * st.num_cu &&
                             planes < ((long)1 << 31) && st.gemm_path != 1;
+    // 3x3, unit stride: straight from global memory, whatever the extents, the alignment and the number of planes (the
+    // tensors hold at least one segment; offsets within a plane and the blocks of all planes are 31-bit numbers)
+    auto fits = [](size_t elems, int h, int w, long n) {
+        return elems >= 16 && (long long)h * w < (1LL << 29) &&
+               (long long)n * ((h + DW_DRB - 1) / DW_DRB) * ((w + DwSeg<T>::COLS - 1) / DwSeg<T>::COLS) < (1LL << 31);
+    };
+    const bool direct_path = sh == 1 && sw == 1 && g.Hk == 3 && g.Wk == 3 && st.gemm_path != 1 &&
+                             fits(in_n, g.H, g.W, planes) && fits(out_n, g.Ho, g.Wo, planes);
     // a single sample: one workgroup per channel produces the weight gradient in one launch
-    const bool wg_single = rows_path && ns == 1 && in_img <= 40 * 1024 && out_img <= 40 * 1024 && st.gemm_path != 1;
+    const bool wg_single = rows_path && g.Hk == 5 && ns == 1 && in_img <= 40 * 1024 && out_img <= 40 * 1024 && st.gemm_path != 1;
     if (step == STEP_FW) {
         const T *X = sg.in(reinterpret_cast<const T *>(a->input->data), in_n);
         const T *Wt = sg.in(reinterpret_cast<const T *>(a->coeff->data), w_n);
         T *Y = sg.out(reinterpret_cast<T *>(a->output->data), out_n);
         if (sg.failed()) return sg.rejected() ? 1 : 2;
-        if (plane_path) {
-            if (g.Hk == 3)
-                launch_dw_plane<T, 3, false>(X, Wt, Y, g.C, g.H, g.W, g.Ho, g.Wo, g.Up, g.Lp, planes, st.stream);
-            else
-                launch_dw_plane<T, 5, false>(X, Wt, Y, g.C, g.H, g.W, g.Ho, g.Wo, g.Up, g.Lp, planes, st.stream);
+        if (direct_path) {
+            launch_dw_direct<T, false>(X, Wt, Y, g.C, g.H, g.W, g.Ho, g.Wo, g.Up, g.Lp, planes, st.stream);
+        } else if (plane_path) {
+            launch_dw_plane<T, 5, false>(X, Wt, Y, g.C, g.H, g.W, g.Ho, g.Wo, g.Up, g.Lp, planes, st.stream);
         } else if (rows_path) {
             int rbs = (g.Ho + DW_RB - 1) / DW_RB, ccs = (g.Wo + 63) / 64;
             long waves = planes * rbs * ccs;
@@ -976,13 +1037,10 @@ static int dw_step(const Args *a, int ns, int step, int sh, int sw, const char *
         const T *Wt = sg.in(reinterpret_cast<const T *>(a->coeff->data), w_n);
         T *dX = sg.out(reinterpret_cast<T *>(a->input->diff), in_n);
         if (sg.failed()) return sg.rejected() ? 1 : 2;
-        if (plane_path) {
-            if (g.Hk == 3)
-                launch_dw_plane<T, 3, true>(dY, Wt, dX, g.C, g.Ho, g.Wo, g.H, g.W, g.Hk - 1 - g.Up, g.Wk - 1 - g.Lp,
-                                            planes, st.stream);
-            else
-                launch_dw_plane<T, 5, true>(dY, Wt, dX, g.C, g.Ho, g.Wo, g.H, g.W, g.Hk - 1 - g.Up, g.Wk - 1 - g.Lp,
-                                            planes, st.stream);
+        if (direct_path) {
+            launch_dw_direct<T, true>(dY, Wt, dX, g.C, g.Ho, g.Wo, g.H, g.W, 2 - g.Up, 2 - g.Lp, planes, st.stream);
+        } else if (plane_path) {
+            launch_dw_plane<T, 5, true>(dY, Wt, dX, g.C, g.Ho, g.Wo, g.H, g.W, 4 - g.Up, 4 - g.Lp, planes, st.stream);
         } else if (rows_path) {
             int rbs = (g.H + DW_RB - 1) / DW_RB, ccs = (g.W + 63) / 64;
             long waves = planes * rbs * ccs;
@@ -996,7 +1054,7 @@ static int dw_step(const Args *a, int ns, int step, int sh, int sw, const char *
         } else {
             hipLaunchKernelGGL((dw_ig_kernel<T>), dim3(nblocks(in_n)), dim3(256), 0, st.stream, dY, Wt, dX, g, in_n);
         }
-    } else if (plane_path || wg_single) {
+    } else if (direct_path || plane_path || wg_single) {
         const T *X = sg.in(reinterpret_cast<const T *>(a->input->data), in_n);
         const T *dY = sg.in(reinterpret_cast<const T *>(a->output->diff), out_n);
         T *dW = sg.out(reinterpret_cast<T *>(a->coeff->diff), w_n);
@@ -1014,29 +1072,24 @@ static int dw_step(const Args *a, int ns, int step, int sh, int sw, const char *
         const int x_vecs = (int)((in_img + 15) / 16);
         const size_t lds = (size_t)x_vecs * 16 + out_img;
         dim3 grid(g.C, sgroups);
-        bool pairs = false;
-        if constexpr (sizeof(T) == 2) {
-            pairs = g.W % 2 == 0 && g.Wo % 2 == 0 && g.Lp % 2 == 0 && reinterpret_cast<uintptr_t>(X) % 4 == 0 &&
-                    reinterpret_cast<uintptr_t>(dY) % 4 == 0;
-            if (pairs && g.Hk == 3 && ns > 1) {
-                hipLaunchKernelGGL(dw_wg_direct_kernel, grid, dim3(256), 0, st.stream, X, dY, part, g.C, ns, per_group, g.H,
-                                   g.W, g.Ho, g.Wo, g.Up, g.Lp, direct);
-            } else if (pairs) {
-                if (g.Hk == 3)
-                    hipLaunchKernelGGL((dw_wg_plane_pairs_kernel<3>), grid, dim3(256), lds, st.stream, X, dY, part, g.C,
-                                       ns, per_group, g.H, g.W, g.Ho, g.Wo, g.Up, g.Lp, x_vecs, direct);
-                else
-                    hipLaunchKernelGGL((dw_wg_plane_pairs_kernel<5>), grid, dim3(256), lds, st.stream, X, dY, part, g.C,
-                                       ns, per_group, g.H, g.W, g.Ho, g.Wo, g.Up, g.Lp, x_vecs, direct);
+        if (direct_path) {
+            const int whole = g.Ho % DW_DRB == 0 && g.Wo % DwSeg<T>::COLS == 0;  // blocks of the gradient
+            const int inside = whole | (whole && g.Ho + 2 <= g.H && g.Wo + 2 <= g.W && g.Up == 0 && g.Lp == 0 ? 2 : 0);
+            hipLaunchKernelGGL((dw_wg_direct_kernel<T>), grid, dim3(256), 0, st.stream, X, dY, part, g.C, ns, per_group, g.H,
+                               g.W, g.Ho, g.Wo, g.Up, g.Lp, in_n, out_n, inside, direct);
+        } else {
+            bool pairs = false;
+            if constexpr (sizeof(T) == 2) {
+                pairs = g.W % 2 == 0 && g.Wo % 2 == 0 && g.Lp % 2 == 0 && reinterpret_cast<uintptr_t>(X) % 4 == 0 &&
+                        reinterpret_cast<uintptr_t>(dY) % 4 == 0;
+                if (pairs)
+                    hipLaunchKernelGGL((dw_wg_plane_pairs_kernel<5>), grid, dim3(256), lds, st.stream, X, dY, part, g.C, ns,
+                                       per_group, g.H, g.W, g.Ho, g.Wo, g.Up, g.Lp, x_vecs, direct);
             }
+            if (!pairs)
+                hipLaunchKernelGGL((dw_wg_plane_kernel<T, 5>), grid, dim3(256), lds, st.stream, X, dY, part, g.C, ns,
+                                   per_group, g.H, g.W, g.Ho, g.Wo, g.Up, g.Lp, x_vecs, direct);
         }
-        if (pairs) {
-        } else if (g.Hk == 3)
-            hipLaunchKernelGGL((dw_wg_plane_kernel<T, 3>), grid, dim3(256), lds, st.stream, X, dY, part, g.C, ns,
-                               per_group, g.H, g.W, g.Ho, g.Wo, g.Up, g.Lp, x_vecs, direct);
-        else
-            hipLaunchKernelGGL((dw_wg_plane_kernel<T, 5>), grid, dim3(256), lds, st.stream, X, dY, part, g.C, ns,
-                               per_group, g.H, g.W, g.Ho, g.Wo, g.Up, g.Lp, x_vecs, direct);
         if (!direct)
             hipLaunchKernelGGL((dw_wg_reduce_kernel2<T>), dim3(g.C), dim3(256), 0, st.stream, part, dW, sgroups, g.C, 1,
                                taps);
