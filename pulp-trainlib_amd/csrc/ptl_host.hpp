@@ -20,7 +20,8 @@ struct StageBlock;  // pinned host memory and device memory of one size, from a 
 // finish() synchronises only when something was staged.
 // Small host tensors share one pinned block: the CPU copies them into it as they are mapped, failed() - which every
 // caller asks after its mappings and before its launches - enqueues one kernel that fetches all of them, and finish()
-// one that writes all results back.
+// one that writes all results back.  Larger ones have a pinned block each and move part by part, the CPU's copies beside
+// the bus's.
 class Stager {
    public:
     // device_only: host pointers are rejected instead of staged (callers that may not allocate)
@@ -58,8 +59,9 @@ class Stager {
         size_t bytes;
         bool copy_out;
         bool copied_in;
-        bool in_block;   // dev lies in block_
-        bool pending;    // in the pinned half of the block, to be fetched
+        bool own;           // block is this tensor's alone
+        bool pending;       // in the pinned half of the shared block, to be fetched
+        StageBlock *block;  // dev lies in it; NULL: a buffer of its own
     };
     void *map(const void *p, size_t bytes, bool copy_in, bool copy_out);
     bool launch_block_copy(bool in);
@@ -69,7 +71,7 @@ class Stager {
     Stager *root_;
     std::vector<size_t> marked_;  // items of root_ that this step is the first to write
     StageBlock *block_ = nullptr;
-    size_t block_used_ = 0;
+    size_t block_used_ = 0, own_bytes_ = 0;
     bool pending_ = false;
     bool failed_ = false;
     bool finished_ = false;

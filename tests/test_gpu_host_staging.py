@@ -57,3 +57,19 @@ def test_a_rejected_step_returns_nothing_and_the_other_still_runs(pkg, gpu):
     ref = torch.nn.grad.conv2d_input((1, Ci, H, H), torch.from_numpy(w).double(), torch.from_numpy(dy).double()[None],
                                      stride=s, padding=1)[0]
     assert np.all(dw == 3) and hp.rel_l2(dx, ref.numpy()) <= 1e-4
+
+
+# (two parts and an odd end; the largest tensor with a block of its own: 32 MiB; one row beyond)
+@pytest.mark.parametrize("n_in,n_out", [(525, 1001), (2896, 2896), (2897, 2897)])
+def test_large_host_tensors_travel_in_parts(pkg, gpu, n_in, n_out):
+    res = []
+    for place in (lambda a: a.copy(), lambda a: torch.from_numpy(a).to(DEV)):
+        t = [place(a) for a in (hp.uniform(1, (n_in,)), np.zeros(n_in, np.float32), hp.uniform(2, (n_out, n_in)),
+                                np.full((n_out, n_in), 3, np.float32), np.zeros(n_out, np.float32), hp.uniform(3, (n_out,)))]
+        a, keep = hp.linear_args(pkg, *t, n_in, n_out)
+        pkg.call("pulp_linear_fp32_fw_cl", a)
+        pkg.call("pulp_linear_fp32_bw_cl", a)
+        assert gpu.ptl_sync() == 0
+        res.append([v if isinstance(v, np.ndarray) else v.cpu().numpy() for v in t])
+    for h, d in zip(*res):
+        assert np.array_equal(h, d)
