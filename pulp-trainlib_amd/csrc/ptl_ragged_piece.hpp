@@ -1,0 +1,58 @@
+// Which bytes a workgroup of the kernel for any size and alignment (ptl_ragged.inc) reads of a matrix that is contiguous
+// along k: plain C++ for the host and the device, so that a test can walk every address on the CPU.
+#pragma once
+
+#ifdef __HIP__
+#define PTL_BOTH __host__ __device__
+#else
+#define PTL_BOTH
+#endif
+
+namespace ptl {
+
+// A thread's piece of VEC elements at position `pos` (0 .. 7) of a slab, where the last slab of a run has `left` elements.
+// Every load has its 16 bytes inside the run, which holds at least one piece:
+//   * a piece that reaches over the end of the run is read so that it ENDS there and shifted down by `cut`;
+//   * one that does not exist is read from the last slab's first k - or, where that slab itself is shorter than a piece,
+//     from the run's last one (`gap`) - and replaced by zeros.
+struct RagPiece {
+    int tail;       // elements from the piece's first k on in the last slab
+    unsigned gap;   // bytes that the last slab lacks of one piece: in it every thread reads this much earlier, ...
+    unsigned back;  // ... and this one as much again
+    unsigned cut;   // bytes
+};
+template <int VEC>
+PTL_BOTH inline RagPiece rag_piece(int left, int pos) {
+    constexpr unsigned ES = 16 / VEC;
+    RagPiece r;
+    r.tail = left - pos * VEC;
+    r.gap = left < VEC ? (unsigned)(VEC - left) * ES : 0u;
+    r.cut = r.tail > 0 && r.tail < VEC ? (unsigned)(VEC - r.tail) * ES : 0u;
+    r.back = r.tail <= 0 ? (unsigned)pos * 16u : r.cut - (r.cut ? r.gap : 0u);
+    return r;
+}
+// Bytes before the slab's start that the offset `rag_piece_off` counts from.  want: ~0, or 0 where nothing is needed any
+// more and every lane reads the same piece.
+PTL_BOTH inline unsigned rag_piece_back(unsigned gap, unsigned back, bool last, unsigned want) { return last ? gap + (back & want) : 0u; }
+// Bytes of the piece from the start of row r0 of the slab; rows beyond the end repeat the last one.
+PTL_BOTH inline unsigned rag_piece_off(int row, int r0, int rows, unsigned row_b, int pos) {
+    return ((unsigned)(row < rows ? row : rows - 1) - (unsigned)r0) * row_b + (unsigned)pos * 16u;
+}
+
+// The slabs of a workgroup in order: position in their run, and the run.  A workgroup asks for more slabs than it has, so
+// that every step waits for the same number of loads: behind the last one the walk stands still and `want` is 0.
+struct RagWalk {
+    int pos, run, per_run, left;
+    PTL_BOTH inline bool last() const { return pos + 1 == per_run; }
+    PTL_BOTH inline unsigned want() const { return left > 0 ? ~0u : 0u; }
+    // On to the next slab, if there is one.
+    PTL_BOTH inline bool next() {
+        if (--left <= 0) return false;
+        const bool end = last();
+        pos = end ? 0 : pos + 1;
+        run += end ? 1 : 0;
+        return true;
+    }
+};
+
+}  // namespace ptl
