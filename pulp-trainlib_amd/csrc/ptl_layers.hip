@@ -58,14 +58,16 @@ __global__ __launch_bounds__(256) void zero_kernel(T *__restrict__ dst, size_t n
 
 // out[b][c][pix] += bias[c] (CHW) or out[b][pix][c] += bias[c] (HWC: inner = 1): a thread adds to one 16-byte piece, the
 // elements of which start at channel and position of the first and walk on (element by element and with a 64-bit
-// division each it took 16 us for 7.6 M elements in fp16, 4.9 this way).
+// division each it took 16 us for 7.6 M elements in fp16, 4.9 this way).  `total` <= 2^30 elements, the first of which has
+// channel c0 and position p0 < 2^31: every index fits 32 bits.
+constexpr size_t BIAS_ADD_MOST = (size_t)1 << 30;
 template <typename T>
 __global__ __launch_bounds__(256) void bias_add_kernel(T *__restrict__ out, const T *__restrict__ bias, unsigned total,
-                                                       unsigned C, unsigned inner) {
+                                                       unsigned C, unsigned inner, unsigned c0, unsigned p0) {
     constexpr unsigned V = 16 / sizeof(T);
     const unsigned i0 = (blockIdx.x * 256 + threadIdx.x) * V;
     if (i0 >= total) return;
-    unsigned q = i0 / inner, p = i0 - q * inner, c = q % C;
+    unsigned q = (p0 + i0) / inner, p = p0 + i0 - q * inner, c = (c0 + q) % C;
     T v[V];
     const bool whole = i0 + V <= total;
     if (whole) __builtin_memcpy(v, out + i0, 16);
@@ -184,12 +186,15 @@ static int bias_grad(const T *dy, T *db, int ns, int C, int pix, int hwc) {
     return hip_ok(hipGetLastError(), "bias grad launch") ? 0 : 2;
 }
 
-// (the piece index of a tensor below 2^31 elements fits 32 bits)
+// (a matrix may have up to 2^62 elements: one launch for each 2^30 of them)
 template <typename T>
 static void launch_bias_add(T *out, const T *bias, size_t total, int C, int inner) {
     constexpr size_t V = 16 / sizeof(T);
-    hipLaunchKernelGGL((bias_add_kernel<T>), dim3((unsigned)((total + 256 * V - 1) / (256 * V))), dim3(256), 0, state().stream, out,
-                       bias, (unsigned)total, (unsigned)C, (unsigned)inner);
+    for (size_t at = 0; at < total; at += BIAS_ADD_MOST) {
+        const size_t n = total - at < BIAS_ADD_MOST ? total - at : BIAS_ADD_MOST, q = at / inner;
+        hipLaunchKernelGGL((bias_add_kernel<T>), dim3((unsigned)((n + 256 * V - 1) / (256 * V))), dim3(256), 0, state().stream,
+                           out + at, bias, (unsigned)n, (unsigned)C, (unsigned)inner, (unsigned)(q % C), (unsigned)(at - q * inner));
+    }
 }
 
 static inline unsigned blocks_for(size_t n) { return (unsigned)((n + 255) / 256); }

@@ -146,6 +146,24 @@ def test_mm_bias_add_transposed(pkg, gpu, dt, H, W):
         assert np.array_equal(host(g), bias_sum(mat, bias, t))
 
 
+# 2^32 - 1 elements, and rows that lie across 2^30, 2^31 and 2^32 of them; small whole numbers: exact
+@pytest.mark.gpu
+@pytest.mark.parametrize("H,W", [(65535, 65537), (65537, 65543), (3, 1500000007)])
+@pytest.mark.parametrize("t", [0, 1])
+def test_mm_bias_add_transposed_of_more_elements_than_32_bits_count(pkg, gpu, H, W, t):
+    mat = torch.full((H, W), 1, dtype=torch.float16, device="cuda:0")
+    bias = (torch.arange(H if t else W, device="cuda:0") % 97).to(torch.float16)
+    a = pkg.MMBiasAddArgs()
+    a.mat, a.bias, a.H, a.W, a.t = mat.data_ptr(), bias.data_ptr(), H, W, t
+    pkg.call("mm_bias_add_transposed_fp16", a)
+    assert gpu.ptl_sync() == 0
+    want = bias + 1
+    step = max(1, (1 << 29) // W)
+    for r in range(0, H, step):
+        assert bool((mat[r:r + step] == (want[r:r + step].view(-1, 1) if t else want)).all()), (r, H, W, t)
+
+
+
 @pytest.mark.parametrize("dt", ["fp32", "fp16"])
 @pytest.mark.parametrize("N,M,K", [(32, 1024, 144), (7, 5, 3), (130, 70, 515)])
 def test_mm_M_and_manager_bias_epilogue(pkg, orc, gpu, dt, N, M, K):
