@@ -804,6 +804,19 @@ static unsigned outer_blocks(int N, int M, int V) {
     return (unsigned)(((size_t)((N + 3) / 4) * ((M + V - 1) / V) + GV_NT - 1) / GV_NT);
 }
 
+// (a launch takes the rows whose units are 31-bit numbers: all of them below 2^35 outputs of 4 bytes)
+template <typename T, int V>
+static int outer(const T *a, const T *b, T *C, int N, int M) {
+    const RagDiv per_row = rag_div((M + V - 1) / V);
+    const long long most = ((1ll << 31) - GV_NT) / per_row.d * 4;
+    for (long long n = 0; n < N; n += most) {
+        const int rows = (int)(N - n < most ? N - n : most);
+        hipLaunchKernelGGL((outer_kernel<T, V>), dim3(outer_blocks(rows, M, V)), dim3(GV_NT), 0, state().stream, a + n, b,
+                           C + (size_t)n * M, rows, M, per_row);
+    }
+    return hip_ok(hipGetLastError(), "outer launch") ? 0 : 2;
+}
+
 template <typename T, int V>
 static int linear_one_bw_v(const T *x, const T *W, const T *dy, T *dW, T *dx, T *db, int in, int out) {
     const int cols = (in + 4 * V - 1) / (4 * V);
@@ -831,14 +844,7 @@ int mm_dispatch(const T *A, const T *B, T *C, int N, int M, int K, int trans_B, 
     if (N <= 0 || M <= 0 || K <= 0) return 0;  // K == 0 leaves C untouched, as mm() does
     State &st = state();
     constexpr int VEC = Traits<T>::VEC;
-    if (K == 1 && !bias) {
-        if (M >= VEC)
-            hipLaunchKernelGGL((outer_kernel<T, VEC>), dim3(outer_blocks(N, M, VEC)), dim3(GV_NT), 0, st.stream, A, B, C, N, M,
-                               rag_div((M + VEC - 1) / VEC));
-        else
-            hipLaunchKernelGGL((outer_kernel<T, 1>), dim3(outer_blocks(N, M, 1)), dim3(GV_NT), 0, st.stream, A, B, C, N, M, rag_div(M));
-        return hip_ok(hipGetLastError(), "outer launch") ? 0 : 2;
-    }
+    if (K == 1 && !bias) return M >= VEC ? outer<T, VEC>(A, B, C, N, M) : outer<T, 1>(A, B, C, N, M);
     if (M == 1 && !bias) return gemv_rowdot<T>(A, B, C, nullptr, N, K);  // B is K x 1 or 1 x K: the same vector
     if (N == 1 && trans_B) return gemv_rowdot<T>(B, A, C, bias, M, K);
     if (N == 1 && !bias) {

@@ -44,6 +44,23 @@ def test_plain_products(pkg, gpu, dt, trans, N, M, K, shift):
     assert rel(Cm, A.double() @ (B.double().t() if trans else B.double())) <= TOL[dt]
 
 
+def test_outer_product_of_more_pieces_than_31_bits_count(pkg, gpu):
+    """A column times a row, 65 540 x 1 048 584 in fp16: 137 GB, 2^31 units of four rows x one piece and some more."""
+    N, M = 65540, (1 << 20) + 8
+    torch.cuda.empty_cache()
+    if torch.cuda.mem_get_info()[0] < 160e9:
+        pytest.skip("less than 160 GB of memory free")
+    a = (torch.arange(N, device=DEV) % 31).to(torch.float16)  # (products are whole numbers below 2^11: exact)
+    b = (torch.arange(M, device=DEV) % 61).to(torch.float16)
+    C = torch.full((N, M), -1, dtype=torch.float16, device=DEV)
+    assert gpu.ptl_mm_fp16(a.data_ptr(), b.data_ptr(), C.data_ptr(), N, M, 1, 0) == 0, gpu.ptl_last_error().decode()
+    assert gpu.ptl_sync() == 0
+    for r in range(0, N, 4096):
+        assert bool((C[r:r + 4096] == a[r:r + 4096].view(-1, 1) * b).all()), r
+    del C
+    torch.cuda.empty_cache()
+
+
 @pytest.mark.parametrize("dt", ["fp32", "fp16"])
 @pytest.mark.parametrize("ns,n_in,n_out,shift", [(1, 33, 9, 1), (1, 5, 3, 0), (1, 4101, 5, 3), (2, 64, 10, 0), (33, 127, 65, 1),
                                                 (391, 785, 333, 0), (5000, 40, 12, 0), (3, 6, 5, 0), (130, 513, 256, 0)])
