@@ -17,8 +17,8 @@ namespace ptl {
 //     from the run's last one (`gap`) - and replaced by zeros.
 struct RagPiece {
     int tail;       // elements from the piece's first k on in the last slab
-    unsigned gap;   // bytes that the last slab lacks of one piece: in it every thread reads this much earlier, ...
-    unsigned back;  // ... and this one as much again
+    unsigned gap;   // bytes that the last slab lacks of one piece
+    unsigned back;  // bytes that the piece is read earlier in the last slab (at least `gap`)
     unsigned cut;   // bytes
 };
 template <int VEC>
@@ -28,15 +28,18 @@ PTL_BOTH inline RagPiece rag_piece(int left, int pos) {
     r.tail = left - pos * VEC;
     r.gap = left < VEC ? (unsigned)(VEC - left) * ES : 0u;
     r.cut = r.tail > 0 && r.tail < VEC ? (unsigned)(VEC - r.tail) * ES : 0u;
-    r.back = r.tail <= 0 ? (unsigned)pos * 16u : r.cut - (r.cut ? r.gap : 0u);
+    r.back = r.tail <= 0 ? (unsigned)pos * 16u + r.gap : r.cut;
     return r;
 }
-// Bytes before the slab's start that the offset `rag_piece_off` counts from.  want: ~0, or 0 where nothing is needed any
-// more and every lane reads the same piece.
-PTL_BOTH inline unsigned rag_piece_back(unsigned gap, unsigned back, bool last, unsigned want) { return last ? gap + (back & want) : 0u; }
-// Bytes of the piece from the start of row r0 of the slab; rows beyond the end repeat the last one.
+// Offsets are counted from a piece before the slab, so that they are never negative: a scalar address and 32 bits a lane.
+constexpr unsigned RAG_AHEAD = 16;
+// Of the piece at `pos` of a row, from the start of row r0 of the slab; rows beyond the end repeat the last one.
 PTL_BOTH inline unsigned rag_piece_off(int row, int r0, int rows, unsigned row_b, int pos) {
-    return ((unsigned)(row < rows ? row : rows - 1) - (unsigned)r0) * row_b + (unsigned)pos * 16u;
+    return ((unsigned)(row < rows ? row : rows - 1) - (unsigned)r0) * row_b + (unsigned)pos * 16u + RAG_AHEAD;
+}
+// Where it is read.  want: nothing is needed any more where this is 0, every lane reads the same piece.
+PTL_BOTH inline unsigned rag_piece_at(unsigned off, unsigned back, unsigned gap, bool last, unsigned want) {
+    return want ? off - (last ? back : 0u) : RAG_AHEAD - (last ? gap : 0u);
 }
 
 // The slabs of a workgroup in order: position in their run, and the run.  A workgroup asks for more slabs than it has, so

@@ -21,8 +21,8 @@ static bool walk(int rows, int K, int runs, int r0, int s0, int ns) {
         for (int pos = 0; pos < 8; ++pos) {
             const ptl::RagPiece q = ptl::rag_piece<VEC>(left, pos);
             for (int row = r0; row < r0 + R; ++row) {
-                const long long at = base - ptl::rag_piece_back(q.gap, q.back, last, want) +
-                                     (ptl::rag_piece_off(row, r0, rows, (unsigned)row_b, pos) & want);
+                const long long at = base - (long long)ptl::RAG_AHEAD +
+                                     ptl::rag_piece_at(ptl::rag_piece_off(row, r0, rows, (unsigned)row_b, pos), q.back, q.gap, last, want);
                 bool ok = at >= 0 && at + 16 <= bytes;
                 const long long mine = w.run * run_b + (row < rows ? row : rows - 1) * row_b;
                 if (want) {
