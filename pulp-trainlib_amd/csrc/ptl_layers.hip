@@ -11,6 +11,7 @@
 #include "ptl_common.hpp"
 #include "ptl_host.hpp"
 #include "ptl_conv_tile.hpp"
+#include "ptl_sum.hpp"
 
 #define STEP_BW_BOTH 3  // weight and input gradient together (library-internal step code)
 #include "ptl_api.h"
@@ -91,7 +92,8 @@ __global__ __launch_bounds__(256) void bias_grad_kernel(const T *__restrict__ dy
     constexpr int V = 16 / (int)sizeof(T);
     const int c = blockIdx.x, b0 = blockIdx.y * per_share, b1 = min(ns, b0 + per_share);
     const int pieces = (pix + V - 1) / V;  // per sample
-    float s = 0.f;
+    LongSum<T> s;
+    s.clear();
     for (int i = threadIdx.x; i < (b1 - b0) * pieces; i += 256) {
         const int b = i / pieces, p = (i - b * pieces) * V;
         const T *src = dy + ((size_t)(b0 + b) * C + c) * pix + p;
@@ -99,20 +101,21 @@ __global__ __launch_bounds__(256) void bias_grad_kernel(const T *__restrict__ dy
             T v[V];
             __builtin_memcpy(v, src, 16);
 #pragma unroll
-            for (int e = 0; e < V; ++e) s += (float)v[e];
+            for (int e = 0; e < V; ++e) s.add((float)v[e]);
         } else {
-            for (int e = 0; p + e < pix; ++e) s += (float)src[e];
+            for (int e = 0; p + e < pix; ++e) s.add((float)src[e]);
         }
     }
-    __shared__ float red[4];
+    __shared__ LongSum<T> red[4];
 #pragma unroll
-    for (int o = 32; o > 0; o >>= 1) s += __shfl_down(s, o, 64);
+    for (int o = 32; o > 0; o >>= 1) s.fold(o);
     if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = s;
     __syncthreads();
     if (threadIdx.x == 0) {
-        s = red[0] + red[1] + red[2] + red[3];
-        if (gridDim.y == 1) db[c] = (T)s;
-        else part[(size_t)blockIdx.y * C + c] = s;
+#pragma unroll
+        for (int w = 1; w < 4; ++w) s.add(red[w]);
+        if (gridDim.y == 1) db[c] = (T)s.value();
+        else part[(size_t)blockIdx.y * C + c] = s.value();
     }
 }
 
@@ -123,7 +126,8 @@ __global__ __launch_bounds__(256) void bias_grad_rows_kernel(const T *__restrict
                                                              int rows, int C, int per_share) {
     const int o = threadIdx.x & 63, w = threadIdx.x >> 6, c = blockIdx.x * 64 + o;
     const int r0 = blockIdx.y * per_share, r1 = min(rows, r0 + per_share);
-    float s = 0.f;
+    LongSum<T> s;
+    s.clear();
     if (c < C) {
         int r = r0 + w;
         for (; r + 12 < r1; r += 16) {
@@ -131,30 +135,36 @@ __global__ __launch_bounds__(256) void bias_grad_rows_kernel(const T *__restrict
 #pragma unroll
             for (int u = 0; u < 4; ++u) v[u] = (float)dy[(size_t)(r + 4 * u) * C + c];
 #pragma unroll
-            for (int u = 0; u < 4; ++u) s += v[u];
+            for (int u = 0; u < 4; ++u) s.add(v[u]);
         }
-        for (; r < r1; r += 4) s += (float)dy[(size_t)r * C + c];
+        for (; r < r1; r += 4) s.add((float)dy[(size_t)r * C + c]);
     }
-    __shared__ float red[4][64];
+    __shared__ LongSum<T> red[4][64];
     red[w][o] = s;
     __syncthreads();
     if (w == 0 && c < C) {
-        s = red[0][o] + red[1][o] + red[2][o] + red[3][o];
-        if (gridDim.y == 1) db[c] = (T)s;
-        else part[(size_t)blockIdx.y * C + c] = s;
+#pragma unroll
+        for (int q = 1; q < 4; ++q) s.add(red[q][o]);
+        if (gridDim.y == 1) db[c] = (T)s.value();
+        else part[(size_t)blockIdx.y * C + c] = s.value();
     }
 }
 
 template <typename T>
 __global__ __launch_bounds__(256) void bias_grad_sum_kernel(const float *__restrict__ part, T *__restrict__ db, int C, int shares) {
     const int o = threadIdx.x & 63, w = threadIdx.x >> 6, c = blockIdx.x * 64 + o;
-    float s = 0.f;
+    LongSum<T> s;
+    s.clear();
     if (c < C)
-        for (int z = w; z < shares; z += 4) s += part[(size_t)z * C + c];
-    __shared__ float red[4][64];
+        for (int z = w; z < shares; z += 4) s.add(part[(size_t)z * C + c]);
+    __shared__ LongSum<T> red[4][64];
     red[w][o] = s;
     __syncthreads();
-    if (w == 0 && c < C) db[c] = (T)(red[0][o] + red[1][o] + red[2][o] + red[3][o]);
+    if (w == 0 && c < C) {
+#pragma unroll
+        for (int q = 1; q < 4; ++q) s.add(red[q][o]);
+        db[c] = (T)s.value();
+    }
 }
 
 // db[c] = sum of dY over samples and positions: one launch where the channels alone fill the chip or little is to be read,

@@ -74,7 +74,7 @@ struct RagProd {
     int bias_n;
     int whole_k;       // the contraction is not split
     int add;           // C keeps what it holds, the product is added to it
-    void *row_sum;     // sum over k of a(n, k), as an extra column of ones in b (RC, GR, XR)
+    void *row_sum;     // sum over k of a(n, k); in the first product of (RC, RC) before (KC, RC), and with b gathered along k
     // set by the launcher
     float *ws;         // partial sums [split][N][pitch]
     int pitch, splits, slabs_per_split;
