@@ -18,7 +18,10 @@
 //     second kernel sums them in a fixed order (deterministic).
 #include "ptl_common.hpp"
 #include "ptl_ragged.hpp"
+#include "ptl_sum.hpp"
 #include "ptl_gemm_async.hpp"
+
+#include <algorithm>
 
 namespace ptl {
 
@@ -701,12 +704,21 @@ __global__ __launch_bounds__(256) void gemv_rowdot_kernel(const T *__restrict__ 
     if (lane == 0) y[row] = (T)(bias ? s + (float)bias[row] : s);
 }
 
-// y[m] = sum_k x[k] * Mx[k*M + m] for the four pieces of columns of workgroup `block`: thread (kl, cv) sums rows kl,
-// kl + 256, ... of piece cv with four loads in flight, the rows meet in LDS (first eight, then the rest).
+// How the rows of a column sum are shared out: `cols` workgroups side by side, each share `chunk` rows.
+struct GvShares {
+    int cols, shares, chunk;
+    float *part;  // [share][M]; one share: the kernel writes the result
+};
+
+// Workgroup `block` sums share block / cols of four pieces of columns of y[m] = sum_k x[k] * Mx[k*M + m]: thread (kl, cv)
+// takes rows kl, kl + 256, ... of piece cv with four loads in flight, the rows meet in LDS (first eight, then the rest).
 template <typename T, int V>
 __device__ inline void gemv_coldot_block(const T *__restrict__ x, const T *__restrict__ Mx, T *__restrict__ y, int K, int M,
-                                         int block, float *red) {
+                                         int block, const GvShares &sh, float *red) {
     constexpr int CV = 4, KL = GV_NT / CV, U = 4;
+    const int share = block / sh.cols;
+    block -= share * sh.cols;
+    const int k0 = share * sh.chunk, k1 = min(K, k0 + sh.chunk);
     const int cv = threadIdx.x % CV, kl = threadIdx.x / CV;
     const int want = (block * CV + cv) * V, col = want + V <= M ? want : M - V;
     float acc[V];
@@ -714,18 +726,18 @@ __device__ inline void gemv_coldot_block(const T *__restrict__ x, const T *__res
     for (int i = 0; i < V; ++i) acc[i] = 0.f;
     const T *p = Mx + col;
     if (want < M) {
-        for (int k = kl; k < K; k += U * KL) {
+        for (int k = k0 + kl; k < k1; k += U * KL) {
             GvPiece<T, V> v[U];
             float xv[U];
 #pragma unroll
-            for (int u = 0; u < U; ++u) {  // (rows beyond the end: the last one, times zero)
-                const int kk = k + u * KL < K ? k + u * KL : K - 1;
+            for (int u = 0; u < U; ++u) {  // (rows beyond the end: the last one is loaded and left out)
+                const int kk = k + u * KL < k1 ? k + u * KL : k1 - 1;
                 v[u] = gv_load<T, V>(p + (size_t)kk * M);
                 xv[u] = (float)x[kk];
             }
 #pragma unroll
             for (int u = 0; u < U; ++u) {
-                if (k + u * KL >= K) break;
+                if (k + u * KL >= k1) break;
 #pragma unroll
                 for (int i = 0; i < V; ++i) acc[i] += xv[u] * (float)v[u].e[i];
             }
@@ -743,19 +755,22 @@ __device__ inline void gemv_coldot_block(const T *__restrict__ x, const T *__res
     }
     __syncthreads();
     if ((int)threadIdx.x < CV * V) {
-        const int c = threadIdx.x / V, first = (block * CV + c) * V, at = first + V <= M ? first : M - V;
+        const int c = threadIdx.x / V, first = (block * CV + c) * V, at = (first + V <= M ? first : M - V) + threadIdx.x % V;
         float s = 0.f;
 #pragma unroll
         for (int w = 0; w < GV_NT / 64; ++w) s += red[w * (CV * V) + threadIdx.x];
-        if (first < M) y[at + threadIdx.x % V] = (T)s;
+        if (first < M) {
+            if (sh.shares > 1) sh.part[(size_t)share * M + at] = s;
+            else y[at] = (T)s;
+        }
     }
 }
 
 template <typename T, int V>
 __global__ __launch_bounds__(GV_NT) void gemv_coldot_kernel(const T *__restrict__ x, const T *__restrict__ Mx, T *__restrict__ y,
-                                                            int K, int M) {
+                                                            int K, int M, const GvShares sh) {
     __shared__ float red[GV_NT / 64 * 4 * V];
-    gemv_coldot_block<T, V>(x, Mx, y, K, M, blockIdx.x, red);
+    gemv_coldot_block<T, V>(x, Mx, y, K, M, blockIdx.x, sh, red);
 }
 
 // C[n*M + m] = a[n] * b[m]: unit `i` is a piece of columns of four consecutive rows; the first piece of a row also copies
@@ -788,16 +803,35 @@ __global__ __launch_bounds__(GV_NT) void outer_kernel(const T *__restrict__ a, c
 }
 
 // Both gradients of a dense layer on one sample in one launch (1024 x 1024 in fp32: 5.9 us as two launches, bound by the
-// host; 3.3 as one): the first `cols` workgroups sum columns for dX, the rest write dW (and db = dY).
+// host; 3.3 as one): the first workgroups sum columns for dX, the rest write dW (and db = dY).
 template <typename T, int V>
 __global__ __launch_bounds__(GV_NT) void linear_one_bw_kernel(const T *__restrict__ x, const T *__restrict__ W,
                                                               const T *__restrict__ dy, T *__restrict__ dW, T *__restrict__ dx,
-                                                              T *__restrict__ db, int in, int out, RagDiv per_row, int cols) {
+                                                              T *__restrict__ db, int in, int out, RagDiv per_row,
+                                                              const GvShares sh) {
     __shared__ float red[GV_NT / 64 * 4 * V];
-    if ((int)blockIdx.x < cols)
-        gemv_coldot_block<T, V>(dy, W, dx, out, in, blockIdx.x, red);
+    const int sums = sh.cols * sh.shares;
+    if ((int)blockIdx.x < sums)
+        gemv_coldot_block<T, V>(dy, W, dx, out, in, blockIdx.x, sh, red);
     else
-        outer_unit<T, V>(dy, x, dW, db, out, in, per_row, (blockIdx.x - cols) * GV_NT + threadIdx.x);
+        outer_unit<T, V>(dy, x, dW, db, out, in, per_row, (blockIdx.x - sums) * GV_NT + threadIdx.x);
+}
+
+// Few columns leave most CUs without a workgroup, and each has a trip to memory for every 1024 of its rows.  The rows are
+// shared out where that saves three such trips, since adding the shares is a launch (2.3 us): as many shares as give every
+// CU a workgroup, of 512 rows and more, at most 32.  In us, one share against these, fp32: 64 columns of 4096 rows 5.8, 5.9; of
+// 16384 rows 23.9, 6.1; of 65536 88.7, 9.2; 256 columns of 4096 rows 10.0, 6.0; 1024 of 4096 10.9, 9.1; 2048 of 4096
+// 13.0, 13.9 (not taken), of 8192 32.4, 25.3.  Ten columns of 4096 rows lose (4.5, 5.8), of 8192 gain (6.6, 5.8).
+template <typename T, int V>
+static GvShares gv_shares(int K, int M) {
+    GvShares sh = {(M + 4 * V - 1) / (4 * V), 1, K, nullptr};
+    const int cu = state().num_cu, trips = (K + 1023) / 1024;
+    const int z = std::min({(cu + sh.cols - 1) / sh.cols, K / 512, 32});
+    if (z < 2 || trips - trips / z < 3 || (sh.cols < 4 && K <= 4096)) return sh;
+    const int chunk = (K + z - 1) / z, shares = (K + chunk - 1) / chunk;
+    // (a stream that is being captured cannot get a workspace: one share then)
+    if (float *part = workspace((size_t)shares * M * sizeof(float))) sh = {sh.cols, shares, chunk, part};
+    return sh;
 }
 
 static unsigned outer_blocks(int N, int M, int V) {
@@ -819,9 +853,10 @@ static int outer(const T *a, const T *b, T *C, int N, int M) {
 
 template <typename T, int V>
 static int linear_one_bw_v(const T *x, const T *W, const T *dy, T *dW, T *dx, T *db, int in, int out) {
-    const int cols = (in + 4 * V - 1) / (4 * V);
-    hipLaunchKernelGGL((linear_one_bw_kernel<T, V>), dim3(cols + outer_blocks(out, in, V)), dim3(GV_NT), 0, state().stream, x, W,
-                       dy, dW, dx, db, in, out, rag_div((in + V - 1) / V), cols);
+    const GvShares sh = gv_shares<T, V>(out, in);
+    hipLaunchKernelGGL((linear_one_bw_kernel<T, V>), dim3(sh.cols * sh.shares + outer_blocks(out, in, V)), dim3(GV_NT), 0,
+                       state().stream, x, W, dy, dW, dx, db, in, out, rag_div((in + V - 1) / V), sh);
+    if (sh.shares > 1) launch_share_sum<T>(sh.part, dx, in, sh.shares, state().stream);
     return hip_ok(hipGetLastError(), "linear backward launch") ? 0 : 2;
 }
 template <typename T>
@@ -838,22 +873,23 @@ static int gemv_rowdot(const T *Mx, const T *x, T *y, const T *bias, int R, int 
     return hip_ok(hipGetLastError(), "gemv launch") ? 0 : 2;
 }
 
+template <typename T, int V>
+static int gemv_coldot(const T *x, const T *Mx, T *y, int K, int M) {
+    const GvShares sh = gv_shares<T, V>(K, M);
+    hipLaunchKernelGGL((gemv_coldot_kernel<T, V>), dim3(sh.cols * sh.shares), dim3(GV_NT), 0, state().stream, x, Mx, y, K, M, sh);
+    if (sh.shares > 1) launch_share_sum<T>(sh.part, y, M, sh.shares, state().stream);
+    return hip_ok(hipGetLastError(), "gemv launch") ? 0 : 2;
+}
+
 template <typename T>
 int mm_dispatch(const T *A, const T *B, T *C, int N, int M, int K, int trans_B, const T *bias) {
     if (!ensure_init()) return 2;
     if (N <= 0 || M <= 0 || K <= 0) return 0;  // K == 0 leaves C untouched, as mm() does
-    State &st = state();
     constexpr int VEC = Traits<T>::VEC;
     if (K == 1 && !bias) return M >= VEC ? outer<T, VEC>(A, B, C, N, M) : outer<T, 1>(A, B, C, N, M);
     if (M == 1 && !bias) return gemv_rowdot<T>(A, B, C, nullptr, N, K);  // B is K x 1 or 1 x K: the same vector
     if (N == 1 && trans_B) return gemv_rowdot<T>(B, A, C, bias, M, K);
-    if (N == 1 && !bias) {
-        if (M >= VEC)
-            hipLaunchKernelGGL((gemv_coldot_kernel<T, VEC>), dim3((M + 4 * VEC - 1) / (4 * VEC)), dim3(GV_NT), 0, st.stream, A, B, C, K, M);
-        else
-            hipLaunchKernelGGL((gemv_coldot_kernel<T, 1>), dim3((M + 3) / 4), dim3(GV_NT), 0, st.stream, A, B, C, K, M);
-        return hip_ok(hipGetLastError(), "gemv launch") ? 0 : 2;
-    }
+    if (N == 1 && !bias) return M >= VEC ? gemv_coldot<T, VEC>(A, B, C, K, M) : gemv_coldot<T, 1>(A, B, C, K, M);
     GemmArgs g = {};
     g.A = A;
     g.B = B;

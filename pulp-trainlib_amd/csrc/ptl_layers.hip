@@ -150,23 +150,6 @@ __global__ __launch_bounds__(256) void bias_grad_rows_kernel(const T *__restrict
     }
 }
 
-template <typename T>
-__global__ __launch_bounds__(256) void bias_grad_sum_kernel(const float *__restrict__ part, T *__restrict__ db, int C, int shares) {
-    const int o = threadIdx.x & 63, w = threadIdx.x >> 6, c = blockIdx.x * 64 + o;
-    LongSum<T> s;
-    s.clear();
-    if (c < C)
-        for (int z = w; z < shares; z += 4) s.add(part[(size_t)z * C + c]);
-    __shared__ LongSum<T> red[4][64];
-    red[w][o] = s;
-    __syncthreads();
-    if (w == 0 && c < C) {
-#pragma unroll
-        for (int q = 1; q < 4; ++q) s.add(red[q][o]);
-        db[c] = (T)s.value();
-    }
-}
-
 // db[c] = sum of dY over samples and positions: one launch where the channels alone fill the chip or little is to be read,
 // else shares of it and their sum (45 channels of 27 753 positions in fp32: 37.6 us with one workgroup per channel and a
 // 64-bit division per element, 8.5 this way).
@@ -191,8 +174,7 @@ static int bias_grad(const T *dy, T *db, int ns, int C, int pix, int hwc) {
                            (int)rows, C, (int)per);
     else
         hipLaunchKernelGGL((bias_grad_kernel<T>), dim3(C, (unsigned)shares), dim3(256), 0, st.stream, dy, part, db, ns, C, pix, (int)per);
-    if (shares > 1)
-        hipLaunchKernelGGL((bias_grad_sum_kernel<T>), dim3((C + 63) / 64), dim3(256), 0, st.stream, part, db, C, (int)shares);
+    if (shares > 1) launch_share_sum<T>(part, db, C, (int)shares, st.stream);
     return hip_ok(hipGetLastError(), "bias grad launch") ? 0 : 2;
 }
 

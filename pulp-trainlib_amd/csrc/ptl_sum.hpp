@@ -1,4 +1,4 @@
-// Sums over the rows of a tensor (bias gradients).
+// Sums over the rows of a tensor (bias gradients), and of the shares that workgroups have of such sums.
 #pragma once
 #include <hip/hip_runtime.h>
 
@@ -35,5 +35,37 @@ struct LongSum {
     // (after an infinity the errors are no numbers: the plain sum counts)
     __device__ inline float value() const { return EXACT && fabsf(c) < __builtin_inff() ? s + c : s; }
 };
+
+// out[c] = sum over the shares of part[share][c]: 64 columns a workgroup, four shares at a time with four loads in flight.
+template <typename T>
+__global__ __launch_bounds__(256) void share_sum_kernel(const float *__restrict__ part, T *__restrict__ out, int C, int shares) {
+    const int o = threadIdx.x & 63, w = threadIdx.x >> 6, c = blockIdx.x * 64 + o;
+    LongSum<T> s;
+    s.clear();
+    if (c < C) {
+        int z = w;
+        for (; z + 12 < shares; z += 16) {
+            float v[4];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) v[u] = part[(size_t)(z + 4 * u) * C + c];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) s.add(v[u]);
+        }
+        for (; z < shares; z += 4) s.add(part[(size_t)z * C + c]);
+    }
+    __shared__ LongSum<T> red[4][64];
+    red[w][o] = s;
+    __syncthreads();
+    if (w == 0 && c < C) {
+#pragma unroll
+        for (int q = 1; q < 4; ++q) s.add(red[q][o]);
+        out[c] = (T)s.value();
+    }
+}
+
+template <typename T>
+static inline void launch_share_sum(const float *part, T *out, int C, int shares, hipStream_t stream) {
+    hipLaunchKernelGGL((share_sum_kernel<T>), dim3((C + 63) / 64), dim3(256), 0, stream, part, out, C, shares);
+}
 
 }  // namespace ptl

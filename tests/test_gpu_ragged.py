@@ -33,7 +33,9 @@ def rel(got, ref):
 @pytest.mark.parametrize("trans", [0, 1])
 # one element over and under a tile, a slab, a piece; k shorter than a slab; a k split; rows shorter than a piece
 @pytest.mark.parametrize("N,M,K,shift", [(33, 65, 65, 0), (31, 63, 127, 1), (129, 127, 33, 3), (300, 201, 2051, 1), (64, 9, 70, 0),
-                                         (8, 8, 8, 1), (9, 1030, 9, 5), (5, 3, 700, 1), (700, 3, 5, 1)])
+                                         (8, 8, 8, 1), (9, 1030, 9, 5), (5, 3, 700, 1), (700, 3, 5, 1),
+                                         # one row: columns summed in shares of the rows (the last of 2, of 8, of 32; none)
+                                         (1, 2049, 8193, 1), (1, 257, 4097, 0), (1, 67, 16411, 3), (1, 10, 8195, 1), (1, 3, 4096, 0)])
 def test_plain_products(pkg, gpu, dt, trans, N, M, K, shift):
     g = torch.Generator(device=DEV).manual_seed(N * 7 + M)
     A, B = tensor(g, (N, K), dt, shift), tensor(g, (M, K) if trans else (K, M), dt, shift)
@@ -63,7 +65,8 @@ def test_outer_product_of_more_pieces_than_31_bits_count(pkg, gpu):
 
 @pytest.mark.parametrize("dt", ["fp32", "fp16"])
 @pytest.mark.parametrize("ns,n_in,n_out,shift", [(1, 33, 9, 1), (1, 5, 3, 0), (1, 4101, 5, 3), (2, 64, 10, 0), (33, 127, 65, 1),
-                                                (391, 785, 333, 0), (5000, 40, 12, 0), (3, 6, 5, 0), (130, 513, 256, 0)])
+                                                (391, 785, 333, 0), (5000, 40, 12, 0), (3, 6, 5, 0), (130, 513, 256, 0),
+                                                (1, 71, 16387, 1), (1, 1031, 4099, 0), (1, 6, 9001, 1)])
 @pytest.mark.parametrize("bias", [0, 1])
 def test_dense_layers(pkg, gpu, dt, ns, n_in, n_out, shift, bias):
     g = torch.Generator(device=DEV).manual_seed(ns + n_in)
