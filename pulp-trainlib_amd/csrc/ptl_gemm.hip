@@ -671,7 +671,7 @@ template int gemm<half_t>(const GemmArgs &);
 // one that ends with it (columns it shares with the piece before are worked out twice, with the same result), rows
 // shorter than a piece go element by element (V = 1).
 // ---------------------------------------------------------------------------
-constexpr int GV_NT = 1024;
+constexpr int GV_NT = 512;
 
 template <typename T, int V>
 struct GvPiece {
@@ -710,36 +710,55 @@ struct GvShares {
     float *part;  // [share][M]; one share: the kernel writes the result
 };
 
-// Workgroup `block` sums share block / cols of four pieces of columns of y[m] = sum_k x[k] * Mx[k*M + m]: thread (kl, cv)
-// takes rows kl, kl + 256, ... of piece cv with four loads in flight, the rows meet in LDS (first eight, then the rest).
+// Workgroup `block` sums share block / cols of eight pieces of columns (a 128-byte line: four, of which two workgroups
+// on different XCDs share a line, take up to twice as long from 8 MB on) of y[m] = sum_k x[k] * Mx[k*M + m]: thread (kl, cv)
+// takes rows kl, kl + 64, ... of piece cv with four loads in flight, the rows meet in LDS (first eight, then the rest).
+constexpr int GV_CV = 8, GV_ROWS = GV_NT / GV_CV, GV_U = 4;
 template <typename T, int V>
 __device__ inline void gemv_coldot_block(const T *__restrict__ x, const T *__restrict__ Mx, T *__restrict__ y, int K, int M,
                                          int block, const GvShares &sh, float *red) {
-    constexpr int CV = 4, KL = GV_NT / CV, U = 4;
+    constexpr int CV = GV_CV, KL = GV_ROWS, U = GV_U, NT = GV_NT;
     const int share = block / sh.cols;
     block -= share * sh.cols;
-    const int k0 = share * sh.chunk, k1 = min(K, k0 + sh.chunk);
+    const unsigned k0 = (unsigned)share * (unsigned)sh.chunk, k1 = min((unsigned)K, k0 + (unsigned)sh.chunk);
     const int cv = threadIdx.x % CV, kl = threadIdx.x / CV;
     const int want = (block * CV + cv) * V, col = want + V <= M ? want : M - V;
     float acc[V];
 #pragma unroll
     for (int i = 0; i < V; ++i) acc[i] = 0.f;
-    const T *p = Mx + col;
     if (want < M) {
-        for (int k = k0 + kl; k < k1; k += U * KL) {
+        // (addresses by additions of a uniform step: a 64-bit product per load takes a fifth of the time of short columns)
+        const size_t step = (size_t)KL * M;
+        unsigned k = k0 + kl;
+        const T *q = Mx + (size_t)k * M + col, *xq = x + k;
+        for (; k + (U - 1) * KL < k1; k += U * KL, q += U * step, xq += U * KL) {
             GvPiece<T, V> v[U];
-            float xv[U];
-#pragma unroll
-            for (int u = 0; u < U; ++u) {  // (rows beyond the end: the last one is loaded and left out)
-                const int kk = k + u * KL < k1 ? k + u * KL : k1 - 1;
-                v[u] = gv_load<T, V>(p + (size_t)kk * M);
-                xv[u] = (float)x[kk];
-            }
+            T xv[U];
 #pragma unroll
             for (int u = 0; u < U; ++u) {
-                if (k + u * KL >= k1) break;
+                v[u] = gv_load<T, V>(q + u * step);
+                xv[u] = xq[u * KL];
+            }
 #pragma unroll
-                for (int i = 0; i < V; ++i) acc[i] += xv[u] * (float)v[u].e[i];
+            for (int u = 0; u < U; ++u)
+#pragma unroll
+                for (int i = 0; i < V; ++i) acc[i] += (float)xv[u] * (float)v[u].e[i];
+        }
+        if (k < k1) {  // (rows beyond the end: the first one, replaced by zeros; a branch around them would take each load into it)
+            GvPiece<T, V> v[U - 1];
+            T xv[U - 1];
+            bool in[U - 1];
+#pragma unroll
+            for (int u = 0; u < U - 1; ++u) {
+                in[u] = k + u * KL < k1;
+                v[u] = gv_load<T, V>(q + (in[u] ? u * step : 0));
+                xv[u] = xq[in[u] ? u * KL : 0];
+            }
+#pragma unroll
+            for (int u = 0; u < U - 1; ++u) {
+                const float f = in[u] ? (float)xv[u] : 0.f;
+#pragma unroll
+                for (int i = 0; i < V; ++i) acc[i] += f * (in[u] ? (float)v[u].e[i] : 0.f);
             }
         }
     }
@@ -758,7 +777,7 @@ __device__ inline void gemv_coldot_block(const T *__restrict__ x, const T *__res
         const int c = threadIdx.x / V, first = (block * CV + c) * V, at = (first + V <= M ? first : M - V) + threadIdx.x % V;
         float s = 0.f;
 #pragma unroll
-        for (int w = 0; w < GV_NT / 64; ++w) s += red[w * (CV * V) + threadIdx.x];
+        for (int w = 0; w < NT / 64; ++w) s += red[w * (CV * V) + threadIdx.x];
         if (first < M) {
             if (sh.shares > 1) sh.part[(size_t)share * M + at] = s;
             else y[at] = (T)s;
@@ -769,7 +788,7 @@ __device__ inline void gemv_coldot_block(const T *__restrict__ x, const T *__res
 template <typename T, int V>
 __global__ __launch_bounds__(GV_NT) void gemv_coldot_kernel(const T *__restrict__ x, const T *__restrict__ Mx, T *__restrict__ y,
                                                             int K, int M, const GvShares sh) {
-    __shared__ float red[GV_NT / 64 * 4 * V];
+    __shared__ float red[GV_NT / 64 * GV_CV * V];
     gemv_coldot_block<T, V>(x, Mx, y, K, M, blockIdx.x, sh, red);
 }
 
@@ -809,7 +828,7 @@ __global__ __launch_bounds__(GV_NT) void linear_one_bw_kernel(const T *__restric
                                                               const T *__restrict__ dy, T *__restrict__ dW, T *__restrict__ dx,
                                                               T *__restrict__ db, int in, int out, RagDiv per_row,
                                                               const GvShares sh) {
-    __shared__ float red[GV_NT / 64 * 4 * V];
+    __shared__ float red[GV_NT / 64 * GV_CV * V];
     const int sums = sh.cols * sh.shares;
     if ((int)blockIdx.x < sums)
         gemv_coldot_block<T, V>(dy, W, dx, out, in, blockIdx.x, sh, red);
@@ -817,17 +836,16 @@ __global__ __launch_bounds__(GV_NT) void linear_one_bw_kernel(const T *__restric
         outer_unit<T, V>(dy, x, dW, db, out, in, per_row, (blockIdx.x - sums) * GV_NT + threadIdx.x);
 }
 
-// Few columns leave most CUs without a workgroup, and each has a trip to memory for every 1024 of its rows.  The rows are
-// shared out where that saves three such trips, since adding the shares is a launch (2.3 us): as many shares as give every
-// CU a workgroup, of 512 rows and more, at most 32.  In us, one share against these, fp32: 64 columns of 4096 rows 5.8, 5.9; of
-// 16384 rows 23.9, 6.1; of 65536 88.7, 9.2; 256 columns of 4096 rows 10.0, 6.0; 1024 of 4096 10.9, 9.1; 2048 of 4096
-// 13.0, 13.9 (not taken), of 8192 32.4, 25.3.  Ten columns of 4096 rows lose (4.5, 5.8), of 8192 gain (6.6, 5.8).
+// Few columns leave CUs without a workgroup, and a workgroup has a trip to memory for every 256 of its rows.  Columns of 4096
+// rows and more are shared out over two workgroups a CU, 512 rows and more each, at most 32 shares, where that is two
+// shares at least; adding them is a launch (2.3 us).  In us, one share against these, fp32: 64 columns of 2048 rows 4.0, 6.1
+// (not taken), of 4096 6.8, 6.1, of 16384 25.3, 6.4; 1024 columns of 2048 rows 5.8, 6.6 (not taken), of 4096 9.9, 6.7; 4096
+// of 4096 18.8, 15.7; 6144 of 4096 21.5, 21.9 (not taken).
 template <typename T, int V>
 static GvShares gv_shares(int K, int M) {
-    GvShares sh = {(M + 4 * V - 1) / (4 * V), 1, K, nullptr};
-    const int cu = state().num_cu, trips = (K + 1023) / 1024;
-    const int z = std::min({(cu + sh.cols - 1) / sh.cols, K / 512, 32});
-    if (z < 2 || trips - trips / z < 3 || (sh.cols < 4 && K <= 4096)) return sh;
+    GvShares sh = {(int)(((long long)M + GV_CV * V - 1) / (GV_CV * V)), 1, K, nullptr};
+    const int cu = state().num_cu, z = std::min({2 * cu / sh.cols, K / 512, 32});
+    if (K < 4096 || sh.cols > cu / 2 || z < 2) return sh;
     const int chunk = (K + z - 1) / z, shares = (K + chunk - 1) / chunk;
     // (a stream that is being captured cannot get a workspace: one share then)
     if (float *part = workspace((size_t)shares * M * sizeof(float))) sh = {sh.cols, shares, chunk, part};
