@@ -11,6 +11,7 @@
 #include "ptl_api.h"
 
 #include <stdio.h>
+#include <algorithm>
 
 namespace ptl {
 
@@ -804,9 +805,10 @@ __global__ __launch_bounds__(256) void dw_direct_kernel(const T *__restrict__ sr
     }
 }
 
-// Weight gradient the same way: a workgroup owns a channel and a group of samples and deals the blocks of DW_DRB
-// gradient rows x COLS columns of all its planes to its lanes, the nine tap sums stay in registers; one reduction
-// per workgroup at the end.  part[(grp * C + ch) * 9 + tap], or the gradient itself when there is one group.
+// Weight gradient the same way: a workgroup owns a channel and a group of samples - or, of large planes, a share of the
+// blocks of one - and deals the blocks of DW_DRB gradient rows x COLS columns of all its planes to its lanes, the nine tap
+// sums stay in registers; one reduction per workgroup at the end.  part[((grp * shares + share) * C + ch) * 9 + tap], or
+// the gradient itself when there is one workgroup per channel.
 template <typename T>
 __global__ __launch_bounds__(256) void dw_wg_direct_kernel(const T *__restrict__ X, const T *__restrict__ dY,
                                                            float *__restrict__ part, int C, int ns, int per_group, int H,
@@ -825,7 +827,7 @@ __global__ __launch_bounds__(256) void dw_wg_direct_kernel(const T *__restrict__
     const unsigned per_plane = (unsigned)(groups * rblocks);
     const int b0 = grp * per_group;
     const unsigned items = per_plane * (unsigned)(min(ns, b0 + per_group) - b0);
-    for (unsigned it = tid; it < items; it += 256) {
+    for (unsigned it = blockIdx.z * 256 + tid; it < items; it += 256 * gridDim.z) {
         const unsigned b = it / per_plane, item = it - b * per_plane;
         const int rb = (int)(item / (unsigned)groups), c0 = (int)(item - (unsigned)rb * groups) * NC, r0 = rb * RB;
         const size_t plane = (size_t)(b0 + b) * C + ch;
@@ -876,7 +878,7 @@ __global__ __launch_bounds__(256) void dw_wg_direct_kernel(const T *__restrict__
         if (direct)
             direct[(size_t)ch * 9 + tid] = (T)sum;
         else
-            part[((size_t)grp * C + ch) * 9 + tid] = sum;
+            part[(((size_t)grp * gridDim.z + blockIdx.z) * C + ch) * 9 + tid] = sum;
     }
 }
 
@@ -1066,15 +1068,26 @@ static int dw_step(const Args *a, int ns, int step, int sh, int sw, const char *
         if (sgroups < 1) sgroups = 1;
         const int per_group = (ns + sgroups - 1) / sgroups;
         sgroups = (ns + per_group - 1) / per_group;
-        float *part = partials((size_t)sgroups * g.C * taps * sizeof(float));
+        // Few large planes: their blocks shared out, up to two workgroups a CU, while those of whole planes would leave three
+        // CUs in four idle; one workgroup a channel only from four blocks a lane on, since adding shares is a launch.
+        // fp32, us: 16 channels of 512 x 512 66.6 -> 10.8, of 256 x 256 20.9 -> 8.3, of 128 x 128 9.0, 9.9 (two shares; not
+        // taken), 64 of 224 x 224 11.8 -> 8.6, 128 13.4, 14.2 (not taken); 2 x 16 of 128 x 128 11.6 -> 8.0.
+        int shares = 1;
+        const long wgs = (long)sgroups * g.C;
+        if (direct_path && 4 * wgs <= st.num_cu) {
+            const int blocks = ((g.Ho + DW_DRB - 1) / DW_DRB) * ((g.Wo + DwSeg<T>::COLS - 1) / DwSeg<T>::COLS);
+            if (sgroups > 1 || blocks >= 4 * 256) shares = (int)std::min(2 * st.num_cu / wgs, (blocks + 255L) / 256);
+        }
+        float *part = partials((size_t)sgroups * shares * g.C * taps * sizeof(float));
         if (!part) return sg.finish(too_big ? 1 : 2);
-        T *direct = sgroups == 1 ? dW : nullptr;  // one group: the kernel writes the gradient, no second launch
+        T *direct = sgroups * shares == 1 ? dW : nullptr;  // one workgroup a channel writes the gradient, no second launch
         const int x_vecs = (int)((in_img + 15) / 16);
         const size_t lds = (size_t)x_vecs * 16 + out_img;
         dim3 grid(g.C, sgroups);
         if (direct_path) {
             const int whole = g.Ho % DW_DRB == 0 && g.Wo % DwSeg<T>::COLS == 0;  // blocks of the gradient
             const int inside = whole | (whole && g.Ho + 2 <= g.H && g.Wo + 2 <= g.W && g.Up == 0 && g.Lp == 0 ? 2 : 0);
+            grid.z = (unsigned)shares;
             hipLaunchKernelGGL((dw_wg_direct_kernel<T>), grid, dim3(256), 0, st.stream, X, dY, part, g.C, ns, per_group, g.H,
                                g.W, g.Ho, g.Wo, g.Up, g.Lp, in_n, out_n, inside, direct);
         } else {
@@ -1091,7 +1104,7 @@ static int dw_step(const Args *a, int ns, int step, int sh, int sw, const char *
                                    per_group, g.H, g.W, g.Ho, g.Wo, g.Up, g.Lp, x_vecs, direct);
         }
         if (!direct)
-            hipLaunchKernelGGL((dw_wg_reduce_kernel2<T>), dim3(g.C), dim3(256), 0, st.stream, part, dW, sgroups, g.C, 1,
+            hipLaunchKernelGGL((dw_wg_reduce_kernel2<T>), dim3(g.C), dim3(256), 0, st.stream, part, dW, sgroups * shares, g.C, 1,
                                taps);
     } else if (rows_path) {
         const T *X = sg.in(reinterpret_cast<const T *>(a->input->data), in_n);

@@ -19,7 +19,9 @@ def placed(t, n):
 @pytest.mark.parametrize("dt", ["fp32", "fp16"])
 @pytest.mark.parametrize("b,C,H,W,pad,shift", [(1, 1, 3, 14, 0, 0), (2, 3, 6, 9, 1, 1), (3, 5, 9, 9, 0, 1), (1, 7, 9, 12, 1, 0),
                                               (5, 2, 16, 33, 2, 3), (2, 9, 15, 58, 0, 0), (3, 2, 4, 5, 1, 1), (37, 17, 30, 31, 1, 0),
-                                              (1, 16, 58, 113, 0, 1), (2, 2, 5, 4, 3, 1)])
+                                              (1, 16, 58, 113, 0, 1), (2, 2, 5, 4, 3, 1),
+                                              # the blocks of a plane in shares, the last one short
+                                              (1, 3, 230, 131, 1, 1), (1, 2, 301, 299, 0, 1), (2, 3, 60, 150, 1, 3), (5, 1, 257, 129, 2, 0)])
 def test_depthwise_blocks(pkg, gpu, dt, b, C, H, W, pad, shift):
     tdt = torch.float32 if dt == "fp32" else torch.float16
     Ho, Wo = H + 2 * pad - 2, W + 2 * pad - 2
