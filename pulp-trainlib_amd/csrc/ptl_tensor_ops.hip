@@ -809,58 +809,86 @@ __global__ __launch_bounds__(256) void dw_direct_kernel(const T *__restrict__ sr
 // blocks of one - and deals the blocks of DW_DRB gradient rows x COLS columns of all its planes to its lanes, the nine tap
 // sums stay in registers; one reduction per workgroup at the end.  part[((grp * shares + share) * C + ch) * 9 + tap], or
 // the gradient itself when there is one workgroup per channel.
-template <typename T>
-__global__ __launch_bounds__(256) void dw_wg_direct_kernel(const T *__restrict__ X, const T *__restrict__ dY,
-                                                           float *__restrict__ part, int C, int ns, int per_group, int H,
-                                                           int W, int Ho, int Wo, int pu, int pl, size_t x_elems,
-                                                           size_t y_elems, int inside, T *__restrict__ direct) {
-    constexpr int RB = DW_DRB, NC = DwSeg<T>::COLS;
-    __shared__ float red[4][9];
-    const int ch = blockIdx.x, grp = blockIdx.y;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    float acc[3][3];
+// A block that reaches over the end of the gradient multiplies what the source has there with zeros, which of an infinity
+// makes no number: a lane whose sums end as one goes over its blocks again, row by row and without the columns that do
+// not exist (STRICT; leaving them out always took 3 to 9 % longer, whole blocks need too many registers for four waves).
+struct DwWgWalk {
+    int C, H, W, Ho, Wo, pu, pl, inside;
+    size_t x_elems, y_elems;
+};
+template <typename T, bool STRICT>
+__device__ inline void dw_wg_blocks(const T *__restrict__ X, const T *__restrict__ dY, const DwWgWalk &w, int ch, int b0, unsigned first,
+                                    unsigned step, unsigned items, float (&acc)[3][3]) {
+    constexpr int RB = STRICT ? 1 : DW_DRB, NC = DwSeg<T>::COLS;
+    const unsigned groups = (unsigned)(w.Wo + NC - 1) / NC, per_plane = groups * ((unsigned)(w.Ho + DW_DRB - 1) / DW_DRB);
 #pragma unroll
     for (int i = 0; i < 3; ++i)
 #pragma unroll
         for (int j = 0; j < 3; ++j) acc[i][j] = 0.f;
-    const int groups = (Wo + NC - 1) / NC, rblocks = (Ho + RB - 1) / RB;
-    const unsigned per_plane = (unsigned)(groups * rblocks);
-    const int b0 = grp * per_group;
-    const unsigned items = per_plane * (unsigned)(min(ns, b0 + per_group) - b0);
-    for (unsigned it = blockIdx.z * 256 + tid; it < items; it += 256 * gridDim.z) {
+    for (unsigned it = first; it < items; it += step) {
         const unsigned b = it / per_plane, item = it - b * per_plane;
-        const int rb = (int)(item / (unsigned)groups), c0 = (int)(item - (unsigned)rb * groups) * NC, r0 = rb * RB;
-        const size_t plane = (size_t)(b0 + b) * C + ch;
-        unsigned G[RB][DwSeg<T>::OUT];
-        dw_segments<T>(dY, plane * Ho * Wo, y_elems, Ho, Wo, r0, c0, inside & 1, G);
-        unsigned P[RB + 2][DwSeg<T>::SRC];
-        dw_segments<T>(X, plane * H * W, x_elems, H, W, r0 - pu, c0 - pl, inside & 2, P);
+        const int rb = (int)(item / groups), c0 = (int)(item - (unsigned)rb * groups) * NC, end = STRICT ? min(w.Ho, (rb + 1) * DW_DRB) : 0;
+        const size_t plane = (size_t)(b0 + b) * w.C + ch;
+        int r0 = rb * DW_DRB;
+#pragma unroll 1
+        do {
+            unsigned G[RB][DwSeg<T>::OUT];
+            dw_segments<T>(dY, plane * w.Ho * w.Wo, w.y_elems, w.Ho, w.Wo, r0, c0, w.inside & 1, G);
+            unsigned P[RB + 2][DwSeg<T>::SRC];
+            dw_segments<T>(X, plane * w.H * w.W, w.x_elems, w.H, w.W, r0 - w.pu, c0 - w.pl, w.inside & 2, P);
 #pragma unroll
-        for (int hr = 0; hr < RB + 2; ++hr) {  // source row r0 - pu + hr meets gradient rows r0 + hr - i
-            unsigned U[4];  // (fp16: the pairs that start one element later)
-            if constexpr (sizeof(T) == 2) {
-#pragma unroll
-                for (int m = 0; m < 4; ++m) U[m] = __builtin_amdgcn_alignbit(P[hr][m + 1], P[hr][m], 16);
-            }
-#pragma unroll
-            for (int i = 0; i < 3; ++i) {
-                if (hr - i < 0 || hr - i >= RB) continue;
+            for (int hr = 0; hr < RB + 2; ++hr) {  // source row r0 - pu + hr meets gradient rows r0 + hr - i
 #pragma unroll
                 for (int j = 0; j < 3; ++j) {
-                    float a = acc[i][j];
+                    unsigned S[4];  // what tap column j reads (fp16, the odd one: the pairs that start one element later)
 #pragma unroll
                     for (int m = 0; m < 4; ++m) {
-                        const unsigned g = G[hr - i][m];
-                        if constexpr (sizeof(T) == 2)
-                            a = __builtin_amdgcn_fdot2(__builtin_bit_cast(dw_h2, j == 1 ? U[m] : P[hr][m + j / 2]),
-                                                       __builtin_bit_cast(dw_h2, g), a, false);
-                        else
-                            a = fmaf(__builtin_bit_cast(float, P[hr][m + j]), __builtin_bit_cast(float, g), a);
+                        if constexpr (sizeof(T) == 2) {
+                            S[m] = j == 1 ? __builtin_amdgcn_alignbit(P[hr][m + 1], P[hr][m], 16) : P[hr][m + j / 2];
+                            if (STRICT) S[m] &= (c0 + 2 * m < w.Wo ? 0xffffu : 0u) | (c0 + 2 * m + 1 < w.Wo ? 0xffff0000u : 0u);
+                        } else {
+                            S[m] = P[hr][m + j];
+                            if (STRICT) S[m] = c0 + m < w.Wo ? S[m] : 0u;
+                        }
                     }
-                    acc[i][j] = a;
+#pragma unroll
+                    for (int i = 0; i < 3; ++i) {
+                        if (hr - i < 0 || hr - i >= RB) continue;
+                        float a = acc[i][j];
+#pragma unroll
+                        for (int m = 0; m < 4; ++m) {
+                            const unsigned g = G[hr - i][m];
+                            if constexpr (sizeof(T) == 2)
+                                a = __builtin_amdgcn_fdot2(__builtin_bit_cast(dw_h2, S[m]), __builtin_bit_cast(dw_h2, g), a, false);
+                            else
+                                a = fmaf(__builtin_bit_cast(float, S[m]), __builtin_bit_cast(float, g), a);
+                        }
+                        acc[i][j] = a;
+                    }
                 }
             }
-        }
+        } while (STRICT && ++r0 < end);
+    }
+}
+
+template <typename T>
+__global__ __launch_bounds__(256) void dw_wg_direct_kernel(const T *__restrict__ X, const T *__restrict__ dY,
+                                                           float *__restrict__ part, int ns, int per_group, const DwWgWalk w,
+                                                           T *__restrict__ direct) {
+    constexpr int RB = DW_DRB, NC = DwSeg<T>::COLS;
+    __shared__ float red[4][9];
+    const int ch = blockIdx.x, grp = blockIdx.y;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int b0 = grp * per_group;
+    const unsigned per_plane = (unsigned)(((w.Wo + NC - 1) / NC) * ((w.Ho + RB - 1) / RB));
+    const unsigned items = per_plane * (unsigned)(min(ns, b0 + per_group) - b0), first = blockIdx.z * 256 + tid, step = 256 * gridDim.z;
+    float acc[3][3];
+    dw_wg_blocks<T, false>(X, dY, w, ch, b0, first, step, items, acc);
+    if (!(w.inside & 1)) {
+        bool none = false;
+#pragma unroll
+        for (int i = 0; i < 9; ++i) none = none || __builtin_isnan(acc[i / 3][i % 3]);
+        if (none) dw_wg_blocks<T, true>(X, dY, w, ch, b0, first, step, items, acc);
     }
 #pragma unroll
     for (int i = 0; i < 3; ++i)
@@ -878,7 +906,7 @@ __global__ __launch_bounds__(256) void dw_wg_direct_kernel(const T *__restrict__
         if (direct)
             direct[(size_t)ch * 9 + tid] = (T)sum;
         else
-            part[(((size_t)grp * gridDim.z + blockIdx.z) * C + ch) * 9 + tid] = sum;
+            part[(((size_t)grp * gridDim.z + blockIdx.z) * w.C + ch) * 9 + tid] = sum;
     }
 }
 
@@ -1088,8 +1116,8 @@ static int dw_step(const Args *a, int ns, int step, int sh, int sw, const char *
             const int whole = g.Ho % DW_DRB == 0 && g.Wo % DwSeg<T>::COLS == 0;  // blocks of the gradient
             const int inside = whole | (whole && g.Ho + 2 <= g.H && g.Wo + 2 <= g.W && g.Up == 0 && g.Lp == 0 ? 2 : 0);
             grid.z = (unsigned)shares;
-            hipLaunchKernelGGL((dw_wg_direct_kernel<T>), grid, dim3(256), 0, st.stream, X, dY, part, g.C, ns, per_group, g.H,
-                               g.W, g.Ho, g.Wo, g.Up, g.Lp, in_n, out_n, inside, direct);
+            const DwWgWalk w = {g.C, g.H, g.W, g.Ho, g.Wo, g.Up, g.Lp, inside, in_n, out_n};
+            hipLaunchKernelGGL((dw_wg_direct_kernel<T>), grid, dim3(256), 0, st.stream, X, dY, part, ns, per_group, w, direct);
         } else {
             bool pairs = false;
             if constexpr (sizeof(T) == 2) {
