@@ -28,12 +28,11 @@ void pulp_conv2d_fp32_bw_cl(void *p) {
     struct Conv2D_args *a = (struct Conv2D_args *)p;
     int rc = 0;
     ptl_internal_stage_begin();
-    if (a && a->skip_wg_grad == 0) rc = ptl_conv2d_fp32_bw_batched(a, 1);
-    /* (the weight gradient wants strides that divide the extent, the input gradient alone does not) */
-    if (a && a->skip_in_grad == 0 && (rc != 0 || a->skip_wg_grad != 0)) {
-        int r2 = ptl_conv2d_fp32_ig_batched(a, 1);
-        if (rc == 0) rc = r2;
-    }
+    if (a && !(a->skip_wg_grad && a->skip_in_grad)) rc = ptl_conv2d_fp32_bw_batched(a, 1);
+    /* a step that is refused leaves the other one (the weight gradient wants strides that divide the extent, the input
+     * gradient does not; a gradient's buffer may be missing) */
+    if (rc != 0 && a->skip_wg_grad == 0 && a->skip_in_grad == 0 && ptl_conv2d_fp32_ig_batched(a, 1) != 0)
+        (void)ptl_conv2d_fp32_wg_batched(a, 1);
     ptl_internal_set_status(ptl_internal_stage_end(a ? rc : 1));
 }
 
@@ -45,12 +44,11 @@ void pulp_conv2d_fp16_bw_cl(void *p) {
     struct Conv2D_args_fp16 *a = (struct Conv2D_args_fp16 *)p;
     int rc = 0;
     ptl_internal_stage_begin();
-    if (a && a->skip_wg_grad == 0) rc = ptl_conv2d_fp16_bw_batched(a, 1);
-    /* (the weight gradient wants strides that divide the extent, the input gradient alone does not) */
-    if (a && a->skip_in_grad == 0 && (rc != 0 || a->skip_wg_grad != 0)) {
-        int r2 = ptl_conv2d_fp16_ig_batched(a, 1);
-        if (rc == 0) rc = r2;
-    }
+    if (a && !(a->skip_wg_grad && a->skip_in_grad)) rc = ptl_conv2d_fp16_bw_batched(a, 1);
+    /* a step that is refused leaves the other one (the weight gradient wants strides that divide the extent, the input
+     * gradient does not; a gradient's buffer may be missing) */
+    if (rc != 0 && a->skip_wg_grad == 0 && a->skip_in_grad == 0 && ptl_conv2d_fp16_ig_batched(a, 1) != 0)
+        (void)ptl_conv2d_fp16_wg_batched(a, 1);
     ptl_internal_set_status(ptl_internal_stage_end(a ? rc : 1));
 }
 
@@ -205,6 +203,9 @@ void pulp_linear_fp32_bw_cl(void *p) {
     struct Linear_args *a = (struct Linear_args *)p;
     int rc = 0;
     if (a && !(a->skip_wg_grad && a->skip_in_grad)) rc = ptl_linear_fp32_bw_batched(a, 1);
+    /* a step that is refused (a buffer that it needs is missing) leaves the other one */
+    if (rc != 0 && a->skip_wg_grad == 0 && a->skip_in_grad == 0 && ptl_linear_fp32_ig_batched(a, 1) != 0)
+        (void)ptl_linear_fp32_wg_batched(a, 1);
     ptl_internal_set_status(a ? rc : 1);
 }
 
@@ -216,6 +217,9 @@ void pulp_linear_fp16_bw_cl(void *p) {
     struct Linear_args_fp16 *a = (struct Linear_args_fp16 *)p;
     int rc = 0;
     if (a && !(a->skip_wg_grad && a->skip_in_grad)) rc = ptl_linear_fp16_bw_batched(a, 1);
+    /* a step that is refused (a buffer that it needs is missing) leaves the other one */
+    if (rc != 0 && a->skip_wg_grad == 0 && a->skip_in_grad == 0 && ptl_linear_fp16_ig_batched(a, 1) != 0)
+        (void)ptl_linear_fp16_wg_batched(a, 1);
     ptl_internal_set_status(a ? rc : 1);
 }
 

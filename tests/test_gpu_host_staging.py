@@ -59,6 +59,54 @@ def test_a_rejected_step_returns_nothing_and_the_other_still_runs(pkg, gpu):
     assert np.all(dw == 3) and hp.rel_l2(dx, ref.numpy()) <= 1e-4
 
 
+@pytest.mark.parametrize("dt", ["fp32", "fp16"])
+@pytest.mark.parametrize("layer", ["linear", "conv2d", "conv2d_any"])
+@pytest.mark.parametrize("place", ["host", "device"])
+def test_a_step_without_a_buffer_leaves_the_other_one(pkg, gpu, dt, layer, place):
+    """A gradient's buffer (or the input that the weight gradient reads) is missing: the call fails, and the step that has
+    all of its tensors has run."""
+    nd = hp.np_dtype(dt)
+    n_in, n_out, Ci, Co, H = 24, 17, 16, 8, 8
+    conv = layer != "linear"
+    if layer == "conv2d_any":  # (the layer that the products with patch matrices take)
+        Ci, Co, H = 24, 40, 21
+    sh = ((Ci, H, H), (Co, Ci, 3, 3), (Co, H, H)) if conv else ((n_in,), (n_out, n_in), (n_out,))
+    x, w, dy = (hp.uniform(20 + i, s, dtype=nd) for i, s in enumerate(sh))
+    put = (lambda v: v.copy()) if place == "host" else (lambda v: torch.from_numpy(v).to(DEV))
+    get = lambda v: v if isinstance(v, np.ndarray) else v.cpu().numpy()
+
+    def run(missing):
+        tx, tdx, tw, tdw, ty, tdy = (put(v) for v in (x, np.full(sh[0], 3, nd), w, np.full(sh[1], 3, nd), np.zeros(sh[2], nd), dy))
+        if missing == "x":
+            tx = None
+        if missing == "dw":
+            tdw = None
+        if missing == "dx":
+            tdx = None
+        if conv:
+            a, keep = hp.conv2d_args(pkg, tx, tdx, tw, tdw, ty, tdy, Ci, H, H, Co, 3, 3, H, H, pad=(1, 1, 1, 1))
+        else:
+            a, keep = hp.linear_args(pkg, tx, tdx, tw, tdw, ty, tdy, n_in, n_out)
+        gpu.ptl_set_gemm_path(7 if layer == "conv2d_any" else 0)
+        try:
+            if missing:
+                with pytest.raises(RuntimeError):
+                    pkg.call("pulp_%s_%s_bw_cl" % ("conv2d" if conv else "linear", dt), a)
+            else:
+                pkg.call("pulp_%s_%s_bw_cl" % ("conv2d" if conv else "linear", dt), a)
+        finally:
+            gpu.ptl_set_gemm_path(0)
+        assert gpu.ptl_sync() == 0
+        return [None if t is None else get(t) for t in (tdx, tdw)]
+
+    dx, dw = run("")
+    for missing in ("x", "dw"):
+        got = run(missing)
+        assert hp.rel_l2(got[0], dx) <= (1e-3 if dt == "fp16" else 1e-5)
+        assert got[1] is None or np.all(got[1] == 3)
+    assert hp.rel_l2(run("dx")[1], dw) <= (1e-3 if dt == "fp16" else 1e-5)
+
+
 # (two parts and an odd end; the largest tensor with a block of its own: 32 MiB; one row beyond)
 @pytest.mark.parametrize("n_in,n_out", [(525, 1001), (2896, 2896), (2897, 2897)])
 def test_large_host_tensors_travel_in_parts(pkg, gpu, n_in, n_out):
