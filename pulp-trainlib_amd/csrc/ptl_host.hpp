@@ -12,6 +12,27 @@ void set_status(int s);
 int init_device(int device);
 int dw_noalloc_setup(int device);  // looks up the fixed partial-sum array of the current device
 
+// Whether two tensors (n elements of T each) share memory.  A launch that forms two gradients at once wants tensors that do
+// not: where they do, the steps run one after the other, each complete before the next (an input gradient may be
+// written over the input).
+template <typename T>
+inline bool share_memory(const T *a, size_t na, const T *b, size_t nb) {
+    return a && b && a < b + nb && b < a + na;
+}
+// Of a backward call: the gradients dW, dX and db against what the call reads and against each other.
+template <typename T>
+inline bool backward_shares_memory(const T *X, size_t nx, const T *W, size_t nw, const T *dY, size_t ny, const T *dW, const T *dX,
+                                   const T *db, size_t nb) {
+    const T *in[3] = {X, W, dY}, *out[3] = {dX, dW, db};
+    const size_t n_in[3] = {nx, nw, ny}, n_out[3] = {nx, nw, nb};
+    for (int o = 0; o < 3; ++o) {
+        for (int i = 0; i < 3; ++i)
+            if (share_memory(out[o], n_out[o], in[i], n_in[i])) return true;
+        if (share_memory(out[o], n_out[o], out[(o + 1) % 3], n_out[(o + 1) % 3])) return true;
+    }
+    return false;
+}
+
 struct StageBlock;  // pinned host memory and device memory of one size, from a pool (ptl_runtime.hip)
 
 // Maps caller pointers to device pointers.  Device pointers pass through;

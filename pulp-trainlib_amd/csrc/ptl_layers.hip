@@ -18,6 +18,7 @@
 #include "ptl_internal.h"
 
 #include <stdio.h>
+#include <algorithm>
 
 namespace ptl {
 
@@ -786,7 +787,16 @@ static int conv2d_bw(const Args *a, int ns, const char *fn) {
         return 1;
     }
     const bool wg = a->skip_wg_grad == 0, ig = a->skip_in_grad == 0;
-    if (wg && ig && a->USE_BIASES != 1 && ns >= 1 && a->input && a->coeff && a->output) {
+    bool apart = false;
+    if (wg && ig && ns >= 1 && a->input && a->coeff && a->output) {
+        auto at = [](const void *p) { return static_cast<const T *>(p); };
+        auto n = [&](const auto *b) { return (size_t)ns * (size_t)std::max(b->C, 0) * std::max(b->H, 0) * std::max(b->W, 0); };
+        const size_t nw = (size_t)std::max(a->output->C, 0) * std::max(a->input->C, 0) * std::max(a->coeff->H, 0) * std::max(a->coeff->W, 0);
+        apart = !backward_shares_memory<T>(at(a->input->data), n(a->input), at(a->coeff->data), nw, at(a->output->diff), n(a->output),
+                                           at(a->coeff->diff), at(a->input->diff),
+                                           a->USE_BIASES == 1 && a->bias ? at(a->bias->diff) : nullptr, (size_t)std::max(a->output->C, 0));
+    }
+    if (apart && a->USE_BIASES != 1) {
         ConvGeom g;
         if (int rc = conv_geom(a, g, fn, true)) return rc;
         const int P = g.Ho * g.Wo, Pk = g.Hk * g.Wk, K = g.Ci * Pk;
@@ -841,7 +851,7 @@ static int conv2d_bw(const Args *a, int ns, const char *fn) {
     // Both gradients as products with patch matrices, except where one of them has a kernel of its own that is ahead: the
     // resident-tile kernels, and the raw-tile weight gradient of large unit-stride 3x3 and 1x1 layers (26 us against 48 for
     // 128 -> 32 channels on 22 x 32 at batch 94).
-    if (wg && ig && ns >= 1 && a->input && a->coeff && a->output && (a->USE_BIASES != 1 || a->bias)) {
+    if (apart && (a->USE_BIASES != 1 || a->bias)) {
         ConvGeom g;
         if (int rc = conv_geom(a, g, fn, true)) return rc;
         if (!ensure_init()) return 2;
@@ -1024,7 +1034,8 @@ static int linear_step(const Args *a, int ns, int step, const char *fn) {
         T *dX = sg.out(reinterpret_cast<T *>(a->input->diff), (size_t)ns * in);
         T *db = use_bias ? sg.out(reinterpret_cast<T *>(a->bias->diff), (size_t)out) : nullptr;
         if (sg.failed()) return 2;
-        if (ns == 1) return sg.finish(linear_one_bw<T>(X, Wt, dY, dW, dX, db, in, out));
+        const bool apart = !backward_shares_memory<T>(X, (size_t)ns * in, Wt, (size_t)out * in, dY, (size_t)ns * out, dW, dX, db, (size_t)out);
+        if (ns == 1 && apart) return sg.finish(linear_one_bw<T>(X, Wt, dY, dW, dX, db, in, out));
         GemmArgs q = {}, r = {};
         q.A = dY;  // dW[o][i] = sum_b dY[b][o] * X[b][i]
         q.B = X;
@@ -1057,6 +1068,11 @@ static int linear_step(const Args *a, int ns, int step, const char *fn) {
         // size up to the work at which the look-up-free kernels' larger tiles make up for two launches.
         const double flops = 4.0 * ns * in * out;
         rc = -1;
+        if (!apart) {
+            rc = ns == 1 ? mm_dispatch<T>(dY, X, dW, out, in, 1, 0) : gemm<T>(q);
+            if (rc == 0 && db) rc = bias_grad<T>(dY, db, ns, out, 1, 1);
+            return sg.finish(rc ? rc : mm_dispatch<T>(dY, Wt, dX, ns, in, out, 0));
+        }
         if (!db || flops > 4e9) rc = gemm_pair_lean<T>(q, r);
         if (rc < 0 && state().gemm_path == 0 && flops <= (sizeof(T) == 2 ? 3e10 : 1e10)) {
             rc = linear_bw_ragged<T>(X, Wt, dY, dW, dX, db, ns, in, out);

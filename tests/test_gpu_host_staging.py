@@ -107,6 +107,37 @@ def test_a_step_without_a_buffer_leaves_the_other_one(pkg, gpu, dt, layer, place
     assert hp.rel_l2(run("dx")[1], dw) <= (1e-3 if dt == "fp16" else 1e-5)
 
 
+@pytest.mark.parametrize("dt", ["fp32", "fp16"])
+@pytest.mark.parametrize("place", ["host", "device"])
+# dense layers: one sample, a batch on whole tiles, one on none; convolutions: small, wide, with patch matrices
+@pytest.mark.parametrize("layer,ns,Ci,Co,H", [("linear", 1, 300, 5000, 0), ("linear", 64, 256, 256, 0), ("linear", 33, 127, 65, 0),
+                                              ("conv2d", 1, 16, 32, 32), ("conv2d", 8, 64, 64, 16), ("conv2d", 5, 40, 130, 21)])
+def test_an_input_gradient_written_over_the_input(pkg, gpu, dt, place, layer, ns, Ci, Co, H):
+    """The weight gradient still is that of the input."""
+    nd = hp.np_dtype(dt)
+    conv = layer == "conv2d"
+    sh = ((ns, Ci, H, H), (Co, Ci, 3, 3), (ns, Co, H, H)) if conv else ((ns, Ci), (Co, Ci), (ns, Co))
+    x, w, dy = (hp.uniform(30 + i, s, dtype=nd) for i, s in enumerate(sh))
+    put = (lambda v: v.copy()) if place == "host" else (lambda v: torch.from_numpy(v).to(DEV))
+    get = lambda v: v if isinstance(v, np.ndarray) else v.cpu().numpy()
+    res = []
+    for alias in (0, 1):
+        tx, tw, tdw, ty, tdy = (put(v) for v in (x, w, np.full(sh[1], 3, nd), np.zeros(sh[2], nd), dy))
+        tdx = tx if alias else put(np.full(sh[0], 3, nd))
+        if conv:
+            a, keep = hp.conv2d_args(pkg, tx, tdx, tw, tdw, ty, tdy, Ci, H, H, Co, 3, 3, H, H, pad=(1, 1, 1, 1))
+        else:
+            a, keep = hp.linear_args(pkg, tx, tdx, tw, tdw, ty, tdy, Ci, Co)
+        if ns == 1:
+            pkg.call("pulp_%s_%s_bw_cl" % (layer, dt), a)
+        else:
+            pkg.call("ptl_%s_%s_bw_batched" % (layer, dt), a, ns)
+        assert gpu.ptl_sync() == 0
+        res.append([get(tdx), get(tdw)])
+    for got, want in zip(res[1], res[0]):
+        assert hp.rel_l2(got, want) <= (1e-3 if dt == "fp16" else 1e-5)
+
+
 # (two parts and an odd end; the largest tensor with a block of its own: 32 MiB; one row beyond)
 @pytest.mark.parametrize("n_in,n_out", [(525, 1001), (2896, 2896), (2897, 2897)])
 def test_large_host_tensors_travel_in_parts(pkg, gpu, n_in, n_out):
