@@ -70,7 +70,9 @@ class Stager {
     void discard();
 
     // The Stager that those made on this thread from now on share (NULL: each its own): a call made of several steps
-    // fetches every host tensor once and waits once, at the end.  A step that fails still returns nothing.
+    // fetches every host tensor once and waits once, at the end.  A step that fails still returns nothing.  What a step
+    // has written is what the next one reads, at the same address; host tensors of a call that overlap in part are taken
+    // for different ones.
     static Stager *&scope();
 
    private:
@@ -80,6 +82,7 @@ class Stager {
         size_t bytes;
         bool copy_out;
         bool copied_in;
+        bool written;       // by a step that succeeded: the device's copy is the valid one
         bool own;           // block is this tensor's alone
         bool pending;       // in the pinned half of the shared block, to be fetched
         StageBlock *block;  // dev lies in it; NULL: a buffer of its own

@@ -374,10 +374,9 @@ bool Stager::failed() {
     return failed_;
 }
 
-// What a step of a shared call wrote goes back to the caller only if the step succeeded.
+// What a step of a shared call wrote goes back to the caller, and is what later steps read, only if the step succeeded.
 void Stager::keep_outputs(bool keep) {
-    if (!keep)
-        for (size_t i : marked_) root_->items_[i].copy_out = false;
+    for (size_t i : marked_) (keep ? root_->items_[i].written : root_->items_[i].copy_out) = keep;
     marked_.clear();
 }
 
@@ -446,8 +445,8 @@ void *Stager::map(const void *host_or_dev, size_t bytes, bool copy_in, bool copy
         hit->copy_out = true;
         if (root_) marked_.push_back((size_t)(hit - r.items_.data()));
     }
-    // a tensor first mapped as an output and later as an input still gets its contents
-    if (copy_in && !hit->copied_in) {
+    // a tensor first mapped as an output and later as an input of the same step still gets its contents
+    if (copy_in && !hit->copied_in && !hit->written) {
         if (hit->own) {
             if (!block_send(hit->block, host_or_dev, hit->bytes)) {
                 failed_ = true;

@@ -138,6 +138,24 @@ def test_an_input_gradient_written_over_the_input(pkg, gpu, dt, place, layer, ns
         assert hp.rel_l2(got, want) <= (1e-3 if dt == "fp16" else 1e-5)
 
 
+# (small tensors, which share a block; one with a block of its own)
+@pytest.mark.parametrize("Ci,Co,P", [(12, 20, 35), (700, 600, 9)])
+def test_a_step_reads_what_the_step_before_it_wrote(pkg, gpu, Ci, Co, P):
+    """The weight gradient written over the weights: the input gradient is formed with it, on the host as on the device."""
+    x, w, dy = (hp.uniform(40 + i, s) for i, s in enumerate(((Ci, P), (Co, Ci), (Co, P))))
+    res = []
+    for put in (lambda v: v.copy(), lambda v: torch.from_numpy(v).to(DEV)):
+        tx, tdx, tw, ty, tdy = (put(v) for v in (x, np.zeros_like(x), w, np.zeros_like(dy), dy))
+        a, keep = hp.pw_args(pkg, tx, tdx, tw, tw, ty, tdy, Ci, Co, 1, P)
+        pkg.call("pulp_conv_pw_fp32_bw_cl", a)
+        assert gpu.ptl_sync() == 0
+        res.append([v if isinstance(v, np.ndarray) else v.cpu().numpy() for v in (tdx, tw)])
+    dw = dy.astype(np.float64) @ x.T.astype(np.float64)
+    assert hp.rel_l2(res[0][1], dw) <= 1e-5 and hp.rel_l2(res[0][0], dw.T @ dy) <= 1e-5
+    for h, d in zip(*res):
+        assert np.array_equal(h, d)
+
+
 # (two parts and an odd end; the largest tensor with a block of its own: 32 MiB; one row beyond)
 @pytest.mark.parametrize("n_in,n_out", [(525, 1001), (2896, 2896), (2897, 2897)])
 def test_large_host_tensors_travel_in_parts(pkg, gpu, n_in, n_out):
