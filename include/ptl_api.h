@@ -315,9 +315,11 @@ int ptl_sync(void);
  * the tap route kept its input tile in LDS (1), or ran the small-layer kernels
  * (2: forward, either gradient, or both gradients in one call; 3: the forward
  * kernel that also applied the normalisation in front of the layer, see
- * ptl_conv2d_*_fw_batched_normed);
+ * ptl_conv2d_*_fw_batched_normed), or products with patch matrices on channel-
+ * minor copies of channel-major tensors (4);
  * ptl_last_gemm_tile() the output tile of the last product that ran a tile-per-workgroup kernel of the
- * look-up-free pipelined GEMM, as rows * 1000 + columns (256256 = 256 x 256, 128064 = 128 x 64). */
+ * look-up-free pipelined GEMM or of the kernel for any size and alignment (of several products in one launch, all of
+ * them), as rows * 1000 + columns (256256 = 256 x 256, 128064 = 128 x 64). */
 void ptl_set_gemm_path(int path);
 int ptl_last_conv_direct(void);
 int ptl_last_gemm_streamed(void);

@@ -196,6 +196,7 @@ int conv_any_fw(const ConvTileDesc &d, const void *X, const void *Wt, const void
     if (!any_fits(d, ES) || (d.in_hwc ? d.Cin < VEC : K < VEC)) return -1;
     const AnyPlan &plan = any_plan<T>(d, ANY_FW);
     const bool turn = plan.turn, minor = d.in_hwc || turn;
+    state().last_conv_resident = turn ? 4 : 0;
     const int Cp = any_padded(d.Cin, ES), Kp = taps * Cp;
     RagConvArgs r = {};
     if (turn || (d.in_hwc && Kp != K)) {  // filters tap by tap, whole pieces of channels; the image channel-minor
@@ -284,6 +285,7 @@ int conv_any_bw(const ConvTileDesc &d, const void *X, const void *dY, const void
     if (!any_fits(d, ES) || (d.in_hwc && (d.Cin < VEC || d.Cout < VEC))) return -1;
     const AnyPlan &plan = any_plan<T>(d, (dW ? ANY_WG : 0) | (dX ? ANY_IG : 0));
     const bool turn = plan.turn && d.Cout >= VEC, minor = d.in_hwc || turn;
+    state().last_conv_resident = turn ? 4 : 0;
     const int Cip = any_padded(d.Cin, ES), Cop = any_padded(d.Cout, ES);
     // scratch: the filters as the input gradient reads them; channel-minor copies of the gradient and of the input
     const size_t w_bytes = dX ? ((size_t)d.Cin * taps * (minor ? Cop : d.Cout) * ES + 255) / 256 * 256 : 0;
