@@ -1406,7 +1406,8 @@ static int mhsa_bw(const Mhsa_args *a, int ns, const char *fn) {
     const float *P = sg.in(a->softmax_buffer->data, pe);
     float *dP = sg.out(a->softmax_buffer->diff, pe);
     if (sg.failed()) return 2;
-    const size_t p1 = panel_part_floats(1, E, F, ns), p3 = panel_part_floats(3, F, E, ns);
+    const bool rag = rag_takes(m);  // (its partial sums, where there are any, are in the workspace)
+    const size_t p1 = rag ? 0 : panel_part_floats(1, E, F, ns), p3 = rag ? 0 : panel_part_floats(3, F, E, ns);
     float *rs = static_cast<float *>(scratch((rows + p1 + p3) * sizeof(float)));
     if (!rs) return 2;
     float *part_o = rs + rows, *part_i = part_o + p1;  // sample-group sums of the output / the input weights' gradients
@@ -1414,7 +1415,6 @@ static int mhsa_bw(const Mhsa_args *a, int ns, const char *fn) {
     // dWout[E x F] = sum over samples of dY . att^T (:742-760) and datt[F x L] = Wout^T . dY (:816-834), one launch;
     // the sample groups of dWout are added up at the end, together with those of the input weights' gradients
     PanelArgs pwo = acts_times_acts(E, F, L, ns);
-    const bool rag = rag_takes(m);
     if (rag) {  // (dWout comes with the other weights' gradients)
         RagArgs r = {};
         r.shape = rag_tile_of(L);

@@ -29,6 +29,22 @@ def test_reserve_grows_and_reports(pkg, gpu):
     assert ws2 == ws1 and sc2 >= max(sc1, 1)
 
 
+def test_attention_reserves_no_partial_sums_of_kernels_it_does_not_run(pkg, gpu):
+    """The backward pass keeps a row of sums (12 KB here) in the scratch buffer; the partial sums of the panel products, which
+    only layers of fewer than four tokens or features run, would be 8.7 MB, more than the buffer's first size of 8 MiB."""
+    ns, L, E, F, heads = 64, 16, 192, 192, 3
+    sh = hp.mhsa_shapes(ns, L, E, F, heads)
+    data = {n: torch.rand(s, device=DEV) for n, s in sh.items()}
+    diff = {n: torch.zeros(s, device=DEV) for n, s in sh.items()}
+    for n in ("wq", "wk", "wv"):
+        diff[n] = torch.zeros((F, E), device=DEV)
+    a, keep = hp.mhsa_args(pkg, data, diff, L, E, F, heads)
+    _, before = reserved(gpu)
+    assert gpu.ptl_mhsa_fp32_bw_batched(ctypes.byref(a), ns) == 0, gpu.ptl_last_error().decode()
+    assert gpu.ptl_sync() == 0
+    assert reserved(gpu)[1] <= max(before, 8 << 20)
+
+
 def test_growth_and_stream_switch_are_refused_under_capture_and_reserve_makes_the_call_capturable(pkg, gpu):
     """A strided input gradient on the general GEMM route zero-stuffs the output gradient into the library's scratch
     buffer.  Captured when that buffer is too small, the call fails with status 2 and names ptl_reserve; the capture
