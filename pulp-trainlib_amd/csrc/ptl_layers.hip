@@ -292,12 +292,24 @@ static ConvTileDesc forward_desc(const ConvGeom &g, int ns) {
 }
 
 // Whether the products with patch matrices (ptl_conv_any.hip) go before the kernels for small problems (raw tiles of one
-// image, the gathering product): by the multiplications of a step, counted by how full its tiles are.  Measured on 300
-// layers from 1 x 3 -> 8 channels on 7 x 7 to 200 x 500 -> 500 on 64 x 64; below these lines they are 10-30 % behind (their
-// launches cost 2-3 us more: addresses of patches before the first load), above 1.1 to 6 times as fast.  Strides: the other
-// route of the input gradient runs over a zero-stuffed tensor.  Channel-minor layers whose channels are no whole pieces have
-// their filters re-laid first, as all have for the input gradient (not worth it for a handful of pixels).  A bias is a launch
-// of its own on the other routes.
+// image, the gathering product): by the millions of multiplications of a step, counted by how full its tiles are.  Strides:
+// the other route of the input gradient runs over a zero-stuffed tensor.  Channel-minor layers whose channels are no whole
+// pieces (`odd`) have their filters re-laid first, as all have for the input gradient.  A bias is a launch of its own on
+// the other routes.  Both routes were timed on 5000 layers (1 to 128 samples, 3 to 512 channels on 7 to 64 pixels, 1 to 25
+// taps, strides 1 and 2, tensors in turn), forced one after the other.  Time of the other route over this one's, mean of
+// the layers between a third of the line and the line; between the line and three times it; and what the rule loses to the
+// better of the two for each layer, in the mean:
+//   forward         fp16 240: 1.14, 1.16, 13 %; fp32 5: 1.23, 1.12, 8 %; channel-minor fp16 5: 1.43, 1.40, 6 %, odd 200:
+//                   0.89, 1.01, 4 %; fp32 60: 1.13, 1.19, 10 %, odd 600: 0.90, 1.08, 2 %
+//   weight gradient 300: 0.96, 1.07, 4 %; strided 200: 1.00, 1.05, 7 %; channel-minor fp16 20: 1.16, 1.20, 7 %, fp32 300:
+//                   1.02, 1.15, 8 %
+//   input gradient  strided 15: 1.22, 1.40, 7 %; fp16 300: 0.93, 1.17, 4 %, channel-minor 240: 0.89, 1.13, 3 %; fp32 320:
+//                   0.90, 1.11, 4 %, channel-minor 1500: 1.15, 1.16, 4 %; few pixels under many filters, whose re-laying
+//                   takes longer than the product, are left out: 0.70
+//   both            by the input gradient's lines: strided 1.39, 1.49, 11 %; fp16 1.07, 1.21, 6 %, channel-minor 1.26, 1.50,
+//                   13 %; fp32 1.04, 1.21, 5 %, channel-minor 1.32, 1.39, 11 %
+// Where a line lies higher than these figures ask for, layers keep the route they had; for fp32 there is a reason to: these
+// tiles add in longer chains, which leaves results 14 to 18 % further from 64 bits in the mean (1.6e-7 against 1.4e-7).
 template <typename T>
 static bool any_pays(const ConvGeom &g, int ns, int steps, bool bias) {
     if (state().gemm_path == 7) return true;
@@ -309,10 +321,7 @@ static bool any_pays(const ConvGeom &g, int ns, int steps, bool bias) {
     double mflop = 2e-6 * ns * g.Co * g.Ho * g.Wo * K * fill(g.Co, 32) * fill(K, 64);
     if (g.hwc) mflop *= fill(g.Ci, VEC);
     if (bias) mflop *= steps == 1 ? 4 : 1.5;
-    if (steps == 1) {
-        if (half && !g.hwc && !strided && g.Co <= 16) return false;  // (the raw tiles: 31 against 42 us for 38 -> 16 on 50 x 37)
-        return mflop >= (g.hwc ? (odd ? (half ? 200 : 600) : half ? 5 : 60) : half ? 240 : 5);
-    }
+    if (steps == 1) return mflop >= (g.hwc ? (odd ? (half ? 200 : 600) : half ? 5 : 60) : half ? 240 : 5);
     if (steps == 2) return mflop >= (g.hwc ? (half ? 20 : 300) : strided ? 200 : 300);
     if ((long long)ns * g.H * g.W < 256 && (long long)g.Co * K > (1 << 18)) return false;
     return mflop >= (strided ? 15 : half ? (g.hwc ? 240 : 300) : g.hwc ? 1500 : 320);
