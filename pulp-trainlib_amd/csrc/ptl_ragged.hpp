@@ -77,6 +77,7 @@ struct RagProd {
     void *row_sum;     // sum over k of a(n, k); in the first product of (RC, RC) before (KC, RC), and with b gathered along k
     // set by the launcher
     float *ws;         // partial sums [split][N][pitch]
+    float *ws_sums;    // of the row sums [split][N]
     int pitch, splits, slabs_per_split;
     int tiles_n, tiles_m, tiles_in;  // tiles along n, along m, along m inside one outer digit
 };
@@ -96,6 +97,7 @@ struct RagSums {  // the products whose contraction was split
     RagProd p[5];
     int first[6];
     int count;
+    int sums;  // the one whose row sums are wanted, or -1
 };
 
 // The products in one launch (plus one for their partial sums where the contraction is split).  The first product has
