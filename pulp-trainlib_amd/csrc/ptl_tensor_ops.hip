@@ -810,8 +810,10 @@ __global__ __launch_bounds__(256) void dw_direct_kernel(const T *__restrict__ sr
 // sums stay in registers; one reduction per workgroup at the end.  part[((grp * shares + share) * C + ch) * 9 + tap], or
 // the gradient itself when there is one workgroup per channel.
 // A block that reaches over the end of the gradient multiplies what the source has there with zeros, which of an infinity
-// makes no number: a lane whose sums end as one goes over its blocks again, row by row and without the columns that do
-// not exist (STRICT; leaving them out always took 3 to 9 % longer, whole blocks need too many registers for four waves).
+// makes no number.  Where sums end as one, the blocks are gone over again, row by row and without the columns that do not
+// exist (STRICT): by the lanes of the kernel that writes the gradient, which is this one if a channel has one workgroup and
+// the one that adds the workgroups' sums otherwise.  (Leaving these products out always took 3 to 9 % longer, code for
+// a second pass in the kernel of many workgroups 1 of 10 us.)
 struct DwWgWalk {
     int C, H, W, Ho, Wo, pu, pl, inside;
     size_t x_elems, y_elems;
@@ -871,25 +873,9 @@ __device__ inline void dw_wg_blocks(const T *__restrict__ X, const T *__restrict
     }
 }
 
-template <typename T>
-__global__ __launch_bounds__(256) void dw_wg_direct_kernel(const T *__restrict__ X, const T *__restrict__ dY,
-                                                           float *__restrict__ part, int ns, int per_group, const DwWgWalk w,
-                                                           T *__restrict__ direct) {
-    constexpr int RB = DW_DRB, NC = DwSeg<T>::COLS;
-    __shared__ float red[4][9];
-    const int ch = blockIdx.x, grp = blockIdx.y;
+// Tap sums of the lanes -> those of the workgroup, in its first nine threads.
+__device__ inline float dw_wg_fold(const float (&acc)[3][3], float (*red)[9]) {
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int b0 = grp * per_group;
-    const unsigned per_plane = (unsigned)(((w.Wo + NC - 1) / NC) * ((w.Ho + RB - 1) / RB));
-    const unsigned items = per_plane * (unsigned)(min(ns, b0 + per_group) - b0), first = blockIdx.z * 256 + tid, step = 256 * gridDim.z;
-    float acc[3][3];
-    dw_wg_blocks<T, false>(X, dY, w, ch, b0, first, step, items, acc);
-    if (!(w.inside & 1)) {
-        bool none = false;
-#pragma unroll
-        for (int i = 0; i < 9; ++i) none = none || __builtin_isnan(acc[i / 3][i % 3]);
-        if (none) dw_wg_blocks<T, true>(X, dY, w, ch, b0, first, step, items, acc);
-    }
 #pragma unroll
     for (int i = 0; i < 3; ++i)
 #pragma unroll
@@ -900,14 +886,68 @@ __global__ __launch_bounds__(256) void dw_wg_direct_kernel(const T *__restrict__
             if (lane == 0) red[wave][i * 3 + j] = v;
         }
     __syncthreads();
-    if (tid < 9) {
-        const float *r = &red[0][0] + tid;
-        const float sum = (r[0] + r[9]) + (r[18] + r[27]);
-        if (direct)
-            direct[(size_t)ch * 9 + tid] = (T)sum;
-        else
-            part[(((size_t)grp * gridDim.z + blockIdx.z) * w.C + ch) * 9 + tid] = sum;
+    const float *r = &red[0][0] + min(tid, 8);
+    return (r[0] + r[9]) + (r[18] + r[27]);
+}
+
+// ALONE: one workgroup a channel, which writes the gradient.
+template <typename T, bool ALONE>
+__global__ __launch_bounds__(256) void dw_wg_direct_kernel(const T *__restrict__ X, const T *__restrict__ dY,
+                                                           float *__restrict__ part, int ns, int per_group, const DwWgWalk w,
+                                                           T *__restrict__ dW) {
+    constexpr int RB = DW_DRB, NC = DwSeg<T>::COLS;
+    __shared__ float red[4][9];
+    const int ch = blockIdx.x, grp = blockIdx.y, tid = threadIdx.x, b0 = grp * per_group;
+    const unsigned per_plane = (unsigned)(((w.Wo + NC - 1) / NC) * ((w.Ho + RB - 1) / RB));
+    const unsigned items = per_plane * (unsigned)(min(ns, b0 + per_group) - b0), first = blockIdx.z * 256 + tid, step = 256 * gridDim.z;
+    float acc[3][3];
+    dw_wg_blocks<T, false>(X, dY, w, ch, b0, first, step, items, acc);
+    if constexpr (ALONE) {
+        if (!(w.inside & 1)) {
+            bool none = false;
+#pragma unroll
+            for (int i = 0; i < 9; ++i) none = none || __builtin_isnan(acc[i / 3][i % 3]);
+            if (none) dw_wg_blocks<T, true>(X, dY, w, ch, b0, first, step, items, acc);
+        }
     }
+    const float sum = dw_wg_fold(acc, red);
+    if (tid < 9) {
+        if constexpr (ALONE) dW[(size_t)ch * 9 + tid] = (T)sum;
+        else part[(((size_t)grp * gridDim.z + blockIdx.z) * w.C + ch) * 9 + tid] = sum;
+    }
+}
+
+// dW[ch][tap] = sum over the shares of part[(share * C + ch) * 9 + tap]: nine consecutive threads read one share.
+template <typename T>
+__global__ __launch_bounds__(256) void dw_wg_direct_sum_kernel(const T *__restrict__ X, const T *__restrict__ dY,
+                                                               const float *__restrict__ part, int ns, int shares, const DwWgWalk w,
+                                                               T *__restrict__ dW) {
+    constexpr int SL = 256 / 9;
+    __shared__ float red[SL][9];
+    __shared__ float wide[4][9];
+    __shared__ int strict;
+    const int ch = blockIdx.x, tid = threadIdx.x, tap = tid % 9, slice = tid / 9;
+    float s = 0.f;
+    if (slice < SL) {
+        for (int z = slice; z < shares; z += SL) s += part[((size_t)z * w.C + ch) * 9 + tap];
+        red[slice][tap] = s;
+    }
+    if (tid == 0) strict = 0;
+    __syncthreads();
+    if (tid < 9) {
+        s = 0.f;
+        for (int k = 0; k < SL; ++k) s += red[k][tid];
+        if (__builtin_isnan(s) && !(w.inside & 1)) strict = 1;
+    }
+    __syncthreads();
+    if (strict) {
+        constexpr int RB = DW_DRB, NC = DwSeg<T>::COLS;
+        const unsigned items = (unsigned)(((w.Wo + NC - 1) / NC) * ((w.Ho + RB - 1) / RB)) * (unsigned)ns;
+        float acc[3][3];
+        dw_wg_blocks<T, true>(X, dY, w, ch, 0, tid, 256, items, acc);
+        s = dw_wg_fold(acc, wide);
+    }
+    if (tid < 9) dW[(size_t)ch * 9 + tid] = (T)s;
 }
 
 template <typename Args>
@@ -1117,7 +1157,12 @@ static int dw_step(const Args *a, int ns, int step, int sh, int sw, const char *
             const int inside = whole | (whole && g.Ho + 2 <= g.H && g.Wo + 2 <= g.W && g.Up == 0 && g.Lp == 0 ? 2 : 0);
             grid.z = (unsigned)shares;
             const DwWgWalk w = {g.C, g.H, g.W, g.Ho, g.Wo, g.Up, g.Lp, inside, in_n, out_n};
-            hipLaunchKernelGGL((dw_wg_direct_kernel<T>), grid, dim3(256), 0, st.stream, X, dY, part, ns, per_group, w, direct);
+            if (direct) {
+                hipLaunchKernelGGL((dw_wg_direct_kernel<T, true>), grid, dim3(256), 0, st.stream, X, dY, part, ns, per_group, w, dW);
+            } else {
+                hipLaunchKernelGGL((dw_wg_direct_kernel<T, false>), grid, dim3(256), 0, st.stream, X, dY, part, ns, per_group, w, dW);
+                hipLaunchKernelGGL((dw_wg_direct_sum_kernel<T>), dim3(g.C), dim3(256), 0, st.stream, X, dY, part, ns, sgroups * shares, w, dW);
+            }
         } else {
             bool pairs = false;
             if constexpr (sizeof(T) == 2) {
@@ -1131,9 +1176,8 @@ static int dw_step(const Args *a, int ns, int step, int sh, int sw, const char *
                 hipLaunchKernelGGL((dw_wg_plane_kernel<T, 5>), grid, dim3(256), lds, st.stream, X, dY, part, g.C, ns,
                                    per_group, g.H, g.W, g.Ho, g.Wo, g.Up, g.Lp, x_vecs, direct);
         }
-        if (!direct)
-            hipLaunchKernelGGL((dw_wg_reduce_kernel2<T>), dim3(g.C), dim3(256), 0, st.stream, part, dW, sgroups * shares, g.C, 1,
-                               taps);
+        if (!direct && !direct_path)
+            hipLaunchKernelGGL((dw_wg_reduce_kernel2<T>), dim3(g.C), dim3(256), 0, st.stream, part, dW, sgroups, g.C, 1, taps);
     } else if (rows_path) {
         const T *X = sg.in(reinterpret_cast<const T *>(a->input->data), in_n);
         const T *dY = sg.in(reinterpret_cast<const T *>(a->output->diff), out_n);
