@@ -301,6 +301,9 @@ static ConvTileDesc forward_desc(const ConvGeom &g, int ns) {
 // better of the two for each layer, in the mean:
 //   forward         fp16 240: 1.14, 1.16, 13 %; fp32 5: 1.23, 1.12, 8 %; channel-minor fp16 5: 1.43, 1.40, 6 %, odd 200:
 //                   0.89, 1.01, 4 %; fp32 60: 1.13, 1.19, 10 %, odd 600: 0.90, 1.08, 2 %
+//                   (fp16, at most 16 filters at unit stride: 1.17 in the mean of 163 layers, but 0.99 (0.92 to 1.07) of the
+//                   four over more than 10^5 pixels, where the raw tiles read each input once for their few filters; 68 -> 8
+//                   on 42 x 42, 143 samples, bias: 171.8 us there, 183.6 here.  Those stay there.)
 //   weight gradient 300: 0.96, 1.07, 4 %; strided 200: 1.00, 1.05, 7 %; channel-minor fp16 20: 1.16, 1.20, 7 %, fp32 300:
 //                   1.02, 1.15, 8 %
 //   input gradient  strided 15: 1.22, 1.40, 7 %; fp16 300: 0.93, 1.17, 4 %, channel-minor 240: 0.89, 1.13, 3 %; fp32 320:
@@ -321,7 +324,10 @@ static bool any_pays(const ConvGeom &g, int ns, int steps, bool bias) {
     double mflop = 2e-6 * ns * g.Co * g.Ho * g.Wo * K * fill(g.Co, 32) * fill(K, 64);
     if (g.hwc) mflop *= fill(g.Ci, VEC);
     if (bias) mflop *= steps == 1 ? 4 : 1.5;
-    if (steps == 1) return mflop >= (g.hwc ? (odd ? (half ? 200 : 600) : half ? 5 : 60) : half ? 240 : 5);
+    if (steps == 1) {
+        if (half && !g.hwc && !strided && g.Co <= 16 && (long long)ns * g.Ho * g.Wo > 100000) return false;
+        return mflop >= (g.hwc ? (odd ? (half ? 200 : 600) : half ? 5 : 60) : half ? 240 : 5);
+    }
     if (steps == 2) return mflop >= (g.hwc ? (half ? 20 : 300) : strided ? 200 : 300);
     if ((long long)ns * g.H * g.W < 256 && (long long)g.Co * K > (1 << 18)) return false;
     return mflop >= (strided ? 15 : half ? (g.hwc ? 240 : 300) : g.hwc ? 1500 : 320);
