@@ -304,7 +304,12 @@ int ptl_sync(void);
  * stride 1 or 2, at most 64 channels on either side, fp16 and fp32; by default
  * only up to four - for layers narrower than 64 channels sixteen - workgroups
  * per compute unit, and for the weight gradient only up to 262144 positions)
- * are taken whenever the geometry fits them.
+ * are taken whenever the geometry fits them; self-attention runs its products
+ * as resident panels (by default only for fewer than four tokens, channels or
+ * channels per head);
+ * 7 = a Conv2D runs as products with patch matrices (any filter, stride and
+ * padding; by default where they measured better) wherever its offsets fit 31
+ * bits; self-attention runs its panel products one to a launch.
  * All routes compute the same products.
  * ptl_last_conv_direct() tells whether the last Conv2D call ran one of the
  * convolution kernels (1) or the implicit-im2col GEMM (0);

@@ -1071,7 +1071,8 @@ static int dw_step(const Args *a, int ns, int step, int sh, int sw, const char *
     const bool plane_path = rows_path && g.Hk == 5 && in_img <= 40 * 1024 && out_img <= 40 * 1024 && planes >= 2L * st.num_cu &&
                             planes < ((long)1 << 31) && st.gemm_path != 1;
     // 3x3, unit stride: straight from global memory, whatever the extents, the alignment and the number of planes (the
-    // tensors hold at least one segment; offsets within a plane and the blocks of all planes are 31-bit numbers)
+    // tensors hold at least one segment; offsets within a plane and the blocks of all planes are 31-bit numbers: planes of
+    // 2^29 elements and more, and calls that ask for the kernels without fast paths, keep the row kernels)
     auto fits = [](size_t elems, int h, int w, long n) {
         return elems >= 16 && (long long)h * w < (1LL << 29) &&
                (long long)n * ((h + DW_DRB - 1) / DW_DRB) * ((w + DwSeg<T>::COLS - 1) / DwSeg<T>::COLS) < (1LL << 31);
