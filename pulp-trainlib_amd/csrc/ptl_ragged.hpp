@@ -76,8 +76,7 @@ struct RagProd {
     int add;           // C keeps what it holds, the product is added to it
     void *row_sum;     // sum over k of a(n, k); in the first product of (RC, RC) before (KC, RC), and with b gathered along k
     // set by the launcher
-    float *ws;         // partial sums [split][N][pitch]
-    float *ws_sums;    // of the row sums [split][N]
+    float *ws;         // partial sums [split][N][pitch], behind them those of the row sums [split][N]
     int pitch, splits, slabs_per_split;
     int tiles_n, tiles_m, tiles_in;  // tiles along n, along m, along m inside one outer digit
 };
