@@ -847,8 +847,9 @@ static GvShares gv_shares(int K, int M) {
     const int cu = state().num_cu, z = std::min({2 * cu / sh.cols, K / 512, 32});
     if (K < 4096 || sh.cols > cu / 2 || z < 2) return sh;
     const int chunk = (K + z - 1) / z, shares = (K + chunk - 1) / chunk;
-    // (a stream that is being captured cannot get a workspace: one share then)
+    // (a stream that is being captured, or a full device, cannot get a workspace: one share then, and no error behind it)
     if (float *part = workspace((size_t)shares * M * sizeof(float))) sh = {sh.cols, shares, chunk, part};
+    else (void)hipGetLastError();
     return sh;
 }
 
