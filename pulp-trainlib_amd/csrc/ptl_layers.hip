@@ -311,8 +311,7 @@ static ConvTileDesc forward_desc(const ConvGeom &g, int ns) {
 //                   takes longer than the product, are left out: 0.70
 //   both            by the input gradient's lines: strided 1.39, 1.49, 11 %; fp16 1.07, 1.21, 6 %, channel-minor 1.26, 1.50,
 //                   13 %; fp32 1.04, 1.21, 5 %, channel-minor 1.32, 1.39, 11 %
-// Where a line lies higher than these figures ask for, layers keep the route they had; for fp32 there is a reason to: these
-// tiles add in longer chains, which leaves results 14 to 18 % further from 64 bits in the mean (1.6e-7 against 1.4e-7).
+// Where a line lies higher than these figures ask for, layers keep the route they had.
 template <typename T>
 static bool any_pays(const ConvGeom &g, int ns, int steps, bool bias) {
     if (state().gemm_path == 7) return true;

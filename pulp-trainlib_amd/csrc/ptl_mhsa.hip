@@ -1278,7 +1278,7 @@ static int rag_tile_of(int L) { return L <= 128 ? 32 : 64; }
 // Rows and runs of k hold whole pieces (the panels take what has shorter ones, and what paths 6 and 7 ask of them).  Against
 // the panels: 83 -> 65 us for 7 x 6 heads of 48 and 19 tokens, 507 -> 430 for 46 x 6 and 192, 123 -> 96 for 8 x 8 of 64 and 64
 // tokens, 222 -> 195 for 32 x 3 of 64 and 197, all forward + backward.  Single samples of up to some hundred tokens would be
-// faster there (61.7 against 71.7 us for 3 heads of 64 and 197 tokens), but a sample's results are the same bits in every
+// faster there (61.7 against 73.0 us for 3 heads of 64 and 197 tokens), but a sample's results are the same bits in every
 // batch, so that both cannot be had.
 static bool rag_takes(const MhsaDims &m) {
     const int path = state().gemm_path;
