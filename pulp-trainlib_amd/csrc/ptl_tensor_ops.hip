@@ -814,6 +814,8 @@ __global__ __launch_bounds__(256) void dw_direct_kernel(const T *__restrict__ sr
 // exist (STRICT): by the lanes of the kernel that writes the gradient, which is this one if a channel has one workgroup and
 // the one that adds the workgroups' sums otherwise.  (Leaving these products out always took 3 to 9 % longer, code for
 // a second pass in the kernel of many workgroups 1 of 10 us.)
+// In fp32 the four products of a row and the workgroups' sums are added apart: as one chain each they lay 1.39e-7 from 64
+// bits over 12 layers (one sample of 513 x 511: 1.0e-6), this way 1.03e-7 (1.4e-7); the passes take as long within 2 %.
 struct DwWgWalk {
     int C, H, W, Ho, Wo, pu, pl, inside;
     size_t x_elems, y_elems;
@@ -856,7 +858,7 @@ __device__ inline void dw_wg_blocks(const T *__restrict__ X, const T *__restrict
 #pragma unroll
                     for (int i = 0; i < 3; ++i) {
                         if (hr - i < 0 || hr - i >= RB) continue;
-                        float a = acc[i][j];
+                        float a = sizeof(T) == 2 ? acc[i][j] : 0.f;  // (fp32: a row's four apart, chains of a quarter)
 #pragma unroll
                         for (int m = 0; m < 4; ++m) {
                             const unsigned g = G[hr - i][m];
@@ -865,7 +867,7 @@ __device__ inline void dw_wg_blocks(const T *__restrict__ X, const T *__restrict
                             else
                                 a = fmaf(__builtin_bit_cast(float, S[m]), __builtin_bit_cast(float, g), a);
                         }
-                        acc[i][j] = a;
+                        acc[i][j] = sizeof(T) == 2 ? a : acc[i][j] + a;
                     }
                 }
             }
@@ -935,8 +937,14 @@ __global__ __launch_bounds__(256) void dw_wg_direct_sum_kernel(const T *__restri
     if (tid == 0) strict = 0;
     __syncthreads();
     if (tid < 9) {
-        s = 0.f;
-        for (int k = 0; k < SL; ++k) s += red[k][tid];
+        float t[SL];
+#pragma unroll
+        for (int k = 0; k < SL; ++k) t[k] = red[k][tid];
+#pragma unroll
+        for (int n = SL; n > 1; n = (n + 1) / 2)
+#pragma unroll
+            for (int k = 0; k < n / 2; ++k) t[k] += t[n - 1 - k];
+        s = t[0];
         if (__builtin_isnan(s) && !(w.inside & 1)) strict = 1;
     }
     __syncthreads();

@@ -62,3 +62,23 @@ def test_conv(pkg, gpu, b, c, co, h, k, s, hwc):
     assert error(chw(dw), rw.view(co, c, k, k)) <= bound(b * ho * ho)
     rx = torch.nn.functional.fold(torch.matmul(W.t().contiguous(), G), (h, h), k, padding=p, stride=s)
     assert error(chw(dx), rx) <= bound(co * k * k)
+
+
+@pytest.mark.parametrize("b,c,h,w", [(3, 5, 67, 45), (40, 16, 33, 29), (200, 3, 18, 23), (1, 2, 513, 511)])
+def test_depthwise_weight_gradient(pkg, gpu, b, c, h, w):
+    """Rows of four products apart, a lane's rows in a chain of at most all rows over 64 lanes, then trees."""
+    r = lambda *s: torch.rand(*s, device=DEV) * 2 - 1
+    x, dy = r(b, c, h + 2, w + 2), r(b, c, h, w)
+    k, dw = torch.zeros(c, 3, 3, device=DEV), torch.zeros(c, 3, 3, device=DEV)
+    a = pkg.DepthWiseConvArgs()
+    keep = [pkg.blob(x, None, c, h + 2, w + 2), pkg.blob(k, dw, 1, 3, 3, c * 9), pkg.blob(dy, dy, c, h, w)]
+    a.input, a.coeff, a.output = [pkg.structs.C.pointer(t) for t in keep]
+    a.stride_h = a.stride_w = 1
+    pkg.call("ptl_conv_dw_fp32_wg_batched", a, b)
+    assert gpu.ptl_sync() == 0
+    X, G = x.double(), dy.double()
+    want = torch.stack([(X[:, :, i:i + h, j:j + w] * G).sum((0, 2, 3)) for i in range(3) for j in range(3)], 1).view(c, 3, 3)
+    n = b * h * w
+    # four products, a chain of rows in a workgroup of 256 lanes of 4 columns (blocks of seven rows: at least that many), trees
+    rows = max(7, n / (4 * 256))
+    assert error(dw, want) <= 2.0 ** -24 / math.sqrt(3) * math.sqrt((4 + rows) / 2 + math.log2(n))
