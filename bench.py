@@ -215,7 +215,7 @@ def main():
         check(fw(ha_ref, ns)); check(bw(ha_ref, ns))
     host_ms = (time.perf_counter() - t0) * 1e3 / 5
     result["host_staged"] = {"ms_per_step": round(host_ms, 4), "TFLOP/s": round(flops_step / (host_ms * 1e-3) / 1e12, 3),
-                             "note": "same step with host pointers: per call hipMalloc + H2D + kernel + D2H + sync"}
+                             "note": "same step with host pointers: per call: pinned blocks or parts over the bus, kernel, back, one wait"}
 
     # ------------------------------------------------------------------------ CPU baseline
     if not args.no_cpu:
