@@ -309,7 +309,10 @@ int ptl_sync(void);
  * channels per head);
  * 7 = a Conv2D runs as products with patch matrices (any filter, stride and
  * padding; by default where they measured better) wherever its offsets fit 31
- * bits; self-attention runs its panel products one to a launch.
+ * bits, each gradient in launches of its own; self-attention runs its panel
+ * products one to a launch.  8, 9 = as 7, but the input gradient in one launch
+ * with the weight gradient, on the tensors as they are (8) or on channel-minor
+ * copies of channel-major ones (9).
  * All routes compute the same products.
  * ptl_last_conv_direct() tells whether the last Conv2D call ran one of the
  * convolution kernels (1) or the implicit-im2col GEMM (0);

@@ -1,9 +1,11 @@
 // Conv2D layers of any geometry (up to 25 taps, strides up to 2 x 2, any size and alignment) as products with implicit
 // patch matrices (ptl_ragged_conv.inc): what the descriptions of their operands say.
-//   * forward: one launch.  Weight gradient: one launch.  Input gradient: a strided layer's is split into its phases (the
+//   * backward, small and middling layers: both gradients in one launch and one more for the partial sums of both; the
+//     filters are read where they are, or re-laid together with channel-minor copies of the tensors.
+//   * forward: one launch.  Weight gradient alone: one launch.  Input gradient: a strided layer's is split into its phases (the
 //     pixels that the same taps reach), each a unit-stride product with its share of the taps - a pass over a zero-stuffed
-//     gradient has stride^2 times the work - all in one launch.  The filters the input gradient reads are re-laid by
-//     spare blocks of the weight gradient's launch.
+//     gradient has stride^2 times the work - all in one launch.  The filters it reads are re-laid by spare blocks of the
+//     weight gradient's launch.
 #include "ptl_common.hpp"
 #include "ptl_conv_tile.hpp"
 #include "ptl_ragged.hpp"
@@ -137,11 +139,12 @@ static int any_sizes(const ConvTileDesc &d, int step, bool minor, RagProd (&p)[R
     return count;
 }
 
-// What a call does: by channel-minor copies of channel-major tensors or on the tensors themselves, and the tiles of its
-// products.  Looked up by the layer's geometry, since weighing the choices takes the host 1-3 us.
+// What a call does: by channel-minor copies of channel-major tensors or on the tensors themselves, both gradients in one
+// launch (64 x 64 tiles; small layers) or one after the other, and the tiles of its products.  Looked up by the layer's geometry, since weighing the choices takes the host 1-3 us.
 struct AnyPlan {
-    bool turn;
+    bool turn, one;     // one: both gradients in one launch
     RagPlan first, ig;  // forward or weight gradient; input gradient
+    RagBackPlan back;
     double clocks;
 };
 template <typename T>
@@ -152,37 +155,47 @@ static const AnyPlan &any_plan(const ConvTileDesc &d, int steps) {
     };
     constexpr int ENTRIES = 64, KEYS = 17;
     static thread_local Entry table[ENTRIES] = {};
-    const int key[KEYS] = {steps, d.in_hwc, d.batch, d.Cin, d.Hin, d.Win, d.Cout, d.Ho, d.Wo, d.KH, d.KW, d.sh, d.sw, d.padU, d.padL, d.padD, d.padR};
+    const int path = state().gemm_path;  // 7 to 9: see ptl_set_gemm_path
+    const int key[KEYS] = {steps + 8 * path, d.in_hwc, d.batch, d.Cin, d.Hin, d.Win, d.Cout, d.Ho, d.Wo, d.KH, d.KW, d.sh, d.sw, d.padU, d.padL, d.padD, d.padR};
     unsigned h = 0;
     for (int i = 0; i < KEYS; ++i) h = h * 31 + (unsigned)key[i];
     Entry &e = table[(h ^ h >> 7) % ENTRIES];
     if (memcmp(e.key, key, sizeof(key)) == 0) return e.plan;
     constexpr int ES = (int)sizeof(T);
     AnyPlan best = {};
-    for (int turn = 0; turn <= (d.in_hwc ? 0 : 1); ++turn) {
-        const bool minor = d.in_hwc || turn;
+    for (int way = 0; way < 4; ++way) {
+        const bool turn = (way & 1) != 0, one = way > 1, minor = d.in_hwc || turn;
+        if ((turn && d.in_hwc) || (one && (path == 7 || !(steps & ANY_IG)))) continue;
+        if (path > 7 && (steps & ANY_IG) && (!one || (!d.in_hwc && turn != (path == 9)))) continue;
         AnyPlan a = {};
-        a.turn = turn != 0;
-        RagProd p[RAG_CONV_MAX] = {};
-        if (steps & (ANY_FW | ANY_WG)) {
+        a.turn = turn;
+        a.one = one;
+        RagProd p[RAG_CONV_MAX] = {}, w[RAG_CONV_MAX] = {};
+        if (one) {
+            if (steps & ANY_WG) any_sizes<T>(d, ANY_WG, minor, w);
+            const int n = any_sizes<T>(d, ANY_IG, minor, p);
+            a.back = ragged_back_plan<T>(steps & ANY_WG ? w : nullptr, p, n, turn ? RAG_BACK_COPIES : minor ? RAG_BACK_MINOR : RAG_BACK_MAJOR);
+            a.clocks = a.back.clocks;
+        }
+        if (!one && (steps & (ANY_FW | ANY_WG))) {
             const int n = any_sizes<T>(d, steps & (ANY_FW | ANY_WG), minor, p);
             a.first = steps & ANY_FW ? ragged_conv_plan<T>(p, n, d.in_hwc ? RAG_GK : RAG_KC, d.in_hwc ? RAG_KC : turn ? RAG_GK : RAG_XK)
                                      : ragged_conv_plan<T>(p, n, RAG_RC, minor ? RAG_GR : RAG_XR);
             a.clocks += a.first.clocks;
         }
-        if (steps & ANY_IG) {
+        if (!one && (steps & ANY_IG)) {
             const int n = any_sizes<T>(d, ANY_IG, minor, p);
             a.ig = ragged_conv_plan<T>(p, n, d.in_hwc ? RAG_GK : RAG_KC, d.in_hwc ? RAG_KC : turn ? RAG_GK : RAG_XK);
             a.clocks += a.ig.clocks;
         }
         // a launch for the layouts, and the bytes it moves (clocks fitted like those of the tiles)
-        if (turn || (d.in_hwc && steps == ANY_FW && any_padded(d.Cin, ES) != d.Cin) || steps == ANY_IG) a.clocks += 12500;
+        if (turn || (d.in_hwc && steps == ANY_FW && any_padded(d.Cin, ES) != d.Cin) || (steps == ANY_IG && !one)) a.clocks += 12500;
         if (turn) {
             const double x = steps == ANY_IG ? 0 : (double)d.batch * d.Hin * d.Win * (d.Cin + any_padded(d.Cin, ES)) * ES;
             const double y = steps == ANY_FW ? 0 : (double)d.batch * d.Ho * d.Wo * (d.Cout + any_padded(d.Cout, ES)) * ES;
             a.clocks += (x + y) / (ES == 2 ? 1500 : 2000);
         }
-        if (turn == 0 || a.clocks < best.clocks) best = a;
+        if (best.clocks == 0 || a.clocks < best.clocks) best = a;
     }
     memcpy(e.key, key, sizeof(key));
     e.plan = best;
@@ -238,10 +251,42 @@ int conv_any_fw(const ConvTileDesc &d, const void *X, const void *Wt, const void
     return ragged_conv<T>(r, RAG_KC, turn ? RAG_GK : RAG_XK, plan.first);
 }
 
-// The products of the input gradient, one per phase, and the filters they read (laid at `filters_at`).  turn: dY is the
-// channel-minor copy of a channel-major gradient.
+// The filters of a phase in place, for the input gradient: as a patch matrix whose pixels are the input channels and whose
+// channels the output channels (channel-major), or by tap and output channel (channel-minor).
 template <typename T>
-static int any_input_gradient(const ConvTileDesc &d, const void *dY, const void *Wt, void *dX, bool turn, char *W, RagConvArgs &r, RagConvArgs &filters) {
+static void any_filters(const ConvTileDesc &d, const void *Wt, const AnyPhase &f, RagGeo &g, RagOp &o) {
+    constexpr int ES = (int)sizeof(T), VEC = 16 / ES;
+    const int taps = d.KH * d.KW, t = f.th * f.tw, c = d.in_hwc ? d.Cin : 1;
+    const int tap_at = (f.ky * d.KW + f.kx) * c * ES, tap_y = d.sh * d.KW * c * ES, tap_x = d.sw * c * ES;
+    o = {};
+    o.p = static_cast<const char *>(Wt) + tap_at;
+    o.rows = d.Cin;
+    g.plane = (unsigned)(d.Cin * taps * ES);
+    g.d_kw = rag_div(f.tw);
+    if (d.in_hwc) {
+        g.d_cb = rag_div((d.Cout + VEC - 1) / VEC);
+        g.py = (unsigned)tap_y;
+        g.px = (unsigned)tap_x;
+        g.size = (unsigned)d.Cout;
+        return;
+    }
+    g.d_x = g.d_y = rag_div(1 << 30);
+    g.px = (unsigned)(taps * ES);
+    g.ty = g.tx = 1;
+    g.H = g.W = 1 << 30;
+    g.d_t = rag_div(t);
+    for (int i = 0; i < t; i += f.tw) g.every_row |= 1u << i;
+    for (int i = 0; i < 32 && t > 0; i += t) g.every_channel |= 1u << i;
+    g.all_taps = (1u << t) - 1u;
+    g.size = (unsigned)((long long)d.Cout * d.Cin * taps * ES - tap_at);
+    for (int j = 0; j < RAG_TAB && t > 0; ++j) g.tab[j] = j / t * (int)g.plane + j % t / f.tw * tap_y + j % t % f.tw * tap_x;
+}
+
+// The products of the input gradient, one per phase, and the filters they read: in place (geometry to `in_place`) or re-laid at
+// W as `filters` says.  turn: dY is the channel-minor copy of a channel-major gradient.
+template <typename T>
+static int any_input_gradient(const ConvTileDesc &d, const void *dY, const void *Wt, void *dX, bool turn, char *W, RagConvArgs &r, RagConvArgs &filters,
+                              RagGeo *in_place) {
     constexpr int ES = (int)sizeof(T), VEC = 16 / ES;
     const bool minor = d.in_hwc || turn;
     const int taps = d.KH * d.KW, Cp = any_padded(d.Cout, ES), inner = minor ? Cp : 1, outer = minor ? 1 : d.Cout;
@@ -258,14 +303,15 @@ static int any_input_gradient(const ConvTileDesc &d, const void *dY, const void 
         RagOp &patch = d.in_hwc ? p.a : p.b, &weight = d.in_hwc ? p.b : p.a;
         if (any_geo<T>(r.geo[i], patch, dY, img, f.qh, f.qw, f.y0, f.x0, 1, 1, f.th, f.tw, -1)) return -1;
         patch.rows = d.batch * f.qh * f.qw;
-        weight = any_rows<T>(W, d.Cin, (long long)K * ES);
+        if (in_place) any_filters<T>(d, Wt, f, in_place[i], weight);
+        else weight = any_rows<T>(W, d.Cin, (long long)K * ES);
         const int pix = d.in_hwc ? d.Cin : 1, img_n = d.Cin * d.Hin * d.Win;
         p.C = static_cast<T *>(dX) + (f.ph * d.Win + f.pw) * pix;
         const RagAxis pixels = d.sh == 1 && d.sw == 1 ? rag_axis2(d.Hin * d.Win, pix, img_n) : rag_axis3(f.qw, f.qh, d.sw * pix, d.sh * d.Win * pix, img_n);
         const RagAxis chans = rag_axis(d.Cin, d.in_hwc ? 1 : d.Hin * d.Win);
         p.cn = d.in_hwc ? pixels : chans;
         p.cm = d.in_hwc ? chans : pixels;
-        if (t == 0) continue;
+        if (t == 0 || in_place) continue;
         RagRelay &l = filters.relay[filters.relays++];
         const int c = d.in_hwc ? d.Cin : 1;  // from tap to tap
         l.dst = W;
@@ -288,7 +334,8 @@ int conv_any_bw(const ConvTileDesc &d, const void *X, const void *dY, const void
     state().last_conv_resident = turn ? 4 : 0;
     const int Cip = any_padded(d.Cin, ES), Cop = any_padded(d.Cout, ES);
     // scratch: the filters as the input gradient reads them; channel-minor copies of the gradient and of the input
-    const size_t w_bytes = dX ? ((size_t)d.Cin * taps * (minor ? Cop : d.Cout) * ES + 255) / 256 * 256 : 0;
+    const bool relaid = dX && (turn || !plan.one);
+    const size_t w_bytes = relaid ? ((size_t)d.Cin * taps * (minor ? Cop : d.Cout) * ES + 255) / 256 * 256 : 0;
     const size_t y_bytes = turn ? ((size_t)npix * Cop * ES + 255) / 256 * 256 : 0, x_bytes = turn && dW ? (size_t)d.batch * d.Hin * d.Win * Cip * ES : 0;
     char *buf = nullptr;
     if (w_bytes + y_bytes + x_bytes && !(buf = static_cast<char *>(scratch(w_bytes + y_bytes + x_bytes)))) return 2;
@@ -335,13 +382,15 @@ int conv_any_bw(const ConvTileDesc &d, const void *X, const void *dY, const void
             }
         }
     }
+    RagGeo in_place[RAG_CONV_MAX] = {};
     if (dX)
-        if (int rc = any_input_gradient<T>(d, dY, Wt, dX, turn, buf, x, w)) return rc;
+        if (int rc = any_input_gradient<T>(d, dY, Wt, dX, turn, buf, x, w, relaid ? nullptr : in_place)) return rc;
     // the filters: together with the channel-minor copies, else by spare blocks of the weight gradient's launch
-    if (turn || !dW) {
+    if (turn || (!dW && relaid)) {
         if (int rc = ragged_relay<T>(w, t, turn ? (dW ? 2 : 1) : 0)) return rc;
         w.relays = 0;
     }
+    if (plan.one && dX) return ragged_back<T>(w, x, in_place, turn ? RAG_BACK_COPIES : minor ? RAG_BACK_MINOR : RAG_BACK_MAJOR, am, plan.back);
     if (dW)
         if (int rc = ragged_conv<T>(w, am, bm, plan.first)) return rc;
     return dX ? ragged_conv<T>(x, d.in_hwc ? RAG_GK : RAG_KC, d.in_hwc ? RAG_KC : turn ? RAG_GK : RAG_XK, plan.ig) : 0;

@@ -309,12 +309,10 @@ static ConvTileDesc forward_desc(const ConvGeom &g, int ns) {
 //   input gradient  strided 15: 1.22, 1.40, 7 %; fp16 300: 0.93, 1.17, 4 %, channel-minor 240: 0.89, 1.13, 3 %; fp32 320:
 //                   0.90, 1.11, 4 %, channel-minor 1500: 1.15, 1.16, 4 %; few pixels under many filters, whose re-laying
 //                   takes longer than the product, are left out: 0.70
-//   both            by the input gradient's lines: strided 1.39, 1.49, 11 %; fp16 1.07, 1.21, 6 %, channel-minor 1.26, 1.50,
-//                   13 %; fp32 1.04, 1.21, 5 %, channel-minor 1.32, 1.39, 11 %
 // Where a line lies higher than these figures ask for, layers keep the route they had.
 template <typename T>
 static bool any_pays(const ConvGeom &g, int ns, int steps, bool bias) {
-    if (state().gemm_path == 7) return true;
+    if (state().gemm_path >= 7) return true;
     if (state().gemm_path != 0) return false;
     constexpr int VEC = 16 / (int)sizeof(T);
     auto fill = [](double n, int unit) { return n / ((long long)((n + unit - 1) / unit) * unit); };
@@ -420,7 +418,7 @@ static int conv2d_fw(const Args *a, int ns, const char *fn) {
             c.n = axis_plain(ns * P, g.Co);
             c.m = axis_plain(g.Co, 1);
         }
-        if (state().gemm_path == 7 && (rc = conv_any_fw<T>(d, X, Wt, bias, Y)) >= 0) return sg.finish(rc);
+        if (state().gemm_path >= 7 && (rc = conv_any_fw<T>(d, X, Wt, bias, Y)) >= 0) return sg.finish(rc);
         if (!g.hwc) rc = conv_small<T>(d, X, Wt, Y);
         // (a normalisation to apply on the way in is the small-layer kernel's business alone: nothing was launched)
         if (rc == CONV_PRE_REFUSED || conv_small_pre_pending()) return CONV_PRE_REFUSED;
@@ -503,7 +501,7 @@ static int conv2d_wg(const Args *a, int ns, const char *fn) {
         // else (or on request) the sum over taps.  From 256 channels on either side and 16384 output pixels the sum
         // over taps goes before the output tile kernel (measured: 81 against 91 us for 256 -> 256 on 14x14 at batch
         // 128, 455 against 533 us on 28x28 at batch 256; at batch 8 the output tile kernel takes 26 against 34 us)
-        if (state().gemm_path == 7 && (rc = conv_any_bw<T>(d, X, dY, nullptr, dW, nullptr, db)) >= 0) return sg.finish(rc);
+        if (state().gemm_path >= 7 && (rc = conv_any_bw<T>(d, X, dY, nullptr, dW, nullptr, db)) >= 0) return sg.finish(rc);
         const bool taps_first = d.Cin >= 128 && d.Cout >= 128 && (d.Cin >= 256 || d.Cout >= 256) &&
                                 (long long)ns * g.Ho * g.Wo >= 16384;
         if (g.hwc) {  // channel-minor tensors: the sum over taps from 64 channels on, else the gathering GEMM below
@@ -622,7 +620,7 @@ static int conv2d_ig(const Args *a, int ns, const char *fn) {
         return sg.finish(gemm<T>(q));
     }
 
-    if (state().gemm_path == 7) {
+    if (state().gemm_path >= 7) {
         ConvTileDesc d = {};
         d.in_hwc = g.hwc ? 1 : 0;
         d.batch = ns; d.Cin = g.Ci; d.Hin = g.H; d.Win = g.W;
@@ -862,9 +860,13 @@ static int conv2d_bw(const Args *a, int ns, const char *fn) {
             }
         }
     }
-    // Both gradients as products with patch matrices, except where one of them has a kernel of its own that is ahead: the
-    // resident-tile kernels, and the raw-tile weight gradient of large unit-stride 3x3 and 1x1 layers (26 us against 48 for
-    // 128 -> 32 channels on 22 x 32 at batch 94).
+    // Both gradients as products with patch matrices (small and middling layers: in one launch), whatever the size: over 2300
+    // layers of 1 to 250 samples the other routes take 1.2 to 1.7 times as long in the mean of each group of type, layout,
+    // stride and bias, and taking the better one of each layer would give 1 % more.  Except where one of the gradients
+    // has a kernel of its own that is ahead: the raw-tile weight gradient of unit-stride 3x3 layers from 10 GFLOP on (other over
+    // this: 1.18 in the mean at 3 to 6 GFLOP, 1.06 at 6 to 10, 0.98 at 10 to 20, 0.94 above; 1x1 layers 1.2 above 10), the
+    // resident-tile one wherever it is preferred (a call then has the bits of its two steps), and those of channel-minor
+    // layers from 20 on (1.77, 1.26 and 1.22 at 4, 10 and 19, 0.92 and 0.82 at 31 and 39).
     if (apart && (a->USE_BIASES != 1 || a->bias)) {
         ConvGeom g;
         if (int rc = conv_geom(a, g, fn, true)) return rc;
@@ -872,11 +874,12 @@ static int conv2d_bw(const Args *a, int ns, const char *fn) {
         const int P = g.Ho * g.Wo, K = g.Ci * g.Hk * g.Wk;
         const size_t in_n = (size_t)ns * g.Ci * g.H * g.W, out_n = (size_t)ns * g.Co * P;
         const ConvTileDesc d = forward_desc(g, ns);
-        const bool unit = g.sh == 1 && g.sw == 1, scatter = K == g.Ci && !unit;
-        const bool own_wg = unit && sizeof(T) == 2 && !g.hwc && g.Hk <= 3 && 2e-9 * ns * g.Co * P * K >= 1;
-        const bool resident = sizeof(T) == 2 && g.hwc && conv_halo_wg_hwc_fits(d, nullptr, nullptr) && conv_halo_wg_hwc_preferred(d);
-        const bool forced = state().gemm_path == 7;
-        if ((forced || (!own_wg && !resident && !scatter)) && fits_int(in_n) && fits_int(out_n) && any_pays<T>(g, ns, 6, a->USE_BIASES == 1)) {
+        const double gflop = 2e-9 * ns * g.Co * P * K;
+        const bool own_wg = g.sh == 1 && g.sw == 1 && sizeof(T) == 2 && !g.hwc && K > g.Ci && g.Hk <= 3 &&
+                            (gflop >= 10 || (g.Hk == 3 && g.Wk == 3 && conv_halo_wg_preferred(d)));
+        const bool resident = sizeof(T) == 2 && g.hwc && gflop >= 20 && conv_halo_wg_hwc_fits(d, nullptr, nullptr) && conv_halo_wg_hwc_preferred(d);
+        const bool forced = state().gemm_path >= 7;
+        if ((forced || (state().gemm_path == 0 && !own_wg && !resident)) && fits_int(in_n) && fits_int(out_n)) {
             Stager sg;
             const T *X = sg.in(reinterpret_cast<const T *>(a->input->data), in_n);
             const T *dY = sg.in(reinterpret_cast<const T *>(a->output->diff), out_n);

@@ -23,8 +23,9 @@ inline RagDiv rag_div(long long dv) {
 // contiguous.  The others are implicit patch matrices (RagGeo): XK and XR gather a channel-major tensor element by element,
 // neighbouring lanes at neighbouring pixels, with pixels as the rows and (channel, tap) as k (XK) or the other way round
 // (XR); GK and GR read channel-minor tensors in pieces of VEC channels of one tap at one pixel, with pixels as the rows
-// and (tap, piece) as k (GK) or the other way round (GR).
-enum RagMode : int { RAG_KC = 0, RAG_RC = 1, RAG_GK = 2, RAG_GR = 3, RAG_XK = 4, RAG_XR = 5 };
+// and (tap, piece) as k (GK) or the other way round (GR).  WR: the filters of a channel-minor layer in place, input channels
+// (contiguous) as the rows and (tap, piece of output channels) as k, beside GK.
+enum RagMode : int { RAG_KC = 0, RAG_RC = 1, RAG_GK = 2, RAG_GR = 3, RAG_XK = 4, RAG_XR = 5, RAG_WR = 6 };
 
 struct RagOp {
     const char *p;     // first element (XK, XR: see RagGeo)
@@ -38,6 +39,8 @@ struct RagOp {
 // An implicit patch matrix: pixel q = (b, qy, qx), tap t = (jy, jx), element at row qy*sy + y0 + ty*jy and column
 // qx*sx + x0 + tx*jx of channel c of image b, zero outside of the H x W image.  ty = tx = 1 for a forward pass, -1 for the
 // input gradient.  Offsets are unsigned: the tensor pointer is moved back by what the smallest of them would lack.
+// XK also reads filters in place, the input channels as its pixels and the output channels as its channels; WR has the
+// bytes from tap to tap in py and px, from output channel to output channel in plane, and in size how many there are.
 constexpr int RAG_TAPS = 25;          // one validity bit per tap and for the seven taps after the last of a channel
 constexpr int RAG_TAB = RAG_TAPS + 7;
 struct RagGeo {
@@ -145,6 +148,18 @@ template <typename T>
 RagPlan ragged_conv_plan(const RagProd *p, int count, int a, int b);
 template <typename T>
 int ragged_conv(RagConvArgs &r, int a, int b, const RagPlan &plan);
+// Both gradients of a layer in one launch (plus one for partial sums): the weight gradient of w (modes a, b; none where its
+// count is 0), then the products of x, whose filters are read in place as f says - channel-major by XK, channel-minor by WR -
+// or, where b is GR and the tensors of x are channel-minor copies (KC, GK), re-laid.
+struct RagBackPlan {
+    int per_w, per_x;  // slabs per workgroup
+    double clocks;
+};
+enum RagBack : int { RAG_BACK_MAJOR = 0, RAG_BACK_MINOR = 1, RAG_BACK_COPIES = 2 };
+template <typename T>
+RagBackPlan ragged_back_plan(const RagProd *w, const RagProd *x, int count, RagBack kind);
+template <typename T>
+int ragged_back(RagConvArgs &w, RagConvArgs &x, const RagGeo *f, RagBack kind, int a, const RagBackPlan &plan);
 // The re-laying alone, filters of r and tensors (n <= 2).
 template <typename T>
 int ragged_relay(RagConvArgs &r, const RagTurn *turn, int n);
