@@ -81,9 +81,11 @@ __device__ inline void static_for(F &&f) {
 // (every wave has then left stage s - 1).
 template <int NS>
 __host__ __device__ constexpr int pipe_pieces(int sidx) {
-    // 12 tile pieces per wave and unit over the first E stages; none in the last NS - 2 stages, so that the
-    // loads behind the first filter stages of a unit are the same in the prologue and in steady state
-    constexpr int E = 9 - (NS - 2) < 6 ? 9 - (NS - 2) : 6;
+    // 12 tile pieces per wave and unit over the first E stages; none in the last NS - 1 stages, which issue the filters
+    // of the next unit's stages 0 .. NS - 2: the wait that certifies its stage 0 lets what is issued behind those
+    // filters be in flight, and must have seen the whole tile land (also, the loads behind the first filter stages of a
+    // unit are then the same in the prologue and in steady state)
+    constexpr int E = 9 - (NS - 1) < 6 ? 9 - (NS - 1) : 6;
     return sidx < E ? 12 / E + (sidx < 12 % E ? 1 : 0) : 0;
 }
 template <int NS>
@@ -91,6 +93,12 @@ __host__ __device__ constexpr int pipe_piece0(int sidx) {
     int n = 0;
     for (int j = 0; j < sidx; ++j) n += pipe_pieces<NS>(j);
     return n;
+}
+template <int NS>
+__host__ __device__ constexpr bool pipe_tile_first() {  // no piece behind the filters of the next unit's first stage
+    for (int s = 9 - (NS - 1); s < 9; ++s)
+        if (pipe_pieces<NS>(s) > 0) return false;
+    return pipe_piece0<NS>(9) == 12;
 }
 template <int NS, int LB>
 __host__ __device__ constexpr int pipe_wait(int sidx) {
@@ -143,7 +151,7 @@ __global__ __launch_bounds__(HALO_NT) void conv_halo_kernel(const HaloArgs a) {
     constexpr int FM = BN / 16, FN = 4;  // fragments per wave: filters x positions (64 positions per wave)
     constexpr int MID = 1;               // half of a stage in front of which the next stage is certified
     constexpr int NR = FM + FN, NM = FM * FN;  // fragment reads / MFMAs per half stage (one k-step of 32)
-    static_assert(NS >= 3 && NS <= 7, "ring depth");
+    static_assert(NS >= 3 && NS <= 7 && pipe_tile_first<NS>(), "ring depth");
     extern __shared__ __align__(16) char smem[];
     const unsigned halo_lds = (unsigned)(uintptr_t)(lds_char *)smem, ring_lds = halo_lds + 2 * HALO_BYTES;
     const char *const halo = smem, *const ring = smem + 2 * HALO_BYTES;
