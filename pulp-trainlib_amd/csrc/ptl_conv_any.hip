@@ -189,7 +189,7 @@ static const AnyPlan &any_plan(const ConvTileDesc &d, int steps) {
             a.clocks += a.ig.clocks;
         }
         // a launch for the layouts, and the bytes it moves (clocks fitted like those of the tiles)
-        if (turn || (d.in_hwc && steps == ANY_FW && any_padded(d.Cin, ES) != d.Cin) || (steps == ANY_IG && !one)) a.clocks += 12500;
+        if (turn || (steps == ANY_IG && !one)) a.clocks += 12500;
         if (turn) {
             const double x = steps == ANY_IG ? 0 : (double)d.batch * d.Hin * d.Win * (d.Cin + any_padded(d.Cin, ES)) * ES;
             const double y = steps == ANY_FW ? 0 : (double)d.batch * d.Ho * d.Wo * (d.Cout + any_padded(d.Cout, ES)) * ES;
@@ -212,9 +212,9 @@ int conv_any_fw(const ConvTileDesc &d, const void *X, const void *Wt, const void
     state().last_conv_resident = turn ? 4 : 0;
     const int Cp = any_padded(d.Cin, ES), Kp = taps * Cp;
     RagConvArgs r = {};
-    if (turn || (d.in_hwc && Kp != K)) {  // filters tap by tap, whole pieces of channels; the image channel-minor
-        const size_t w_bytes = ((size_t)d.Cout * Kp * ES + 255) / 256 * 256, x_bytes = turn ? (size_t)d.batch * d.Hin * d.Win * Cp * ES : 0;
-        char *buf = static_cast<char *>(scratch(w_bytes + x_bytes));
+    if (turn) {  // filters tap by tap, whole pieces of channels; the image channel-minor
+        const size_t w_bytes = ((size_t)d.Cout * Kp * ES + 255) / 256 * 256;
+        char *buf = static_cast<char *>(scratch(w_bytes + (size_t)d.batch * d.Hin * d.Win * Cp * ES));
         if (!buf) return 2;
         RagRelay &l = r.relay[0];
         r.relay_src = Wt;
@@ -223,13 +223,13 @@ int conv_any_fw(const ConvTileDesc &d, const void *X, const void *Wt, const void
         l.rows = d.Cout; l.row_s = K;
         l.outer = 1;
         l.taps = taps; l.kw = d.KW;
-        l.tap_x = d.in_hwc ? d.Cin : 1; l.tap_y = d.KW * l.tap_x;
-        l.inner = Cp; l.lim = d.Cin; l.inner_s = d.in_hwc ? 1 : taps;
+        l.tap_x = 1; l.tap_y = d.KW;
+        l.inner = Cp; l.lim = d.Cin; l.inner_s = taps;
         const RagTurn t = {X, buf + w_bytes, d.batch, d.Cin, Cp, d.Hin * d.Win};
-        if (int rc = ragged_relay<T>(r, &t, turn ? 1 : 0)) return rc;
+        if (int rc = ragged_relay<T>(r, &t, 1)) return rc;
         r.relays = 0;
         Wt = buf;
-        if (turn) X = t.dst;
+        X = t.dst;
     }
     RagProd &p = r.p[0];
     r.count = any_sizes<T>(d, ANY_FW, minor, r.p);
@@ -243,6 +243,12 @@ int conv_any_fw(const ConvTileDesc &d, const void *X, const void *Wt, const void
     if (d.in_hwc) {
         p.cn = rag_axis(npix, d.Cout);
         p.cm = rag_axis(d.Cout, 1);
+        if (Kp != K) {  // channels that are no whole pieces: filters in place, their rows as the pixels of images of KH x KW
+            const AnyImage filter = {d.Cin, d.KH, d.KW, 1, (long long)d.Cout * K * ES};
+            if (any_geo<T>(r.geo_a, weight, Wt, filter, 1 << 30, 1 << 30, 0, 0, 0, 0, d.KH, d.KW, 1)) return -1;
+            r.geo_a.px = (unsigned)(K * ES);
+            return ragged_conv<T>(r, RAG_GK, RAG_GK, plan.first);
+        }
         return ragged_conv<T>(r, RAG_GK, RAG_KC, plan.first);
     }
     p.bias_n = 1;

@@ -292,18 +292,17 @@ static ConvTileDesc forward_desc(const ConvGeom &g, int ns) {
 }
 
 // Whether the products with patch matrices (ptl_conv_any.hip) go before the kernels for small problems (raw tiles of one
-// image, the gathering product): by the millions of multiplications of a step, counted by how full its tiles are.  Strides:
-// the other route of the input gradient runs over a zero-stuffed tensor.  Channel-minor layers whose channels are no whole
-// pieces (`odd`) have their filters re-laid first, as all have for the input gradient.  A bias is a launch of its own on
-// the other routes.  Both routes were timed on 5000 layers (1 to 128 samples, 3 to 512 channels on 7 to 64 pixels, 1 to 25
+// image, the gathering product).
+// Forward: always.  Over 2800 layers (1 to 250 samples) the other routes take 1.05 to 1.25 times as long in the mean of each
+// group of type, layout, stride and bias, and the better one of each layer would give 0 to 4 % more.  Except fp16 layers of
+// unit stride with few filters over many pixels and a short contraction, where the raw tiles read each input once: 8 ->
+// 16 1 x 1, 14.2 us there and 17.5 here; 64 -> 16 3 x 3, 42 and 49; but 83 -> 16 1 x 1 24 and 16, 132 -> 15 3 x 3 152 and 129.
+// One gradient alone: by the millions of multiplications of a step, counted by how full its tiles are.  Strides: the
+// other route of the input gradient runs over a zero-stuffed tensor.  A bias gradient is a launch of its own on the other
+// routes.  Both routes were timed on 5000 layers (1 to 128 samples, 3 to 512 channels on 7 to 64 pixels, 1 to 25
 // taps, strides 1 and 2, tensors in turn), forced one after the other.  Time of the other route over this one's, mean of
 // the layers between a third of the line and the line; between the line and three times it; and what the rule loses to the
 // better of the two for each layer, in the mean:
-//   forward         fp16 240: 1.14, 1.16, 13 %; fp32 5: 1.23, 1.12, 8 %; channel-minor fp16 5: 1.43, 1.40, 6 %, odd 200:
-//                   0.89, 1.01, 4 %; fp32 60: 1.13, 1.19, 10 %, odd 600: 0.90, 1.08, 2 %
-//                   (fp16, at most 16 filters at unit stride: 1.17 in the mean of 163 layers, but 0.99 (0.92 to 1.07) of the
-//                   four over more than 10^5 pixels, where the raw tiles read each input once for their few filters; 68 -> 8
-//                   on 42 x 42, 143 samples, bias: 171.8 us there, 183.6 here.  Those stay there.)
 //   weight gradient 300: 0.96, 1.07, 4 %; strided 200: 1.00, 1.05, 7 %; channel-minor fp16 20: 1.16, 1.20, 7 %, fp32 300:
 //                   1.02, 1.15, 8 %
 //   input gradient  strided 15: 1.22, 1.40, 7 %; fp16 300: 0.93, 1.17, 4 %, channel-minor 240: 0.89, 1.13, 3 %; fp32 320:
@@ -317,14 +316,12 @@ static bool any_pays(const ConvGeom &g, int ns, int steps, bool bias) {
     constexpr int VEC = 16 / (int)sizeof(T);
     auto fill = [](double n, int unit) { return n / ((long long)((n + unit - 1) / unit) * unit); };
     const int K = g.Ci * g.Hk * g.Wk;
-    const bool strided = g.sh > 1 || g.sw > 1, odd = g.hwc && g.Ci % VEC != 0, half = sizeof(T) == 2;
+    const bool strided = g.sh > 1 || g.sw > 1, half = sizeof(T) == 2;
+    if (steps == 1)
+        return !(half && !g.hwc && !strided && g.Co <= 16 && K <= (K == g.Ci ? 40 : 700) && (long long)ns * g.Ho * g.Wo > 100000);
     double mflop = 2e-6 * ns * g.Co * g.Ho * g.Wo * K * fill(g.Co, 32) * fill(K, 64);
     if (g.hwc) mflop *= fill(g.Ci, VEC);
-    if (bias) mflop *= steps == 1 ? 4 : 1.5;
-    if (steps == 1) {
-        if (half && !g.hwc && !strided && g.Co <= 16 && (long long)ns * g.Ho * g.Wo > 100000) return false;
-        return mflop >= (g.hwc ? (odd ? (half ? 200 : 600) : half ? 5 : 60) : half ? 240 : 5);
-    }
+    if (bias) mflop *= 1.5;
     if (steps == 2) return mflop >= (g.hwc ? (half ? 20 : 300) : strided ? 200 : 300);
     if ((long long)ns * g.H * g.W < 256 && (long long)g.Co * K > (1 << 18)) return false;
     return mflop >= (strided ? 15 : half ? (g.hwc ? 240 : 300) : g.hwc ? 1500 : 320);
@@ -419,6 +416,10 @@ static int conv2d_fw(const Args *a, int ns, const char *fn) {
             c.m = axis_plain(g.Co, 1);
         }
         if (state().gemm_path >= 7 && (rc = conv_any_fw<T>(d, X, Wt, bias, Y)) >= 0) return sg.finish(rc);
+        // (the small-layer kernel adds no bias, which is a launch of its own: 8 -> 16 channels on 8 x 8, 7 samples, fp16 8.3
+        // against 7.3 us, 8 -> 48 on 40 x 40, 8 samples, fp32 17.5 against 8.4; without one its bits are those of the call
+        // that also forms the output's sums)
+        if (bias && !conv_small_pre_pending() && any_pays<T>(g, ns, 1, true) && (rc = conv_any_fw<T>(d, X, Wt, bias, Y)) >= 0) return sg.finish(rc);
         if (!g.hwc) rc = conv_small<T>(d, X, Wt, Y);
         // (a normalisation to apply on the way in is the small-layer kernel's business alone: nothing was launched)
         if (rc == CONV_PRE_REFUSED || conv_small_pre_pending()) return CONV_PRE_REFUSED;

@@ -132,7 +132,7 @@ struct RagConvOf {
     int first[N + 1];
     int count;
     RagGeo geo[N];          // of each product's patch matrix
-    RagGeo geo_a;           // of a first operand that is gathered too (XR; one product)
+    RagGeo geo_a;           // of the other operand where it is gathered too (one product): a gradient (XR), filters (GK, GK)
     const void *relay_src;  // blocks behind the last product re-lay filters for a later product
     RagRelay relay[RAG_CONV_MAX];
     int relays, relay_first[RAG_CONV_MAX + 1];
