@@ -402,6 +402,79 @@ int conv_any_bw(const ConvTileDesc &d, const void *X, const void *dY, const void
     return dX ? ragged_conv<T>(x, d.in_hwc ? RAG_GK : RAG_KC, d.in_hwc ? RAG_KC : turn ? RAG_GK : RAG_XK, plan.ig) : 0;
 }
 
+// 1 x 1 layers of unit stride without padding on channel-major tensors: products of matrices.  -1: rows or images shorter than
+// a piece.
+template <typename T>
+int conv_point_fw(const ConvTileDesc &d, const void *X, const void *Wt, const void *bias, void *Y) {
+    constexpr int ES = (int)sizeof(T), VEC = 16 / ES;
+    const int P = d.Hin * d.Win;
+    if (!any_fits(d, ES) || P < VEC || d.Cin < VEC) return -1;
+    RagArgs r = {};
+    RagProd &p = r.p[0];
+    r.count = 1;
+    p.N = d.Cout;
+    p.M = d.batch * P;
+    p.m_in = P;
+    p.K = d.Cin;
+    p.a = any_rows<T>(Wt, d.Cout, (long long)d.Cin * ES);
+    p.b = any_rows<T>(X, P, 0);
+    p.b.k_b = (unsigned)(P * ES);
+    p.b.outer_b = (long long)d.Cin * P * ES;
+    p.C = Y;
+    p.cn = rag_axis(d.Cout, P);
+    p.cm = rag_axis2(P, 1, d.Cout * P);
+    p.runs = 1;
+    p.outer = d.batch;
+    p.bias = bias;
+    p.bias_n = 1;
+    return ragged<T>(r, RAG_KC, RAG_RC, RAG_KC, RAG_RC);
+}
+template int conv_point_fw<float>(const ConvTileDesc &, const void *, const void *, const void *, void *);
+template int conv_point_fw<half_t>(const ConvTileDesc &, const void *, const void *, const void *, void *);
+
+// Both gradients in one launch.
+template <typename T>
+int conv_point_bw(const ConvTileDesc &d, const void *X, const void *dY, const void *Wt, void *dW, void *dX, void *db) {
+    constexpr int ES = (int)sizeof(T), VEC = 16 / ES;
+    const int P = d.Hin * d.Win;
+    if (!any_fits(d, ES) || P < VEC || d.Cin < VEC) return -1;
+    RagConvArgs w = {}, x = {};
+    RagProd &p = w.p[0], &q = x.p[0];
+    w.count = x.count = 1;
+    p.N = d.Cout;
+    p.M = p.m_in = d.Cin;
+    p.K = P;
+    p.runs = d.batch;
+    p.a = any_rows<T>(dY, d.Cout, (long long)P * ES);
+    p.a.run_b = (long long)d.Cout * P * ES;
+    p.b = any_rows<T>(X, d.Cin, (long long)P * ES);
+    p.b.run_b = (long long)d.Cin * P * ES;
+    p.C = dW;
+    p.row_sum = db;
+    p.cn = rag_axis(d.Cout, d.Cin);
+    p.cm = rag_axis(d.Cin, 1);
+    q.N = d.Cin;
+    q.M = d.batch * P;
+    q.m_in = P;
+    q.K = d.Cout;
+    q.a = any_rows<T>(Wt, d.Cin, 0);
+    q.a.k_b = (unsigned)(d.Cin * ES);
+    q.b = any_rows<T>(dY, P, 0);
+    q.b.k_b = (unsigned)(P * ES);
+    q.b.outer_b = (long long)d.Cout * P * ES;
+    q.C = dX;
+    q.cn = rag_axis(d.Cin, P);
+    q.cm = rag_axis2(P, 1, d.Cin * P);
+    p.outer = q.runs = 1;
+    q.outer = d.batch;
+    const RagBackPlan plan = ragged_back_plan<T>(&p, &q, 1, RAG_BACK_POINT);
+    state().last_conv_resident = 0;
+    const RagGeo none = {};
+    return ragged_back<T>(w, x, &none, RAG_BACK_POINT, RAG_KC, plan);
+}
+
+template int conv_point_bw<float>(const ConvTileDesc &, const void *, const void *, const void *, void *, void *, void *);
+template int conv_point_bw<half_t>(const ConvTileDesc &, const void *, const void *, const void *, void *, void *, void *);
 template int conv_any_fw<float>(const ConvTileDesc &, const void *, const void *, const void *, void *);
 template int conv_any_fw<half_t>(const ConvTileDesc &, const void *, const void *, const void *, void *);
 template int conv_any_bw<float>(const ConvTileDesc &, const void *, const void *, const void *, void *, void *, void *);

@@ -374,6 +374,174 @@ static AxisMap tap_axis(const ConvGeom &g) {
     return a;
 }
 
+// The product behind a step of a pointwise layer; element (co, ci) of the weights lies at co * w_co + ci * w_ci.
+static GemmArgs pw_product(int step, const void *X, const void *Wt, const void *dY, void *out, int ns, int Ci, int Co, int HW, bool hwc, int w_co,
+                           int w_ci) {
+    GemmArgs q = {};
+    q.a.HL = q.a.WL = q.b.HL = q.b.WL = 1;
+    const int BP = ns * HW;
+    if (step == STEP_FW) {
+        q.C = out;
+        q.K = Ci;
+        if (!hwc) {
+            q.A = Wt;
+            q.B = X;
+            q.N = Co;
+            q.M = BP;
+            q.a.row = axis_plain(Co, Ci);
+            q.a.k = axis_plain(Ci, 1);
+            q.b.row = axis_two(BP, HW, Ci * HW, 1);
+            q.b.k = axis_plain(Ci, HW);
+            q.c.n = axis_plain(Co, HW);
+            q.c.m = axis_two(BP, HW, Co * HW, 1);
+        } else {
+            q.A = X;
+            q.B = Wt;
+            q.N = BP;
+            q.M = Co;
+            q.a.row = axis_plain(BP, Ci);
+            q.a.k = axis_plain(Ci, 1);
+            q.b.row = axis_plain(Co, w_co);
+            q.b.k = axis_plain(Ci, w_ci);
+            q.c.n = axis_plain(BP, Co);
+            q.c.m = axis_plain(Co, 1);
+        }
+    } else if (step == STEP_WGT_GRAD) {
+        q.A = dY;
+        q.B = X;
+        q.C = out;
+        q.N = Co;
+        q.M = Ci;
+        q.K = BP;
+        if (!hwc) {
+            q.a.row = axis_plain(Co, HW);
+            q.a.k = axis_two(BP, HW, Co * HW, 1);
+            q.b.row = axis_plain(Ci, HW);
+            q.b.k = axis_two(BP, HW, Ci * HW, 1);
+        } else {
+            q.a.row = axis_plain(Co, 1);
+            q.a.k = axis_plain(BP, Co);
+            q.b.row = axis_plain(Ci, 1);
+            q.b.k = axis_plain(BP, Ci);
+        }
+        q.c.n = axis_plain(Co, w_co);
+        q.c.m = axis_plain(Ci, w_ci);
+    } else {
+        q.C = out;
+        q.K = Co;
+        if (!hwc) {
+            q.A = Wt;
+            q.B = dY;
+            q.N = Ci;
+            q.M = BP;
+            q.a.row = axis_plain(Ci, w_ci);
+            q.a.k = axis_plain(Co, w_co);
+            q.b.row = axis_two(BP, HW, Co * HW, 1);
+            q.b.k = axis_plain(Co, HW);
+            q.c.n = axis_plain(Ci, HW);
+            q.c.m = axis_two(BP, HW, Ci * HW, 1);
+        } else {
+            q.A = dY;
+            q.B = Wt;
+            q.N = BP;
+            q.M = Ci;
+            q.a.row = axis_plain(BP, Co);
+            q.a.k = axis_plain(Co, 1);
+            q.b.row = axis_plain(Ci, w_ci);
+            q.b.k = axis_plain(Co, w_co);
+            q.c.n = axis_plain(BP, Ci);
+            q.c.m = axis_plain(Ci, 1);
+        }
+    }
+    return q;
+}
+
+// Weight and input gradient (and the bias gradient, where db is not null) of a dense layer over ns samples.  apart: what is
+// written shares no memory with what is read.
+template <typename T>
+static int dense_bw(const T *X, const T *Wt, const T *dY, T *dW, T *dX, T *db, int ns, int in, int out, bool apart) {
+    GemmArgs q = {}, r = {};
+    q.A = dY;  // dW[o][i] = sum_b dY[b][o] * X[b][i]
+    q.B = X;
+    q.C = dW;
+    q.N = out;
+    q.M = in;
+    q.K = ns;
+    q.a.row = axis_plain(out, 1);
+    q.a.k = axis_plain(ns, out);
+    q.b.row = axis_plain(in, 1);
+    q.b.k = axis_plain(ns, in);
+    q.a.HL = q.a.WL = q.b.HL = q.b.WL = 1;
+    q.c.n = axis_plain(out, in);
+    q.c.m = axis_plain(in, 1);
+    r.A = dY;  // dX[b][i] = sum_o dY[b][o] * W[o][i]
+    r.B = Wt;
+    r.C = dX;
+    r.N = ns;
+    r.M = in;
+    r.K = out;
+    r.a.row = axis_plain(ns, out);
+    r.a.k = axis_plain(out, 1);
+    r.b.row = axis_plain(in, 1);
+    r.b.k = axis_plain(out, in);
+    r.a.HL = r.a.WL = r.b.HL = r.b.WL = 1;
+    r.c.n = axis_plain(ns, in);
+    r.c.m = axis_plain(in, 1);
+    // Whole slabs of aligned rows: the look-up-free pair.  Other layers, and small ones with a bias (whose gradient
+    // would be a launch of its own: 2.5-4 us against the 1-2 us that the pair is faster), take the kernel for any
+    // size up to the work at which the look-up-free kernels' larger tiles make up for two launches.
+    const double flops = 4.0 * ns * in * out;
+    int rc = -1;
+    if (!apart) {
+        rc = ns == 1 ? mm_dispatch<T>(dY, X, dW, out, in, 1, 0) : gemm<T>(q);
+        if (rc == 0 && db) rc = bias_grad<T>(dY, db, ns, out, 1, 1);
+        return rc ? rc : mm_dispatch<T>(dY, Wt, dX, ns, in, out, 0);
+    }
+    if (!db || flops > 4e9) rc = gemm_pair_lean<T>(q, r);
+    if (rc < 0 && state().gemm_path == 0 && flops <= (sizeof(T) == 2 ? 3e10 : 1e10)) {
+        rc = linear_bw_ragged<T>(X, Wt, dY, dW, dX, db, ns, in, out);
+        if (rc >= 0) return rc;
+    }
+    if (rc < 0) rc = gemm_pair<T>(q, r);
+    if (rc == 0 && db) rc = bias_grad<T>(dY, db, ns, out, 1, 1);
+    return rc;
+}
+
+// Layers of one tap, unit stride and no padding are products of matrices: channel-minor ones dense layers over the pixels.
+static bool is_point(const ConvGeom &g) {
+    return g.Hk == 1 && g.Wk == 1 && g.sh == 1 && g.sw == 1 && g.H == g.Ho && g.W == g.Wo && g.Up == 0 && g.Lp == 0 && state().gemm_path == 0;
+}
+template <typename T>
+static int point_fw(const ConvGeom &g, int ns, const T *X, const T *Wt, const T *bias, T *Y) {
+    constexpr int VEC = 16 / (int)sizeof(T);
+    const int P = g.H * g.W;
+    if (!is_point(g) || g.Ci < VEC) return -1;
+    if (g.hwc) return mm_dispatch<T>(X, Wt, Y, ns * P, g.Co, g.Ci, 1, bias);
+    if (P < VEC) return -1;
+    if (bias) return conv_point_fw<T>(forward_desc(g, ns), X, Wt, bias, Y);
+    return gemm<T>(pw_product(STEP_FW, X, Wt, nullptr, Y, ns, g.Ci, g.Co, P, false, g.Ci, 1));
+}
+// Channel-major tensors: both gradients in one launch up to 40 MB of input and output, the two products by themselves above
+// (the patch matrices' time over theirs, mean of 400 layers, one launch / two products: fp16 2.4 / 1.6 below 0.3 MB, 1.8 / 1.4 at 3 to
+// 30, 1.5 / 1.4 at 30 to 100, 0.8 / 1.2 above; fp32 1.9 / 1.4, 1.4 / 1.2, 1.05 / 1.11, 1.07 / 1.23).  Channel-minor fp16 layers
+// above 100 MB stay with the patch matrices (0.82).
+template <typename T>
+static int point_bw(const ConvGeom &g, int ns, const T *X, const T *dY, const T *Wt, T *dW, T *dX, T *db) {
+    constexpr int VEC = 16 / (int)sizeof(T);
+    const int P = g.H * g.W;
+    if (!is_point(g) || g.Ci < VEC || g.Co < VEC) return -1;
+    const double mb = 1e-6 * sizeof(T) * ns * P * ((double)g.Ci + g.Co);
+    if (g.hwc) return sizeof(T) == 2 && mb > 100 ? -1 : dense_bw<T>(X, Wt, dY, dW, dX, db, ns * P, g.Ci, g.Co, true);
+    if (P < VEC) return -1;
+    if (mb <= 40) {
+        const int rc = conv_point_bw<T>(forward_desc(g, ns), X, dY, Wt, dW, dX, db);
+        if (rc >= 0) return rc;
+    }
+    int rc = gemm<T>(pw_product(STEP_WGT_GRAD, X, nullptr, dY, dW, ns, g.Ci, g.Co, P, false, g.Ci, 1));
+    if (rc == 0 && db) rc = bias_grad<T>(dY, db, ns, g.Co, P, 0);
+    return rc ? rc : gemm<T>(pw_product(STEP_IN_GRAD, nullptr, Wt, dY, dX, ns, g.Ci, g.Co, P, false, g.Ci, 1));
+}
+
 template <typename T, typename Args>
 static int conv2d_fw(const Args *a, int ns, const char *fn) {
     ConvGeom g;
@@ -419,10 +587,12 @@ static int conv2d_fw(const Args *a, int ns, const char *fn) {
         // (the small-layer kernel adds no bias, which is a launch of its own: 8 -> 16 channels on 8 x 8, 7 samples, fp16 8.3
         // against 7.3 us, 8 -> 48 on 40 x 40, 8 samples, fp32 17.5 against 8.4; without one its bits are those of the call
         // that also forms the output's sums)
+        if (bias && !conv_small_pre_pending() && (rc = point_fw<T>(g, ns, X, Wt, bias, Y)) >= 0) return sg.finish(rc);
         if (bias && !conv_small_pre_pending() && any_pays<T>(g, ns, 1, true) && (rc = conv_any_fw<T>(d, X, Wt, bias, Y)) >= 0) return sg.finish(rc);
         if (!g.hwc) rc = conv_small<T>(d, X, Wt, Y);
         // (a normalisation to apply on the way in is the small-layer kernel's business alone: nothing was launched)
         if (rc == CONV_PRE_REFUSED || conv_small_pre_pending()) return CONV_PRE_REFUSED;
+        if (rc < 0 && (rc = point_fw<T>(g, ns, X, Wt, bias, Y)) >= 0) return sg.finish(rc);
         if (rc < 0) rc = conv_taps<T>(d, X, Wt, Y, c);
         if (rc < 0 && any_pays<T>(g, ns, 1, bias != nullptr) && (rc = conv_any_fw<T>(d, X, Wt, bias, Y)) >= 0) return sg.finish(rc);
         if (rc < 0) rc = conv_tile<T>(d, X, Wt, Y, c);
@@ -891,7 +1061,8 @@ static int conv2d_bw(const Args *a, int ns, const char *fn) {
             if (sg.failed()) return sg.rejected() ? 1 : 2;
             state().last_conv_direct = 0;
             state().last_conv_resident = 0;
-            const int rc = conv_any_bw<T>(d, X, dY, Wt, dW, dX, db);
+            int rc = point_bw<T>(g, ns, X, dY, Wt, dW, dX, db);
+            if (rc < 0) rc = conv_any_bw<T>(d, X, dY, Wt, dW, dX, db);
             if (rc >= 0) return sg.finish(rc);
             sg.discard();
         }
@@ -917,91 +1088,14 @@ static int pw_step(const Args *a, int ns, int step, const char *fn) {
         return 1;
     }
     Stager sg;
-    GemmArgs q = {};
-    q.a.HL = q.a.WL = q.b.HL = q.b.WL = 1;
-    const int BP = ns * HW;
-    if (step == STEP_FW) {
-        const T *X = sg.in(reinterpret_cast<const T *>(a->input->data), in_n);
-        const T *Wt = sg.in(reinterpret_cast<const T *>(a->coeff->data), (size_t)Co * Ci);
-        T *Y = sg.out(reinterpret_cast<T *>(a->output->data), out_n);
-        q.C = Y;
-        q.K = Ci;
-        if (!hwc) {
-            q.A = Wt;
-            q.B = X;
-            q.N = Co;
-            q.M = BP;
-            q.a.row = axis_plain(Co, Ci);
-            q.a.k = axis_plain(Ci, 1);
-            q.b.row = axis_two(BP, HW, Ci * HW, 1);
-            q.b.k = axis_plain(Ci, HW);
-            q.c.n = axis_plain(Co, HW);
-            q.c.m = axis_two(BP, HW, Co * HW, 1);
-        } else {
-            q.A = X;
-            q.B = Wt;
-            q.N = BP;
-            q.M = Co;
-            q.a.row = axis_plain(BP, Ci);
-            q.a.k = axis_plain(Ci, 1);
-            q.b.row = axis_plain(Co, w_co);
-            q.b.k = axis_plain(Ci, w_ci);
-            q.c.n = axis_plain(BP, Co);
-            q.c.m = axis_plain(Co, 1);
-        }
-    } else if (step == STEP_WGT_GRAD) {
-        const T *X = sg.in(reinterpret_cast<const T *>(a->input->data), in_n);
-        const T *dY = sg.in(reinterpret_cast<const T *>(a->output->diff), out_n);
-        T *dW = sg.out(reinterpret_cast<T *>(a->coeff->diff), (size_t)Co * Ci);
-        q.A = dY;
-        q.B = X;
-        q.C = dW;
-        q.N = Co;
-        q.M = Ci;
-        q.K = BP;
-        if (!hwc) {
-            q.a.row = axis_plain(Co, HW);
-            q.a.k = axis_two(BP, HW, Co * HW, 1);
-            q.b.row = axis_plain(Ci, HW);
-            q.b.k = axis_two(BP, HW, Ci * HW, 1);
-        } else {
-            q.a.row = axis_plain(Co, 1);
-            q.a.k = axis_plain(BP, Co);
-            q.b.row = axis_plain(Ci, 1);
-            q.b.k = axis_plain(BP, Ci);
-        }
-        q.c.n = axis_plain(Co, w_co);
-        q.c.m = axis_plain(Ci, w_ci);
-    } else {
-        const T *Wt = sg.in(reinterpret_cast<const T *>(a->coeff->data), (size_t)Co * Ci);
-        const T *dY = sg.in(reinterpret_cast<const T *>(a->output->diff), out_n);
-        T *dX = sg.out(reinterpret_cast<T *>(a->input->diff), in_n);
-        q.C = dX;
-        q.K = Co;
-        if (!hwc) {
-            q.A = Wt;
-            q.B = dY;
-            q.N = Ci;
-            q.M = BP;
-            q.a.row = axis_plain(Ci, w_ci);
-            q.a.k = axis_plain(Co, w_co);
-            q.b.row = axis_two(BP, HW, Co * HW, 1);
-            q.b.k = axis_plain(Co, HW);
-            q.c.n = axis_plain(Ci, HW);
-            q.c.m = axis_two(BP, HW, Ci * HW, 1);
-        } else {
-            q.A = dY;
-            q.B = Wt;
-            q.N = BP;
-            q.M = Ci;
-            q.a.row = axis_plain(BP, Co);
-            q.a.k = axis_plain(Co, 1);
-            q.b.row = axis_plain(Ci, w_ci);
-            q.b.k = axis_plain(Co, w_co);
-            q.c.n = axis_plain(BP, Ci);
-            q.c.m = axis_plain(Ci, 1);
-        }
-    }
+    const size_t w_n = (size_t)Co * Ci;
+    const T *X = step != STEP_IN_GRAD ? sg.in(reinterpret_cast<const T *>(a->input->data), in_n) : nullptr;
+    const T *dY = step != STEP_FW ? sg.in(reinterpret_cast<const T *>(a->output->diff), out_n) : nullptr;
+    const T *Wt = step != STEP_WGT_GRAD ? sg.in(reinterpret_cast<const T *>(a->coeff->data), w_n) : nullptr;
+    T *out = step == STEP_FW ? sg.out(reinterpret_cast<T *>(a->output->data), out_n)
+             : step == STEP_WGT_GRAD ? sg.out(reinterpret_cast<T *>(a->coeff->diff), w_n)
+                                     : sg.out(reinterpret_cast<T *>(a->input->diff), in_n);
+    const GemmArgs q = pw_product(step, X, Wt, dY, out, ns, Ci, Co, HW, hwc, w_co, w_ci);
     if (sg.failed()) return 2;
     return sg.finish(gemm<T>(q));
 }
@@ -1054,50 +1148,7 @@ static int linear_step(const Args *a, int ns, int step, const char *fn) {
         if (sg.failed()) return 2;
         const bool apart = !backward_shares_memory<T>(X, (size_t)ns * in, Wt, (size_t)out * in, dY, (size_t)ns * out, dW, dX, db, (size_t)out);
         if (ns == 1 && apart) return sg.finish(linear_one_bw<T>(X, Wt, dY, dW, dX, db, in, out));
-        GemmArgs q = {}, r = {};
-        q.A = dY;  // dW[o][i] = sum_b dY[b][o] * X[b][i]
-        q.B = X;
-        q.C = dW;
-        q.N = out;
-        q.M = in;
-        q.K = ns;
-        q.a.row = axis_plain(out, 1);
-        q.a.k = axis_plain(ns, out);
-        q.b.row = axis_plain(in, 1);
-        q.b.k = axis_plain(ns, in);
-        q.a.HL = q.a.WL = q.b.HL = q.b.WL = 1;
-        q.c.n = axis_plain(out, in);
-        q.c.m = axis_plain(in, 1);
-        r.A = dY;  // dX[b][i] = sum_o dY[b][o] * W[o][i]
-        r.B = Wt;
-        r.C = dX;
-        r.N = ns;
-        r.M = in;
-        r.K = out;
-        r.a.row = axis_plain(ns, out);
-        r.a.k = axis_plain(out, 1);
-        r.b.row = axis_plain(in, 1);
-        r.b.k = axis_plain(out, in);
-        r.a.HL = r.a.WL = r.b.HL = r.b.WL = 1;
-        r.c.n = axis_plain(ns, in);
-        r.c.m = axis_plain(in, 1);
-        // Whole slabs of aligned rows: the look-up-free pair.  Other layers, and small ones with a bias (whose gradient
-        // would be a launch of its own: 2.5-4 us against the 1-2 us that the pair is faster), take the kernel for any
-        // size up to the work at which the look-up-free kernels' larger tiles make up for two launches.
-        const double flops = 4.0 * ns * in * out;
-        rc = -1;
-        if (!apart) {
-            rc = ns == 1 ? mm_dispatch<T>(dY, X, dW, out, in, 1, 0) : gemm<T>(q);
-            if (rc == 0 && db) rc = bias_grad<T>(dY, db, ns, out, 1, 1);
-            return sg.finish(rc ? rc : mm_dispatch<T>(dY, Wt, dX, ns, in, out, 0));
-        }
-        if (!db || flops > 4e9) rc = gemm_pair_lean<T>(q, r);
-        if (rc < 0 && state().gemm_path == 0 && flops <= (sizeof(T) == 2 ? 3e10 : 1e10)) {
-            rc = linear_bw_ragged<T>(X, Wt, dY, dW, dX, db, ns, in, out);
-            if (rc >= 0) return sg.finish(rc);
-        }
-        if (rc < 0) rc = gemm_pair<T>(q, r);
-        if (rc == 0 && db) rc = bias_grad<T>(dY, db, ns, out, 1, 1);
+        rc = dense_bw<T>(X, Wt, dY, dW, dX, db, ns, in, out, apart);
     } else if (step == STEP_WGT_GRAD) {
         const T *X = sg.in(reinterpret_cast<const T *>(a->input->data), (size_t)ns * in);
         const T *dY = sg.in(reinterpret_cast<const T *>(a->output->diff), (size_t)ns * out);

@@ -150,12 +150,13 @@ template <typename T>
 int ragged_conv(RagConvArgs &r, int a, int b, const RagPlan &plan);
 // Both gradients of a layer in one launch (plus one for partial sums): the weight gradient of w (modes a, b; none where its
 // count is 0), then the products of x, whose filters are read in place as f says - channel-major by XK, channel-minor by WR -
-// or, where b is GR and the tensors of x are channel-minor copies (KC, GK), re-laid.
+// or, where the tensors of x are channel-minor copies (KC, GK), re-laid.  POINT: 1 x 1 layers of unit stride on channel-major
+// tensors, which are matrices (KC, KC before RC, RC).
 struct RagBackPlan {
     int per_w, per_x;  // slabs per workgroup
     double clocks;
 };
-enum RagBack : int { RAG_BACK_MAJOR = 0, RAG_BACK_MINOR = 1, RAG_BACK_COPIES = 2 };
+enum RagBack : int { RAG_BACK_MAJOR = 0, RAG_BACK_MINOR = 1, RAG_BACK_COPIES = 2, RAG_BACK_POINT = 3 };
 template <typename T>
 RagBackPlan ragged_back_plan(const RagProd *w, const RagProd *x, int count, RagBack kind);
 template <typename T>
