@@ -1037,7 +1037,9 @@ static int conv2d_bw(const Args *a, int ns, const char *fn) {
     // has a kernel of its own that is ahead: the raw-tile weight gradient of unit-stride 3x3 layers from 10 GFLOP on (other over
     // this: 1.18 in the mean at 3 to 6 GFLOP, 1.06 at 6 to 10, 0.98 at 10 to 20, 0.94 above; 1x1 layers 1.2 above 10), the
     // resident-tile one wherever it is preferred (a call then has the bits of its two steps), and those of channel-minor
-    // layers from 20 on (1.77, 1.26 and 1.22 at 4, 10 and 19, 0.92 and 0.82 at 31 and 39).
+    // layers from 20 on (1.77, 1.26 and 1.22 at 4, 10 and 19, 0.92 and 0.82 at 31 and 39).  Strided channel-major 1x1 layers,
+    // whose input gradient is a plain product scattered over zeros, from some MB of input and output on (fp16 1.4 in the
+    // mean at 3 to 5 MB, 1.0 at 7 to 30, 0.8 above; fp32 1.4 at 7 to 10, 1.1 at 10 to 30, 0.8 above).
     if (apart && (a->USE_BIASES != 1 || a->bias)) {
         ConvGeom g;
         if (int rc = conv_geom(a, g, fn, true)) return rc;
@@ -1049,8 +1051,9 @@ static int conv2d_bw(const Args *a, int ns, const char *fn) {
         const bool own_wg = g.sh == 1 && g.sw == 1 && sizeof(T) == 2 && !g.hwc && K > g.Ci && g.Hk <= 3 &&
                             (gflop >= 10 || (g.Hk == 3 && g.Wk == 3 && conv_halo_wg_preferred(d)));
         const bool resident = sizeof(T) == 2 && g.hwc && gflop >= 20 && conv_halo_wg_hwc_fits(d, nullptr, nullptr) && conv_halo_wg_hwc_preferred(d);
+        const bool scatter = K == g.Ci && (g.sh > 1 || g.sw > 1) && !g.hwc && sizeof(T) * (in_n + out_n) >= (sizeof(T) == 2 ? 7000000 : 30000000);
         const bool forced = state().gemm_path >= 7;
-        if ((forced || (state().gemm_path == 0 && !own_wg && !resident)) && fits_int(in_n) && fits_int(out_n)) {
+        if ((forced || (state().gemm_path == 0 && !own_wg && !resident && !scatter)) && fits_int(in_n) && fits_int(out_n)) {
             Stager sg;
             const T *X = sg.in(reinterpret_cast<const T *>(a->input->data), in_n);
             const T *dY = sg.in(reinterpret_cast<const T *>(a->output->diff), out_n);
