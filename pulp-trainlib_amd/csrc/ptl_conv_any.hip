@@ -402,8 +402,7 @@ int conv_any_bw(const ConvTileDesc &d, const void *X, const void *dY, const void
     return dX ? ragged_conv<T>(x, d.in_hwc ? RAG_GK : RAG_KC, d.in_hwc ? RAG_KC : turn ? RAG_GK : RAG_XK, plan.ig) : 0;
 }
 
-// 1 x 1 layers of unit stride without padding on channel-major tensors: products of matrices.  -1: rows or images shorter than
-// a piece.
+// 1 x 1 layers of unit stride without padding: products of matrices.  -1: rows or images shorter than a piece.
 template <typename T>
 int conv_point_fw(const ConvTileDesc &d, const void *X, const void *Wt, const void *bias, void *Y) {
     constexpr int ES = (int)sizeof(T), VEC = 16 / ES;
@@ -411,28 +410,36 @@ int conv_point_fw(const ConvTileDesc &d, const void *X, const void *Wt, const vo
     if (!any_fits(d, ES) || P < VEC || d.Cin < VEC) return -1;
     RagArgs r = {};
     RagProd &p = r.p[0];
-    r.count = 1;
+    r.count = p.runs = p.outer = 1;
+    p.K = d.Cin;
+    p.C = Y;
+    p.bias = bias;
+    RagOp &pixels = d.in_hwc ? p.a : p.b, &weight = d.in_hwc ? p.b : p.a;
+    weight = any_rows<T>(Wt, d.Cout, (long long)d.Cin * ES);
+    if (d.in_hwc) {
+        p.N = d.batch * P;
+        p.M = p.m_in = d.Cout;
+        pixels = any_rows<T>(X, p.N, (long long)d.Cin * ES);
+        p.cn = rag_axis(p.N, d.Cout);
+        p.cm = rag_axis(d.Cout, 1);
+        return ragged<T>(r, RAG_KC, RAG_KC, RAG_KC, RAG_KC);
+    }
     p.N = d.Cout;
     p.M = d.batch * P;
     p.m_in = P;
-    p.K = d.Cin;
-    p.a = any_rows<T>(Wt, d.Cout, (long long)d.Cin * ES);
-    p.b = any_rows<T>(X, P, 0);
-    p.b.k_b = (unsigned)(P * ES);
-    p.b.outer_b = (long long)d.Cin * P * ES;
-    p.C = Y;
+    p.outer = d.batch;
+    pixels = any_rows<T>(X, P, 0);
+    pixels.k_b = (unsigned)(P * ES);
+    pixels.outer_b = (long long)d.Cin * P * ES;
     p.cn = rag_axis(d.Cout, P);
     p.cm = rag_axis2(P, 1, d.Cout * P);
-    p.runs = 1;
-    p.outer = d.batch;
-    p.bias = bias;
     p.bias_n = 1;
     return ragged<T>(r, RAG_KC, RAG_RC, RAG_KC, RAG_RC);
 }
 template int conv_point_fw<float>(const ConvTileDesc &, const void *, const void *, const void *, void *);
 template int conv_point_fw<half_t>(const ConvTileDesc &, const void *, const void *, const void *, void *);
 
-// Both gradients in one launch.
+// Both gradients in one launch, channel-major tensors.
 template <typename T>
 int conv_point_bw(const ConvTileDesc &d, const void *X, const void *dY, const void *Wt, void *dW, void *dX, void *db) {
     constexpr int ES = (int)sizeof(T), VEC = 16 / ES;

@@ -236,7 +236,7 @@ template <typename T>
 int conv_any_fw(const ConvTileDesc &d, const void *X, const void *Wt, const void *bias, void *Y);
 template <typename T>
 int conv_any_bw(const ConvTileDesc &d, const void *X, const void *dY, const void *Wt, void *dW, void *dX, void *db);
-// 1 x 1 layers of unit stride without padding, channel-major (see ptl_conv_any.hip).
+// 1 x 1 layers of unit stride without padding; the gradients of channel-major ones (see ptl_conv_any.hip).
 template <typename T>
 int conv_point_fw(const ConvTileDesc &d, const void *X, const void *Wt, const void *bias, void *Y);
 template <typename T>

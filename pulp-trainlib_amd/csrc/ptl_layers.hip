@@ -515,25 +515,28 @@ template <typename T>
 static int point_fw(const ConvGeom &g, int ns, const T *X, const T *Wt, const T *bias, T *Y) {
     constexpr int VEC = 16 / (int)sizeof(T);
     const int P = g.H * g.W;
-    if (!is_point(g) || g.Ci < VEC) return -1;
+    if (!is_point(g) || g.Ci < VEC || P < VEC) return -1;
+    // (fp32 on the kernel for any size: its sums are nearer to 64 bits, 1.1e-7 against 2.0e-7 for 448 -> 47 channels)
+    if (sizeof(T) == 4 || (bias && !g.hwc)) return conv_point_fw<T>(forward_desc(g, ns), X, Wt, bias, Y);
     if (g.hwc) return mm_dispatch<T>(X, Wt, Y, ns * P, g.Co, g.Ci, 1, bias);
-    if (P < VEC) return -1;
-    if (bias) return conv_point_fw<T>(forward_desc(g, ns), X, Wt, bias, Y);
     return gemm<T>(pw_product(STEP_FW, X, Wt, nullptr, Y, ns, g.Ci, g.Co, P, false, g.Ci, 1));
 }
-// Channel-major tensors: both gradients in one launch up to 40 MB of input and output, the two products by themselves above
-// (the patch matrices' time over theirs, mean of 400 layers, one launch / two products: fp16 2.4 / 1.6 below 0.3 MB, 1.8 / 1.4 at 3 to
-// 30, 1.5 / 1.4 at 30 to 100, 0.8 / 1.2 above; fp32 1.9 / 1.4, 1.4 / 1.2, 1.05 / 1.11, 1.07 / 1.23).  Channel-minor fp16 layers
-// above 100 MB stay with the patch matrices (0.82).
+// Channel-major tensors: both gradients in one launch, fp16 up to 40 MB of input and output, the two products by themselves
+// above (the patch matrices' time over theirs, mean of 400 layers, one launch / two products: fp16 2.4 / 1.6 below 0.3 MB,
+// 1.8 / 1.4 at 3 to 30, 1.5 / 1.4 at 30 to 100, 0.8 / 1.2 above).  Channel-minor fp16 layers above 100 MB stay with the
+// patch matrices (0.82).
 template <typename T>
 static int point_bw(const ConvGeom &g, int ns, const T *X, const T *dY, const T *Wt, T *dW, T *dX, T *db) {
     constexpr int VEC = 16 / (int)sizeof(T);
     const int P = g.H * g.W;
     if (!is_point(g) || g.Ci < VEC || g.Co < VEC) return -1;
     const double mb = 1e-6 * sizeof(T) * ns * P * ((double)g.Ci + g.Co);
-    if (g.hwc) return sizeof(T) == 2 && mb > 100 ? -1 : dense_bw<T>(X, Wt, dY, dW, dX, db, ns * P, g.Ci, g.Co, true);
+    if (g.hwc) {
+        if (sizeof(T) == 4) return linear_bw_ragged<T>(X, Wt, dY, dW, dX, db, ns * P, g.Ci, g.Co);
+        return mb > 100 ? -1 : dense_bw<T>(X, Wt, dY, dW, dX, db, ns * P, g.Ci, g.Co, true);
+    }
     if (P < VEC) return -1;
-    if (mb <= 40) {
+    if (mb <= 40 || sizeof(T) == 4) {
         const int rc = conv_point_bw<T>(forward_desc(g, ns), X, dY, Wt, dW, dX, db);
         if (rc >= 0) return rc;
     }

@@ -1,0 +1,65 @@
+"""fp32 products formed from three bf16 pieces of each value: infinities and values below the pieces' range go through the fp32
+instructions, and the bf16 instructions' rounding (towards minus infinity) does not add up over long contractions."""
+import pytest
+import torch
+
+import helpers as hp
+from test_gpu_conv_any import rel, tensor
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+def point_layer(pkg, ns, Ci, Co, P, g):
+    x, dx, dy = tensor(g, (ns, Ci, 1, P), "fp32"), tensor(g, (ns, Ci, 1, P), "fp32"), tensor(g, (ns, Co, 1, P), "fp32")
+    w, dw = tensor(g, (Co, Ci), "fp32"), tensor(g, (Co, Ci), "fp32")
+    a, keep = hp.conv2d_args(pkg, x, dx, w, dw, dy, dy, Ci, 1, P, Co, 1, 1, 1, P, (0, 0, 0, 0), (1, 1), 0)
+    return x, dx, dy, w, dw, a, keep
+
+
+@pytest.mark.parametrize("what", ["infinity", "nan", "huge", "tiny"])
+def test_values_outside_the_range_of_the_pieces(pkg, gpu, what):
+    g = torch.Generator(device=DEV).manual_seed(3)
+    ns, Ci, Co, P = 32, 270, 300, 333  # (contractions of 19 slabs and of 666: sixteen a workgroup or more take pieces)
+    x, dx, dy, w, dw, a, keep = point_layer(pkg, ns, Ci, Co, P, g)
+    if what == "tiny":  # (the third piece of 1e-35 lies below the smallest bf16)
+        x.mul_(1e-35)
+        dy[:, 7].mul_(1e-2)
+    else:  # (huge: rounds up to infinity as a bf16)
+        x[2, 3, 0, 77] = {"infinity": float("inf"), "nan": float("nan"), "huge": 3.4e38}[what]
+        dy[4, 9, 0, 5] = {"infinity": -float("inf"), "nan": float("nan"), "huge": -3.4e38}[what]
+        if what == "huge":
+            dy.mul_(0.25)
+    pkg.call("ptl_conv2d_fp32_bw_batched", a, ns)
+    assert gpu.ptl_sync() == 0 and gpu.ptl_last_gemm_tile() == 64064
+    X, D, W = x.double().reshape(ns, Ci, P), dy.double().reshape(ns, Co, P), w.double()
+    ref_dw = sum(D[b] @ X[b].t().contiguous() for b in range(ns))
+    ref_dx = torch.stack([W.t().contiguous() @ D[b] for b in range(ns)])
+    for got, ref in ((dw, ref_dw), (dx.reshape(ns, Ci, P), ref_dx)):
+        got = got.double()
+        ref = torch.where(ref.abs() > torch.finfo(torch.float32).max, ref * float("inf"), ref)
+        assert torch.equal(got.isnan(), ref.isnan())
+        assert torch.equal(got.isinf(), ref.isinf()) and torch.equal(got[ref.isinf()], ref[ref.isinf()])
+        fin = ref.isfinite()
+        row = ref[fin].abs().max() if what == "huge" else (ref[fin] ** 2).mean().sqrt()
+        # 10 700 products, 660 slabs: sqrt(660 / 3) roundings of 2^-25 and of 2^-24 in eight, five times that for the largest of 81 000
+        assert float((got[fin] - ref[fin]).abs().max()) <= 4e-6 * float(row)
+    if what == "tiny":  # row 7 by itself
+        assert rel(dw[7], ref_dw[7]) <= 1e-6 and rel(dw[8], ref_dw[8]) <= 1e-6
+
+
+def test_long_contractions_have_no_drift(pkg, gpu):
+    """37 000 products a sum.  One rounding of 2^-25 towards minus infinity per instruction (six to 16 products) of sums of
+    the size sqrt(32), added up, would be 3e-7 of a result; what is left of it when every other slab has the other sign is
+    at most one slab's, 1e-8 or less."""
+    g = torch.Generator(device=DEV).manual_seed(4)
+    ns, Ci, Co, P = 64, 31, 300, 576
+    x, dx, dy, w, dw, a, keep = point_layer(pkg, ns, Ci, Co, P, g)
+    pkg.call("ptl_conv2d_fp32_bw_batched", a, ns)
+    assert gpu.ptl_sync() == 0
+    X, D = x.double().reshape(ns, Ci, P), dy.double().reshape(ns, Co, P)
+    ref = sum(D[b] @ X[b].t().contiguous() for b in range(ns))
+    err, rms = dw.double() - ref, float((ref ** 2).mean().sqrt())
+    assert abs(float(err.mean())) <= 5e-8 * rms
+    # random roundings: 8 slabs, then up to 50 sums of eight: sqrt((8 + 50) / 6) 2^-24 / sqrt(12) * 2, and a slab's own 7e-8
+    assert rel(dw, ref) <= 2e-7
