@@ -178,4 +178,30 @@ int gemm_async_pair(GemmArgs &g0, GemmArgs &g1);
 template <typename T>
 int mm_dispatch(const T *A, const T *B, T *C, int N, int M, int K, int trans_B, const T *bias = nullptr);
 
+#ifdef __HIP_DEVICE_COMPILE__
+// Asks for all lines of a kernel's arguments at its start.  They lie in memory, and the compiler loads each where it is
+// needed: a line that is asked for behind an index or a branch that came from another line is one more trip before the first
+// load of data.
+template <typename... A>
+constexpr int args_bytes() {
+    int n = 0;
+    ((n = (n + (int)alignof(A) - 1) / (int)alignof(A) * (int)alignof(A) + (int)sizeof(A)), ...);
+    return n;
+}
+template <typename... A>
+__device__ __forceinline__ void fetch_args(const A &...) {  // all arguments, in their order
+    typedef const unsigned __attribute__((address_space(4))) *Words;
+    const Words p = (Words)__builtin_amdgcn_kernarg_segment_ptr();
+    constexpr int LINES = (args_bytes<A...>() + 63) / 64;
+#pragma unroll
+    for (int l = 0; l < LINES; l += 8) {
+        auto word = [&](int i) { return p[(l + i < LINES ? l + i : LINES - 1) * 16]; };
+        asm volatile("" ::"s"(word(0)), "s"(word(1)), "s"(word(2)), "s"(word(3)), "s"(word(4)), "s"(word(5)), "s"(word(6)), "s"(word(7)));
+    }
+}
+#else
+template <typename... A>
+__device__ inline void fetch_args(const A &...) {}
+#endif
+
 }  // namespace ptl

@@ -18,6 +18,7 @@ inline RagDiv rag_div(long long dv) {
     r.s = l - 1;
     return r;
 }
+__device__ inline unsigned rag_quot(unsigned n, const RagDiv &d) { return d.m ? __umulhi(n, d.m) >> d.s : n; }
 
 // How an operand's tile is filled.  KC and RC: 16-byte pieces of a matrix whose rows (KC) or whose k columns (RC) are
 // contiguous.  The others are implicit patch matrices (RagGeo): XK and XR gather a channel-major tensor element by element,

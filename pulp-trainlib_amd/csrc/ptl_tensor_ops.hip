@@ -8,10 +8,12 @@
 // measured against HBM bandwidth, not the matrix cores.
 #include "ptl_common.hpp"
 #include "ptl_host.hpp"
+#include "ptl_ragged.hpp"
 #include "ptl_api.h"
 
 #include <stdio.h>
 #include <algorithm>
+#include <type_traits>
 
 namespace ptl {
 
@@ -1256,6 +1258,36 @@ struct PatchGeom {
 
 typedef unsigned PatchPiece __attribute__((ext_vector_type(4)));  // (a built-in vector: loads from any address space)
 __device__ const PatchPiece patch_zero = {0u, 0u, 0u, 0u};  // what the window holds outside the tensor
+typedef unsigned PatchRun __attribute__((ext_vector_type(4), aligned(2)));  // (element alignment of the narrower type)
+
+// A piece of a row that was read d elements before (d > 0) or behind the place that is meant: moved there, with zeros.
+template <typename T>
+__device__ inline PatchPiece patch_shift(PatchPiece v, int d) {
+    const int bits = (d < 0 ? -d : d) * 8 * (int)sizeof(T);
+    if (d > 0) {  // towards element 0
+        if (bits & 64) v = PatchPiece{v.z, v.w, 0u, 0u};
+        if (bits & 32) v = PatchPiece{v.y, v.z, v.w, 0u};
+        const unsigned bs = bits & 31;
+        v = PatchPiece{__builtin_amdgcn_alignbit(v.y, v.x, bs), __builtin_amdgcn_alignbit(v.z, v.y, bs),
+                       __builtin_amdgcn_alignbit(v.w, v.z, bs), v.w >> bs};
+    } else if (d < 0) {
+        if (bits & 64) v = PatchPiece{0u, 0u, v.x, v.y};
+        if (bits & 32) v = PatchPiece{0u, v.x, v.y, v.z};
+        const unsigned bs = bits & 31;  // (0 or 16: a left shift by 16 is alignbit(hi, lo, 16) one dword up)
+        if (bs) v = PatchPiece{v.x << 16, __builtin_amdgcn_alignbit(v.y, v.x, 16), __builtin_amdgcn_alignbit(v.z, v.y, 16),
+                               __builtin_amdgcn_alignbit(v.w, v.z, 16)};
+    }
+    return v;
+}
+
+// Which of n tiles workgroup b of n takes, so that every XCD has a run of them: workgroups go to the eight XCDs in turn.
+__device__ inline unsigned xcd_run(unsigned b, unsigned n) {
+    const unsigned xcd = b & 7;
+    return (b >> 3) + xcd * (n >> 3) + min(xcd, n & 7);
+}
+
+// How patch_rows_kernel reads rows of the tensor.
+enum PatchRead { PATCH_SINGLE, PATCH_ALIGNED, PATCH_MOVED };
 
 // buf(p, q) = src[c, hp*h_mul + h_add + hk, wp*w_mul + w_add + wk] or 0 outside,
 // p = hp*Wp + wp, q = (c,hk,wk) for CHW and (hk,wk,c) for HWC.
@@ -1383,22 +1415,32 @@ __global__ __launch_bounds__(256) void patch_kernel(const T *__restrict__ src, T
 // R buffer rows as 16-byte chunks, each gathered from LDS.  Divisions by the runtime extents are multiplications
 // by ceil(2^32 / d) (exact for dividends below 2^16).
 // A vector memory instruction occupies the address unit for its 64 lanes whatever each lane moves, so the window
-// is read in as few instructions as the layout allows: WIDE (rows of the tensor start on 16-byte boundaries) takes
-// the aligned 16-byte pieces that cover the window - the window then starts up to a piece early, `shift` elements
-// that the offsets table skips - and otherwise one element per lane, one wave per window row.
+// is read in as few instructions as the layout allows: pieces of 16 bytes, PATCH_ALIGNED where rows of the tensor start on
+// 16-byte boundaries (the window then starts up to a piece early, `shift` elements that the offsets table skips),
+// PATCH_MOVED from wherever the window starts (a piece that would begin before its row or end behind it is read where it
+// fits and shifted), and one element per lane, one wave per window row, from rows shorter than a piece.
+// The workgroups that write one run of buffer rows follow each other on one XCD (xcd_run): where their parts meet inside a
+// line, it is put together in that L2.
+// Single elements and places in turn over the XCDs before / now, 3 x 3: 111 channels of 237 x 68 in fp16 16.6 / 10.1 us, 16 of
+// 53 x 33 4.05 / 2.9; 192 of 97 x 76 in fp32, aligned, 15.2 / 12.4.
 // The writes bound it (a 3x3 filter writes nine elements per one read), and whole chunks serve rows of any length and
 // start: the last chunk of a row piece ends with the piece, the channels are split into equal pieces whatever their
-// number.  154 channels of 60 x 253 in fp16, 3 x 3: 47.6 us, 106.6 one element at a time;
-// 186 channels of 212 x 154 in fp32: 110 us, before 258.
-template <typename T, bool WIDE>
+// number.
+template <typename T, PatchRead READ>
 __global__ __launch_bounds__(256) void patch_rows_kernel(const T *__restrict__ src, T *__restrict__ buf, PatchGeom g, int R,
-                                                         int CB, int LW, unsigned m_pk, unsigned m_wk, unsigned m_hk) {
+                                                         int CB, int LW, unsigned m_pk, unsigned m_wk, unsigned m_hk, int np, unsigned m_np,
+                                                         RagDiv by_nx, RagDiv by_nz, unsigned tiles) {
+    fetch_args(src, buf, g, R, CB, LW, m_pk, m_wk, m_hk, np, m_np, by_nx, by_nz, tiles);
+    const int nx = (int)by_nx.d, nz = (int)by_nz.d;
+    constexpr bool WIDE = READ == PATCH_ALIGNED;
     constexpr int VEC = 16 / (int)sizeof(T);
     // (as global-memory pointers: a generic one would load through the flat path, whose waits are shared with LDS)
     typedef const T __attribute__((address_space(1))) *GlobalT;
     typedef const PatchPiece __attribute__((address_space(1))) *GlobalPiece;
+    typedef const PatchRun __attribute__((address_space(1))) *GlobalRun;
     extern __shared__ __attribute__((aligned(16))) char smem[];
-    const int wp0 = blockIdx.x * R, hp = blockIdx.y, c0 = blockIdx.z * CB;
+    const unsigned tile = xcd_run(blockIdx.x, tiles), place = rag_quot(tile, by_nz), row_of = rag_quot(place, by_nx);
+    const int c0 = (int)(tile - place * nz) * CB, hp = (int)row_of, wp0 = (int)(place - row_of * nx) * R;
     CB = min(CB, g.C - c0);
     const int PK = g.Hk * g.Wk, Q = g.C * PK, nq = CB * PK;  // (at least a chunk)
     unsigned short *offs = reinterpret_cast<unsigned short *>(smem);                    // [nq]
@@ -1417,28 +1459,45 @@ __global__ __launch_bounds__(256) void patch_rows_kernel(const T *__restrict__ s
     // Every lane always loads and always stores: a load under a condition becomes a branch with a wait of its own,
     // and the compiler moves a load into the branch that holds its only use.  What lies outside the tensor is read
     // from a piece of zeros; what lies outside the window is written to the spare slot behind it.
-    if (WIDE) {
-        const int np = (shift + width + VEC - 1) / VEC, items = rows * np;  // pieces per row; LW holds np whole pieces
-        const unsigned m_np = (unsigned)((((unsigned long long)1 << 32) + np - 1) / np);
-        for (int i0 = threadIdx.x; i0 < items; i0 += 4 * 256) {
-            PatchPiece v[4];
-            int at[4];
+    if (READ != PATCH_SINGLE) {
+        const int items = rows * np;  // (np pieces cover a row of the window, LW holds them)
+        auto stage = [&](auto count, int i0) {  // items i0, i0 + 256, ...
+            constexpr int U = decltype(count)::value;
+            PatchPiece v[U];
+            int at[U], moved[U];
 #pragma unroll
-            for (int u = 0; u < 4; ++u) {
+            for (int u = 0; u < U; ++u) {
                 const int item = i0 + u * 256;
                 const int r = (int)div_magic((unsigned)min(item, items - 1), m_np), piece = min(item, items - 1) - r * np;
                 const int c_l = (int)div_magic((unsigned)r, m_hk), h = h_first + (r - c_l * g.Hk), w = w_start + piece * VEC;
-                const bool ok = (unsigned)h < (unsigned)g.Hs && (unsigned)w < (unsigned)g.Ws;  // (a piece is all in or all out)
-                const int off = ((c0 + c_l) * g.Hs + h) * g.Ws + w;  // (below 2^31: the host checks the tensor's size)
-                v[u] = *(ok ? (GlobalPiece)(src + off) : (GlobalPiece)&patch_zero);
+                const int row = ((c0 + c_l) * g.Hs + h) * g.Ws;  // (below 2^31: the host checks the tensor's size)
+                if (WIDE) {
+                    const bool ok = (unsigned)h < (unsigned)g.Hs && (unsigned)w < (unsigned)g.Ws;  // (a piece is all in or all out)
+                    v[u] = *(ok ? (GlobalPiece)(src + row + w) : (GlobalPiece)&patch_zero);
+                } else {
+                    const int w_in = min(max(w, 0), g.Ws - VEC);
+                    moved[u] = w - w_in;
+                    const bool ok = (unsigned)h < (unsigned)g.Hs && moved[u] > -VEC && moved[u] < VEC;
+                    const PatchRun run = *(ok ? (GlobalRun)(src + row + w_in) : (GlobalRun)&patch_zero);
+                    v[u] = PatchPiece{run.x, run.y, run.z, run.w};
+                }
                 at[u] = item < items ? r * LW + piece * VEC : rows * LW;
             }
+            if (!WIDE) {
 #pragma unroll
-            for (int u = 0; u < 4; ++u) {  // (rows start on 4-byte boundaries only: their pitch is an odd number of dwords)
+                for (int u = 0; u < U; ++u) v[u] = patch_shift<T>(v[u], moved[u]);
+            }
+#pragma unroll
+            for (int u = 0; u < U; ++u) {  // (rows start on 4-byte boundaries only: their pitch is an odd number of dwords)
                 unsigned *dst = reinterpret_cast<unsigned *>(lds + at[u]);
                 dst[0] = v[u].x; dst[1] = v[u].y; dst[2] = v[u].z; dst[3] = v[u].w;
             }
-        }
+        };
+        const int tid = threadIdx.x;
+        if (items <= 256) stage(std::integral_constant<int, 1>(), tid);
+        else if (items <= 512) stage(std::integral_constant<int, 2>(), tid);
+        else
+            for (int i0 = tid; i0 - tid < items; i0 += 4 * 256) stage(std::integral_constant<int, 4>(), i0);
     } else {
         const int w_lane = w_first + lane;
         const bool col_ok = (unsigned)w_lane < (unsigned)g.Ws && lane < width;
@@ -1505,9 +1564,8 @@ struct PatchCols {
 template <typename T>
 __global__ __launch_bounds__(256) void patch_cols_kernel(const T *__restrict__ src, T *__restrict__ buf, PatchGeom g,
                                                          PatchCols k, unsigned chunks) {
-    constexpr int VEC = 16 / (int)sizeof(T), EB = 8 * (int)sizeof(T);
-    typedef unsigned Run __attribute__((ext_vector_type(4), aligned(2)));  // (element alignment of the narrower type)
-    typedef const Run __attribute__((address_space(1))) *GlobalRun;
+    constexpr int VEC = 16 / (int)sizeof(T);
+    typedef const PatchRun __attribute__((address_space(1))) *GlobalRun;
     const unsigned B = blockIdx.x * 256u, i = B + threadIdx.x;
     if (i >= chunks) return;
     const int PK = g.Hk * g.Wk;
@@ -1521,23 +1579,9 @@ __global__ __launch_bounds__(256) void patch_cols_kernel(const T *__restrict__ s
     const int w_in = min(max(w0, 0), g.Ws - VEC), d = w0 - w_in;  // d > 0: the run ends behind the row
     const bool ok = (unsigned)h < (unsigned)g.Hs && d > -VEC && d < VEC;
     const unsigned off = ((unsigned)c * g.Hs + h) * g.Ws + w_in;
-    Run v = *(ok ? (GlobalRun)(src + off) : (GlobalRun)&patch_zero);
-    const int bits = (d < 0 ? -d : d) * EB;
-    if (d > 0) {  // towards element 0
-        if (bits & 64) v = Run{v.z, v.w, 0u, 0u};
-        if (bits & 32) v = Run{v.y, v.z, v.w, 0u};
-        const unsigned bs = bits & 31;
-        v = Run{__builtin_amdgcn_alignbit(v.y, v.x, bs), __builtin_amdgcn_alignbit(v.z, v.y, bs),
-                __builtin_amdgcn_alignbit(v.w, v.z, bs), v.w >> bs};
-    } else if (d < 0) {
-        if (bits & 64) v = Run{0u, 0u, v.x, v.y};
-        if (bits & 32) v = Run{0u, v.x, v.y, v.z};
-        const unsigned bs = bits & 31;  // (0 or 16: a left shift by 16 is alignbit(hi, lo, 16) one dword up)
-        if (bs) v = Run{v.x << 16, __builtin_amdgcn_alignbit(v.y, v.x, 16), __builtin_amdgcn_alignbit(v.z, v.y, 16),
-                        __builtin_amdgcn_alignbit(v.w, v.z, 16)};
-    }
-    typedef unsigned Chunk __attribute__((ext_vector_type(4)));
-    *reinterpret_cast<Chunk *>(buf + (size_t)i * VEC) = Chunk{v.x, v.y, v.z, v.w};
+    const PatchRun run = *(ok ? (GlobalRun)(src + off) : (GlobalRun)&patch_zero);
+    const PatchPiece v = patch_shift<T>(PatchPiece{run.x, run.y, run.z, run.w}, d);
+    *reinterpret_cast<PatchPiece *>(buf + (size_t)i * VEC) = v;
 }
 
 // The column-major patch matrix at unit strides from the source's side: a row (c, hk, wk) of the matrix is the image
@@ -1646,15 +1690,17 @@ static int patch_rows(const T *src, T *buf, const PatchGeom &g) {
     // positions per workgroup: a window row of at most 64 elements (one pass of a wave) - half that with pieces,
     // whose loads are few either way: more and shorter workgroups overlap their load and store phases better -
     // and then the same number for every workgroup of a grid row
+    const PatchRead read = wide ? PATCH_ALIGNED : g.Ws >= VEC ? PATCH_MOVED : PATCH_SINGLE;
     int R = (64 - g.Wk) / g.w_mul + 1;
-    if (wide && R >= 32) R = (R + 1) / 2;
+    if (read != PATCH_SINGLE && R >= 32) R = (R + 1) / 2;
     if (R > g.Wp) R = g.Wp;
     R = (g.Wp + (g.Wp + R - 1) / R - 1) / ((g.Wp + R - 1) / R);
     // row pitch of the window: an odd number of dwords, so that the rows the lanes of a wave gather from (every
     // Hk-th one for neighbouring channels) spread over the LDS banks; with pieces, room for the whole pieces that
     // cover a window starting anywhere in its first piece
     int LW = (R - 1) * g.w_mul + g.Wk;
-    if (wide) LW = (VEC - 1 + LW + VEC - 1) / VEC * VEC;
+    const int np = ((wide ? VEC - 1 : 0) + LW + VEC - 1) / VEC;
+    if (read != PATCH_SINGLE) LW = np * VEC;
     LW = ES == 2 ? (((LW + 1) & ~1) | 2) : (LW | 1);
     // (table of column offsets, window, one spare slot)
     auto bytes = [&](int cb) { return (((size_t)cb * PK * 2 + 15) & ~(size_t)15) + (size_t)cb * g.Hk * LW * ES + 16; };
@@ -1669,13 +1715,15 @@ static int patch_rows(const T *src, T *buf, const PatchGeom &g) {
     nz = (g.C + CB - 1) / CB;
     if (bytes(CB) > 64 * 1024 || last * PK < VEC || CB * g.Hk * LW >= 65536 || nz >= 65536) return -1;
     auto magic = [](unsigned d) { return (unsigned)((((unsigned long long)1 << 32) + d - 1) / d); };
-    dim3 grid((g.Wp + R - 1) / R, g.Hp, nz);
-    if (wide)
-        hipLaunchKernelGGL((patch_rows_kernel<T, true>), grid, dim3(256), bytes(CB), state().stream, src, buf, g, R, CB, LW,
-                           magic(PK), magic(g.Wk), magic(g.Hk));
-    else
-        hipLaunchKernelGGL((patch_rows_kernel<T, false>), grid, dim3(256), bytes(CB), state().stream, src, buf, g, R, CB,
-                           LW, magic(PK), magic(g.Wk), magic(g.Hk));
+    const int nx = (g.Wp + R - 1) / R;
+    if ((long long)nx * g.Hp * nz >= 1LL << 31) return -1;
+    const dim3 grid((unsigned)(nx * g.Hp * nz));
+    auto launch = [&](auto kern) {
+        hipLaunchKernelGGL(kern, grid, dim3(256), bytes(CB), state().stream, src, buf, g, R, CB, LW, magic(PK), magic(g.Wk), magic(g.Hk), np, magic(np), rag_div(nx), rag_div(nz), grid.x);
+    };
+    if (read == PATCH_ALIGNED) launch(patch_rows_kernel<T, PATCH_ALIGNED>);
+    else if (read == PATCH_MOVED) launch(patch_rows_kernel<T, PATCH_MOVED>);
+    else launch(patch_rows_kernel<T, PATCH_SINGLE>);
     return hip_ok(hipGetLastError(), "patch launch") ? 0 : 2;
 }
 
@@ -1935,14 +1983,21 @@ static int blocktransp(const Args *a, const char *fn) {
             const long long groups = (long long)(((a->Cin + td - 1) / td + 1) / 2) * (((a->Cout + td - 1) / td + 1) / 2);
             return (unsigned)(32 * ((groups + 7) / 8));
         };
-        const int pitch = 32 * P + VEC;  // rows of the tile start on 16-byte boundaries
-        const size_t lds = (size_t)32 * pitch * sizeof(T);
-        const dim3 grid(tile_grid(32));
+        const long long tiles = (long long)((a->Cin + 31) / 32) * ((a->Cout + 31) / 32);
+        // Runs of single elements take more loads than are in flight at a time: a chip that is not full takes smaller tiles,
+        // sixteen times as many (53 x 51 channels, 3 x 3, fp32: 6.65 -> 3.3 us; 320 x 255, fp16: 7.0 -> 4.3).
+        const int td = vecs || tiles >= state().num_cu ? 32 : 8;
+        const int pitch = td * P + VEC;  // rows of the tile start on 16-byte boundaries
+        const size_t lds = (size_t)td * pitch * sizeof(T);
+        const dim3 grid(tile_grid(td));
         if (vecs)
             hipLaunchKernelGGL((blocktransp_tile_kernel<T, true, 32, 256>), grid, dim3(256), lds, state().stream, w, bt,
                                a->Cin, a->Cout, P, m_p, pitch);
-        else
+        else if (td == 32)
             hipLaunchKernelGGL((blocktransp_tile_kernel<T, false, 32, 256>), grid, dim3(256), lds, state().stream, w,
+                               bt, a->Cin, a->Cout, P, m_p, pitch);
+        else
+            hipLaunchKernelGGL((blocktransp_tile_kernel<T, false, 8, 256>), grid, dim3(256), lds, state().stream, w,
                                bt, a->Cin, a->Cout, P, m_p, pitch);
         rc = hip_ok(hipGetLastError(), "blocktranspose launch") ? 0 : 2;
     } else {
@@ -1964,21 +2019,28 @@ static int blocktransp(const Args *a, const char *fn) {
 // out(j, i) = out[out_base + b*out_bs + j*out_rs + i].
 struct Transp2D {
     int N, M;
+    unsigned tiles;
+    RagDiv by_ny;  // tiles along N
     long long in_rs, out_rs, in_bs, out_bs, in_base, out_base;
 };
 
 // 64 x 64 tiles through LDS, 16 bytes per access on both sides wherever the rows start (a wave's eight rows of 128 bytes
 // need no alignment for that); what is left of a row behind its last whole piece moves element by element.  Memory
-// bounds it: over matrices of odd sizes 1.3x the rate of moving each element by itself, aligned ones as before.
+// bounds it: over matrices of odd sizes 1.3x the rate of moving each element by itself, aligned ones as before.  The tiles
+// that write one band of output rows follow each other on one XCD, whose L2 puts together the lines that they share: 75 x
+// 24 249 in fp16, with the copy behind it, 9.3 -> 7.9 us.
 typedef unsigned TranspPiece __attribute__((ext_vector_type(4), aligned(1)));
 template <typename T>
 __global__ __launch_bounds__(256) void transpose2d_kernel(const T *__restrict__ in, T *__restrict__ out, Transp2D g) {
+    fetch_args(in, out, g);
+    const unsigned ny = g.by_ny.d, t = xcd_run(blockIdx.x, g.tiles);
     constexpr int VEC = 16 / (int)sizeof(T), CH = 64 / VEC;  // chunks per tile row
     constexpr int PITCH = sizeof(T) == 2 ? 66 : 65;          // elements
     __shared__ __attribute__((aligned(16))) T tile[64 * PITCH];
     in += g.in_base + (long long)blockIdx.z * g.in_bs;
     out += g.out_base + (long long)blockIdx.z * g.out_bs;
-    const int j0 = blockIdx.x * 64, i0 = blockIdx.y * 64;
+    const unsigned tx = rag_quot(t, g.by_ny);
+    const int j0 = (int)tx * 64, i0 = (int)(t - tx * ny) * 64;
     union Piece {
         TranspPiece u;
         T e[VEC];
@@ -2029,8 +2091,9 @@ __global__ __launch_bounds__(256) void transpose2d_kernel(const T *__restrict__ 
 template <typename T>
 static int transpose2d_strided(const T *in, T *out, int N, int M, long long in_rs, long long out_rs, int batch,
                                long long in_bs, long long out_bs, long long in_base, long long out_base) {
-    const Transp2D g = {N, M, in_rs, out_rs, in_bs, out_bs, in_base, out_base};
-    const dim3 grid((M + 63) / 64, (N + 63) / 64, batch);
+    const int nx = (M + 63) / 64, ny = (N + 63) / 64;
+    const Transp2D g = {N, M, (unsigned)(nx * ny), rag_div(ny), in_rs, out_rs, in_bs, out_bs, in_base, out_base};
+    const dim3 grid(g.tiles, 1, batch);
     hipLaunchKernelGGL((transpose2d_kernel<T>), grid, dim3(256), 0, state().stream, in, out, g);
     return hip_ok(hipGetLastError(), "transpose launch") ? 0 : 2;
 }
