@@ -169,6 +169,12 @@ int gemm_pair_lean(const GemmArgs &g0, const GemmArgs &g1);
 // Weight, input and (where db is given) bias gradient of a dense layer in one launch: on one sample; on a batch.
 template <typename T>
 int linear_one_bw(const T *x, const T *W, const T *dy, T *dW, T *dx, T *db, int in, int out);
+// ... and on two to LINEAR_FEW; the forward pass of two to sixteen.
+constexpr int LINEAR_FEW = 8;
+template <typename T>
+int linear_few_bw(const T *x, const T *W, const T *dy, T *dW, T *dx, T *db, int ns, int in, int out);
+template <typename T>
+int linear_few_fw(const T *x, const T *W, T *y, const T *bias, int ns, int in, int out);
 template <typename T>
 int linear_bw_ragged(const T *X, const T *W, const T *dY, T *dW, T *dX, T *db, int ns, int in, int out);
 template <typename T>
@@ -181,7 +187,8 @@ int mm_dispatch(const T *A, const T *B, T *C, int N, int M, int K, int trans_B, 
 #ifdef __HIP_DEVICE_COMPILE__
 // Asks for all lines of a kernel's arguments at its start.  They lie in memory, and the compiler loads each where it is
 // needed: a line that is asked for behind an index or a branch that came from another line is one more trip before the first
-// load of data.
+// load of data. (Patch rows and transpositions; in row dots, batch norms, convolutions and sums
+// it gave nothing that could be measured.)
 template <typename... A>
 constexpr int args_bytes() {
     int n = 0;

@@ -707,7 +707,7 @@ __global__ __launch_bounds__(256) void gemv_rowdot_kernel(const T *__restrict__ 
 // How the rows of a column sum are shared out: `cols` workgroups side by side, each share `chunk` rows.
 struct GvShares {
     int cols, shares, chunk;
-    float *part;  // [share][M]; one share: the kernel writes the result
+    float *part;  // [share][sample][M]; one share: the kernel writes the result
 };
 
 // Workgroup `block` sums share block / cols of eight pieces of columns (a 128-byte line: four, of which two workgroups
@@ -841,14 +841,17 @@ __global__ __launch_bounds__(GV_NT) void linear_one_bw_kernel(const T *__restric
 // shares at least; adding them is a launch (2.3 us).  In us, one share against these, fp32: 64 columns of 2048 rows 4.0, 6.1
 // (not taken), of 4096 6.8, 6.1, of 16384 25.3, 6.4; 1024 columns of 2048 rows 5.8, 6.6 (not taken), of 4096 9.9, 6.7; 4096
 // of 4096 18.8, 15.7; 6144 of 4096 21.5, 21.9 (not taken).
+// With several samples the sums themselves take a workgroup 1.7 us for every 512 rows: shares from FEW_SHARED rows on (5
+// samples, 1152 -> 3328 in fp16 22.5 us with one share, 12.3 with six).
+constexpr int FEW_SHARED = 1536;
 template <typename T, int V>
-static GvShares gv_shares(int K, int M) {
+static GvShares gv_shares(int K, int M, int ns = 1) {
     GvShares sh = {(int)(((long long)M + GV_CV * V - 1) / (GV_CV * V)), 1, K, nullptr};
     const int cu = state().num_cu, z = std::min({2 * cu / sh.cols, K / 512, 32});
-    if (K < 4096 || sh.cols > cu / 2 || z < 2) return sh;
+    if (K < (ns > 1 ? FEW_SHARED : 4096) || sh.cols > cu / 2 || z < 2) return sh;
     const int chunk = (K + z - 1) / z, shares = (K + chunk - 1) / chunk;
     // (a stream that is being captured, or a full device, cannot get a workspace: one share then, and no error behind it)
-    if (float *part = workspace((size_t)shares * M * sizeof(float))) sh = {sh.cols, shares, chunk, part};
+    if (float *part = workspace((size_t)shares * ns * M * sizeof(float))) sh = {sh.cols, shares, chunk, part};
     else (void)hipGetLastError();
     return sh;
 }
@@ -885,6 +888,273 @@ int linear_one_bw(const T *x, const T *W, const T *dy, T *dW, T *dx, T *db, int 
 }
 template int linear_one_bw<float>(const float *, const float *, const float *, float *, float *, float *, int, int);
 template int linear_one_bw<half_t>(const half_t *, const half_t *, const half_t *, half_t *, half_t *, half_t *, int, int);
+
+// ---- dense layers on a few samples ----------------------------------------------------------------------------------
+// The weights are read, their gradient is written once for all samples; 32 x 32 MFMA tiles would be three quarters padding or
+// more, and a contraction that few tiles share needs partial sums and a second launch.  Sums in fp32 as with one sample.  Bound
+// by a launch and two or three trips to memory up to some MB (3.5 us forward, 4.2 backward), by memory above (3595 -> 3776, 3
+// samples, fp16, backward 24 us, 54 MB; before 30).
+
+// y[b][r] = sum_k W[r][k] * x[b][k] (+ bias[r]): WPR waves a row, a piece of the row and of each sample a lane.
+template <typename T, int V, int NS, int WPR>
+__global__ __launch_bounds__(256) void linear_few_fw_kernel(const T *__restrict__ W, const T *__restrict__ x, T *__restrict__ y,
+                                                            const T *__restrict__ bias, int ns, int in, int out) {
+    constexpr int U = NS <= 4 ? 4 : 2, STEP = WPR * 64 * V;
+    __shared__ float red[4][NS];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int row = blockIdx.x * (4 / WPR) + wave / WPR, part = wave % WPR;
+    float s[NS];
+#pragma unroll
+    for (int b = 0; b < NS; ++b) s[b] = 0.f;
+    if (row < out) {
+        const T *p = W + (size_t)row * in, *xb[NS];
+#pragma unroll
+        for (int b = 0; b < NS; ++b) xb[b] = x + (size_t)min(b, ns - 1) * in;
+        const int whole = in / V * V;
+        int k = (part * 64 + lane) * V;
+        for (; k + (U - 1) * STEP < whole; k += U * STEP) {
+            GvPiece<T, V> w[U], v[U][NS];
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                w[u] = gv_load<T, V>(p + k + u * STEP);
+#pragma unroll
+                for (int b = 0; b < NS; ++b) v[u][b] = gv_load<T, V>(xb[b] + k + u * STEP);
+            }
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+#pragma unroll
+                for (int b = 0; b < NS; ++b)
+#pragma unroll
+                    for (int i = 0; i < V; ++i) s[b] += (float)w[u].e[i] * (float)v[u][b].e[i];
+        }
+        if (k < whole) {  // (pieces beyond the end: the first one, replaced by zeros)
+            GvPiece<T, V> w[U - 1], v[U - 1][NS];
+            bool ok[U - 1];
+#pragma unroll
+            for (int u = 0; u < U - 1; ++u) {
+                ok[u] = k + u * STEP < whole;
+                const int at = ok[u] ? k + u * STEP : k;
+                w[u] = gv_load<T, V>(p + at);
+#pragma unroll
+                for (int b = 0; b < NS; ++b) v[u][b] = gv_load<T, V>(xb[b] + at);
+            }
+#pragma unroll
+            for (int u = 0; u < U - 1; ++u)
+#pragma unroll
+                for (int b = 0; b < NS; ++b)
+#pragma unroll
+                    for (int i = 0; i < V; ++i) s[b] += (ok[u] ? (float)w[u].e[i] : 0.f) * (ok[u] ? (float)v[u][b].e[i] : 0.f);
+        }
+        if (part == 0 && whole + lane < in) {
+#pragma unroll
+            for (int b = 0; b < NS; ++b) s[b] += (float)p[whole + lane] * (float)xb[b][whole + lane];
+        }
+    }
+#pragma unroll
+    for (int b = 0; b < NS; ++b)
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) s[b] += __shfl_xor(s[b], o, 64);
+    float v = s[0];  // lane b: of sample b
+#pragma unroll
+    for (int b = 1; b < NS; ++b) v = lane == b ? s[b] : v;
+    if constexpr (WPR > 1) {
+        if (lane < NS) red[wave][lane] = v;
+        __syncthreads();
+        if (part == 0 && lane < NS) {
+            v = red[wave][lane];
+#pragma unroll
+            for (int w = 1; w < WPR; ++w) v += red[wave + w][lane];
+        }
+    }
+    if (part == 0 && lane < ns && row < out) y[(size_t)lane * out + row] = (T)(bias ? v + (float)bias[row] : v);
+}
+
+// dx[b][m] = sum_k dy[b][k] * W[k][m], as gemv_coldot_block for one sample: eight rows a thread and trip, the dy's of the 512 rows
+// of a trip in LDS, those of a row side by side.
+template <typename T, int V, int NS>
+struct FewSums {
+    static constexpr int U = 8, ROWS = U * GV_ROWS, WAVES = GV_NT / 64, RED = NS * WAVES * GV_CV * V, DY = ROWS * NS;
+    static constexpr int FLOATS = RED > DY ? RED : DY;
+    static_assert(ROWS == GV_NT, "a thread fetches the dy's of a row");
+};
+template <typename T, int V, int NS>
+__device__ inline void linear_few_sums(const T *__restrict__ dy, const T *__restrict__ W, T *__restrict__ dx, int ns, int K, int M, int block,
+                                       const GvShares &sh, float *lds) {
+    typedef FewSums<T, V, NS> S;
+    constexpr int CV = GV_CV, KL = GV_ROWS, U = S::U, NT = GV_NT;
+    const int share = block / sh.cols;
+    block -= share * sh.cols;
+    const int k0 = share * sh.chunk, k1 = min(K, k0 + sh.chunk);
+    const int tid = threadIdx.x, cv = tid % CV, kl = tid / CV;
+    const int want = (block * CV + cv) * V, col = min(want, M - V);
+    float acc[NS][V];
+#pragma unroll
+    for (int b = 0; b < NS; ++b)
+#pragma unroll
+        for (int i = 0; i < V; ++i) acc[b][i] = 0.f;
+    for (int c = k0; c < k1; c += S::ROWS) {
+        const bool whole = c + S::ROWS <= k1;  // (rows beyond the end: the last one, replaced by zeros)
+        GvPiece<T, V> v[U];
+        T d[NS];
+#pragma unroll
+        for (int u = 0; u < U; ++u) v[u] = gv_load<T, V>(W + (size_t)min(c + kl + u * KL, k1 - 1) * M + col);
+#pragma unroll
+        for (int b = 0; b < NS; ++b) d[b] = dy[(size_t)min(b, ns - 1) * K + min(c + tid, k1 - 1)];
+        __syncthreads();
+#pragma unroll
+        for (int b = 0; b < NS; ++b) lds[tid * NS + b] = c + tid < k1 ? (float)d[b] : 0.f;
+        __syncthreads();
+        if (!whole) {
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+#pragma unroll
+                for (int i = 0; i < V; ++i) v[u].e[i] = c + kl + u * KL < k1 ? v[u].e[i] : (T)0.f;
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            if (c + u * KL >= k1) break;
+#pragma unroll
+            for (int b = 0; b < NS; ++b) {
+                const float f = lds[(kl + u * KL) * NS + b];
+#pragma unroll
+                for (int i = 0; i < V; ++i) acc[b][i] += f * (float)v[u].e[i];
+            }
+        }
+    }
+    // Lanes of a wave that share a piece are CV apart.  Two values a time, half of the lanes adds up the one, half the other:
+    // a quarter of the values a lane in the end (with three shuffles a value the sums alone took 5 us, 64 values a lane).
+    constexpr int N = NS * V, Q = N / 4;
+    static_assert(N % 4 == 0 && CV == 8, "quarters");
+    const int lane = tid & 63, wave = tid >> 6;
+    float two[N / 2], one[Q];
+    auto value = [&](int n) { return __float_as_uint(acc[n / V][n % V]); };
+#pragma unroll
+    for (int n = 0; n < N / 2; ++n) {
+        const auto p = __builtin_amdgcn_permlane32_swap(value(n), value(n + N / 2), false, false);
+        two[n] = __uint_as_float(p[0]) + __uint_as_float(p[1]);
+    }
+#pragma unroll
+    for (int n = 0; n < Q; ++n) {
+        const auto p = __builtin_amdgcn_permlane16_swap(__float_as_uint(two[n]), __float_as_uint(two[n + Q]), false, false);
+        one[n] = __uint_as_float(p[0]) + __uint_as_float(p[1]);
+        one[n] += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(one[n]), 0x128, 0xf, 0xf, false));  // lane ^ 8
+    }
+    __syncthreads();
+    if (!(lane & 8)) {
+        const int first = (lane >> 5) * (N / 2) + ((lane >> 4) & 1) * Q;
+#pragma unroll
+        for (int n = 0; n < Q; ++n) {
+            const int b = (first + n) / V, i = (first + n) % V;
+            lds[(b * S::WAVES + wave) * (CV * V) + (lane & 7) * V + i] = one[n];
+        }
+    }
+    __syncthreads();
+    for (int t = tid; t < NS * CV * V; t += NT) {
+        const int b = t / (CV * V), r = t % (CV * V), first = (block * CV + r / V) * V, at = min(first, M - V) + r % V;
+        float s = 0.f;
+#pragma unroll
+        for (int w = 0; w < S::WAVES; ++w) s += lds[(b * S::WAVES + w) * (CV * V) + r];
+        if (first < M && b < ns) {
+            if (sh.shares > 1) sh.part[((size_t)share * ns + b) * M + at] = s;
+            else dx[(size_t)b * M + at] = (T)s;
+        }
+    }
+}
+
+// dW[n][m] = sum_b dy[b][n] * x[b][m]: a wave takes 64 pieces of columns of FEW_ROWS rows; lane (b, row) fetches a dy, which are
+// the same for all lanes.  db[n] = sum_b dy[b][n] where it is wanted.
+constexpr int FEW_ROWS = 8;
+template <typename T, int V, int NS>
+__device__ inline void linear_few_outer(const T *__restrict__ dy, const T *__restrict__ x, T *__restrict__ dW, T *__restrict__ db, int ns,
+                                        int out, int in, RagDiv per_row, unsigned unit) {
+    const unsigned q = rag_quot(unit, per_row);  // units of 64 pieces
+    const int n0 = (int)q * FEW_ROWS, lane = threadIdx.x & 63, want = ((int)(unit - q * per_row.d) * 64 + lane) * V;
+    if (n0 >= out) return;
+    const int m = min(want, in - V);
+    const float mine = (float)dy[(size_t)min(lane / FEW_ROWS, ns - 1) * out + min(n0 + lane % FEW_ROWS, out - 1)];
+    GvPiece<T, V> xv[NS];
+#pragma unroll
+    for (int b = 0; b < NS; ++b) xv[b] = gv_load<T, V>(x + (size_t)min(b, ns - 1) * in + m);
+#pragma unroll
+    for (int r = 0; r < FEW_ROWS; ++r) {
+        float s[V], sum = 0.f;
+#pragma unroll
+        for (int e = 0; e < V; ++e) s[e] = 0.f;
+#pragma unroll
+        for (int b = 0; b < NS; ++b)
+            if (b < ns) {
+                const float d = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(mine), b * FEW_ROWS + r));
+                sum += d;
+#pragma unroll
+                for (int e = 0; e < V; ++e) s[e] += d * (float)xv[b].e[e];
+            }
+        if (n0 + r < out && want < in) {
+            GvPiece<T, V> o;
+#pragma unroll
+            for (int e = 0; e < V; ++e) o.e[e] = (T)s[e];
+            __builtin_memcpy(dW + (size_t)(n0 + r) * in + m, &o, sizeof(o));
+            if (db && want == 0) db[n0 + r] = (T)sum;
+        }
+    }
+}
+
+// Both gradients in one launch: the first workgroups sum columns for dX, the rest write dW and db.
+template <typename T, int V, int NS>
+__global__ __launch_bounds__(GV_NT) void linear_few_bw_kernel(const T *__restrict__ x, const T *__restrict__ W, const T *__restrict__ dy,
+                                                              T *__restrict__ dW, T *__restrict__ dx, T *__restrict__ db, int ns, int in,
+                                                              int out, RagDiv per_row, const GvShares sh) {
+    __shared__ __attribute__((aligned(16))) float lds[FewSums<T, V, NS>::FLOATS];
+    const int sums = sh.cols * sh.shares;
+    if ((int)blockIdx.x < sums)
+        linear_few_sums<T, V, NS>(dy, W, dx, ns, out, in, blockIdx.x, sh, lds);
+    else
+        linear_few_outer<T, V, NS>(dy, x, dW, db, ns, out, in, per_row,
+                                   (blockIdx.x - sums) * (GV_NT / 64) + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6));
+}
+
+template <typename T, int V, int NS>
+static int linear_few_bw_run(const T *x, const T *W, const T *dy, T *dW, T *dx, T *db, int ns, int in, int out) {
+    const GvShares sh = gv_shares<T, V>(out, in, ns);
+    const int per_row = (in + 64 * V - 1) / (64 * V);
+    const long long units = (long long)((out + FEW_ROWS - 1) / FEW_ROWS) * per_row;
+    hipLaunchKernelGGL((linear_few_bw_kernel<T, V, NS>), dim3((unsigned)(sh.cols * sh.shares + (units + GV_NT / 64 - 1) / (GV_NT / 64))),
+                       dim3(GV_NT), 0, state().stream, x, W, dy, dW, dx, db, ns, in, out, rag_div(per_row), sh);
+    if (sh.shares > 1) launch_share_sum<T>(sh.part, dx, ns * in, sh.shares, state().stream);
+    return hip_ok(hipGetLastError(), "linear backward launch") ? 0 : 2;
+}
+template <typename T, int V>
+static int linear_few_bw_v(const T *x, const T *W, const T *dy, T *dW, T *dx, T *db, int ns, int in, int out) {
+    return ns <= 2 && V > 1 ? linear_few_bw_run<T, V, (V > 1 ? 2 : 4)>(x, W, dy, dW, dx, db, ns, in, out)
+         : ns <= 4 ? linear_few_bw_run<T, V, 4>(x, W, dy, dW, dx, db, ns, in, out)
+                   : linear_few_bw_run<T, V, 8>(x, W, dy, dW, dx, db, ns, in, out);
+}
+template <typename T>
+int linear_few_bw(const T *x, const T *W, const T *dy, T *dW, T *dx, T *db, int ns, int in, int out) {
+    constexpr int VEC = Traits<T>::VEC;
+    return in >= VEC ? linear_few_bw_v<T, VEC>(x, W, dy, dW, dx, db, ns, in, out) : linear_few_bw_v<T, 1>(x, W, dy, dW, dx, db, ns, in, out);
+}
+template int linear_few_bw<float>(const float *, const float *, const float *, float *, float *, float *, int, int, int);
+template int linear_few_bw<half_t>(const half_t *, const half_t *, const half_t *, half_t *, half_t *, half_t *, int, int, int);
+
+template <typename T, int NS>
+static int linear_few_fw_run(const T *x, const T *W, T *y, const T *bias, int ns, int in, int out) {
+    constexpr int V = Traits<T>::VEC;
+    hipStream_t s = state().stream;
+    // (rows that would not fill the chip with a wave each, and are long: four waves a row)
+    if (out < 8 * state().num_cu && in > 256 * V)
+        hipLaunchKernelGGL((linear_few_fw_kernel<T, V, NS, 4>), dim3(out), dim3(256), 0, s, W, x, y, bias, ns, in, out);
+    else
+        hipLaunchKernelGGL((linear_few_fw_kernel<T, V, NS, 1>), dim3((out + 3) / 4), dim3(256), 0, s, W, x, y, bias, ns, in, out);
+    return hip_ok(hipGetLastError(), "linear forward launch") ? 0 : 2;
+}
+template <typename T>
+int linear_few_fw(const T *x, const T *W, T *y, const T *bias, int ns, int in, int out) {
+    return ns <= 2 ? linear_few_fw_run<T, 2>(x, W, y, bias, ns, in, out) : ns <= 4 ? linear_few_fw_run<T, 4>(x, W, y, bias, ns, in, out)
+         : ns <= 8 ? linear_few_fw_run<T, 8>(x, W, y, bias, ns, in, out)
+                   : linear_few_fw_run<T, 16>(x, W, y, bias, ns, in, out);
+}
+template int linear_few_fw<float>(const float *, const float *, float *, const float *, int, int, int);
+template int linear_few_fw<half_t>(const half_t *, const half_t *, half_t *, const half_t *, int, int, int);
 
 template <typename T>
 static int gemv_rowdot(const T *Mx, const T *x, T *y, const T *bias, int R, int K) {

@@ -1110,6 +1110,20 @@ static int pw_step(const Args *a, int ns, int step, const char *fn) {
 // W is [out][in] row-major (lib/sources/pulp_linear_fp32.c:39-46); sample b of
 // the input/output blobs is a vector of blob->dim elements.
 
+// Few samples: the kernels of ptl_gemm.hip that read each weight once, against tiles of 32 x 32 and more with partial sums, in a
+// grid of 96 to 3800 inputs and 48 to 4000 outputs.
+// Forward, two to eight samples: 1.1 to 3.5 times as fast (1157 -> 500, 4 samples, fp16 2.9), 0.8 to 1 at worst (96 -> 4000,
+// 3, fp16).  Up to sixteen samples 1.15 to 2.4 times with few outputs, not with many, where all of the samples are read again
+// for every row (1944 -> 320, 16, fp16 10.2 -> 6.7 us; 781 -> 3840, 11, fp32 12.5 and 13.5; 3904 -> 2837, 9: 14.7 and 29.7).
+static bool few_fw(int ns, int out) { return state().gemm_path == 0 && ns >= 2 && (ns <= 8 || (ns <= 16 && out <= 1280)); }
+// Backward: fp32 1.05 to 4 times (2304 -> 2100, 4 samples 45 -> 11 us), fp16 1.03 to 2.3 up to four samples.  With more the
+// matrix instructions of fp16 are as fast until the weights are many (8 samples, 640 -> 48 5.1 and 5.7 us, 1157 -> 500 7.9 ->
+// 7.3, 640 -> 2100 12.3 -> 10.1).
+template <typename T>
+static bool few_bw(int ns, int in, int out) {
+    return state().gemm_path == 0 && ns >= 2 && ns <= LINEAR_FEW && (sizeof(T) == 4 || ns <= 4 || in >= 1024 || out >= 1536);
+}
+
 template <typename T, typename Args>
 static int linear_step(const Args *a, int ns, int step, const char *fn) {
     if (!a || !a->input || !a->coeff || !a->output) {
@@ -1142,6 +1156,7 @@ static int linear_step(const Args *a, int ns, int step, const char *fn) {
         T *Y = sg.out(reinterpret_cast<T *>(a->output->data), (size_t)ns * out);
         const T *bias = use_bias ? sg.in(reinterpret_cast<const T *>(a->bias->data), (size_t)out) : nullptr;
         if (sg.failed()) return 2;
+        if (few_fw(ns, out)) return sg.finish(linear_few_fw<T>(X, Wt, Y, bias, ns, in, out));
         rc = mm_dispatch<T>(X, Wt, Y, ns, out, in, 1, bias);  // Y[b][o] = X[b][:] . W[o][:] + bias[o]
     } else if (step == STEP_BW_BOTH) {
         // weight and input gradient of a batch in one launch
@@ -1153,6 +1168,7 @@ static int linear_step(const Args *a, int ns, int step, const char *fn) {
         T *db = use_bias ? sg.out(reinterpret_cast<T *>(a->bias->diff), (size_t)out) : nullptr;
         if (sg.failed()) return 2;
         const bool apart = !backward_shares_memory<T>(X, (size_t)ns * in, Wt, (size_t)out * in, dY, (size_t)ns * out, dW, dX, db, (size_t)out);
+        if (few_bw<T>(ns, in, out) && apart) return sg.finish(linear_few_bw<T>(X, Wt, dY, dW, dX, db, ns, in, out));
         if (ns == 1 && apart) return sg.finish(linear_one_bw<T>(X, Wt, dY, dW, dX, db, in, out));
         rc = dense_bw<T>(X, Wt, dY, dW, dX, db, ns, in, out, apart);
     } else if (step == STEP_WGT_GRAD) {

@@ -1,0 +1,72 @@
+"""Dense layers on a few samples: weights read once for all of them, sums of rows and of columns in 16-byte pieces."""
+import pytest
+import torch
+
+from test_gpu_patch_rows import DEV, shifted
+
+pytestmark = pytest.mark.gpu
+TDT = {"fp32": torch.float32, "fp16": torch.float16}
+
+
+def run(pkg, gpu, dt, ns, n_in, n_out, bias, shift, spoil=None):
+    g = torch.Generator(device=DEV).manual_seed(n_in * 31 + n_out)
+    r = lambda *s: shifted((torch.rand(*s, generator=g, device=DEV) - 0.5).to(TDT[dt]), shift)[0]
+    x, w, b, dy = r(ns, n_in), r(n_out, n_in), r(n_out), r(ns, n_out)
+    if spoil:
+        w[spoil], x[:, 0] = float("inf"), 1.0
+    guard = {k: shifted(torch.zeros(*s, device=DEV, dtype=TDT[dt]), shift) for k, s in
+             (("y", (ns, n_out)), ("dx", (ns, n_in)), ("dw", (n_out, n_in)), ("db", (n_out,)))}
+    y, dx, dw, db = (guard[k][0] for k in ("y", "dx", "dw", "db"))
+    a = pkg.LinearArgs()
+    keep = [pkg.blob(x, dx, 1, 1, 1, n_in), pkg.blob(w, dw, 1, 1, 1, n_in * n_out), pkg.blob(b, db, 1, 1, 1, n_out), pkg.blob(y, dy, 1, 1, 1, n_out)]
+    a.input, a.coeff, a.bias, a.output = [pkg.structs.C.pointer(k) for k in keep]
+    a.use_biases = bias
+    for k, q in zip(keep, (n_in, n_in * n_out, n_out, n_out)):
+        assert k.dim == q
+    pkg.call("ptl_linear_%s_fw_batched" % dt, a, ns)
+    pkg.call("ptl_linear_%s_bw_batched" % dt, a, ns)
+    assert gpu.ptl_sync() == 0
+    for t, buf in guard.values():
+        assert bool((buf[:shift] == 5).all()) and bool((buf[shift + t.numel():] == 5).all())
+    X, W, B, D = (t.double() for t in (x, w, b, dy))
+    ref = {"y": X @ W.t() + (B if bias else 0), "dx": D @ W, "dw": D.t() @ X, "db": D.sum(0) if bias else torch.zeros_like(B)}
+    size = {"y": X.abs() @ W.abs().t() + B.abs(), "dx": D.abs() @ W.abs(), "dw": D.abs().t() @ X.abs(), "db": D.abs().sum(0)}
+    return {"y": y, "dx": dx, "dw": dw, "db": db}, ref, size
+
+
+def check(dt, got, ref, size, n_in, n_out):
+    for k, v in got.items():
+        # a chain of roundings: the terms of a lane's sum (a 64th of the contraction), of a wave's and of the waves
+        chain = {"y": n_in / 64, "dx": n_out / 64}.get(k, 0) + 40
+        tol = chain * 2.0 ** -24 * size[k] + (2.0 ** -11 * ref[k].abs() + 2.0 ** -25 if dt == "fp16" else 0)
+        assert bool(((v.double() - ref[k]).abs() <= tol).all()), k
+
+
+@pytest.mark.parametrize("dt", ["fp32", "fp16"])
+@pytest.mark.parametrize("ns", [2, 3, 4, 5, 8, 9, 16])
+@pytest.mark.parametrize("n_in,n_out,bias,shift", [(1, 5, 1, 0), (3, 9, 0, 1), (7, 1, 1, 1), (8, 8, 1, 0), (9, 65, 0, 1), (255, 63, 1, 3), (257, 64, 0, 0),
+                                                   (513, 521, 1, 1), (1025, 130, 0, 0), (2049, 7, 1, 1), (300, 2050, 1, 0), (70, 1100, 0, 1),
+                                                   (1031, 1033, 1, 1)])
+def test_few_samples(pkg, gpu, dt, ns, n_in, n_out, bias, shift):
+    check(dt, *run(pkg, gpu, dt, ns, n_in, n_out, bias, shift), n_in, n_out)
+
+
+@pytest.mark.parametrize("dt", ["fp32", "fp16"])
+@pytest.mark.parametrize("ns", [2, 4, 7])
+def test_rows_shared_out(pkg, gpu, dt, ns):
+    """1536 rows and more: shares of the column sums that a second launch adds."""
+    n_in, n_out = 520, 1541
+    check(dt, *run(pkg, gpu, dt, ns, n_in, n_out, 1, 1), n_in, n_out)
+
+
+@pytest.mark.parametrize("dt", ["fp32", "fp16"])
+@pytest.mark.parametrize("n_in,n_out", [(70, 77), (600, 530)])
+def test_infinite_weights_stay_in_their_row_and_column(pkg, gpu, dt, n_in, n_out):
+    """What is read in place of rows and pieces beyond the end does not count: the last row and column hold infinities."""
+    ns = 3
+    got, ref, size = run(pkg, gpu, dt, ns, n_in, n_out, 0, 1, spoil=(n_out - 1, n_in - 1))
+    for k in ("y", "dx"):
+        assert torch.equal(got[k].isfinite(), ref[k].isfinite()) and torch.equal(got[k].isnan(), ref[k].isnan())
+        fin = ref[k].isfinite()
+        got[k], ref[k], size[k] = got[k][fin], ref[k][fin], size[k][fin]
+    check(dt, got, ref, size, n_in, n_out)
