@@ -1170,6 +1170,21 @@ static int gemv_coldot(const T *x, const T *Mx, T *y, int K, int M) {
     return hip_ok(hipGetLastError(), "gemv launch") ? 0 : 2;
 }
 
+// Whether C = A B^T takes the kernel that shares the contraction out over the waves of a 32 x 32 tile, in a grid of 20 to 800
+// samples, 11 to 2600 outputs and 17 to 1280 inputs (us, other routes / this): a chip that is not full two times over
+// (fp32 800 x 785 x 333 16.6 / 13.9, 800 x 1157 x 700 21 / 24), where the other routes have one launch, of larger tiles, not
+// full once (fp16 391 x 512 x 333 9.2 / 5.0, x 700 5.4 / 6.5; fp32 391 x 320 x 700 8.9 / 9.8).  Contractions of at most four trips
+// to memory: fp16 100 x 1024 x 128 8.0 / 6.3, from odd rows, which its scattered pieces cannot read at speed, 100 x 785 x 128
+// 7.1 / 10.6; fp32 100 x 512 x 128 9.2 / 6.7, 100 x 785 x 333 10.6 / 8.0, 100 x 1280 x 128 9.9 / 11.8.
+template <typename T>
+static bool deep_pays(const T *A, const T *B, int N, int M, int K) {
+    constexpr int VEC = Traits<T>::VEC;
+    const long long tiles = (long long)((N + 31) / 32) * ((M + 31) / 32), cu = state().num_cu;
+    if (state().gemm_path != 0 || K < VEC || tiles > 2 * cu) return false;
+    if (sizeof(T) == 4) return K <= 1200 && (K % 16 ? true : tiles <= cu ? K <= 900 || tiles >= 64 : K >= 512);
+    return K % 2 == 0 && ((reinterpret_cast<uintptr_t>(A) | reinterpret_cast<uintptr_t>(B)) & 3) == 0 && K <= (tiles <= cu ? 1024 : 256);
+}
+
 template <typename T>
 int mm_dispatch(const T *A, const T *B, T *C, int N, int M, int K, int trans_B, const T *bias) {
     if (!ensure_init()) return 2;
@@ -1179,6 +1194,7 @@ int mm_dispatch(const T *A, const T *B, T *C, int N, int M, int K, int trans_B, 
     if (M == 1 && !bias) return gemv_rowdot<T>(A, B, C, nullptr, N, K);  // B is K x 1 or 1 x K: the same vector
     if (N == 1 && trans_B) return gemv_rowdot<T>(B, A, C, bias, M, K);
     if (N == 1 && !bias) return M >= VEC ? gemv_coldot<T, VEC>(A, B, C, K, M) : gemv_coldot<T, 1>(A, B, C, K, M);
+    if (trans_B && deep_pays<T>(A, B, N, M, K)) return ragged_deep<T>(A, B, C, N, M, K, bias);
     GemmArgs g = {};
     g.A = A;
     g.B = B;

@@ -166,4 +166,8 @@ int ragged_back(RagConvArgs &w, RagConvArgs &x, const RagGeo *f, RagBack kind, i
 template <typename T>
 int ragged_relay(RagConvArgs &r, const RagTurn *turn, int n);
 
+// C[N][M] = A[N][K] * B[M][K]^T (+ bias[M]) with the contraction shared out over the waves of a tile; K >= 16 bytes.
+template <typename T>
+int ragged_deep(const T *A, const T *B, T *C, int N, int M, int K, const T *bias);
+
 }  // namespace ptl

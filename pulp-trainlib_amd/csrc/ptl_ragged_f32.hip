@@ -3,4 +3,5 @@
 
 namespace ptl {
 template int ragged<float>(RagArgs &, int, int, int, int);
+template int ragged_deep<float>(const float *, const float *, float *, int, int, int, const float *);
 }  // namespace ptl
