@@ -63,3 +63,24 @@ def test_long_contractions_have_no_drift(pkg, gpu):
     assert abs(float(err.mean())) <= 5e-8 * rms
     # random roundings: 8 slabs, then up to 50 sums of eight: sqrt((8 + 50) / 6) 2^-24 / sqrt(12) * 2, and a slab's own 7e-8
     assert rel(dw, ref) <= 2e-7
+
+
+@pytest.mark.parametrize("hwc", [0, 1])
+@pytest.mark.parametrize("ns", [39, 40])
+def test_layers_on_both_sides_of_the_line_between_taps_and_patches(pkg, gpu, hwc, ns):
+    """2.94 and 3.02 GFLOP: tap by tap, and as a product with patch matrices in bf16 pieces."""
+    Ci = Co = 64
+    H = W = 32
+    g = torch.Generator(device=DEV).manual_seed(ns)
+    act = (ns, H, W, Ci) if hwc else (ns, Ci, H, W)
+    x, y, dy, w, dw = (torch.rand(s, generator=g, device=DEV) - 0.5 for s in (act, act, act, (Co, 3, 3, Ci) if hwc else (Co, Ci, 3, 3), (Co, 9 * Ci)))
+    a, keep = hp.conv2d_args(pkg, x, dy, w, dw, y, dy, Ci, H, W, Co, 3, 3, H, W, pad=(1, 1, 1, 1), stride=(1, 1), hwc=hwc)
+    pkg.call("ptl_conv2d_fp32_fw_batched", a, ns)
+    assert gpu.ptl_sync() == 0
+    assert (2e-9 * ns * Co * H * W * Ci * 9 >= 3) == (ns == 40)
+    assert gpu.ptl_last_conv_direct() == (0 if ns == 40 else 1)
+    chw = (lambda t: t.double().permute(0, 3, 1, 2)) if hwc else (lambda t: t.double())
+    cols = torch.nn.functional.unfold(chw(x), 3, padding=1)
+    ref = (chw(w).reshape(Co, -1) @ cols).view(ns, Co, H, W)
+    # 576 products: sqrt(576 / 3) roundings of 2^-25 of a result's size
+    assert rel(chw(y), ref) <= 4.2e-7
