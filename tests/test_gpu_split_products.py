@@ -84,3 +84,22 @@ def test_layers_on_both_sides_of_the_line_between_taps_and_patches(pkg, gpu, hwc
     ref = (chw(w).reshape(Co, -1) @ cols).view(ns, Co, H, W)
     # 576 products: sqrt(576 / 3) roundings of 2^-25 of a result's size
     assert rel(chw(y), ref) <= 4.2e-7
+
+
+@pytest.mark.parametrize("ns,Ci,Co,k,stride", [(3, 24, 45, 5, 2), (9, 24, 45, 5, 2), (33, 24, 45, 5, 2), (18, 32, 38, 3, 1), (16, 4, 189, 3, 1)])
+def test_weight_gradients_in_more_parts(pkg, gpu, ns, Ci, Co, k, stride):
+    """Odd images, from contractions too short for bf16 pieces to ones in parts of some sixteen slabs."""
+    H = W = 57
+    Ho = (H + 2 * (k // 2) - k) // stride + 1
+    g = torch.Generator(device=DEV).manual_seed(ns * Co)
+    x, dy, w, dw = (torch.rand(s, generator=g, device=DEV) - 0.5 for s in ((ns, Ci, H, W), (ns, Co, Ho, Ho), (Co, Ci, k, k), (Co, Ci * k * k)))
+    dx = torch.empty_like(x)
+    a, keep = hp.conv2d_args(pkg, x, dx, w, dw, dy, dy, Ci, H, W, Co, k, k, Ho, Ho, pad=(k // 2,) * 4, stride=(stride, stride), hwc=0)
+    pkg.call("ptl_conv2d_fp32_bw_batched", a, ns)
+    assert gpu.ptl_sync() == 0
+    ref = torch.zeros(Co, Ci * k * k, dtype=torch.float64, device=DEV)
+    for b in range(ns):
+        cols = torch.nn.functional.unfold(x[b : b + 1].double(), k, padding=k // 2, stride=stride)[0]
+        ref += dy[b].double().reshape(Co, -1) @ cols.t().contiguous()
+    # as above, 2e-7, and up to 64 parts added up: sqrt(64 / 3) roundings of 2^-25
+    assert rel(dw, ref) <= 3.4e-7
