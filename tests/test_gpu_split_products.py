@@ -103,3 +103,26 @@ def test_weight_gradients_in_more_parts(pkg, gpu, ns, Ci, Co, k, stride):
         ref += dy[b].double().reshape(Co, -1) @ cols.t().contiguous()
     # as above, 2e-7, and up to 64 parts added up: sqrt(64 / 3) roundings of 2^-25
     assert rel(dw, ref) <= 3.4e-7
+
+
+@pytest.mark.parametrize("size", [2.0 ** -99, 2.0 ** -112, 2.0 ** -115, 2.0 ** -120, 2.0 ** -124])
+@pytest.mark.parametrize("few", [0, 1])
+def test_small_values_times_large_ones(pkg, gpu, size, few):
+    """Values whose lower pieces are below the smallest bf16 (2^-133), times ones of 2^60: results of 2^-40 to 2^-60.  few: one
+    such value in a row, zeros beside it."""
+    g = torch.Generator(device=DEV).manual_seed(5)
+    ns, Ci, Co, P = 32, 270, 300, 333
+    x, dx, dy, w, dw, a, keep = point_layer(pkg, ns, Ci, Co, P, g)
+    dy.mul_(2.0 ** 60)
+    for t in (x, w):
+        t.copy_(torch.where(t < 0, t - 1, t + 1) * size)  # (1 to 2 times size, and with the other sign)
+    if few:
+        one = x[3, :, 0, 50].clone()
+        x.zero_()
+        x[3, :, 0, 50] = one
+    pkg.call("ptl_conv2d_fp32_bw_batched", a, ns)
+    assert gpu.ptl_sync() == 0
+    X, D, W = x.double().reshape(ns, Ci, P), dy.double().reshape(ns, Co, P), w.double()
+    # sums as above, 2e-7 (one product: its rounding)
+    assert rel(dw, sum(D[b] @ X[b].t().contiguous() for b in range(ns))) <= 2e-7
+    assert rel(dx.reshape(ns, Ci, P), torch.stack([W.t().contiguous() @ D[b] for b in range(ns)])) <= 2e-7
