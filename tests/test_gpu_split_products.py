@@ -126,3 +126,20 @@ def test_small_values_times_large_ones(pkg, gpu, size, few):
     # sums as above, 2e-7 (one product: its rounding)
     assert rel(dw, sum(D[b] @ X[b].t().contiguous() for b in range(ns))) <= 2e-7
     assert rel(dx.reshape(ns, Ci, P), torch.stack([W.t().contiguous() @ D[b] for b in range(ns)])) <= 2e-7
+
+
+def test_products_next_to_the_largest_number(pkg, gpu):
+    """1.868e19 * 1.8205e19 = 3.4007e38 is finite, the product of the leading pieces is not."""
+    g = torch.Generator(device=DEV).manual_seed(6)
+    ns, Ci, Co, P = 32, 270, 300, 333
+    x, dx, dy, w, dw, a, keep = point_layer(pkg, ns, Ci, Co, P, g)
+    x.zero_()
+    x[3, 7, 0, 50] = 1.868e19
+    dy[3, 11, 0, 50] = 1.8205e19
+    dy[3, 12, 0, 50] = -1.8205e19
+    dy[3, 13, 0, 50] = 1.83e19
+    pkg.call("ptl_conv2d_fp32_bw_batched", a, ns)
+    assert gpu.ptl_sync() == 0
+    ref = x[3, 7, 0, 50].double() * dy[3, :, 0, 50].double()
+    assert float(dw[13, 7]) == float("inf") and float(ref[13]) > torch.finfo(torch.float32).max
+    assert torch.equal(dw[:13, 7], ref[:13].float()) and float(ref[11]) == -float(ref[12])
