@@ -1175,13 +1175,14 @@ static int gemv_coldot(const T *x, const T *Mx, T *y, int K, int M) {
 // (fp32 800 x 785 x 333 16.6 / 13.9, 800 x 1157 x 700 21 / 24), where the other routes have one launch, of larger tiles, not
 // full once (fp16 391 x 512 x 333 9.2 / 5.0, x 700 5.4 / 6.5; fp32 391 x 320 x 700 8.9 / 9.8).  Contractions of at most four trips
 // to memory: fp16 100 x 1024 x 128 8.0 / 6.3, from odd rows, which its scattered pieces cannot read at speed, 100 x 785 x 128
-// 7.1 / 10.6; fp32 100 x 512 x 128 9.2 / 6.7, 100 x 785 x 333 10.6 / 8.0, 100 x 1280 x 128 9.9 / 11.8.
+// 7.1 / 10.6; fp32 100 x 512 x 128 9.2 / 6.7, 100 x 785 x 333 10.6 / 8.0, 100 x 1280 x 128 9.9 / 11.8.  fp32 up to 900, where its
+// sums are as near to 64 bits as the other routes' (900: 1.19e-7 and 1.21e-7, 1153: 1.30e-7 and 1.18e-7).
 template <typename T>
 static bool deep_pays(const T *A, const T *B, int N, int M, int K) {
     constexpr int VEC = Traits<T>::VEC;
     const long long tiles = (long long)((N + 31) / 32) * ((M + 31) / 32), cu = state().num_cu;
     if (state().gemm_path != 0 || K < VEC || tiles > 2 * cu) return false;
-    if (sizeof(T) == 4) return K <= 1200 && (K % 16 ? true : tiles <= cu ? K <= 900 || tiles >= 64 : K >= 512);
+    if (sizeof(T) == 4) return K <= 900 && (K % 16 || tiles <= cu || K >= 512);
     return K % 2 == 0 && ((reinterpret_cast<uintptr_t>(A) | reinterpret_cast<uintptr_t>(B)) & 3) == 0 && K <= (tiles <= cu ? 1024 : 256);
 }
 

@@ -1,5 +1,7 @@
 """Products of few tiles with the contraction shared out over the waves of a tile, at the edges of pieces, steps, trips and
 tiles, from the C API's forward pass of dense layers."""
+import math
+
 import pytest
 import torch
 
@@ -51,3 +53,15 @@ def test_what_is_cut_away_does_not_count(pkg, gpu, dt, n_in):
     assert torch.equal(y.isnan(), ref.isnan()) and torch.equal(y.isinf(), ref.isinf())
     fin = ref.isfinite()
     assert bool(((y.double() - ref).abs()[fin] <= (2.0 ** -10 if dt == "fp16" else 2e-5) * ref[fin]).all())
+
+
+@pytest.mark.parametrize("ns,n_in,n_out", [(100, 65, 333), (100, 513, 128), (391, 785, 333), (391, 900, 200), (391, 901, 200)])
+def test_sums_are_no_chains(pkg, gpu, ns, n_in, n_out):
+    """fp32: a wave has four chains.  Roundings of at most u = 2^-24 leave u / sqrt(3) * sqrt(n / 2) after a chain of n additions of
+    values of random sign; here a 32nd of the contraction, two more in a wave and the eight waves (beyond 900 slabs of 32)."""
+    g = torch.Generator(device=DEV).manual_seed(n_in)
+    x, w = (torch.rand(s, n_in, generator=g, device=DEV) * 2 - 1 for s in (ns, n_out))
+    y = forward(pkg, gpu, "fp32", x, w, None, 0)
+    ref = x.double() @ w.double().t()
+    bound = 2.0 ** -24 / math.sqrt(3) * math.sqrt((n_in / 32 + 10) / 2)
+    assert float((y.double() - ref).norm() / ref.norm()) <= bound
