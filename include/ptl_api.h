@@ -310,9 +310,9 @@ int ptl_sync(void);
  * 7 = a Conv2D runs as products with patch matrices (any filter, stride and
  * padding; by default where they measured better) wherever its offsets fit 31
  * bits, each gradient in launches of its own; self-attention runs its panel
- * products one to a launch.  8, 9 = as 7, but the input gradient in one launch
- * with the weight gradient, on the tensors as they are (8) or on channel-minor
- * copies of channel-major ones (9).
+ * products one to a launch.  8, 9 = Conv2D as with 7, but the input gradient in
+ * one launch with the weight gradient, on the tensors as they are (8) or on
+ * channel-minor copies of channel-major ones (9); all else as with 0.
  * All routes compute the same products.
  * ptl_last_conv_direct() tells whether the last Conv2D call ran one of the
  * convolution kernels (1) or the implicit-im2col GEMM (0);
@@ -327,12 +327,16 @@ int ptl_sync(void);
  * minor copies of channel-major tensors (4);
  * ptl_last_gemm_tile() the output tile of the last product that ran a tile-per-workgroup kernel of the
  * look-up-free pipelined GEMM or of the kernel for any size and alignment (of several products in one launch, all of
- * them), as rows * 1000 + columns (256256 = 256 x 256, 128064 = 128 x 64). */
+ * them), as rows * 1000 + columns (256256 = 256 x 256, 128064 = 128 x 64);
+ * ptl_last_gemm_form() how the last dense layer, matrix product or Conv2D call formed its sums: an fp32 product of it
+ * from three bf16 pieces of each value (1), the contraction shared out over the waves of a 32 x 32 tile (2), the kernels
+ * for dense layers on a few samples (3), or otherwise (0). */
 void ptl_set_gemm_path(int path);
 int ptl_last_conv_direct(void);
 int ptl_last_gemm_streamed(void);
 int ptl_last_conv_resident(void);
 int ptl_last_gemm_tile(void);
+int ptl_last_gemm_form(void);
 /* A measurement aid (no counterpart in the reference, not on the training path): the rate, in TFLOP/s, that this
  * board sustains on a loop of nothing but fp16 MFMAs - shape 32: v_mfma_f32_32x32x16_f16, 16: v_mfma_f32_16x16x32_f16 -
  * on random (1) or all-zero (0) operands, with one or two waves per SIMD on every compute unit, `iters` x 262144 flops

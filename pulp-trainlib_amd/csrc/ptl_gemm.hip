@@ -1114,6 +1114,7 @@ __global__ __launch_bounds__(GV_NT) void linear_few_bw_kernel(const T *__restric
 
 template <typename T, int V, int NS>
 static int linear_few_bw_run(const T *x, const T *W, const T *dy, T *dW, T *dx, T *db, int ns, int in, int out) {
+    state().last_gemm_form = 3;
     const GvShares sh = gv_shares<T, V>(out, in, ns);
     const int per_row = (in + 64 * V - 1) / (64 * V);
     const long long units = (long long)((out + FEW_ROWS - 1) / FEW_ROWS) * per_row;
@@ -1140,6 +1141,7 @@ template <typename T, int NS>
 static int linear_few_fw_run(const T *x, const T *W, T *y, const T *bias, int ns, int in, int out) {
     constexpr int V = Traits<T>::VEC;
     hipStream_t s = state().stream;
+    state().last_gemm_form = 3;
     // (rows that would not fill the chip with a wave each, and are long: four waves a row)
     if (out < 8 * state().num_cu && in > 256 * V)
         hipLaunchKernelGGL((linear_few_fw_kernel<T, V, NS, 4>), dim3(out), dim3(256), 0, s, W, x, y, bias, ns, in, out);
@@ -1189,6 +1191,7 @@ static bool deep_pays(const T *A, const T *B, int N, int M, int K) {
 template <typename T>
 int mm_dispatch(const T *A, const T *B, T *C, int N, int M, int K, int trans_B, const T *bias) {
     if (!ensure_init()) return 2;
+    state().last_gemm_form = 0;
     if (N <= 0 || M <= 0 || K <= 0) return 0;  // K == 0 leaves C untouched, as mm() does
     constexpr int VEC = Traits<T>::VEC;
     if (K == 1 && !bias) return M >= VEC ? outer<T, VEC>(A, B, C, N, M) : outer<T, 1>(A, B, C, N, M);

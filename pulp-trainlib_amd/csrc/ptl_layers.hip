@@ -551,6 +551,7 @@ static int conv2d_fw(const Args *a, int ns, const char *fn) {
     if (int rc = conv_geom(a, g, fn, true)) return rc;
     if (ns <= 0) return 0;
     if (!ensure_init()) return 2;
+    state().last_gemm_form = 0;
     const int K = g.Ci * g.Hk * g.Wk, P = g.Ho * g.Wo;
     size_t in_n = (size_t)ns * g.Ci * g.H * g.W, out_n = (size_t)ns * g.Co * P;
     if (!fits_int(in_n) || !fits_int(out_n)) {
@@ -652,6 +653,7 @@ static int conv2d_wg(const Args *a, int ns, const char *fn) {
     if (int rc = conv_geom(a, g, fn, true)) return rc;
     if (ns <= 0) return 0;
     if (!ensure_init()) return 2;
+    state().last_gemm_form = 0;
     const int K = g.Ci * g.Hk * g.Wk, P = g.Ho * g.Wo;
     size_t in_n = (size_t)ns * g.Ci * g.H * g.W, out_n = (size_t)ns * g.Co * P;
     if (!fits_int(in_n) || !fits_int(out_n)) {
@@ -733,6 +735,7 @@ static int conv2d_ig(const Args *a, int ns, const char *fn) {
     if (int rc = conv_geom(a, g, fn, false)) return rc;
     if (ns <= 0) return 0;
     if (!ensure_init()) return 2;
+    state().last_gemm_form = 0;
     const int Pk = g.Hk * g.Wk, K = g.Co * Pk, P = g.Ho * g.Wo;
     size_t in_n = (size_t)ns * g.Ci * g.H * g.W, out_n = (size_t)ns * g.Co * P;
     const int Hd = (g.Ho - 1) * g.sh + 1, Wd = (g.Wo - 1) * g.sw + 1;
@@ -988,6 +991,7 @@ static int conv2d_bw(const Args *a, int ns, const char *fn) {
                                            at(a->coeff->diff), at(a->input->diff),
                                            a->USE_BIASES == 1 && a->bias ? at(a->bias->diff) : nullptr, (size_t)std::max(a->output->C, 0));
     }
+    state().last_gemm_form = 0;
     if (apart && a->USE_BIASES != 1) {
         ConvGeom g;
         if (int rc = conv_geom(a, g, fn, true)) return rc;
@@ -1090,6 +1094,7 @@ static int pw_step(const Args *a, int ns, int step, const char *fn) {
     if (int rc = pw_geom(a, fn)) return rc;
     if (ns <= 0) return 0;
     if (!ensure_init()) return 2;
+    state().last_gemm_form = 0;
     const int Ci = a->input->C, Co = a->output->C, HW = a->input->H * a->input->W;
     const bool hwc = a->HWC == 1;
     const bool w_ci_major = hwc && sizeof(T) == 4;  // fp32 HWC stores [Ci][Co]
@@ -1145,6 +1150,7 @@ static int linear_step(const Args *a, int ns, int step, const char *fn) {
     }
     if (ns <= 0) return 0;
     if (!ensure_init()) return 2;
+    state().last_gemm_form = 0;
     if (!fits_int((size_t)ns * in) || !fits_int((size_t)ns * out) || !fits_int((size_t)in * out)) {
         set_error("%s: tensor larger than 2^31 elements", fn);
         return 1;

@@ -33,7 +33,8 @@ def test_edges(pkg, gpu, dt, ns, n_out, n_in):
     r = lambda *s: shifted((torch.rand(*s, generator=g, device=DEV) - 0.5).to(TDT[dt]), shift)[0]
     x, w, b = r(ns, n_in), r(n_out, n_in), (r(n_out) if ns & 1 else None)
     y = forward(pkg, gpu, dt, x, w, b, shift)
-    assert n_in < 8 or gpu.ptl_last_gemm_tile() == 32032
+    takes = 4 <= n_in <= 900 if dt == "fp32" else n_in >= 8 and n_in % 2 == 0
+    assert (gpu.ptl_last_gemm_form() == 2) == takes
     X, W, B = x.double(), w.double(), 0 if b is None else b.double()
     ref, size = X @ W.t() + B, X.abs() @ W.abs().t() + abs(B)
     # a wave's chain of n_in / 8 additions at most, the sum of eight waves and the bias
@@ -49,6 +50,7 @@ def test_what_is_cut_away_does_not_count(pkg, gpu, dt, n_in):
     x, w = ((torch.rand(s, n_in, generator=g, device=DEV) + 0.5).to(TDT[dt]) for s in (40, 50))
     x[7, n_in - 1], w[11, n_in - 1], x[39, 0] = float("inf"), -float("inf"), float("nan")
     y = forward(pkg, gpu, dt, x, w, None, 0)
+    assert gpu.ptl_last_gemm_form() == 2
     ref = x.double() @ w.double().t()
     assert torch.equal(y.isnan(), ref.isnan()) and torch.equal(y.isinf(), ref.isinf())
     fin = ref.isfinite()
@@ -62,6 +64,7 @@ def test_sums_are_no_chains(pkg, gpu, ns, n_in, n_out):
     g = torch.Generator(device=DEV).manual_seed(n_in)
     x, w = (torch.rand(s, n_in, generator=g, device=DEV) * 2 - 1 for s in (ns, n_out))
     y = forward(pkg, gpu, "fp32", x, w, None, 0)
+    assert gpu.ptl_last_gemm_form() == (2 if n_in <= 900 else 0)
     ref = x.double() @ w.double().t()
     bound = 2.0 ** -24 / math.sqrt(3) * math.sqrt((n_in / 32 + 10) / 2)
     assert float((y.double() - ref).norm() / ref.norm()) <= bound

@@ -24,8 +24,12 @@ def run(pkg, gpu, dt, ns, n_in, n_out, bias, shift, spoil=None):
     for k, q in zip(keep, (n_in, n_in * n_out, n_out, n_out)):
         assert k.dim == q
     pkg.call("ptl_linear_%s_fw_batched" % dt, a, ns)
+    forms = [gpu.ptl_last_gemm_form()]
     pkg.call("ptl_linear_%s_bw_batched" % dt, a, ns)
     assert gpu.ptl_sync() == 0
+    forms.append(gpu.ptl_last_gemm_form())
+    few_bw = ns <= 8 and (dt == "fp32" or ns <= 4 or n_in >= 1024 or n_out >= 1536)
+    assert [f == 3 for f in forms] == [ns <= 8 or n_out <= 1280, few_bw]
     for t, buf in guard.values():
         assert bool((buf[:shift] == 5).all()) and bool((buf[shift + t.numel():] == 5).all())
     X, W, B, D = (t.double() for t in (x, w, b, dy))

@@ -31,7 +31,7 @@ def test_values_outside_the_range_of_the_pieces(pkg, gpu, what):
         if what == "huge":
             dy.mul_(0.25)
     pkg.call("ptl_conv2d_fp32_bw_batched", a, ns)
-    assert gpu.ptl_sync() == 0 and gpu.ptl_last_gemm_tile() == 64064
+    assert gpu.ptl_sync() == 0 and (gpu.ptl_last_gemm_tile(), gpu.ptl_last_gemm_form()) == (64064, 1)
     X, D, W = x.double().reshape(ns, Ci, P), dy.double().reshape(ns, Co, P), w.double()
     ref_dw = sum(D[b] @ X[b].t().contiguous() for b in range(ns))
     ref_dx = torch.stack([W.t().contiguous() @ D[b] for b in range(ns)])
@@ -56,7 +56,7 @@ def test_long_contractions_have_no_drift(pkg, gpu):
     ns, Ci, Co, P = 64, 31, 300, 576
     x, dx, dy, w, dw, a, keep = point_layer(pkg, ns, Ci, Co, P, g)
     pkg.call("ptl_conv2d_fp32_bw_batched", a, ns)
-    assert gpu.ptl_sync() == 0
+    assert gpu.ptl_sync() == 0 and gpu.ptl_last_gemm_form() == 1
     X, D = x.double().reshape(ns, Ci, P), dy.double().reshape(ns, Co, P)
     ref = sum(D[b] @ X[b].t().contiguous() for b in range(ns))
     err, rms = dw.double() - ref, float((ref ** 2).mean().sqrt())
@@ -78,7 +78,7 @@ def test_layers_on_both_sides_of_the_line_between_taps_and_patches(pkg, gpu, hwc
     pkg.call("ptl_conv2d_fp32_fw_batched", a, ns)
     assert gpu.ptl_sync() == 0
     assert (2e-9 * ns * Co * H * W * Ci * 9 >= 3) == (ns == 40)
-    assert gpu.ptl_last_conv_direct() == (0 if ns == 40 else 1)
+    assert gpu.ptl_last_conv_direct() == (0 if ns == 40 else 1) and gpu.ptl_last_gemm_form() == (1 if ns == 40 else 0)
     chw = (lambda t: t.double().permute(0, 3, 1, 2)) if hwc else (lambda t: t.double())
     cols = torch.nn.functional.unfold(chw(x), 3, padding=1)
     ref = (chw(w).reshape(Co, -1) @ cols).view(ns, Co, H, W)
@@ -88,7 +88,7 @@ def test_layers_on_both_sides_of_the_line_between_taps_and_patches(pkg, gpu, hwc
 
 @pytest.mark.parametrize("ns,Ci,Co,k,stride", [(3, 24, 45, 5, 2), (9, 24, 45, 5, 2), (33, 24, 45, 5, 2), (18, 32, 38, 3, 1), (16, 4, 189, 3, 1)])
 def test_weight_gradients_in_more_parts(pkg, gpu, ns, Ci, Co, k, stride):
-    """Odd images, from contractions too short for bf16 pieces to ones in parts of some sixteen slabs."""
+    """Odd images, from contractions too short for bf16 pieces (up to nine samples) to ones in parts of some sixteen slabs."""
     H = W = 57
     Ho = (H + 2 * (k // 2) - k) // stride + 1
     g = torch.Generator(device=DEV).manual_seed(ns * Co)
@@ -96,7 +96,7 @@ def test_weight_gradients_in_more_parts(pkg, gpu, ns, Ci, Co, k, stride):
     dx = torch.empty_like(x)
     a, keep = hp.conv2d_args(pkg, x, dx, w, dw, dy, dy, Ci, H, W, Co, k, k, Ho, Ho, pad=(k // 2,) * 4, stride=(stride, stride), hwc=0)
     pkg.call("ptl_conv2d_fp32_bw_batched", a, ns)
-    assert gpu.ptl_sync() == 0
+    assert gpu.ptl_sync() == 0 and gpu.ptl_last_gemm_form() == (1 if ns > 9 else 0)
     ref = torch.zeros(Co, Ci * k * k, dtype=torch.float64, device=DEV)
     for b in range(ns):
         cols = torch.nn.functional.unfold(x[b : b + 1].double(), k, padding=k // 2, stride=stride)[0]
@@ -121,7 +121,7 @@ def test_small_values_times_large_ones(pkg, gpu, size, few):
         x.zero_()
         x[3, :, 0, 50] = one
     pkg.call("ptl_conv2d_fp32_bw_batched", a, ns)
-    assert gpu.ptl_sync() == 0
+    assert gpu.ptl_sync() == 0 and gpu.ptl_last_gemm_form() == 1
     X, D, W = x.double().reshape(ns, Ci, P), dy.double().reshape(ns, Co, P), w.double()
     # sums as above, 2e-7 (one product: its rounding)
     assert rel(dw, sum(D[b] @ X[b].t().contiguous() for b in range(ns))) <= 2e-7
@@ -139,7 +139,7 @@ def test_products_next_to_the_largest_number(pkg, gpu):
     dy[3, 12, 0, 50] = -1.8205e19
     dy[3, 13, 0, 50] = 1.83e19
     pkg.call("ptl_conv2d_fp32_bw_batched", a, ns)
-    assert gpu.ptl_sync() == 0
+    assert gpu.ptl_sync() == 0 and gpu.ptl_last_gemm_form() == 1
     ref = x[3, 7, 0, 50].double() * dy[3, :, 0, 50].double()
     assert float(dw[13, 7]) == float("inf") and float(ref[13]) > torch.finfo(torch.float32).max
     assert torch.equal(dw[:13, 7], ref[:13].float()) and float(ref[11]) == -float(ref[12])
