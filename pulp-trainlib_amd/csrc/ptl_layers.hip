@@ -1122,17 +1122,35 @@ static int pw_step(const Args *a, int ns, int step, const char *fn) {
 // the input/output blobs is a vector of blob->dim elements.
 
 // Few samples: the kernels of ptl_gemm.hip that read each weight once, against tiles of 32 x 32 and more with partial sums, in a
-// grid of 96 to 3800 inputs and 48 to 4000 outputs.
-// Forward, two to eight samples: 1.1 to 3.5 times as fast (1157 -> 500, 4 samples, fp16 2.9), 0.8 to 1 at worst (96 -> 4000,
-// 3, fp16).  Up to sixteen samples 1.15 to 2.4 times with few outputs, not with many, where all of the samples are read again
-// for every row (1944 -> 320, 16, fp16 10.2 -> 6.7 us; 781 -> 3840, 11, fp32 12.5 and 13.5; 3904 -> 2837, 9: 14.7 and 29.7).
-static bool few_fw(int ns, int out) { return state().gemm_path == 0 && ns >= 2 && (ns <= 8 || (ns <= 16 && out <= 1280)); }
-// Backward: fp32 1.05 to 4 times (2304 -> 2100, 4 samples 45 -> 11 us), fp16 1.03 to 2.3 up to four samples.  With more the
-// matrix instructions of fp16 are as fast until the weights are many (8 samples, 640 -> 48 5.1 and 5.7 us, 1157 -> 500 7.9 ->
-// 7.3, 640 -> 2100 12.3 -> 10.1).
+// grid of 64 to 65536 inputs and 64 to 65536 outputs.  Other routes' time over theirs:
+// Forward, up to sixteen samples: 1.1 to 2.2 while the weights are few.  Every row reads all samples again, 4 to 16 times the
+// weights' own bytes out of L2, which bounds it beyond
+//   two samples        nothing (8192 x 8192 fp32 1.13, fp16 1.11)
+//   three and four     70 MB (64 MB: fp32 1.07 to 1.24, fp16 0.97 to 1.13; 128 MB: 0.83 to 1.07)
+//   five to eight      24 MB of rows up to 16384 (16 MB: 1.08 to 1.36; 32 MB: 0.62 to 1.0; 65536 -> 64 0.78 and 0.96)
+//   up to sixteen      5.5 MB of rows up to 12 KB and 4096, 1280 outputs (5 MB: 1.01 to 1.12; 10 MB and 4096 -> 320: 0.7 to 0.9)
+// and rows by the thousand, of which each is a wave's chain of shuffles: 8192 of less than 1 KB take 0.75 to 0.92, 65536 of any
+// length 0.2 to 0.8, 16384 0.5 to 0.9 but with two samples from 4 KB on (1.1 to 2.0) and in fp32 with up to four from 2 KB on,
+// where the other routes are behind up to 256 MB (1.3 to 1.75).
+template <typename T>
+static bool few_fw(int ns, int in, int out) {
+    if (state().gemm_path != 0 || ns < 2 || ns > 16) return false;
+    const double bytes = (double)sizeof(T) * in * out, row = (double)sizeof(T) * in;
+    if (ns > 8) return out <= 1280 && in <= 4096 && row <= 12288 && bytes <= 5.5e6;
+    const bool more = out > 8192;
+    if (more && !(ns == 2 && row >= 4096) && !(sizeof(T) == 4 && ns <= 4 && out <= 16384 && row >= 2048)) return false;
+    if (out > 4096 && row < 1024) return false;
+    if (ns > 4) return in <= 16384 && bytes <= 24e6;
+    return ns == 2 || bytes <= (more ? 270e6 : 70e6);
+}
+// Backward: fp32 1.0 to 3.7 (2304 -> 2100, 4 samples 45 -> 11 us; 4096 -> 64 0.85 to 0.93), fp16 1.0 to 2.7 up to four samples.  With
+// more the matrix instructions of fp16 are as fast until the weights are many (8 samples, 640 -> 48 5.1 and 5.7 us, 1157 -> 500
+// 7.9 -> 7.3, 640 -> 2100 12.3 -> 10.1), and with one side long and the other short (65536 -> 64 0.74, 16384 -> 64 0.83, 64 ->
+// 65536 0.9; 8192 -> 64 1.02, 64 -> 16384 1.08).
 template <typename T>
 static bool few_bw(int ns, int in, int out) {
-    return state().gemm_path == 0 && ns >= 2 && ns <= LINEAR_FEW && (sizeof(T) == 4 || ns <= 4 || in >= 1024 || out >= 1536);
+    if (state().gemm_path != 0 || ns < 2 || ns > LINEAR_FEW) return false;
+    return sizeof(T) == 4 || ns <= 4 || ((in >= 1024 || out >= 1536) && in <= 128LL * out && out <= 512LL * in);
 }
 
 template <typename T, typename Args>
@@ -1168,7 +1186,7 @@ static int linear_step(const Args *a, int ns, int step, const char *fn) {
         T *Y = sg.out(reinterpret_cast<T *>(a->output->data), (size_t)ns * out);
         const T *bias = use_bias ? sg.in(reinterpret_cast<const T *>(a->bias->data), (size_t)out) : nullptr;
         if (sg.failed()) return 2;
-        if (few_fw(ns, out)) return sg.finish(linear_few_fw<T>(X, Wt, Y, bias, ns, in, out));
+        if (few_fw<T>(ns, in, out)) return sg.finish(linear_few_fw<T>(X, Wt, Y, bias, ns, in, out));
         rc = mm_dispatch<T>(X, Wt, Y, ns, out, in, 1, bias);  // Y[b][o] = X[b][:] . W[o][:] + bias[o]
     } else if (step == STEP_BW_BOTH) {
         // weight and input gradient of a batch in one launch

@@ -8,7 +8,7 @@ pytestmark = pytest.mark.gpu
 TDT = {"fp32": torch.float32, "fp16": torch.float16}
 
 
-def run(pkg, gpu, dt, ns, n_in, n_out, bias, shift, spoil=None):
+def run(pkg, gpu, dt, ns, n_in, n_out, bias, shift, spoil=None, takes=None):
     g = torch.Generator(device=DEV).manual_seed(n_in * 31 + n_out)
     r = lambda *s: shifted((torch.rand(*s, generator=g, device=DEV) - 0.5).to(TDT[dt]), shift)[0]
     x, w, b, dy = r(ns, n_in), r(n_out, n_in), r(n_out), r(ns, n_out)
@@ -28,8 +28,8 @@ def run(pkg, gpu, dt, ns, n_in, n_out, bias, shift, spoil=None):
     pkg.call("ptl_linear_%s_bw_batched" % dt, a, ns)
     assert gpu.ptl_sync() == 0
     forms.append(gpu.ptl_last_gemm_form())
-    few_bw = ns <= 8 and (dt == "fp32" or ns <= 4 or n_in >= 1024 or n_out >= 1536)
-    assert [f == 3 for f in forms] == [ns <= 8 or n_out <= 1280, few_bw]
+    few_bw = ns <= 8 and (dt == "fp32" or ns <= 4 or ((n_in >= 1024 or n_out >= 1536) and n_in <= 128 * n_out))
+    assert [f == 3 for f in forms] == list(takes or (ns <= 8 or n_out <= 1280, few_bw))
     for t, buf in guard.values():
         assert bool((buf[:shift] == 5).all()) and bool((buf[shift + t.numel():] == 5).all())
     X, W, B, D = (t.double() for t in (x, w, b, dy))
@@ -74,3 +74,30 @@ def test_infinite_weights_stay_in_their_row_and_column(pkg, gpu, dt, n_in, n_out
         fin = ref[k].isfinite()
         got[k], ref[k], size[k] = got[k][fin], ref[k][fin], size[k][fin]
     check(dt, got, ref, size, n_in, n_out)
+
+
+@pytest.mark.parametrize("dt,ns,n_in,n_out,fw,bw", [
+    ("fp32", 4, 4096, 4096, 1, 1), ("fp32", 3, 4352, 4096, 0, 1),      # 70 MB of weights
+    ("fp16", 8, 2928, 4096, 1, 1), ("fp16", 5, 2936, 4096, 0, 1),      # 24 MB
+    ("fp32", 8, 16384, 64, 1, 1), ("fp32", 8, 16388, 64, 0, 1),        # long rows
+    ("fp32", 16, 1024, 1280, 1, 0), ("fp32", 9, 1076, 1280, 0, 0),     # 5.5 MB
+    ("fp16", 16, 4096, 64, 1, 0), ("fp16", 9, 4104, 64, 0, 0), ("fp32", 12, 3076, 64, 0, 0), ("fp16", 9, 512, 1281, 0, 0),
+    ("fp32", 2, 255, 4096, 1, 1), ("fp32", 2, 255, 4097, 0, 1), ("fp32", 8, 256, 4097, 1, 1),  # many short rows
+    ("fp16", 2, 2048, 8193, 1, 1), ("fp16", 2, 2040, 8193, 0, 1), ("fp16", 4, 2048, 8193, 0, 1),
+    ("fp32", 4, 512, 16384, 1, 1), ("fp32", 4, 511, 16384, 0, 1), ("fp32", 4, 512, 16385, 0, 1), ("fp32", 5, 512, 8193, 0, 1),
+    ("fp16", 8, 8192, 64, 1, 1), ("fp16", 8, 8200, 64, 1, 0), ("fp16", 8, 20, 10240, 0, 1), ("fp16", 8, 20, 10248, 0, 0)])
+def test_lines_to_the_other_routes(pkg, gpu, dt, ns, n_in, n_out, fw, bw):
+    check(dt, *run(pkg, gpu, dt, ns, n_in, n_out, 1, 0, takes=(fw, bw)), n_in, n_out)
+
+
+def test_more_outputs_than_one_launch_of_row_sums_has_threads_for(pkg, gpu):
+    """2^26 rows, a wave each: such a launch left the outputs as they were."""
+    ns, n_out = 2, 2 ** 26 + 5
+    x, w = torch.tensor([[2.0], [-3.0]], device=DEV).half(), (torch.arange(n_out, device=DEV) % 511).half()
+    y = torch.zeros(ns, n_out, device=DEV).half()
+    a = pkg.LinearArgs()
+    keep = [pkg.blob(x, None, dim=1), pkg.blob(w, None, dim=n_out), pkg.blob(y, None, dim=n_out)]
+    a.input, a.coeff, a.output = [pkg.structs.C.pointer(k) for k in keep]
+    pkg.call("ptl_linear_fp16_fw_batched", a, ns)
+    assert gpu.ptl_sync() == 0
+    assert torch.equal(y, x * w)
