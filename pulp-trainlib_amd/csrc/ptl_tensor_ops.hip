@@ -1286,6 +1286,11 @@ __device__ inline unsigned xcd_run(unsigned b, unsigned n) {
     return (b >> 3) + xcd * (n >> 3) + min(xcd, n & 7);
 }
 
+// Workgroup b of n tiles in a launch of tile_grid(n): a launch of 256 threads has room for 2^24 of them along one axis.
+constexpr int TILE_GRID = 23;
+static dim3 tile_grid(long long n) { return dim3((unsigned)std::min(n, 1LL << TILE_GRID), (unsigned)((n + (1LL << TILE_GRID) - 1) >> TILE_GRID)); }
+__device__ inline unsigned tile_of_grid() { return blockIdx.y << TILE_GRID | blockIdx.x; }
+
 // How patch_rows_kernel reads rows of the tensor.
 enum PatchRead { PATCH_SINGLE, PATCH_ALIGNED, PATCH_MOVED };
 
@@ -1439,7 +1444,8 @@ __global__ __launch_bounds__(256) void patch_rows_kernel(const T *__restrict__ s
     typedef const PatchPiece __attribute__((address_space(1))) *GlobalPiece;
     typedef const PatchRun __attribute__((address_space(1))) *GlobalRun;
     extern __shared__ __attribute__((aligned(16))) char smem[];
-    const unsigned tile = xcd_run(blockIdx.x, tiles), place = rag_quot(tile, by_nz), row_of = rag_quot(place, by_nx);
+    if (tile_of_grid() >= tiles) return;
+    const unsigned tile = xcd_run(tile_of_grid(), tiles), place = rag_quot(tile, by_nz), row_of = rag_quot(place, by_nx);
     const int c0 = (int)(tile - place * nz) * CB, hp = (int)row_of, wp0 = (int)(place - row_of * nx) * R;
     CB = min(CB, g.C - c0);
     const int PK = g.Hk * g.Wk, Q = g.C * PK, nq = CB * PK;  // (at least a chunk)
@@ -1717,9 +1723,10 @@ static int patch_rows(const T *src, T *buf, const PatchGeom &g) {
     auto magic = [](unsigned d) { return (unsigned)((((unsigned long long)1 << 32) + d - 1) / d); };
     const int nx = (g.Wp + R - 1) / R;
     if ((long long)nx * g.Hp * nz >= 1LL << 31) return -1;
-    const dim3 grid((unsigned)(nx * g.Hp * nz));
+    const unsigned tiles = (unsigned)(nx * g.Hp * nz);
     auto launch = [&](auto kern) {
-        hipLaunchKernelGGL(kern, grid, dim3(256), bytes(CB), state().stream, src, buf, g, R, CB, LW, magic(PK), magic(g.Wk), magic(g.Hk), np, magic(np), rag_div(nx), rag_div(nz), grid.x);
+        hipLaunchKernelGGL(kern, tile_grid(tiles), dim3(256), bytes(CB), state().stream, src, buf, g, R, CB, LW, magic(PK), magic(g.Wk), magic(g.Hk), np, magic(np), rag_div(nx),
+                           rag_div(nz), tiles);
     };
     if (read == PATCH_ALIGNED) launch(patch_rows_kernel<T, PATCH_ALIGNED>);
     else if (read == PATCH_MOVED) launch(patch_rows_kernel<T, PATCH_MOVED>);
@@ -1979,7 +1986,7 @@ static int blocktransp(const Args *a, const char *fn) {
         // runs of whole 16-byte chunks: every run starts on a chunk (rows of Ci x P and Co x P elements, tiles of 32 x P)
         const bool vecs = ((size_t)a->Cin * P * sizeof(T)) % 16 == 0 && ((size_t)a->Cout * P * sizeof(T)) % 16 == 0 &&
                           reinterpret_cast<uintptr_t>(w) % 16 == 0 && reinterpret_cast<uintptr_t>(bt) % 16 == 0;
-        auto tile_grid = [&](int td) {  // (groups of four tiles, rounded up to eight groups)
+        auto block_grid = [&](int td) {  // (groups of four tiles, rounded up to eight groups)
             const long long groups = (long long)(((a->Cin + td - 1) / td + 1) / 2) * (((a->Cout + td - 1) / td + 1) / 2);
             return (unsigned)(32 * ((groups + 7) / 8));
         };
@@ -1989,7 +1996,7 @@ static int blocktransp(const Args *a, const char *fn) {
         const int td = vecs || tiles >= state().num_cu ? 32 : 8;
         const int pitch = td * P + VEC;  // rows of the tile start on 16-byte boundaries
         const size_t lds = (size_t)td * pitch * sizeof(T);
-        const dim3 grid(tile_grid(td));
+        const dim3 grid(block_grid(td));
         if (vecs)
             hipLaunchKernelGGL((blocktransp_tile_kernel<T, true, 32, 256>), grid, dim3(256), lds, state().stream, w, bt,
                                a->Cin, a->Cout, P, m_p, pitch);
@@ -2033,7 +2040,8 @@ typedef unsigned TranspPiece __attribute__((ext_vector_type(4), aligned(1)));
 template <typename T>
 __global__ __launch_bounds__(256) void transpose2d_kernel(const T *__restrict__ in, T *__restrict__ out, Transp2D g) {
     fetch_args(in, out, g);
-    const unsigned ny = g.by_ny.d, t = xcd_run(blockIdx.x, g.tiles);
+    if (tile_of_grid() >= g.tiles) return;
+    const unsigned ny = g.by_ny.d, t = xcd_run(tile_of_grid(), g.tiles);
     constexpr int VEC = 16 / (int)sizeof(T), CH = 64 / VEC;  // chunks per tile row
     constexpr int PITCH = sizeof(T) == 2 ? 66 : 65;          // elements
     __shared__ __attribute__((aligned(16))) T tile[64 * PITCH];
@@ -2093,7 +2101,8 @@ static int transpose2d_strided(const T *in, T *out, int N, int M, long long in_r
                                long long in_bs, long long out_bs, long long in_base, long long out_base) {
     const int nx = (M + 63) / 64, ny = (N + 63) / 64;
     const Transp2D g = {N, M, (unsigned)(nx * ny), rag_div(ny), in_rs, out_rs, in_bs, out_bs, in_base, out_base};
-    const dim3 grid(g.tiles, 1, batch);
+    dim3 grid = tile_grid(g.tiles);
+    grid.z = batch;
     hipLaunchKernelGGL((transpose2d_kernel<T>), grid, dim3(256), 0, state().stream, in, out, g);
     return hip_ok(hipGetLastError(), "transpose launch") ? 0 : 2;
 }
