@@ -1172,20 +1172,23 @@ static int gemv_coldot(const T *x, const T *Mx, T *y, int K, int M) {
     return hip_ok(hipGetLastError(), "gemv launch") ? 0 : 2;
 }
 
-// Whether C = A B^T takes the kernel that shares the contraction out over the waves of a 32 x 32 tile, in a grid of 20 to 800
-// samples, 11 to 2600 outputs and 17 to 1280 inputs (us, other routes / this): a chip that is not full two times over
-// (fp32 800 x 785 x 333 16.6 / 13.9, 800 x 1157 x 700 21 / 24), where the other routes have one launch, of larger tiles, not
-// full once (fp16 391 x 512 x 333 9.2 / 5.0, x 700 5.4 / 6.5; fp32 391 x 320 x 700 8.9 / 9.8).  Contractions of at most four trips
-// to memory: fp16 100 x 1024 x 128 8.0 / 6.3, from odd rows, which its scattered pieces cannot read at speed, 100 x 785 x 128
-// 7.1 / 10.6; fp32 100 x 512 x 128 9.2 / 6.7, 100 x 785 x 333 10.6 / 8.0, 100 x 1280 x 128 9.9 / 11.8.  fp32 up to 900, where its
-// sums are as near to 64 bits as the other routes' (900: 1.19e-7 and 1.21e-7, 1153: 1.30e-7 and 1.18e-7).
+// Whether C = A B^T takes the kernel that shares the contraction out over the waves of a 32 x 32 tile, in a grid of 17 to 8192
+// samples, 8 to 8192 outputs and 16 to 1300 inputs (us, other routes / this): 1.3 times as fast in the mean of 233 fp32 layers,
+// 1.2 of 189 in fp16.  As many tiles as the chip has compute units: contractions of at most four trips to memory (fp16 100 x 1024
+// x 128 8.0 / 6.3, but from odd rows, which its scattered pieces cannot read at speed, 100 x 785 x 128 7.1 / 10.6; fp32 100 x 512 x
+// 128 9.2 / 6.7, 100 x 785 x 333 10.6 / 8.0), fp32 up to 900, where its sums are as near to 64 bits as the other routes' (900:
+// 1.19e-7 and 1.21e-7, 1153: 1.30e-7 and 1.18e-7).  Up to two tiles a compute unit, where the other routes have one launch of
+// larger tiles: fp32 from rows that they cannot read in whole slabs up to 800 (714 16.6 / 13.9, 886 19.4 / 20.5), aligned ones
+// of 512 to 600 (512 12.9 / 10.8, 240 9.0 / 8.9, 576 14.4 / 14.4, 832 18.0 / 18.9, 1152 15.5 / 22.8); fp16 up to 256 but for whole
+// slabs (128 4.7 / 6.4, 192 5.0 / 6.6; 64 5.0 / 4.9).
 template <typename T>
 static bool deep_pays(const T *A, const T *B, int N, int M, int K) {
     constexpr int VEC = Traits<T>::VEC;
     const long long tiles = (long long)((N + 31) / 32) * ((M + 31) / 32), cu = state().num_cu;
     if (state().gemm_path != 0 || K < VEC || tiles > 2 * cu) return false;
-    if (sizeof(T) == 4) return K <= 900 && (K % 16 || tiles <= cu || K >= 512);
-    return K % 2 == 0 && ((reinterpret_cast<uintptr_t>(A) | reinterpret_cast<uintptr_t>(B)) & 3) == 0 && K <= (tiles <= cu ? 1024 : 256);
+    if (sizeof(T) == 4) return tiles <= cu ? K <= 900 : K % 16 ? K <= 800 : K >= 512 && K <= 600;
+    return K % 2 == 0 && ((reinterpret_cast<uintptr_t>(A) | reinterpret_cast<uintptr_t>(B)) & 3) == 0 &&
+           (tiles <= cu ? K <= 1024 : K <= 256 && (K % 64 != 0 || K == 64));
 }
 
 template <typename T>

@@ -68,3 +68,19 @@ def test_sums_are_no_chains(pkg, gpu, ns, n_in, n_out):
     ref = x.double() @ w.double().t()
     bound = 2.0 ** -24 / math.sqrt(3) * math.sqrt((n_in / 32 + 10) / 2)
     assert float((y.double() - ref).norm() / ref.norm()) <= bound
+
+
+@pytest.mark.parametrize("dt,n_in,n_out,takes", [
+    ("fp32", 512, 864, 1), ("fp32", 496, 864, 0), ("fp32", 608, 864, 0), ("fp32", 800, 864, 0), ("fp32", 799, 864, 1), ("fp32", 801, 864, 0),
+    ("fp32", 800, 512, 1), ("fp32", 20, 1376, 0), ("fp16", 64, 864, 1), ("fp16", 128, 864, 0), ("fp16", 130, 864, 1), ("fp16", 192, 864, 0),
+    ("fp16", 192, 512, 1), ("fp16", 258, 864, 0)])
+def test_lines_to_the_other_routes(pkg, gpu, dt, n_in, n_out, takes):
+    """378 samples: twelve tiles in height, 192 to 516 of them on 256 compute units."""
+    g = torch.Generator(device=DEV).manual_seed(n_in)
+    x, w = ((torch.rand(s, n_in, generator=g, device=DEV) - 0.5).to(TDT[dt]) for s in (378, n_out))
+    y = forward(pkg, gpu, dt, x, w, None, 0)
+    assert (gpu.ptl_last_gemm_form() == 2) == takes
+    ref = x.double() @ w.double().t()
+    # fp32: as above, and one chain of additions on routes that look nothing up; fp16: roundings of the result, 2^-12 in the mean
+    bound = 2.0 ** -24 / math.sqrt(3) * math.sqrt((n_in / 32 + 10 if takes else n_in) / 2)
+    assert float((y.double() - ref).norm() / ref.norm()) <= (bound if dt == "fp32" else 2.5e-4)
