@@ -511,11 +511,34 @@ static int dense_bw(const T *X, const T *Wt, const T *dY, T *dW, T *dX, T *db, i
 static bool is_point(const ConvGeom &g) {
     return g.Hk == 1 && g.Wk == 1 && g.sh == 1 && g.sw == 1 && g.H == g.Ho && g.W == g.Wo && g.Up == 0 && g.Lp == 0 && state().gemm_path == 0;
 }
+// Where the other routes are ahead (over 1800 fp32 and 900 fp16 layers; elsewhere they take 1.2 to 1.3 times as long in the mean):
+//   * fp32, channel-major, from 1 GFLOP on: 33 to 128 channels into 256 and more, whose panels of filters each stream the image again
+//     (their time over this one's 0.72 to 0.88 in the mean; 128 -> 335, 103 samples of 36 x 25 119 and 241 us); more channels into at
+//     most 32, whose tiles are half empty (0.88); and from 2 GFLOP on images of up to 1024 pixels, with which the tiles end (0.94).
+//     Images of at most 48 pixels whatever the work from two tiles a compute unit on (0.43 to 0.86; 128 -> 448, 203 samples of 5 x 3
+//     15 and 61; one tile 1.0);
+//   * fp32, channel-minor, eight to sixteen channels in whole pieces, no bias: the gathering product, which reads each pixel once (8 ->
+//     16, 436 samples of 59 x 59 37.5 and 132, 16 -> 320, 98 000 pixels 48.1 and 50.6; 20 -> 184 14.5 and 14.6);
+//   * fp16, channel-minor with a bias, at most 32 filters over 2^17 pixels and more, 0.79: the patch products (32 -> 24, 1.7 million
+//     pixels 95 and 128; 33 filters and more 1.1).
+template <typename T>
+static bool point_shallow(const ConvGeom &g, bool bias) {
+    return sizeof(T) == 4 && g.hwc && !bias && g.Ci >= 8 && g.Ci <= 16 && g.Ci % 4 == 0 && g.Co % 4 == 0 && is_point(g);
+}
+template <typename T>
+static bool point_fw_behind(const ConvGeom &g, int ns, bool bias) {
+    const int P = g.H * g.W;
+    if (sizeof(T) == 2) return g.hwc && bias && g.Co <= 32 && (long long)ns * P >= 1 << 17;
+    if (g.hwc) return point_shallow<T>(g, bias);
+    const double gflop = 2e-9 * ns * P * g.Ci * g.Co;
+    if (P <= 48 && (long long)ns * ((g.Co + 63) / 64) >= 2 * state().num_cu) return true;
+    return gflop >= 1 && g.Ci > 32 && (g.Ci <= 128 ? g.Co >= 256 : g.Co <= 32 || (P <= 1024 && gflop >= 2));
+}
 template <typename T>
 static int point_fw(const ConvGeom &g, int ns, const T *X, const T *Wt, const T *bias, T *Y) {
     constexpr int VEC = 16 / (int)sizeof(T);
     const int P = g.H * g.W;
-    if (!is_point(g) || g.Ci < VEC || P < VEC) return -1;
+    if (!is_point(g) || g.Ci < VEC || P < VEC || point_fw_behind<T>(g, ns, bias != nullptr)) return -1;
     // (fp32 on the kernel for any size: its sums are nearer to 64 bits, 1.1e-7 against 2.0e-7 for 448 -> 47 channels)
     if (sizeof(T) == 4 || (bias && !g.hwc)) return conv_point_fw<T>(forward_desc(g, ns), X, Wt, bias, Y);
     if (g.hwc) return mm_dispatch<T>(X, Wt, Y, ns * P, g.Co, g.Ci, 1, bias);
@@ -600,11 +623,12 @@ static int conv2d_fw(const Args *a, int ns, const char *fn) {
         // Large fp32 layers are bound by the matrix instructions, of which products with patch matrices form theirs from bf16
         // pieces: from 3 GFLOP on 1.2 to 1.7 times as fast as tap by tap, 0.96 at worst (60 samples, 128 -> 128, 32 x 32, 3 x 3 175
         // -> 139 us; 4, 512 -> 64, 28 x 28, 5 x 5 channel-minor 145 -> 85), 0.75 to 1.26 from 1 to 2.5 GFLOP.
-        if (rc < 0 && sizeof(T) == 4 && state().gemm_path == 0 && 2.0 * ns * g.Co * g.Ho * g.Wo * K >= 3e9 &&
+        const bool gather = point_shallow<T>(g, bias != nullptr);
+        if (rc < 0 && !gather && sizeof(T) == 4 && state().gemm_path == 0 && 2.0 * ns * g.Co * g.Ho * g.Wo * K >= 3e9 &&
             any_pays<T>(g, ns, 1, bias != nullptr) && (rc = conv_any_fw<T>(d, X, Wt, bias, Y)) >= 0)
             return sg.finish(rc);
         if (rc < 0) rc = conv_taps<T>(d, X, Wt, Y, c);
-        if (rc < 0 && any_pays<T>(g, ns, 1, bias != nullptr) && (rc = conv_any_fw<T>(d, X, Wt, bias, Y)) >= 0) return sg.finish(rc);
+        if (rc < 0 && !gather && any_pays<T>(g, ns, 1, bias != nullptr) && (rc = conv_any_fw<T>(d, X, Wt, bias, Y)) >= 0) return sg.finish(rc);
         if (rc < 0) rc = conv_tile<T>(d, X, Wt, Y, c);
         if (rc > 0) return sg.finish(rc);
         if (rc == 0) state().last_conv_direct = 1;

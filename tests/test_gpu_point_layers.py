@@ -43,3 +43,21 @@ def test_layer(pkg, gpu, dt, hwc, bias, case):
     assert rel(dw, D.t() @ X) <= TOL[dt]
     if bias:
         assert rel(db, D.sum(0)) <= TOL[dt]
+
+
+@pytest.mark.parametrize("dt,hwc,bias,ns,Ci,Co,H,W", [
+    ("fp32", 0, 0, 120, 33, 256, 25, 25), ("fp32", 0, 1, 30, 128, 260, 25, 25), ("fp32", 0, 1, 30, 128, 255, 25, 25), ("fp32", 0, 1, 120, 32, 256, 25, 25),
+    ("fp32", 0, 1, 90, 132, 32, 41, 37), ("fp32", 0, 0, 90, 132, 33, 41, 37), ("fp32", 0, 1, 60, 129, 128, 32, 32), ("fp32", 0, 1, 60, 129, 128, 33, 32),
+    ("fp32", 0, 0, 512, 65, 64, 6, 8), ("fp32", 0, 1, 260, 20, 70, 1, 15), ("fp32", 0, 0, 511, 65, 64, 7, 7),  # images of 48 pixels
+    ("fp32", 1, 0, 9, 8, 20, 41, 37), ("fp32", 1, 0, 9, 16, 64, 41, 37), ("fp32", 1, 0, 9, 20, 64, 41, 37), ("fp32", 1, 0, 9, 12, 66, 41, 37),
+    ("fp32", 1, 0, 600, 16, 32, 72, 72),                                                                         # 3.2 GFLOP
+    ("fp16", 1, 1, 33, 24, 32, 64, 64), ("fp16", 1, 1, 32, 9, 17, 64, 64), ("fp16", 1, 1, 31, 24, 32, 64, 64), ("fp16", 1, 1, 33, 24, 33, 64, 64)])
+def test_forward_on_both_sides_of_the_lines(pkg, gpu, dt, hwc, bias, ns, Ci, Co, H, W):
+    g = torch.Generator(device=DEV).manual_seed(Ci + Co)
+    act = (lambda c: (ns, H, W, c)) if hwc else (lambda c: (ns, c, H, W))
+    x, y, w, b = tensor(g, act(Ci), dt), tensor(g, act(Co), dt), tensor(g, (Co, Ci), dt), tensor(g, (Co,), dt)
+    a, keep = hp.conv2d_args(pkg, x, x, w, w, y, y, Ci, H, W, Co, 1, 1, H, W, (0, 0, 0, 0), (1, 1), hwc, bias=b if bias else None)
+    pkg.call("ptl_conv2d_%s_fw_batched" % dt, a, ns)
+    assert gpu.ptl_sync() == 0
+    rows = (lambda t, c: t.double().reshape(-1, c)) if hwc else (lambda t, c: t.double().reshape(ns, c, H * W).permute(0, 2, 1).reshape(-1, c))
+    assert rel(rows(y, Co), rows(x, Ci) @ w.double().t() + (b.double() if bias else 0)) <= TOL[dt]
