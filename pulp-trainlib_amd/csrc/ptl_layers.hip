@@ -544,6 +544,11 @@ static int point_fw(const ConvGeom &g, int ns, const T *X, const T *Wt, const T 
     if (g.hwc) return mm_dispatch<T>(X, Wt, Y, ns * P, g.Co, g.Ci, 1, bias);
     return gemm<T>(pw_product(STEP_FW, X, Wt, nullptr, Y, ns, g.Ci, g.Co, P, false, g.Ci, 1));
 }
+// fp32 layers of 128 channels and more into fewer than 64, from 64 MB of input and output on: half of a tile of the weight gradient
+// is empty, and the patch products (channel-major: 0.63 to 0.93 of the time here) or the steps one after the other (channel-minor: 0.67
+// to 0.93) are ahead (480 -> 9, 257 samples of 27 x 27 272 and 422 us; 704 -> 16, 12 of 93 x 65 140 and 199; 64 filters 1.0 to 1.2).
+template <typename T>
+static bool point_bw_behind(const ConvGeom &g, double mb) { return sizeof(T) == 4 && mb >= 64 && g.Co < 64 && g.Ci >= 128; }
 // Channel-major tensors: both gradients in one launch, fp16 up to 40 MB of input and output, the two products by themselves
 // above (the patch matrices' time over theirs, mean of 400 layers, one launch / two products: fp16 2.4 / 1.6 below 0.3 MB,
 // 1.8 / 1.4 at 3 to 30, 1.5 / 1.4 at 30 to 100, 0.8 / 1.2 above).  Channel-minor fp16 layers above 100 MB stay with the
@@ -554,6 +559,7 @@ static int point_bw(const ConvGeom &g, int ns, const T *X, const T *dY, const T 
     const int P = g.H * g.W;
     if (!is_point(g) || g.Ci < VEC || g.Co < VEC) return -1;
     const double mb = 1e-6 * sizeof(T) * ns * P * ((double)g.Ci + g.Co);
+    if (point_bw_behind<T>(g, mb)) return -1;
     if (g.hwc) {
         if (sizeof(T) == 4) return linear_bw_ragged<T>(X, Wt, dY, dW, dX, db, ns * P, g.Ci, g.Co);
         return mb > 100 ? -1 : dense_bw<T>(X, Wt, dY, dW, dX, db, ns * P, g.Ci, g.Co, true);
@@ -1076,7 +1082,11 @@ static int conv2d_bw(const Args *a, int ns, const char *fn) {
     // resident-tile one wherever it is preferred (a call then has the bits of its two steps), and those of channel-minor
     // layers from 20 on (1.77, 1.26 and 1.22 at 4, 10 and 19, 0.92 and 0.82 at 31 and 39).  Strided channel-major 1x1 layers,
     // whose input gradient is a plain product scattered over zeros, from some MB of input and output on (fp16 1.4 in the
-    // mean at 3 to 5 MB, 1.0 at 7 to 30, 0.8 above; fp32 1.4 at 7 to 10, 1.1 at 10 to 30, 0.8 above).
+    // mean at 3 to 5 MB, 1.0 at 7 to 30, 0.8 above; fp32 1.4 at 7 to 10, 1.1 at 10 to 30, 0.8 above).  Channel-minor ones of whole
+    // groups of 32 filters, for the same reason: fp16 from 32768 output pixels on (0.73 to 0.99 of the time here in the mean; 40 -> 64, 196
+    // samples of 109 x 75 81 and 192 us), fp32 without a bias from 32 MB on with at most 32 channels on one side (0.87 and 0.94; more 1.07).
+    // And fp16 layers of up to sixteen channels on rows of whole pieces, from 60000 pixels on, whose gradients both have kernels on raw
+    // tiles (6 -> 8, 449 samples of 40 x 40 58 and 107, 9 -> 7, 29 of 160 x 112 64 and 100, 11 -> 4, 4 of 160 x 160 36 and 36).
     if (apart && (a->USE_BIASES != 1 || a->bias)) {
         ConvGeom g;
         if (int rc = conv_geom(a, g, fn, true)) return rc;
@@ -1089,8 +1099,15 @@ static int conv2d_bw(const Args *a, int ns, const char *fn) {
                             (gflop >= 10 || (g.Hk == 3 && g.Wk == 3 && conv_halo_wg_preferred(d)));
         const bool resident = sizeof(T) == 2 && g.hwc && gflop >= 20 && conv_halo_wg_hwc_fits(d, nullptr, nullptr) && conv_halo_wg_hwc_preferred(d);
         const bool scatter = K == g.Ci && (g.sh > 1 || g.sw > 1) && !g.hwc && sizeof(T) * (in_n + out_n) >= (sizeof(T) == 2 ? 7000000 : 30000000);
-        const bool forced = state().gemm_path >= 7;
-        if ((forced || (state().gemm_path == 0 && !own_wg && !resident && !scatter)) && fits_int(in_n) && fits_int(out_n)) {
+        const bool forced = state().gemm_path >= 7, bias = a->USE_BIASES == 1;
+        const double mb = 1e-6 * sizeof(T) * (in_n + out_n);
+        const bool point_steps = is_point(g) && g.hwc && point_bw_behind<T>(g, mb);
+        const bool minor_steps = g.hwc && K == g.Ci && (g.sh > 1 || g.sw > 1) && g.Co % 32 == 0 &&
+                                 (sizeof(T) == 2 ? (long long)ns * P >= 32768 : !bias && mb >= 32 && std::min(g.Ci, g.Co) <= 32);
+        const bool small_steps = sizeof(T) == 2 && !g.hwc && g.Hk == 3 && g.Wk == 3 && g.sh == 1 && g.sw == 1 && g.W % 8 == 0 && g.Ci <= 16 &&
+                                 g.Co <= 16 && (long long)ns * P >= 60000;
+        const bool steps = own_wg || resident || scatter || point_steps || minor_steps || small_steps;
+        if ((forced || (state().gemm_path == 0 && !steps)) && fits_int(in_n) && fits_int(out_n)) {
             Stager sg;
             const T *X = sg.in(reinterpret_cast<const T *>(a->input->data), in_n);
             const T *dY = sg.in(reinterpret_cast<const T *>(a->output->diff), out_n);

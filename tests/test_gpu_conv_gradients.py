@@ -58,3 +58,29 @@ def test_gradients(pkg, gpu, dt, hwc, path, bias, case):
     assert rel(chw(dw), ref_dw) <= TOL[dt]
     if bias:
         assert rel(db, D.sum((0, 2))) <= TOL[dt]
+
+
+@pytest.mark.parametrize("dt,hwc,bias,ns,Ci,Co,H,W,k,s", [
+    ("fp32", 0, 1, 82, 128, 63, 32, 32, 1, 1), ("fp32", 0, 0, 81, 128, 63, 32, 32, 1, 1), ("fp32", 0, 0, 83, 128, 64, 32, 32, 1, 1),  # 64 MB
+    ("fp32", 1, 1, 82, 128, 63, 32, 32, 1, 1), ("fp32", 1, 0, 83, 127, 63, 32, 32, 1, 1),
+    ("fp16", 1, 0, 32, 24, 32, 63, 63, 1, 2), ("fp16", 1, 1, 33, 9, 96, 63, 63, 1, 2), ("fp16", 1, 0, 31, 24, 32, 63, 63, 1, 2),  # 32768 pixels
+    ("fp32", 1, 0, 82, 16, 32, 63, 63, 1, 2), ("fp32", 1, 0, 85, 16, 32, 63, 63, 1, 2), ("fp32", 1, 1, 85, 16, 32, 63, 63, 1, 2),  # 32 MB
+    ("fp16", 0, 0, 15, 9, 7, 64, 64, 3, 1), ("fp16", 0, 1, 15, 16, 16, 64, 64, 3, 1), ("fp16", 0, 1, 14, 16, 16, 64, 64, 3, 1)])  # 60000
+def test_gradients_on_both_sides_of_the_lines_to_single_steps(pkg, gpu, dt, hwc, bias, ns, Ci, Co, H, W, k, s):
+    p, Ho, Wo = k // 2, (H - 1) // s + 1, (W - 1) // s + 1
+    g = torch.Generator(device=DEV).manual_seed(Ci * Co + ns)
+    act = (lambda c, h, w: (ns, h, w, c)) if hwc else (lambda c, h, w: (ns, c, h, w))
+    x, dx, dy = tensor(g, act(Ci, H, W), dt), tensor(g, act(Ci, H, W), dt), tensor(g, act(Co, Ho, Wo), dt)
+    w, dw = (tensor(g, (Co, k, k, Ci) if hwc else (Co, Ci, k, k), dt) for _ in range(2))
+    b, db = (tensor(g, (Co,), dt), tensor(g, (Co,), dt)) if bias else (None, None)
+    a, keep = hp.conv2d_args(pkg, x, dx, w, dw, dy, dy, Ci, H, W, Co, k, k, Ho, Wo, pad=(p, p, p, p), stride=(s, s), hwc=hwc, bias=b, dbias=db)
+    pkg.call("ptl_conv2d_%s_bw_batched" % dt, a, ns)
+    assert gpu.ptl_sync() == 0
+    chw = (lambda t: t.double().permute(0, 3, 1, 2)) if hwc else (lambda t: t.double())
+    cols, D, Wm = F.unfold(chw(x), k, padding=p, stride=s), chw(dy).reshape(ns, Co, -1), chw(w).reshape(Co, -1)
+    assert rel(chw(dw).reshape(Co, -1), D.permute(1, 0, 2).reshape(Co, -1) @ cols.permute(0, 2, 1).reshape(-1, Ci * k * k)) <= TOL[dt]
+    assert rel(chw(dx), F.fold(Wm.t() @ D, (H, W), k, padding=p, stride=s)) <= TOL[dt]
+    if bias:
+        assert rel(db, D.sum((0, 2))) <= TOL[dt]
+    if k == 3:
+        assert gpu.ptl_last_conv_direct() == (ns == 15)
