@@ -87,3 +87,31 @@ def test_infinities(pkg, gpu, dt, ns, n_in, n_out, step):
     db = run_dense(pkg, gpu, ns, n_in, n_out, dy, step)
     assert float(db[1]) == inf and float(db[2]) == -inf and bool(db[3:5].isnan().all())
     assert bool(db[0].isfinite()) and bool(db[5:].isfinite().all())
+
+
+# both gradients in one launch, by whole images and by pixels, on copies, channel-minor in pieces, of one tap, tiles of 32 to 128
+BOTH = [(57, 35, 40, 15, 15, 5, 1, 0, 0), (72, 8, 40, 23, 23, 3, 2, 0, 0), (49, 244, 33, 10, 10, 1, 1, 0, 0), (9, 20, 45, 5, 5, 3, 1, 0, 0),
+        (20, 39, 72, 19, 19, 1, 1, 1, 0), (30, 24, 40, 21, 20, 3, 1, 1, 0), (13, 64, 150, 16, 16, 3, 1, 0, 9), (64, 96, 256, 14, 14, 3, 1, 0, 7),
+        (33, 24, 45, 57, 57, 5, 2, 0, 0), (40, 64, 256, 30, 30, 1, 1, 0, 0)]
+
+
+@pytest.mark.parametrize("ns,Ci,Co,H,W,k,s,hwc,path", BOTH)
+def test_backward_calls_of_convolutions_round_once(pkg, gpu, ns, Ci, Co, H, W, k, s, hwc, path):
+    """Values of both signs, so that the sums are small beside their terms."""
+    p = k // 2
+    Ho, Wo = (H + 2 * p - k) // s + 1, (W + 2 * p - k) // s + 1
+    g = torch.Generator(device=DEV).manual_seed(Ci)
+    act = (lambda c, h, w: (ns, h, w, c)) if hwc else (lambda c, h, w: (ns, c, h, w))
+    x, dy = (torch.rand(sh, generator=g, device=DEV) * 2 - 1 for sh in (act(Ci, H, W), act(Co, Ho, Wo)))
+    wsh = (Co, k, k, Ci) if hwc else (Co, Ci, k, k)
+    w, dw, y, dx, b, db = (torch.zeros(sh, device=DEV) for sh in (wsh, wsh, dy.shape, x.shape, (Co,), (Co,)))
+    a, keep = hp.conv2d_args(pkg, x, dx, w, dw, y, dy, Ci, H, W, Co, k, k, Ho, Wo, pad=(p, p, p, p), stride=(s, s), hwc=hwc, bias=b, dbias=db)
+    gpu.ptl_set_gemm_path(path)
+    try:
+        pkg.call("ptl_conv2d_fp32_bw_batched", a, ns)
+        assert gpu.ptl_sync() == 0
+    finally:
+        gpu.ptl_set_gemm_path(0)
+    ref = (dy.reshape(-1, Co) if hwc else dy.permute(0, 2, 3, 1).reshape(-1, Co)).double().sum(0)
+    # the rounding of a result is 2^-24 of it at most, 0.42 of that in the root mean square over all mantissas
+    assert float((db.double() - ref).norm() / ref.norm()) <= 0.6 * 2.0 ** -24
