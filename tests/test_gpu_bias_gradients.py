@@ -115,3 +115,11 @@ def test_backward_calls_of_convolutions_round_once(pkg, gpu, ns, Ci, Co, H, W, k
     ref = (dy.reshape(-1, Co) if hwc else dy.permute(0, 2, 3, 1).reshape(-1, Co)).double().sum(0)
     # the rounding of a result is 2^-24 of it at most, 0.42 of that in the root mean square over all mantissas
     assert float((db.double() - ref).norm() / ref.norm()) <= 0.6 * 2.0 ** -24
+
+
+@pytest.mark.parametrize("ns,n_in,n_out", [(2, 1, 77), (3, 600, 130), (4, 86, 259), (5, 4100, 65), (7, 177, 646), (8, 144, 1001)])
+def test_few_samples_round_once(pkg, gpu, ns, n_in, n_out):
+    dy = torch.rand((ns, n_out), generator=torch.Generator(device=DEV).manual_seed(n_in), device=DEV) * 2 - 1
+    db = run_dense(pkg, gpu, ns, n_in, n_out, dy, "bw")
+    assert gpu.ptl_last_gemm_form() == 3
+    assert torch.equal(db, dy.double().sum(0).float())
