@@ -1,5 +1,5 @@
-"""fp32 products formed from three bf16 pieces of each value: infinities and values below the pieces' range go through the fp32
-instructions, and the bf16 instructions' rounding (towards minus infinity) does not add up over long contractions."""
+"""fp32 products formed from three bf16 pieces of each value: infinities and values above the pieces' range go through the fp32
+instructions, small ones keep their bits, and the bf16 instructions' rounding (towards minus infinity) does not add up over long contractions."""
 import pytest
 import torch
 
@@ -22,7 +22,7 @@ def test_values_outside_the_range_of_the_pieces(pkg, gpu, what):
     g = torch.Generator(device=DEV).manual_seed(3)
     ns, Ci, Co, P = 32, 270, 300, 333  # (contractions of 19 slabs and of 666: sixteen a workgroup or more take pieces)
     x, dx, dy, w, dw, a, keep = point_layer(pkg, ns, Ci, Co, P, g)
-    if what == "tiny":  # (the third piece of 1e-35 lies below the smallest bf16)
+    if what == "tiny":  # (the third piece of 1e-35 would lie below the smallest bf16)
         x.mul_(1e-35)
         dy[:, 7].mul_(1e-2)
     else:  # (huge: rounds up to infinity as a bf16)
@@ -105,17 +105,17 @@ def test_weight_gradients_in_more_parts(pkg, gpu, ns, Ci, Co, k, stride):
     assert rel(dw, ref) <= 3.4e-7
 
 
-@pytest.mark.parametrize("size", [2.0 ** -99, 2.0 ** -112, 2.0 ** -115, 2.0 ** -120, 2.0 ** -124])
+@pytest.mark.parametrize("size,other", [(-99, 60), (-112, 60), (-115, 60), (-120, 60), (-124, 60), (-130, 60), (-135, 60), (-149, 60), (-60, -60)])
 @pytest.mark.parametrize("few", [0, 1])
-def test_small_values_times_large_ones(pkg, gpu, size, few):
-    """Values whose lower pieces are below the smallest bf16 (2^-133), times ones of 2^60: results of 2^-40 to 2^-60.  few: one
-    such value in a row, zeros beside it."""
+def test_small_values_times_large_ones(pkg, gpu, size, other, few):
+    """Values whose lower pieces, or that themselves, are below the smallest bf16 (2^-133), times ones of 2^60: results of 2^-40 to
+    2^-85; and products that the smaller pieces leave below the smallest fp32 number.  few: one such value in a row, zeros beside it."""
     g = torch.Generator(device=DEV).manual_seed(5)
     ns, Ci, Co, P = 32, 270, 300, 333
     x, dx, dy, w, dw, a, keep = point_layer(pkg, ns, Ci, Co, P, g)
-    dy.mul_(2.0 ** 60)
+    dy.mul_(2.0 ** other)
     for t in (x, w):
-        t.copy_(torch.where(t < 0, t - 1, t + 1) * size)  # (1 to 2 times size, and with the other sign)
+        t.copy_(torch.where(t < 0, t - 1, t + 1) * 2.0 ** (size // 2) * 2.0 ** (size - size // 2))  # (1 to 2 times 2^size, with both signs)
     if few:
         one = x[3, :, 0, 50].clone()
         x.zero_()
