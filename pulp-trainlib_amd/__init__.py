@@ -118,7 +118,7 @@ NORMED_ENTRY_POINTS = ["ptl_conv2d_%s_fw_batched_normed" % dt for dt in ("fp16",
 HEAD_ENTRY_POINTS = ["ptl_pool_linear_loss_%s_batched" % dt for dt in ("fp16", "fp32")]
 
 OTHER_ENTRY_POINTS = ["ptl_init", "ptl_last_error", "ptl_last_status", "ptl_set_stream", "ptl_sync", "ptl_set_gemm_path",
-                      "ptl_last_conv_direct", "ptl_last_gemm_streamed", "ptl_last_conv_resident", "ptl_last_gemm_tile", "ptl_last_gemm_form", "ptl_timer_begin", "ptl_timer_end_ms", "ptl_mm_fp32", "ptl_mm_fp16", "ptl_copy_bytes",
+                      "ptl_last_conv_direct", "ptl_last_gemm_streamed", "ptl_last_conv_resident", "ptl_last_gemm_tile", "ptl_last_gemm_form", "ptl_staging_copies", "ptl_timer_begin", "ptl_timer_end_ms", "ptl_mm_fp32", "ptl_mm_fp16", "ptl_copy_bytes",
                       "ptl_reserve", "ptl_reserved", "ptl_probe_mfma_fp16"]
 
 
@@ -213,6 +213,8 @@ def load():
     lib.ptl_last_gemm_tile.restype = ctypes.c_int
     lib.ptl_last_gemm_form.argtypes = []
     lib.ptl_last_gemm_form.restype = ctypes.c_int
+    lib.ptl_staging_copies.argtypes = []
+    lib.ptl_staging_copies.restype = ctypes.c_longlong
     lib.ptl_sync.argtypes = []
     lib.ptl_sync.restype = ctypes.c_int
     lib.ptl_timer_begin.argtypes = []

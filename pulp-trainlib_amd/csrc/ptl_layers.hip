@@ -1006,11 +1006,7 @@ static int pw_geom(const Args *a, const char *fn) {
 // Weight and input gradient of one call (the batched twin of pulp_conv2d_*_bw_cl): honours skip_wg_grad /
 // skip_in_grad; where both run on the resident-tile kernels they share the blocked copy of the output gradient.
 template <typename T, typename Args>
-static int conv2d_bw(const Args *a, int ns, const char *fn) {
-    if (!a) {
-        set_error("%s: null argument structure", fn);
-        return 1;
-    }
+static int conv2d_bw_routes(const Args *a, int ns, const char *fn) {
     const bool wg = a->skip_wg_grad == 0, ig = a->skip_in_grad == 0;
     bool apart = false;
     if (wg && ig && ns >= 1 && a->input && a->coeff && a->output) {
@@ -1124,10 +1120,18 @@ static int conv2d_bw(const Args *a, int ns, const char *fn) {
             sg.discard();
         }
     }
-    ptl_internal_stage_begin();  // (host tensors: fetched once for both steps)
-    int rc = wg ? conv2d_wg<T>(a, ns, fn) : 0;
-    if (rc == 0 && ig) rc = conv2d_ig<T>(a, ns, fn);
-    return ptl_internal_stage_end(rc);
+    const int rc = wg ? conv2d_wg<T>(a, ns, fn) : 0;
+    return rc == 0 && ig ? conv2d_ig<T>(a, ns, fn) : rc;
+}
+
+template <typename T, typename Args>
+static int conv2d_bw(const Args *a, int ns, const char *fn) {
+    if (!a) {
+        set_error("%s: null argument structure", fn);
+        return 1;
+    }
+    ptl_internal_stage_begin();  // (host tensors: fetched once for both steps, and for a route that was asked before them)
+    return ptl_internal_stage_end(conv2d_bw_routes<T>(a, ns, fn));
 }
 
 template <typename T, typename Args>

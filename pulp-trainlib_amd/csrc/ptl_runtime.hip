@@ -346,6 +346,7 @@ bool Stager::launch_block_copy(bool in) {
     auto flush = [&]() {
         if (c.n == 0) return true;
         hipLaunchKernelGGL(stage_copy_kernel, dim3((c.first[c.n] + 255) / 256), dim3(256), 0, state().stream, c);
+        ++state().staging_copies;
         c.n = 0;
         return hip_ok(hipGetLastError(), "staging launch");
     };
@@ -452,6 +453,7 @@ void *Stager::map(const void *host_or_dev, size_t bytes, bool copy_in, bool copy
                 failed_ = true;
                 return nullptr;
             }
+            ++state().staging_copies;
         } else if (hit->block) {
             memcpy(r.block_->host + (static_cast<char *>(hit->dev) - r.block_->dev), host_or_dev, hit->bytes);
             hit->pending = r.pending_ = true;
@@ -459,6 +461,8 @@ void *Stager::map(const void *host_or_dev, size_t bytes, bool copy_in, bool copy
                            "hipMemcpy(H2D)")) {
             failed_ = true;
             return nullptr;
+        } else {
+            ++state().staging_copies;
         }
         hit->copied_in = true;
     }
@@ -572,6 +576,7 @@ int ptl_last_gemm_streamed(void) { return ptl::state().last_gemm_streamed; }
 int ptl_last_conv_resident(void) { return ptl::state().last_conv_resident; }
 int ptl_last_gemm_tile(void) { return ptl::state().last_gemm_tile; }
 int ptl_last_gemm_form(void) { return ptl::state().last_gemm_form; }
+long long ptl_staging_copies(void) { return ptl::state().staging_copies; }
 
 int ptl_sync(void) {
     if (!ptl::ensure_init()) return 2;

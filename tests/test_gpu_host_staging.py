@@ -170,3 +170,24 @@ def test_large_host_tensors_travel_in_parts(pkg, gpu, n_in, n_out):
         res.append([v if isinstance(v, np.ndarray) else v.cpu().numpy() for v in t])
     for h, d in zip(*res):
         assert np.array_equal(h, d)
+
+
+# (layers that the route of both gradients in one launch takes, and ones that it is asked for and leaves to the two steps: few
+# channels, channel-minor; the last one's tensors are a transfer each)
+@pytest.mark.parametrize("dt,ns,Ci,Co,H,K,s,copies", [("fp16", 4, 24, 48, 29, 1, 1, 2), ("fp32", 2, 9, 8, 12, 3, 1, 2), ("fp16", 4, 3, 48, 29, 1, 1, 2),
+                                                      ("fp16", 4, 4, 93, 15, 3, 2, 2), ("fp16", 4, 3, 64, 181, 1, 1, 3)])
+def test_a_backward_call_fetches_a_host_tensor_once(pkg, gpu, dt, ns, Ci, Co, H, K, s, copies):
+    nd, p = hp.np_dtype(dt), K // 2
+    Ho = hp.conv_out(H, K, p, p, s)
+    x, w, dy = (hp.uniform(31 + i, sh, dtype=nd) for i, sh in enumerate(((ns, H, H, Ci), (Co, K, K, Ci), (ns, Ho, Ho, Co))))
+    res = []
+    for place in (lambda a: a.copy(), lambda a: torch.from_numpy(a).to(DEV)):
+        t = [place(a) for a in (x, np.full_like(x, 3), w, np.full_like(w, 3), np.zeros_like(dy), dy)]
+        a, keep = hp.conv2d_args(pkg, *t, Ci, H, H, Co, K, K, Ho, Ho, (p,) * 4, (s, s), hwc=1)
+        before = gpu.ptl_staging_copies()
+        pkg.call("ptl_conv2d_%s_bw_batched" % dt, a, ns)
+        assert gpu.ptl_sync() == 0
+        assert gpu.ptl_staging_copies() - before == (0 if res else copies)
+        res.append([v if isinstance(v, np.ndarray) else v.cpu().numpy() for v in t])
+    for h, d in zip(*res):
+        assert np.array_equal(h, d)
