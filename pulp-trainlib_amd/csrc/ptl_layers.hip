@@ -297,6 +297,10 @@ static ConvTileDesc forward_desc(const ConvGeom &g, int ns) {
 // group of type, layout, stride and bias, and the better one of each layer would give 0 to 4 % more.  Except fp16 layers of
 // unit stride with few filters over many pixels and a short contraction, where the raw tiles read each input once: 8 ->
 // 16 1 x 1, 14.2 us there and 17.5 here; 64 -> 16 3 x 3, 42 and 49; but 83 -> 16 1 x 1 24 and 16, 132 -> 15 3 x 3 152 and 129.
+// And channel-major fp16 layers of several taps without a bias whose few tiles have a long contraction, which takes its partial
+// sums through memory here: 58 layers of more than 32 filters, 550 terms and up to 30 tiles of 64 x 64 0.88 of the time by
+// the gathering product in the mean, 1.02 at worst (2 samples, 64 -> 152, 13 x 13, 5 x 5 12.6 and 15.2 us; 4, 64 -> 128, 12 x 12,
+// 3 x 3 10.7 and 12.1); above 33 tiles 1.00, below 550 terms 1.10, up to 32 filters 0.99, with a bias 1.04.
 // One gradient alone: by the millions of multiplications of a step, counted by how full its tiles are.  Strides: the
 // other route of the input gradient runs over a zero-stuffed tensor.  A bias gradient is a launch of its own on the other
 // routes.  Both routes were timed on 5000 layers (1 to 128 samples, 3 to 512 channels on 7 to 64 pixels, 1 to 25
@@ -317,8 +321,11 @@ static bool any_pays(const ConvGeom &g, int ns, int steps, bool bias) {
     auto fill = [](double n, int unit) { return n / ((long long)((n + unit - 1) / unit) * unit); };
     const int K = g.Ci * g.Hk * g.Wk;
     const bool strided = g.sh > 1 || g.sw > 1, half = sizeof(T) == 2;
-    if (steps == 1)
-        return !(half && !g.hwc && !strided && g.Co <= 16 && K <= (K == g.Ci ? 40 : 700) && (long long)ns * g.Ho * g.Wo > 100000);
+    if (steps == 1) {
+        const long long pix = (long long)ns * g.Ho * g.Wo, tiles = (g.Co + 63) / 64 * ((pix + 63) / 64);
+        if (half && !g.hwc && !bias && K > g.Ci && K >= 550 && g.Co > 32 && tiles <= 30) return false;
+        return !(half && !g.hwc && !strided && g.Co <= 16 && K <= (K == g.Ci ? 40 : 700) && pix > 100000);
+    }
     double mflop = 2e-6 * ns * g.Co * g.Ho * g.Wo * K * fill(g.Co, 32) * fill(K, 64);
     if (g.hwc) mflop *= fill(g.Ci, VEC);
     if (bias) mflop *= 1.5;

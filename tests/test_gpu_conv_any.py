@@ -70,3 +70,17 @@ def test_convolution(pkg, gpu, dt, hwc, bias, case):
     assert rel(chw(dx), ref_dx) <= TOL[dt]
     if bias:
         assert rel(db, D.sum((0, 2))) <= TOL[dt]
+
+
+# (channel-major fp16 layers without a bias: at 30 tiles of 64 x 64 and 550 terms the gathering product takes them)
+@pytest.mark.parametrize("ns,Ci,Co,H,k,s,p", [(4, 62, 65, 15, 3, 1, 1), (4, 61, 65, 15, 3, 1, 1), (4, 62, 32, 15, 3, 1, 1), (4, 62, 33, 15, 3, 1, 1),
+                                              (3, 64, 160, 25, 3, 1, 1), (2, 40, 130, 25, 5, 2, 2), (1, 512, 156, 5, 5, 2, 2), (8, 62, 256, 11, 3, 1, 1)])
+def test_forward_on_few_tiles(pkg, gpu, ns, Ci, Co, H, k, s, p):
+    Ho = (H + 2 * p - k) // s + 1
+    g = torch.Generator(device=DEV).manual_seed(Ci * Co + H)
+    x, y, w = (tensor(g, sh, "fp16") for sh in ((ns, Ci, H, H), (ns, Co, Ho, Ho), (Co, Ci, k, k)))
+    a, keep = hp.conv2d_args(pkg, x, x, w, w, y, y, Ci, H, H, Co, k, k, Ho, Ho, pad=(p,) * 4, stride=(s, s))
+    pkg.call("ptl_conv2d_fp16_fw_batched", a, ns)
+    assert gpu.ptl_sync() == 0
+    ref = w.double().reshape(Co, -1) @ F.unfold(x.double(), k, padding=p, stride=s)
+    assert rel(y.double().reshape(ns, Co, -1), ref) <= TOL["fp16"]
