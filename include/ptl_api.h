@@ -339,7 +339,7 @@ int ptl_last_gemm_tile(void);
 int ptl_last_gemm_form(void);
 /* Transfers that have been made so far for host tensors: to the device, one for the small tensors that are fetched together and one for
  * each large one; back, one for the small ones. */
-long long ptl_staging_copies(void);
+int ptl_staging_copies(void);
 /* A measurement aid (no counterpart in the reference, not on the training path): the rate, in TFLOP/s, that this
  * board sustains on a loop of nothing but fp16 MFMAs - shape 32: v_mfma_f32_32x32x16_f16, 16: v_mfma_f32_16x16x32_f16 -
  * on random (1) or all-zero (0) operands, with one or two waves per SIMD on every compute unit, `iters` x 262144 flops

@@ -214,7 +214,7 @@ def load():
     lib.ptl_last_gemm_form.argtypes = []
     lib.ptl_last_gemm_form.restype = ctypes.c_int
     lib.ptl_staging_copies.argtypes = []
-    lib.ptl_staging_copies.restype = ctypes.c_longlong
+    lib.ptl_staging_copies.restype = ctypes.c_int
     lib.ptl_sync.argtypes = []
     lib.ptl_sync.restype = ctypes.c_int
     lib.ptl_timer_begin.argtypes = []

@@ -576,7 +576,7 @@ int ptl_last_gemm_streamed(void) { return ptl::state().last_gemm_streamed; }
 int ptl_last_conv_resident(void) { return ptl::state().last_conv_resident; }
 int ptl_last_gemm_tile(void) { return ptl::state().last_gemm_tile; }
 int ptl_last_gemm_form(void) { return ptl::state().last_gemm_form; }
-long long ptl_staging_copies(void) { return ptl::state().staging_copies; }
+int ptl_staging_copies(void) { return ptl::state().staging_copies; }
 
 int ptl_sync(void) {
     if (!ptl::ensure_init()) return 2;
