@@ -187,28 +187,53 @@ template <typename T>
 int mm_dispatch(const T *A, const T *B, T *C, int N, int M, int K, int trans_B, const T *bias = nullptr);
 
 #ifdef __HIP_DEVICE_COMPILE__
-// Asks for all lines of a kernel's arguments at its start.  They lie in memory, and the compiler loads each where it is
-// needed: a line that is asked for behind an index or a branch that came from another line is one more trip before the first
-// load of data. (Patch rows and transpositions; in row dots, batch norms, convolutions and sums
-// it gave nothing that could be measured.)
+// Asks for lines of a kernel's arguments together.  They lie in memory and the compiler loads each where it is needed: a line
+// that is asked for behind an index or a branch that came from another line is one more trip, of about 1000 clocks, before
+// the first load of data.  Worth it where there are many lines or trips: products of any size, whose arguments are 300 to 4000
+// bytes (9 samples, 22 -> 8 channels, 13 x 13, 3 x 3 in fp16, forward and backward 23.1 -> 20.8 us; 200 drawn passes 1.02 in the mean,
+// convolutions 1.04), patch rows, transpositions.  In row dots, batch norms, tiled convolutions and sums it gave nothing
+// that could be measured, and lines that a workgroup does not need cost (all five products' for a pair: 24.2 -> 24.8 us).
 template <typename... A>
 constexpr int args_bytes() {
     int n = 0;
     ((n = (n + (int)alignof(A) - 1) / (int)alignof(A) * (int)alignof(A) + (int)sizeof(A)), ...);
     return n;
 }
+// B0 bytes from a0 on, B1 from a1 and B2 from a2: whole words.
+template <int B0, int B1 = 0, int B2 = 0>
+__device__ __forceinline__ void fetch_args_at(int a0, int a1 = 0, int a2 = 0) {
+    typedef const char __attribute__((address_space(4))) *Bytes;
+    const Bytes p = (Bytes)__builtin_amdgcn_kernarg_segment_ptr();
+    unsigned word;
+    asm volatile(
+        ".macro ptl_fetch base, lines, last\n"
+        ".set ptl_arg, 0\n"
+        ".rept \\lines\n"
+        "s_load_dword %0, \\base, ptl_arg\n"
+        ".set ptl_arg, ptl_arg + 64\n"
+        ".endr\n"
+        "s_load_dword %0, \\base, \\last\n"
+        ".endm\n"
+        "ptl_fetch %1, %c4, %c7\n"
+        ".if %c5\n"
+        "ptl_fetch %2, %c5, %c8\n"
+        ".endif\n"
+        ".if %c6\n"
+        "ptl_fetch %3, %c6, %c9\n"
+        ".endif\n"
+        ".purgem ptl_fetch\n"
+        "s_waitcnt lgkmcnt(0)"
+        : "=&s"(word)
+        : "s"(p + a0), "s"(p + a1), "s"(p + a2), "i"((B0 + 63) / 64), "i"((B1 + 63) / 64), "i"((B2 + 63) / 64), "i"(B0 - 4), "i"(B1 - 4), "i"(B2 - 4)
+        : "memory");
+}
 template <typename... A>
 __device__ __forceinline__ void fetch_args(const A &...) {  // all arguments, in their order
-    typedef const unsigned __attribute__((address_space(4))) *Words;
-    const Words p = (Words)__builtin_amdgcn_kernarg_segment_ptr();
-    constexpr int LINES = (args_bytes<A...>() + 63) / 64;
-#pragma unroll
-    for (int l = 0; l < LINES; l += 8) {
-        auto word = [&](int i) { return p[(l + i < LINES ? l + i : LINES - 1) * 16]; };
-        asm volatile("" ::"s"(word(0)), "s"(word(1)), "s"(word(2)), "s"(word(3)), "s"(word(4)), "s"(word(5)), "s"(word(6)), "s"(word(7)));
-    }
+    fetch_args_at<args_bytes<A...>()>(0);
 }
 #else
+template <int, int = 0, int = 0>
+__device__ inline void fetch_args_at(int, int = 0, int = 0) {}
 template <typename... A>
 __device__ inline void fetch_args(const A &...) {}
 #endif

@@ -87,20 +87,20 @@ struct RagProd {
 
 constexpr int RAG_MAX = 5;
 struct RagArgs {
-    RagProd p[RAG_MAX];
     int first[RAG_MAX + 1];  // first workgroup of each product
     int count;
     int shape;  // 32, 64: that tile, whatever it costs (sums in the same order at every size); 0: the cheapest
     // of the first product of (KC, RC) before (KC, KC) only: up to three runs of k lie anywhere, run r + 1 hop_a[r],
     // hop_b[r] bytes behind run r (its run_b is not used)
     long long hop_a[2], hop_b[2];
+    RagProd p[RAG_MAX];
 };
 
 struct RagSums {  // the products whose contraction was split
-    RagProd p[5];
     int first[6];
     int count;
     int sums;  // the one whose row sums are wanted, or -1
+    RagProd p[5];
 };
 
 // The products in one launch (plus one for their partial sums where the contraction is split).  The first product has
@@ -129,14 +129,14 @@ struct RagTurn {
 constexpr int RAG_CONV_MAX = 4;
 template <int N>
 struct RagConvOf {
-    RagProd p[N];
     int first[N + 1];
     int count;
+    int relays, relay_first[RAG_CONV_MAX + 1];
+    RagProd p[N];
     RagGeo geo[N];          // of each product's patch matrix
     RagGeo geo_a;           // of the other operand where it is gathered too (one product): a gradient (XR), filters (GK, GK)
     const void *relay_src;  // blocks behind the last product re-lay filters for a later product
     RagRelay relay[RAG_CONV_MAX];
-    int relays, relay_first[RAG_CONV_MAX + 1];
 };
 typedef RagConvOf<RAG_CONV_MAX> RagConvArgs;
 // The tiles and slabs per workgroup that ragged_conv() would choose for the products (of which sizes and runs count), and the clocks of
