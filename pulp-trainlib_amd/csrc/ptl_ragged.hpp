@@ -31,8 +31,9 @@ enum RagMode : int { RAG_KC = 0, RAG_RC = 1, RAG_GK = 2, RAG_GR = 3, RAG_XK = 4,
 struct RagOp {
     const char *p;     // first element (XK, XR: see RagGeo)
     int rows;          // extent along the output (GR: taps x pieces x VEC)
-    unsigned row_b;    // KC: bytes from row to row
+    unsigned row_b;    // KC: bytes from row to row; RC with `pad`: rows in all
     unsigned k_b;      // RC: bytes from k to k
+    RagDiv pad;        // RC, d > 0: the outer digits follow each other, each filled up to so many rows (rag_row_up)
     long long run_b;   // bytes from one run of k to the next (KC, RC)
     long long outer_b; // RC: bytes between the outer digits of the rows
 };
