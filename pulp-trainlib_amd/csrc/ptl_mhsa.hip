@@ -16,6 +16,8 @@
 // addresses.
 #include <float.h>
 
+#include <type_traits>
+
 #include "ptl_api.h"
 #include "ptl_gemm_async.hpp"
 #include "ptl_gemm_async.inc"
@@ -40,6 +42,12 @@ __device__ inline float fastexp_gist(float x) {
     x = __fadd_rn(__fmul_rn(12102203.17133801f, x), 1064986823.010288f);
     if (x < 8388608.f || x > 2139095040.f) x = (x < 8388608.f) ? 0.0f : 2139095040.f;
     return __builtin_bit_cast(float, (uint32_t)x);
+}
+
+// The same for x <= 0 or NaN, which have no upper end to be kept from.
+__device__ inline float fastexp_below(float x) {
+    x = __fadd_rn(__fmul_rn(12102203.17133801f, x), 1064986823.010288f);
+    return x < 8388608.f ? 0.f : __builtin_bit_cast(float, (uint32_t)x);
 }
 
 // 1/sqrt by the magic-constant estimate and one Newton step (q_rsqrt,
@@ -459,6 +467,7 @@ struct AttnArgs {
     const float *zero;       // 256 zero bytes: source of elements that do not exist
     int L, H, heads, F, LP, ns;
     float scale;
+    RagDiv d_tiles, d_heads;  // of the kernels up to SQ_L tokens
 };
 
 // Forward: o0 = probabilities, o1 = attention_map.  grid (query tiles, heads, samples).
@@ -627,11 +636,14 @@ __global__ __launch_bounds__(ATT_NT) void attn_bw_key_kernel(AttnArgs a) {
 
 // ---------------------------------------------------------------------------------------------------------
 // Sequences of at most 256 tokens and heads of at most 64 (HB = 1: 32): the score tile of 32 queries and the one operand
-// that a product needs along its other axis are in LDS, everything else goes from global memory to the matrix cores'
-// registers (lanes along the tokens: whole lines), since no other wave of the workgroup needs it.  78 KB for 197 tokens,
-// so that two workgroups share a CU and one's loads hide behind the other's products; with all three operands resident
-// (150 KB, one workgroup of 16 waves) the phases followed one another: 37 / 37 / 41 us for 32 x 3 heads of 64 and 197
-// tokens, 29 / 28 / 30 this way, of which the products take 7 / 9 / 7 at the matrix rate.
+// that a product needs along its other axis are in LDS (the panel): 78 KB for 197 tokens, so that two workgroups share a CU
+// and one's loads hide behind the other's products.  32 x 3 heads of 64 and 197 tokens: 37 / 37 / 41 us with all three
+// operands resident (150 KB, one workgroup of 16 waves), 30 / 28 / 30 with two workgroups, now 25.7 / 26.0 / 24.6, of which the
+// products take 7 / 9 / 7 at the matrix rate.  A workgroup of the forward kernel then took 28 k clocks: 12 until its operands
+// were there and multiplied (a CU takes a vector load of 64 lanes every 10 to 20 clocks, whatever its width), 5 of softmax, 4 of
+// the value mix, 2 until that was stored.  So what is the same in all lanes is worked out in scalar registers, a wave's four rows
+// are reduced side by side, and a head whose [H][L] block starts on 16 bytes and has whole pieces of 16 (LINE) comes in such
+// pieces, 50 loads instead of 64 rows of unaligned ones (or of 448 loads of single elements for the scores).
 constexpr int SQ_NW = 8;           // waves
 constexpr int SQ_NT = SQ_NW * 64;  // threads
 constexpr int SQ_RPW = 32 / SQ_NW; // score rows per wave
@@ -645,56 +657,145 @@ constexpr size_t sq_lds(int L, bool key) {
     return (tiles > parked ? tiles : parked) * sizeof(float);
 }
 
+static_assert(SQ_RPW == 4 && SQ_L == 256, "the softmax's registers");
+
 // Workgroups go to the eight XCDs in turn, each with an L2 of its own: all tiles of a head take ids of the same XCD, so that
 // its operands come from memory once and not once per tile.  False: no head for this workgroup.
 struct SqPlace {
     int tile, h, b, part;
 };
-__device__ inline bool sq_place(const AttnArgs &a, int parts, SqPlace &p) {
-    const unsigned tiles = (unsigned)(a.L + 31) / 32u * (unsigned)parts, j = blockIdx.x >> 3, group = j / tiles, t = j - group * tiles;
+template <int PARTS>
+__device__ inline bool sq_place(const AttnArgs &a, SqPlace &p) {
+    const unsigned j = blockIdx.x >> 3, group = rag_quot(j, a.d_tiles), t = j - group * a.d_tiles.d;
     const unsigned head = group * 8u + (blockIdx.x & 7u);
     if (head >= (unsigned)(a.heads * a.ns)) return false;
-    p.b = (int)(head / (unsigned)a.heads);
-    p.h = (int)(head - (unsigned)p.b * a.heads);
-    p.tile = (int)(t / (unsigned)parts);
-    p.part = (int)(t % (unsigned)parts);
+    p.b = (int)rag_quot(head, a.d_heads);
+    p.h = (int)(head - (unsigned)p.b * a.d_heads.d);
+    p.tile = (int)(t / (unsigned)PARTS);
+    p.part = (int)(t % (unsigned)PARTS);
     return true;
 }
 
-// S[r][c] = scale * sum_d R[d][r0 + r] * C[d][c] for c < L, zero up to the next group of eight; R and C are [H][L] in
-// global memory.  One block of 32 columns per wave.
-// then(): what is asked for behind the operands.
-template <int HB, typename Then>
-__device__ inline void sq_scores(const float *__restrict__ R, const float *__restrict__ C, int L, int H, int r0, float scale,
-                                 float *S, int wave, int l32, int half, Then then) {
-    constexpr int STEPS = 16 * HB;
-    const int pitch = sq_pitch(L), blocks = (L + 31) >> 5;
-    const unsigned r = (unsigned)min(r0 + l32, L - 1);
-    if (wave >= blocks) then();
-    static_assert(SQ_L / 32 <= SQ_NW, "a block per wave");
-    if (wave < blocks) {
-        const int c = wave * 32 + l32;
-        const unsigned cc = (unsigned)min(c, L - 1);
-        mh_f32x16 acc = {0};
-        float af[STEPS], bf[STEPS];
+// The element `off` bytes behind g, which is the same in all lanes: the load takes it from scalar registers.
+__device__ inline float sq_load(const float *g, unsigned off) { return *reinterpret_cast<const float *>(reinterpret_cast<const char *>(g) + off); }
+__device__ inline void sq_put(float *g, unsigned off, float v) { *reinterpret_cast<float *>(reinterpret_cast<char *>(g) + off) = v; }
+
+// wave_max and wave_sum of a wave's four rows side by side: one instruction a step and row, its wait states filled by the other
+// rows (one after the other, with what the compiler adds for signalling NaNs, 110 more instructions a wave and kernel).
+#define SQ_STEP(op, how) op " %0, %0, %0 " how "\n" op " %1, %1, %1 " how "\n" op " %2, %2, %2 " how "\n" op " %3, %3, %3 " how "\n"
+#define SQ_ROWS(op)                                                                                                            \
+    "s_nop 1\n" SQ_STEP(op, "row_shr:1 row_mask:0xf bank_mask:0xf") SQ_STEP(op, "row_shr:2 row_mask:0xf bank_mask:0xf")         \
+        SQ_STEP(op, "row_shr:4 row_mask:0xf bank_mask:0xf") SQ_STEP(op, "row_shr:8 row_mask:0xf bank_mask:0xf")                 \
+            SQ_STEP(op, "row_bcast:15 row_mask:0xa bank_mask:0xf") SQ_STEP(op, "row_bcast:31 row_mask:0xc bank_mask:0xf") "s_nop 1"
+__device__ inline void sq_max(float (&v)[SQ_RPW]) {
+    asm("" SQ_ROWS("v_max_f32_dpp") : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]), "+v"(v[3]));
 #pragma unroll
-        for (int s = 0; s < STEPS; ++s) {
-            const unsigned row = (unsigned)(min(2 * s + half, H - 1) * L);
-            af[s] = R[row + r];
-            bf[s] = C[row + cc];
-        }
-        __builtin_amdgcn_sched_barrier(0);  // (all of them in flight before the first is waited for)
-        then();
+    for (int i = 0; i < SQ_RPW; ++i) v[i] = last_lane(v[i]);
+}
+__device__ inline void sq_sum(float (&v)[SQ_RPW]) {
+    asm("" SQ_ROWS("v_add_f32_dpp") : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]), "+v"(v[3]));
 #pragma unroll
-        for (int s = 0; s < STEPS; ++s) {
-            const bool in = 2 * s + half < H;  // (beyond the head: zeros)
-            acc = __builtin_amdgcn_mfma_f32_32x32x2f32(in ? af[s] : 0.f, in ? bf[s] : 0.f, acc, 0, 0, 0);
-        }
-        if (c < pitch - 4) {
-#pragma unroll
-            for (int v = 0; v < 16; ++v) S[(8 * (v / 4) + 4 * half + (v % 4)) * pitch + c] = c < L ? acc[v] * scale : 0.f;
-        }
+    for (int i = 0; i < SQ_RPW; ++i) v[i] = last_lane(v[i]);
+}
+
+// Rows of V ([H][L]) on their way into the panel: complete once they have been waited for and the edge has been stored, and
+// behind a barrier.  LINE: as they lie in memory, a row of L floats behind the other and nothing beyond the last; otherwise at
+// sq_pitch(L) with zeros beyond L and H.
+template <int HB, bool LINE>
+__device__ inline TileEdge sq_fetch(const float *g, int L, int H, float *lds, const float *zero, int tid, int wave, int lane) {
+    if (LINE) {
+        const int pieces = (H * L) >> 2;  // (in [0, 4096])
+        const unsigned to = (unsigned)(uintptr_t)(lds_char *)lds;
+        for (int j = wave; j * 64 < pieces; j += SQ_NW)
+            if (j * 64 + lane < pieces) lds_dma<16>(g + (j * 64 + lane) * 4, to + (unsigned)j * 1024u);
+        return TileEdge{make_float4(0.f, 0.f, 0.f, 0.f), nullptr};
     }
+    const int cols = (L + 7) / 8 * 8, col = lane * 4;
+    const unsigned to = (unsigned)(uintptr_t)(lds_char *)lds;
+    for (int d = wave; d < 32 * HB; d += SQ_NW) {
+        const bool full = d < H && col + 4 <= L;
+        if (col < cols && (full || d >= H || col >= L)) lds_dma<16>(full ? g + d * L + col : zero, to + (unsigned)(d * sq_pitch(L)) * 4u);
+    }
+    return tile_edge_load(g, L, 32 * HB, cols, H, L, lds, sq_pitch(L), tid);
+}
+
+// S[r][c] = scale * sum_d R[d][r0 + r] * C[d][c] for c < L, zero up to the next group of eight; R and C are [H][L] in
+// global memory.  One block of 32 columns per wave.  then(): asks for what the panel holds afterwards; ahead(): for what is
+// needed behind the scores.
+// LINE: C comes through the panel and R, 32 columns of it, once through LDS; what follows C there arrives during the softmax.
+// Otherwise every wave takes both from global memory into registers, which waits for one trip to memory less: forward, us,
+// through the panel and straight, 32 x 3 heads of 64 and 197 tokens (LINE) 25.7 and 26.9, 8 x 6 of 32 and 250 (LINE) 13.1 and 13.6,
+// 14 x 3 of 64 and 256 22.6 and 21.6, 20 x 4 of 64 and 160 16.6 and 14.6.
+template <int HB, bool LINE, typename Then, typename Ahead>
+__device__ inline void sq_scores(const float *R, const float *C, int L, int H, int r0, float scale, float *S, float *panel, const float *zero,
+                                 int tid, int wave, int lane, Then then, Ahead ahead) {
+    constexpr int STEPS = 16 * HB, MINE = STEPS / SQ_NW;
+    const int l32 = lane & 31, half = lane >> 5;
+    const int pitch = sq_pitch(L), blocks = (L + 31) >> 5;
+    static_assert(SQ_L / 32 <= SQ_NW, "a block per wave");
+    const int c = wave * 32 + l32;
+    const unsigned r = (unsigned)min(r0 + l32, L - 1) * 4u, cc = (unsigned)min(c, L - 1) * 4u, next = half ? (unsigned)L * 4u : 0u;
+    auto store = [&](const mh_f32x16 &acc) {
+        if (c >= pitch - 4) return;
+#pragma unroll
+        for (int v = 0; v < 16; ++v) S[(8 * (v / 4) + 4 * half + (v % 4)) * pitch + c] = c < L ? acc[v] * scale : 0.f;
+    };
+    mh_f32x16 acc = {0};
+    if (LINE) {
+        float *Rs = pitch >= 32 * HB ? S : panel + 32 * HB * pitch;
+        float mine[MINE];
+#pragma unroll
+        for (int s = 0; s < MINE; ++s) {
+            const int d = 2 * (wave + SQ_NW * s);
+            mine[s] = sq_load(R + min(d, H - 1) * L, r + (d + 1 < H ? next : 0u));
+        }
+        sq_fetch<HB, LINE>(C, L, H, panel, zero, tid, wave, lane);
+#pragma unroll
+        for (int s = 0; s < MINE; ++s) Rs[(2 * (wave + SQ_NW * s) + half) * 32 + l32] = mine[s];
+        wait_vmcnt<0>();
+        __syncthreads();
+        ahead();
+        auto form = [&](auto whole) {  // whole: H == 32 HB
+            const float *a = Rs + half * 32 + l32, *b = panel + half * L + min(c, L - 1);
+#pragma unroll
+            for (int s = 0; s < STEPS; ++s) {
+                const bool in = whole.value || 2 * s + half < H;  // (beyond the head: zeros)
+                const float av = a[s * 64], bv = b[2 * s * L];
+                acc = __builtin_amdgcn_mfma_f32_32x32x2f32(in ? av : 0.f, in ? bv : 0.f, acc, 0, 0, 0);
+            }
+        };
+        if (wave < blocks) {
+            if (H == 32 * HB) form(std::true_type{});
+            else form(std::false_type{});
+        }
+        __syncthreads();  // (S takes the place of R, the next panel that of C)
+        then();
+        if (wave < blocks) store(acc);
+    } else {
+        auto form = [&](auto whole) {
+            float af[STEPS], bf[STEPS];
+#pragma unroll
+            for (int s = 0; s < STEPS; ++s) {
+                const int d = whole.value ? 2 * s : min(2 * s, H - 1);
+                const unsigned hop = whole.value || 2 * s + 1 < H ? next : 0u;
+                af[s] = sq_load(R + d * L, r + hop);
+                bf[s] = sq_load(C + d * L, cc + hop);
+            }
+            __builtin_amdgcn_sched_barrier(0);  // (all of them in flight before the first is waited for)
+            then();
+#pragma unroll
+            for (int s = 0; s < STEPS; ++s) {
+                const bool in = whole.value || 2 * s + half < H;
+                acc = __builtin_amdgcn_mfma_f32_32x32x2f32(in ? af[s] : 0.f, in ? bf[s] : 0.f, acc, 0, 0, 0);
+            }
+            store(acc);
+        };
+        if (wave >= blocks) then();
+        else if (H == 32 * HB) form(std::true_type{});
+        else form(std::false_type{});
+        ahead();
+    }
+    __syncthreads();
 }
 
 // Parked partial tiles of the contraction ranges -> out[d][x0 + x] (d < H, x0 + x < L).
@@ -714,8 +815,23 @@ __device__ inline void sq_store(const mh_f32x16 &acc, float *red, int L, int H, 
     }
 }
 
+// V[row][k4 .. k4 + 3] of the panel, zero beyond L.
+template <bool LINE>
+__device__ inline float4 sq_frag(const float *Vs, int row, int k4, int L, int pitch) {
+    if (!LINE) return *reinterpret_cast<const float4 *>(Vs + row * pitch + k4);
+    const float *v = Vs + row * L + k4;
+    float4 f = make_float4(v[0], v[1], v[2], v[3]);
+    if (k4 + 4 > L) {
+        f.x = k4 < L ? f.x : 0.f;
+        f.y = k4 + 1 < L ? f.y : 0.f;
+        f.z = k4 + 2 < L ? f.z : 0.f;
+        f.w = 0.f;
+    }
+    return f;
+}
+
 // out[d][r0 + r] = sum_c V[d][c] * S[r][c]: V and S in LDS, both zero beyond L.  Waves: (block of 32 d) x (range of c).
-template <int HB>
+template <int HB, bool LINE>
 __device__ inline void sq_mix(const float *Vs, const float *S, int L, int H, int r0, float *__restrict__ out, float *red, int tid,
                               int wave, int l32, int half) {
     constexpr int KS = SQ_NW / HB;
@@ -724,90 +840,81 @@ __device__ inline void sq_mix(const float *Vs, const float *S, int L, int H, int
     mh_f32x16 acc = {0};
     for (int g = ks * per; g < end; ++g) {
         const int k4 = g * 8 + half * 4;
-        mfma4(acc, *reinterpret_cast<const float4 *>(Vs + (db * 32 + l32) * pitch + k4),
-              *reinterpret_cast<const float4 *>(S + l32 * pitch + k4));
+        mfma4(acc, sq_frag<LINE>(Vs, db * 32 + l32, k4, L, pitch), *reinterpret_cast<const float4 *>(S + l32 * pitch + k4));
     }
     sq_store<HB>(acc, red, L, H, r0, out, tid, wave, l32, half);
 }
 
-// Rows of V ([H][L], zeros beyond either) on their way into LDS; complete after sq_arrived() and a barrier.
-template <int HB>
-__device__ inline TileEdge sq_fetch(const float *g, int L, int H, float *lds, const float *zero, int tid, int wave, int lane) {
-    const int cols = (L + 7) / 8 * 8;
-    tile_dma<SQ_NW>(g, L, 32 * HB, cols, H, L, lds, sq_pitch(L), zero, wave, lane);
-    return tile_edge_load(g, L, 32 * HB, cols, H, L, lds, sq_pitch(L), tid);
-}
-
-template <int HB>
+template <int HB, bool LINE>
 __global__ __launch_bounds__(SQ_NT, 4) void attn_fw_res_kernel(AttnArgs a) {
     extern __shared__ __attribute__((aligned(16))) float att_lds[];
+    fetch_args(a);
     SqPlace at;
-    if (!sq_place(a, 1, at)) return;
+    if (!sq_place<1>(a, at)) return;
     const int r0 = at.tile * 32, h = at.h, b = at.b, L = a.L, pitch = sq_pitch(L);
     float *S = att_lds, *Vs = S + 32 * pitch;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int l32 = lane & 31, half = lane >> 5;
     const size_t hoff = ((size_t)b * a.F + (size_t)h * a.H) * L;
     TileEdge edge;
-    sq_scores<HB>(a.q + hoff, a.k + hoff, L, a.H, r0, a.scale, S, wave, l32, half,
-                  [&] { edge = sq_fetch<HB>(a.v + hoff, L, a.H, Vs, a.zero, tid, wave, lane); });
-    tile_edge_store(edge);
-    wait_vmcnt<0>();
-    __syncthreads();
+    sq_scores<HB, LINE>(a.q + hoff, a.k + hoff, L, a.H, r0, a.scale, S, Vs, a.zero, tid, wave, lane,
+                        [&] { edge = sq_fetch<HB, LINE>(a.v + hoff, L, a.H, Vs, a.zero, tid, wave, lane); }, [] {});
     // softmax of this wave's rows over the keys (lib/sources/pulp_act_fp32.c:187-225): max, approximate
     // exponential of the difference, sum, division; the rows' reductions run side by side
     float *P = a.o0 + ((size_t)b * a.heads + h) * L * L;
-    float sv[SQ_RPW][4], mx[SQ_RPW], sum[SQ_RPW];
+    const int first = wave * SQ_RPW;
+    const bool live = r0 + first < L;
+    float *rows = S + first * pitch + lane;
+    float sv[SQ_RPW][4], mx[SQ_RPW], sum[SQ_RPW] = {};
+    if (live) {
 #pragma unroll
-    for (int i = 0; i < SQ_RPW; ++i) {
-        const float *srow = S + (wave * SQ_RPW + i) * pitch;
-        mx[i] = -FLT_MAX;
+        for (int i = 0; i < SQ_RPW; ++i) mx[i] = -FLT_MAX;
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const int c = lane + 64 * j;
-            sv[i][j] = c < L ? srow[c] : -FLT_MAX;
-            mx[i] = fmaxf(mx[i], sv[i][j]);
-        }
-    }
+        for (int j = 0; j < 4; ++j)
+            if (lane + 64 * j < L) {
 #pragma unroll
-    for (int i = 0; i < SQ_RPW; ++i) mx[i] = wave_max(mx[i]);
-#pragma unroll
-    for (int i = 0; i < SQ_RPW; ++i) {
-        sum[i] = 0.f;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const int c = lane + 64 * j;
-            sv[i][j] = c < L ? fastexp_gist(sv[i][j] - mx[i]) : 0.f;
-            sum[i] += sv[i][j];
-        }
-    }
-#pragma unroll
-    for (int i = 0; i < SQ_RPW; ++i) sum[i] = wave_sum(sum[i]);
-#pragma unroll
-    for (int i = 0; i < SQ_RPW; ++i) {
-        const int row = wave * SQ_RPW + i;
-        float *srow = S + row * pitch;
-        const bool live = r0 + row < L;
-        const float inv = 1.0f / sum[i];  // one division per row; the products differ from quotients by an ulp at most
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const int c = lane + 64 * j;
-            if (c < L) {
-                const float pv = sv[i][j] * inv;
-                srow[c] = pv;
-                if (live) P[(size_t)(r0 + row) * L + c] = pv;
+                for (int i = 0; i < SQ_RPW; ++i) mx[i] = fmaxf(mx[i], sv[i][j] = rows[i * pitch + 64 * j]);
             }
-        }
+        sq_max(mx);
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+            if (lane + 64 * j < L) {
+#pragma unroll
+                for (int i = 0; i < SQ_RPW; ++i) sum[i] += sv[i][j] = fastexp_below(sv[i][j] - mx[i]);
+            }
+        sq_sum(sum);
+        // (one division for the four rows, in four lanes; the products differ from quotients by an ulp at most)
+        float inv = sum[0];
+#pragma unroll
+        for (int i = 1; i < SQ_RPW; ++i) inv = lane == i ? sum[i] : inv;
+        inv = 1.0f / inv;
+#pragma unroll
+        for (int i = 0; i < SQ_RPW; ++i) sum[i] = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, inv), i));
+    }
+    tile_edge_store(edge);
+    wait_vmcnt<0>();
+    if (live) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+            if (lane + 64 * j < L) {
+#pragma unroll
+                for (int i = 0; i < SQ_RPW; ++i) {
+                    sv[i][j] *= sum[i];
+                    rows[i * pitch + 64 * j] = sv[i][j];
+                    if (r0 + first + i < L) sq_put(P + (r0 + first + i) * L + 64 * j, (unsigned)lane * 4u, sv[i][j]);
+                }
+            }
     }
     __syncthreads();
-    sq_mix<HB>(Vs, S, L, a.H, r0, a.o1 + hoff, att_lds, tid, wave, l32, half);
+    sq_mix<HB, LINE>(Vs, S, L, a.H, r0, a.o1 + hoff, att_lds, tid, wave, l32, half);
 }
 
-template <int HB>
+template <int HB, bool LINE>
 __global__ __launch_bounds__(SQ_NT, 4) void attn_bw_query_res_kernel(AttnArgs a) {
     extern __shared__ __attribute__((aligned(16))) float att_lds[];
+    fetch_args(a);
     SqPlace at;
-    if (!sq_place(a, 1, at)) return;
+    if (!sq_place<1>(a, at)) return;
     const int r0 = at.tile * 32, h = at.h, b = at.b, L = a.L, pitch = sq_pitch(L);
     float *S = att_lds, *Ks = S + 32 * pitch;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -816,112 +923,137 @@ __global__ __launch_bounds__(SQ_NT, 4) void attn_bw_query_res_kernel(AttnArgs a)
     const size_t poff = ((size_t)b * a.heads + h) * L * L;
     // dP[query][key] = sum_d dA[d][query] v[d][key]   (lib/sources/pulp_mhsa_fp32.c:958-1060)
     TileEdge edge;
+    const int first = wave * SQ_RPW;
+    const bool live = r0 + first < L;
     float pr[SQ_RPW][4];  // this wave's probability rows
-    sq_scores<HB>(a.da + hoff, a.v + hoff, L, a.H, r0, 1.0f, S, wave, l32, half, [&] {
-        edge = sq_fetch<HB>(a.k + hoff, L, a.H, Ks, a.zero, tid, wave, lane);
-    });
+    sq_scores<HB, LINE>(
+        a.da + hoff, a.v + hoff, L, a.H, r0, 1.0f, S, Ks, a.zero, tid, wave, lane,
+        [&] {
+            if (LINE) {  // (they are waited for here, so that nothing waits for the panel before it is needed)
 #pragma unroll
-    for (int i = 0; i < SQ_RPW; ++i)
+                for (int i = 0; i < SQ_RPW; ++i) asm volatile("" : "+v"(pr[i][0]), "+v"(pr[i][1]), "+v"(pr[i][2]), "+v"(pr[i][3]));
+            }
+            edge = sq_fetch<HB, LINE>(a.k + hoff, L, a.H, Ks, a.zero, tid, wave, lane);
+        },
+        [&] {
+            if (!live) return;
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const int row = r0 + wave * SQ_RPW + i, c = lane + 64 * j;
-            pr[i][j] = (row < L && c < L) ? a.p[poff + (size_t)row * L + c] : 0.f;
-        }
+            for (int j = 0; j < 4; ++j)
+                if (lane + 64 * j < L) {
+#pragma unroll
+                    for (int i = 0; i < SQ_RPW; ++i) pr[i][j] = sq_load(a.p + poff + min(r0 + first + i, L - 1) * L + 64 * j, (unsigned)lane * 4u);
+                }
+        });
+    // softmax backward (lib/sources/pulp_act_fp32.c:335-390) and the scaling (:1176-1183)
+    float *rows = S + first * pitch + lane;
+    float gv[SQ_RPW][4], sum[SQ_RPW] = {};
+    if (live) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+            if (lane + 64 * j < L) {
+#pragma unroll
+                for (int i = 0; i < SQ_RPW; ++i) sum[i] += (gv[i][j] = rows[i * pitch + 64 * j]) * pr[i][j];
+            }
+        sq_sum(sum);
+    }
     tile_edge_store(edge);
     wait_vmcnt<0>();
-    __syncthreads();
-    // softmax backward (lib/sources/pulp_act_fp32.c:335-390) and the scaling (:1176-1183)
-    float gv[SQ_RPW][4], sum[SQ_RPW];
+    if (live) {
 #pragma unroll
-    for (int i = 0; i < SQ_RPW; ++i) {
-        const float *srow = S + (wave * SQ_RPW + i) * pitch;
-        sum[i] = 0.f;
+        for (int j = 0; j < 4; ++j)
+            if (lane + 64 * j < L) {
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const int c = lane + 64 * j;
-            gv[i][j] = c < L ? srow[c] : 0.f;
-            sum[i] += gv[i][j] * pr[i][j];
-        }
-    }
-#pragma unroll
-    for (int i = 0; i < SQ_RPW; ++i) sum[i] = wave_sum(sum[i]);
-#pragma unroll
-    for (int i = 0; i < SQ_RPW; ++i) {
-        const int row = wave * SQ_RPW + i;
-        float *srow = S + row * pitch;
-        const bool live = r0 + row < L;
-        float *dprow = a.o0 + poff + (size_t)(r0 + row) * L;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const int c = lane + 64 * j;
-            if (c < L) {
-                if (live) dprow[c] = gv[i][j];
-                srow[c] = ((gv[i][j] - sum[i]) * pr[i][j]) * a.scale;
+                for (int i = 0; i < SQ_RPW; ++i) {
+                    if (r0 + first + i < L) sq_put(a.o0 + poff + (r0 + first + i) * L + 64 * j, (unsigned)lane * 4u, gv[i][j]);
+                    rows[i * pitch + 64 * j] = ((gv[i][j] - sum[i]) * pr[i][j]) * a.scale;
+                }
             }
-        }
-        if (live && lane == 0) a.o2[((size_t)b * a.heads + h) * L + r0 + row] = sum[i];
+        if (lane == 0)
+#pragma unroll
+            for (int i = 0; i < SQ_RPW; ++i)
+                if (r0 + first + i < L) a.o2[((size_t)b * a.heads + h) * L + r0 + first + i] = sum[i];
     }
     __syncthreads();
     // dq[d][query] = sum_key k[d][key] dS[query][key]   (:1342-1360)
-    sq_mix<HB>(Ks, S, L, a.H, r0, a.o1 + hoff, att_lds, tid, wave, l32, half);
+    sq_mix<HB, LINE>(Ks, S, L, a.H, r0, a.o1 + hoff, att_lds, tid, wave, l32, half);
 }
 
-// Key side, a tile of 32 keys: one workgroup forms dv, one dk.  dA (q) is resident as [d][query], the key
-// columns of P (and dP) go straight to registers, 128 bytes of a query per half wave.
+// Key side, a tile of 32 keys: one workgroup forms dv, one dk.  dA (q) is the panel, the key columns of P (and dP) go straight
+// to registers, 128 bytes of a query per half wave.  NB: blocks of 32 features a wave forms.  Both (beyond 128 tokens), so that
+// no two waves load the same columns: 30 -> 25 us for 32 x 3 heads of 64 and 197 tokens; with fewer tokens an eighth of them is
+// a group or two, and one block a wave the better (59 x 3 of 48 and 96 tokens 16.7 against 17.7 us).
 //   dv[d][key] = sum_query dA[d][query] P[query][key]                         (:884-902)
 //   dk[d][key] = sum_query q[d][query] dS[query][key], dS = (dP - rs) P scale  (:1244-1330)
-template <int HB, bool DK>
+template <int HB, bool LINE, bool DK, int NB>
 __device__ inline void sq_key(const AttnArgs &a, const SqPlace &at, float *lds) {
-    constexpr int KS = SQ_NW / HB, STEP = 4;
+    constexpr int KS = SQ_NW * NB / HB, PER = 4;  // shares of the queries, groups of eight of them a wave
     const int c0 = at.tile * 32, L = a.L, H = a.H, pitch = sq_pitch(L);
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int l32 = lane & 31, half = lane >> 5;
     const size_t hoff = ((size_t)at.b * a.F + (size_t)at.h * H) * L, row0 = (size_t)at.b * a.heads + at.h;
     const float *P = a.p + row0 * L * L, *G = a.dp + row0 * L * L;
-    const TileEdge edge = sq_fetch<HB>((DK ? a.q : a.da) + hoff, L, H, lds, a.zero, tid, wave, lane);
+    const TileEdge edge = sq_fetch<HB, LINE>((DK ? a.q : a.da) + hoff, L, H, lds, a.zero, tid, wave, lane);
     float *rsl = lds + 32 * HB * pitch;  // (zeros up to the next group of eight)
     if (DK && tid < pitch) rsl[tid] = tid < L ? a.rs[row0 * L + tid] : 0.f;
-    const int db = wave % HB, ks = wave / HB;
-    const unsigned c = (unsigned)min(c0 + l32, L - 1);
+    const int db = NB == 1 ? wave % HB : 0, ks = NB == 1 ? wave / HB : wave;
+    const unsigned c = (unsigned)min(c0 + l32, L - 1) * 4u;
     const int groups = (L + 7) >> 3, per = (groups + KS - 1) / KS, g0 = ks * per, end = min(groups, g0 + per);
     tile_edge_store(edge);
     wait_vmcnt<0>();
     __syncthreads();
-    mh_f32x16 acc = {0};
-    for (int g = g0; g < end; g += STEP) {
-        float p[STEP][4], q[STEP][4];  // of the four queries of a group that this half holds
+    float p[PER][4], q[PER][4];  // of the four queries of a group that this half holds
 #pragma unroll
-        for (int u = 0; u < STEP; ++u)
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const unsigned o = (unsigned)(min(min(g + u, end - 1) * 8 + half * 4 + j, L - 1) * L) + c;
-                p[u][j] = P[o];
-                if (DK) q[u][j] = G[o];
-            }
-        __builtin_amdgcn_sched_barrier(0);  // (all of them in flight before the first is waited for)
-#pragma unroll
-        for (int u = 0; u < STEP; ++u) {
-            if (g + u >= end) break;
-            const int k4 = (g + u) * 8 + half * 4;
-            float o[4];
+    for (int u = 0; u < PER; ++u)
+        if (g0 + u < end) {
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
-                o[j] = DK ? ((q[u][j] - rsl[k4 + j]) * p[u][j]) * a.scale : p[u][j];
-                if (k4 + j >= L) o[j] = 0.f;
+                const unsigned o = (unsigned)min(((g0 + u) * 8 + j) * L + half * 4 * L, (L - 1) * L) * 4u + c;
+                p[u][j] = sq_load(P, o);
+                if (DK) q[u][j] = sq_load(G, o);
             }
-            mfma4(acc, *reinterpret_cast<const float4 *>(lds + (db * 32 + l32) * pitch + k4), make_float4(o[0], o[1], o[2], o[3]));
         }
+    __builtin_amdgcn_sched_barrier(0);  // (all of them in flight before the first is waited for)
+    mh_f32x16 acc[NB];
+#pragma unroll
+    for (int i = 0; i < NB; ++i) acc[i] = mh_f32x16{0};
+#pragma unroll
+    for (int u = 0; u < PER; ++u) {
+        if (g0 + u >= end) break;
+        const int k4 = (g0 + u) * 8 + half * 4;
+        const float4 rs = DK ? *reinterpret_cast<const float4 *>(rsl + k4) : make_float4(0.f, 0.f, 0.f, 0.f);
+        float o[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) o[j] = DK ? ((q[u][j] - (j == 0 ? rs.x : j == 1 ? rs.y : j == 2 ? rs.z : rs.w)) * p[u][j]) * a.scale : p[u][j];
+        if ((g0 + u) * 8 + 8 > L) {
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                if (k4 + j >= L) o[j] = 0.f;
+        }
+#pragma unroll
+        for (int i = 0; i < NB; ++i) mfma4(acc[i], sq_frag<LINE>(lds, (db + i) * 32 + l32, k4, L, pitch), make_float4(o[0], o[1], o[2], o[3]));
     }
-    sq_store<HB>(acc, lds, L, H, c0, (DK ? a.o1 : a.o0) + hoff, tid, wave, l32, half);
+    float *out = (DK ? a.o1 : a.o0) + hoff;
+    if (NB == 1) {
+        sq_store<HB>(acc[0], lds, L, H, c0, out, tid, wave, l32, half);
+    } else {
+#pragma unroll
+        for (int i = 0; i < NB; ++i) sq_store<1>(acc[i], lds, L, H - 32 * i, c0, out + (size_t)32 * i * L, tid, wave, l32, half);
+    }
 }
 
-template <int HB>
-__global__ __launch_bounds__(SQ_NT, 4) void attn_bw_key_res_kernel(AttnArgs a) {
+template <int HB, bool LINE>
+__global__ __launch_bounds__(SQ_NT, HB == 1 ? 8 : 6) void attn_bw_key_res_kernel(AttnArgs a) {
     extern __shared__ __attribute__((aligned(16))) float att_lds[];
+    fetch_args(a);
     SqPlace at;
-    if (!sq_place(a, 2, at)) return;
-    if (at.part == 1) sq_key<HB, true>(a, at, att_lds);
-    else sq_key<HB, false>(a, at, att_lds);
+    if (!sq_place<2>(a, at)) return;
+    if (HB == 2 && a.L > 128) {
+        if (at.part == 1) sq_key<HB, LINE, true, HB>(a, at, att_lds);
+        else sq_key<HB, LINE, false, HB>(a, at, att_lds);
+    } else {
+        if (at.part == 1) sq_key<HB, LINE, true, 1>(a, at, att_lds);
+        else sq_key<HB, LINE, false, 1>(a, at, att_lds);
+    }
 }
 
 // Row softmax over H rows of W (one wave per row).
@@ -1013,9 +1145,9 @@ static int launch_attn(int which, AttnArgs &a, int ns) {
     return hip_ok(hipGetLastError(), "attention launch") ? 0 : 2;
 }
 
-template <int HB>
+template <int HB, bool LINE>
 static int launch_attn_res(int which, AttnArgs &a, int ns) {
-    void (*kern)(AttnArgs) = which == 0 ? attn_fw_res_kernel<HB> : which == 1 ? attn_bw_query_res_kernel<HB> : attn_bw_key_res_kernel<HB>;
+    void (*kern)(AttnArgs) = which == 0 ? attn_fw_res_kernel<HB, LINE> : which == 1 ? attn_bw_query_res_kernel<HB, LINE> : attn_bw_key_res_kernel<HB, LINE>;
     static bool attr_set[3] = {false, false, false};
     if (!attr_set[which]) {
         if (!hip_ok(hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
@@ -1025,6 +1157,8 @@ static int launch_attn_res(int which, AttnArgs &a, int ns) {
         attr_set[which] = true;
     }
     a.ns = ns;
+    a.d_tiles = rag_div((long long)((a.L + 31) / 32) * (which == 2 ? 2 : 1));
+    a.d_heads = rag_div(a.heads);
     const long long blocks = ((long long)ns * a.heads + 7) / 8 * 8 * ((a.L + 31) / 32) * (which == 2 ? 2 : 1);
     if (blocks >= (1ll << 31)) {
         set_error("attention: too many heads");
@@ -1038,7 +1172,10 @@ static int launch_attn_any(int which, AttnArgs &a, int ns) {
     if (a.L <= SQ_L && a.H <= 64) {
         a.zero = static_cast<const float *>(state().zeros);
         if (!a.zero) return 2;
-        return a.H <= 32 ? launch_attn_res<1>(which, a, ns) : launch_attn_res<2>(which, a, ns);
+        // LINE: every head's block in whole pieces of 16 bytes.  Rows of whole pieces (L % 4 == 0) would meet few banks that way.
+        const uintptr_t at = reinterpret_cast<uintptr_t>(which == 2 ? a.q : a.k) | reinterpret_cast<uintptr_t>(which == 2 ? a.da : a.v);
+        if (a.L % 4 && a.H % 4 == 0 && at % 16 == 0) return a.H <= 32 ? launch_attn_res<1, true>(which, a, ns) : launch_attn_res<2, true>(which, a, ns);
+        return a.H <= 32 ? launch_attn_res<1, false>(which, a, ns) : launch_attn_res<2, false>(which, a, ns);
     }
     if (a.H <= 32) return launch_attn<32>(which, a, ns);
     if (a.H <= 64) return launch_attn<64>(which, a, ns);
