@@ -123,9 +123,9 @@ static void *grow(void *&buf, size_t &have, size_t want, const char *what) {
 float *workspace(size_t bytes) {
     State &st = state();
     void *p = st.ws;
-    p = grow(p, st.ws_bytes, bytes, "hipMalloc(workspace)");
-    st.ws = static_cast<float *>(p);
-    return st.ws;
+    void *got = grow(p, st.ws_bytes, bytes, "hipMalloc(workspace)");
+    st.ws = static_cast<float *>(p);  // (a growth that is refused leaves the one that is there)
+    return static_cast<float *>(got);
 }
 
 void *scratch(size_t bytes) {
