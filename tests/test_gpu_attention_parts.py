@@ -1,0 +1,96 @@
+"""The parts that the weight gradients of attention are formed in beside the input gradient: against 64 bits where a part is a few
+slabs, where there are several rounds of workgroups and where nothing is split; and with a workspace too small for them, in a
+capture that must not grow it."""
+import ctypes
+import os
+import subprocess
+import sys
+
+import numpy as np
+import pytest
+import torch
+
+import helpers as hp
+
+pytestmark = pytest.mark.gpu
+
+
+def backward(pkg, gpu, ns, L, E, F, heads, run=None):
+    """Backward from random states; (arguments' tensors, gradients), the gradients of `run` if that calls it."""
+    sh = hp.mhsa_shapes(ns, L, E, F, heads)
+    g = torch.Generator().manual_seed(L + F)
+    data = {n: (torch.rand(s, generator=g) - 0.5).cuda() for n, s in sh.items()}
+    data["p"] /= L
+    diff = {n: torch.full(sh[n], 7.0, device="cuda") for n in ("q", "k", "v", "att", "p", "wo")}
+    diff.update({n: torch.full((F, E), 7.0, device="cuda") for n in ("wq", "wk", "wv")})
+    diff["x"], diff["y"] = torch.zeros(sh["x"], device="cuda"), (torch.rand(sh["y"], generator=g) - 0.5).cuda()
+    a, keep = hp.mhsa_args(pkg, data, diff, L, E, F, heads)
+    call = lambda: gpu.ptl_mhsa_fp32_bw_batched(ctypes.byref(a), ns)
+    if run:
+        run(call, diff)
+    else:
+        assert call() == 0, gpu.ptl_last_error().decode()
+        assert gpu.ptl_sync() == 0
+    return data, diff
+
+
+# samples, tokens, token size, features, heads
+@pytest.mark.parametrize("case", [(1, 5, 8, 8, 1), (64, 17, 192, 192, 3), (40, 33, 70, 96, 2), (31, 128, 64, 64, 2), (12, 131, 192, 192, 3),
+                                  (8, 130, 320, 320, 10), (64, 129, 64, 128, 2), (33, 192, 192, 192, 6)])
+def test_against_64_bits(pkg, gpu, case):
+    ns, L, E, F, heads = case
+    data, diff = backward(pkg, gpu, ns, L, E, F, heads)
+    x, dy, att = data["x"].double(), diff["y"].double(), data["att"].double()
+    flat = lambda t: t.transpose(0, 1).reshape(t.shape[1], -1)  # [rows][samples x tokens]
+    rel = lambda got, ref: float((got.double() - ref).norm() / ref.norm())
+    for w, n in (("wq", "q"), ("wk", "k"), ("wv", "v")):
+        assert rel(diff[w], flat(diff[n].double()) @ flat(x).T) <= 1e-6, w  # (32-bit sums of sums of 32: 2e-7 in the mean)
+    assert rel(diff["wo"].reshape(E, F), flat(dy) @ flat(att).T) <= 1e-6
+    dx = sum(data[w].double().reshape(E, F) @ flat(diff[n].double()) for w, n in (("wq", "q"), ("wk", "k"), ("wv", "v")))
+    assert rel(flat(diff["x"]), dx) <= 1e-6
+
+
+SMALL = (28, 130, 384, 384, 12)  # 22 MiB of partial sums; a fifth of the parts fit in 8
+
+
+def captured_in_a_small_workspace():
+    import __graft_entry__ as ge
+    pkg = ge.load_package()
+    gpu = pkg.load()
+    assert gpu.ptl_init(0) == 0 and gpu.ptl_reserve(1, 8 << 20) == 0
+    ws, sc = ctypes.c_size_t(0), ctypes.c_size_t(0)
+    gpu.ptl_reserved(ctypes.byref(ws), ctypes.byref(sc))
+    assert ws.value == 8 << 20, ws.value
+    side, graph = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+
+    def run(call, diff):
+        torch.cuda.synchronize()
+        gpu.ptl_set_stream(ctypes.c_void_p(side.cuda_stream))
+        with torch.cuda.graph(graph, stream=side):
+            rc = call()
+        assert rc == 0, gpu.ptl_last_error().decode()
+        for _ in range(3):
+            for n, t in diff.items():
+                if n != "y":
+                    t.zero_()
+            torch.cuda.synchronize()
+            graph.replay()
+            torch.cuda.synchronize()
+
+    _, got = backward(pkg, gpu, *SMALL, run=run)
+    gpu.ptl_set_stream(None)
+    gpu.ptl_reserved(ctypes.byref(ws), ctypes.byref(sc))
+    assert ws.value == 8 << 20, ws.value
+    _, ref = backward(pkg, gpu, *SMALL)
+    gpu.ptl_reserved(ctypes.byref(ws), ctypes.byref(sc))
+    assert ws.value > 8 << 20, ws.value  # the parts that a call takes that may grow it
+    for n in ("wq", "wk", "wv", "wo", "x", "q", "k", "v"):
+        assert float((got[n].double() - ref[n].double()).norm() / ref[n].double().norm()) <= 1e-6, n
+    print("captured", flush=True)
+
+
+def test_capture_with_a_small_workspace(gpu):
+    here = os.path.dirname(os.path.abspath(__file__))
+    code = "import sys; sys.path[:0] = [%r, %r]; import test_gpu_attention_parts as t; t.captured_in_a_small_workspace()" % (here, os.path.dirname(here))
+    r = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=100)
+    assert r.returncode == 0 and "captured" in r.stdout, r.stdout + r.stderr
