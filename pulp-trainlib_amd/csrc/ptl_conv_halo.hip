@@ -31,6 +31,7 @@ namespace ptl {
 namespace {
 
 constexpr int HALO_BM = 256;                       // positions per tile
+constexpr int HALO_SHORT = 192;                    // and of a short one: three of a wave's four fragments
 constexpr int HALO_NP = 384;                       // positions held per channel block (tile + 2*Wp + 2, padded)
 constexpr int HALO_BYTES = HALO_NP * 8 * 16;       // one buffer: 8 channel blocks
 constexpr int HALO_NT = 256;
@@ -50,6 +51,7 @@ struct HaloArgs {
     int s_img, s_row;
     int batch, Cin, Cout, Hp, Wp, Ho, Wo;
     int tiles, ct_count;  // tile = position tile * ct_count + filter tile
+    int full_tiles;       // those of HALO_BM rows; the tiles behind them have HALO_SHORT (see halo_tiles)
     int xcd_map;          // 1: the grid is a multiple of 8 and a workgroup's first tile follows its XCD
     // channel-major route, optional: the output once more as the next layer's blocked, padded input
     half_t *yblk;           // [Cout/8][yb_P] chunks of eight filters, nullptr: no such copy
@@ -150,7 +152,12 @@ __global__ __launch_bounds__(HALO_NT) void conv_halo_kernel(const HaloArgs a) {
     constexpr int LB = BN / 32;          // filter chunks per thread and stage
     constexpr int FM = BN / 16, FN = 4;  // fragments per wave: filters x positions (64 positions per wave)
     constexpr int MID = 1;               // half of a stage in front of which the next stage is certified
-    constexpr int NR = FM + FN, NM = FM * FN;  // fragment reads / MFMAs per half stage (one k-step of 32)
+    // SHORT: there are short tiles, and a wave's fourth position fragment is multiplied last, behind a branch.  Every form
+    // of that (also a body for each kind of tile) cost the channel-major tiles 3 to 8 % and gained 7 to 9 in the short ones;
+    // here it costs nothing.
+    constexpr bool SHORT = HWC && BN == 128;
+    constexpr int COLS = SHORT ? FN - 1 : FN;  // fragments among whose MFMAs the reads and loads are issued
+    constexpr int NR = FM + FN, NM = FM * COLS;  // fragment reads / MFMAs of them per half stage (one k-step of 32)
     static_assert(NS >= 3 && NS <= 7 && pipe_tile_first<NS>(), "ring depth");
     extern __shared__ __align__(16) char smem[];
     const unsigned halo_lds = (unsigned)(uintptr_t)(lds_char *)smem, ring_lds = halo_lds + 2 * HALO_BYTES;
@@ -175,12 +182,18 @@ __global__ __launch_bounds__(HALO_NT) void conv_halo_kernel(const HaloArgs a) {
 
     // The divisions that locate a tile and the 64-bit products behind its addresses are about a hundred scalar
     // instructions: once per unit, not once per load.
+    // the first row of a position tile, the rows of a wave
+    auto first_row = [&](unsigned pt) {
+        const unsigned full = SHORT ? (unsigned)a.full_tiles / (unsigned)a.ct_count : pt + 1;
+        return pt < full ? pt * HALO_BM : full * HALO_BM + (pt - full) * HALO_SHORT;
+    };
+    auto span = [&](int tile) { return (unsigned)(!SHORT || tile < a.full_tiles ? HALO_BM / 4 : HALO_SHORT / 4); };
     auto make_unit = [&](int tile, int cs) {
         HaloUnit u;
         u.tile = tile;
         u.cs = cs;
         const unsigned pt = (unsigned)tile / (unsigned)a.ct_count, ct = (unsigned)tile - pt * (unsigned)a.ct_count;
-        const unsigned q0 = pt * HALO_BM, b0 = q0 / a.qimg;
+        const unsigned q0 = first_row(pt), b0 = q0 / a.qimg;
         u.rem0 = q0 - b0 * a.qimg;
         u.p0 = q0 + b0 * a.jump;  // (the host keeps the positions, a tile's reach included, below 2^31)
         u.loc0 = 0;
@@ -198,7 +211,7 @@ __global__ __launch_bounds__(HALO_NT) void conv_halo_kernel(const HaloArgs a) {
     auto lane_rows = [&](const HaloUnit &u, unsigned (&row)[FN]) {
 #pragma unroll
         for (int j = 0; j < FN; ++j) {
-            const unsigned r = (unsigned)(64 * wave + 16 * j + l16), v = u.rem0 + r;
+            const unsigned r = span(u.tile) * (unsigned)wave + (unsigned)(16 * j + l16), v = u.rem0 + r;
             if (!HWC && a.dense) {
                 // pixel (cross samples on, y, x) -> its padded position, from the tile's first one
                 unsigned cross = 0;
@@ -338,7 +351,7 @@ __global__ __launch_bounds__(HALO_NT) void conv_halo_kernel(const HaloArgs a) {
             // order (nothing may cross a sched_barrier): the address arithmetic of a load sits between two MFMAs
             // instead of in front of a run of them.
             static_for<0, NM>([&](auto MI) {
-                constexpr int m = decltype(MI)::value, i = m / FN, j = m % FN;
+                constexpr int m = decltype(MI)::value, i = m / COLS, j = m % COLS;
                 if constexpr (m < NR) read_frag(cur ^ 1, wnext, xbuf, hn, m);
                 mfma16(acc[i][j], wf[cur][i], xf[cur][j]);
                 if constexpr (m >= NR && (m - NR) % dstep == 0) {
@@ -358,6 +371,11 @@ __global__ __launch_bounds__(HALO_NT) void conv_halo_kernel(const HaloArgs a) {
                 }
                 __builtin_amdgcn_sched_barrier(0);
             });
+            if constexpr (SHORT)
+                if (cu.tile < a.full_tiles) {
+                    static_for<0, FM>([&](auto II) { mfma16(acc[decltype(II)::value][FN - 1], wf[cur][decltype(II)::value], xf[cur][FN - 1]); });
+                    __builtin_amdgcn_sched_barrier(0);
+                }
             if constexpr (half == 1) {
                 prev_off = slot_off;
                 slot_off = slot_off + STAGE == NS * STAGE ? 0u : slot_off + STAGE;
@@ -365,16 +383,16 @@ __global__ __launch_bounds__(HALO_NT) void conv_halo_kernel(const HaloArgs a) {
         });
         const bool tile_done = cu.cs + 1 == UC;
         if (tile_done) {
-            const unsigned q0 = ((unsigned)cu.tile / (unsigned)a.ct_count) * HALO_BM;
+            const unsigned q0 = first_row((unsigned)cu.tile / (unsigned)a.ct_count);
             const int co0 = (cu.tile % a.ct_count) * BN;
             const unsigned PO = (unsigned)(a.Ho * a.Wo);
             if constexpr (HWC) {
 #pragma unroll
                 for (int j = 0; j < FN; ++j) {
-                    const unsigned q = q0 + (unsigned)(64 * wave + 16 * j + l16);  // (Q < 2^31 on the host)
+                    const unsigned r = (unsigned)(16 * j + l16), q = q0 + span(cu.tile) * (unsigned)wave + r;  // (Q < 2^31 on the host)
                     const unsigned b = q / a.qimg, rem = q - b * a.qimg;
                     const unsigned yy = rem / (unsigned)a.Wp, xx = rem - yy * (unsigned)a.Wp;
-                    if (q < a.Q && yy < (unsigned)a.Ho && xx < (unsigned)a.Wo) {
+                    if (r < span(cu.tile) && q < a.Q && yy < (unsigned)a.Ho && xx < (unsigned)a.Wo) {
                         // a lane holds four consecutive filters of its position per filter fragment
                         half_t *dst = a.y + ((size_t)b * PO + yy * (unsigned)a.Wo + xx) * (unsigned)a.Cout + co0 + 4 * kq;
 #pragma unroll
@@ -938,6 +956,30 @@ __global__ __launch_bounds__(256) void conv_halo_embed_kernel(const half_t *__re
 
 }  // namespace
 
+// Position tiles of the rows a.Q of the 128-filter channel-minor kernel, and how many tiles are whole.  Every CU takes a tile a
+// round, so that the last round costs a whole one however few tiles it has; where its rows, and those of the rounds before it if
+// need be, cost less in short tiles (0.8 of a whole one: their filters are as many), they have those.  Batch 128, 128 -> 128 on
+// 28 x 28 45 -> 42 us, 100, 128 -> 256 on 20 x 20 45.1 -> 39.1, 77, 192 -> 128 on 33 x 33 58.3 -> 51.5; 40, 512 -> 512 on 14 x 14 (one
+// round of 132 or 176) 65 -> 58.5; layers that keep their tiles as before.
+static long long halo_tiles(HaloArgs &a) {
+    const long long cu = state().num_cu, whole = ((long long)a.Q + HALO_BM - 1) / HALO_BM;
+    auto rounds = [&](long long tiles) { return (tiles * a.ct_count + cu - 1) / cu; };
+    const long long most = rounds(whole);
+    long long best = 10 * most, tiles = whole, full = whole;
+    for (long long k = most - 1; k >= 0 && k + 4 > most; --k) {  // (four short rounds are three whole ones)
+        const long long some = k * cu / a.ct_count, rest = (long long)a.Q - some * HALO_BM;
+        if (rest <= 0) continue;
+        const long long all = some + (rest + HALO_SHORT - 1) / HALO_SHORT, cost = 10 * k + 8 * (rounds(all) - k);
+        if (cost < best) {
+            best = cost;
+            tiles = all;
+            full = some;
+        }
+    }
+    a.full_tiles = (int)(full * a.ct_count);
+    return tiles;
+}
+
 long long conv_halo_margin() { return HALO_BM + HALO_NP; }
 
 bool conv_halo_fits(const ConvTileDesc &d, int Hp, int Wp) {
@@ -1047,8 +1089,9 @@ int conv_halo_hwc_launch(const ConvTileDesc &d, const void *X, const void *wr, v
     magic31((unsigned)a.Wp, &a.m_row, &a.s_row);
     const int bn = d.Cout % 128 == 0 ? 128 : 64;
     a.ct_count = d.Cout / bn;
-    const long long ptiles = ((long long)a.Q + HALO_BM - 1) / HALO_BM;
+    long long ptiles = ((long long)a.Q + HALO_BM - 1) / HALO_BM;
     if (ptiles * a.ct_count >= (1ll << 30)) return -1;
+    if (bn == 128) ptiles = halo_tiles(a);
     a.tiles = (int)(ptiles * a.ct_count);
     const int grid = a.tiles < st.num_cu ? a.tiles : st.num_cu;
     a.xcd_map = grid % 8 == 0;
