@@ -1546,6 +1546,7 @@ static int mhsa_bw(const Mhsa_args *a, int ns, const char *fn) {
     float *dP = sg.out(a->softmax_buffer->diff, pe);
     if (sg.failed()) return 2;
     const bool rag = rag_takes(m);  // (its partial sums, where there are any, are in the workspace)
+    state().last_gemm_form = 0;
     const size_t p1 = rag ? 0 : panel_part_floats(1, E, F, ns), p3 = rag ? 0 : panel_part_floats(3, F, E, ns);
     float *rs = static_cast<float *>(scratch((rows + p1 + p3) * sizeof(float)));
     if (!rs) return 2;
