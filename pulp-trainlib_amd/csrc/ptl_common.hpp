@@ -152,6 +152,7 @@ bool ensure_init();
 void set_error(const char *fmt, ...);
 bool hip_ok(hipError_t e, const char *what);
 float *workspace(size_t bytes);
+float *workspace_if(size_t bytes);  // nullptr, and no error, where it would have to grow and cannot: in a capture, for lack of memory
 void *scratch(size_t bytes);
 
 template <typename T>

@@ -850,9 +850,8 @@ static GvShares gv_shares(int K, int M, int ns = 1) {
     const int cu = state().num_cu, z = std::min({2 * cu / sh.cols, K / 512, 32});
     if (K < (ns > 1 ? FEW_SHARED : 4096) || sh.cols > cu / 2 || z < 2) return sh;
     const int chunk = (K + z - 1) / z, shares = (K + chunk - 1) / chunk;
-    // (a stream that is being captured, or a full device, cannot get a workspace: one share then, and no error behind it)
-    if (float *part = workspace((size_t)shares * ns * M * sizeof(float))) sh = {sh.cols, shares, chunk, part};
-    else (void)hipGetLastError();
+    // (a stream that is being captured, or a full device, cannot get a workspace: one share then)
+    if (float *part = workspace_if((size_t)shares * ns * M * sizeof(float))) sh = {sh.cols, shares, chunk, part};
     return sh;
 }
 

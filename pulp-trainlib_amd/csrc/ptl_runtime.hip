@@ -95,6 +95,8 @@ static bool stream_is_capturing(hipStream_t s) {
     return status != hipStreamCaptureStatusNone;
 }
 
+static size_t grown(size_t want) { return want < (size_t)(8u << 20) ? (size_t)(8u << 20) : want + want / 4; }
+
 static void *grow(void *&buf, size_t &have, size_t want, const char *what) {
     if (want <= have) return buf;
     State &st = state();
@@ -111,7 +113,7 @@ static void *grow(void *&buf, size_t &have, size_t want, const char *what) {
         buf = nullptr;
         have = 0;
     }
-    size_t sz = want < (size_t)(8u << 20) ? (size_t)(8u << 20) : want + want / 4;
+    const size_t sz = grown(want);
     if (!hip_ok(hipMalloc(&buf, sz), what)) {
         buf = nullptr;
         return nullptr;
@@ -126,6 +128,31 @@ float *workspace(size_t bytes) {
     void *got = grow(p, st.ws_bytes, bytes, "hipMalloc(workspace)");
     st.ws = static_cast<float *>(p);  // (a growth that is refused leaves the one that is there)
     return static_cast<float *>(got);
+}
+
+// For a caller that has another way without it.  The larger buffer comes before the present one goes, so that a refusal costs neither
+// that one nor a wait; only a lack of memory is passed over, another HIP error is left for the launch behind to report.
+float *workspace_if(size_t bytes) {
+    State &st = state();
+    if (bytes <= st.ws_bytes) return st.ws;
+    if (stream_is_capturing(st.stream)) return nullptr;
+    const size_t sz = grown(bytes);
+    void *more = nullptr;
+    const hipError_t e = hipMalloc(&more, sz);
+    if (e != hipSuccess) {
+        if (e == hipErrorOutOfMemory) (void)hipGetLastError();
+        return nullptr;
+    }
+    if (st.ws) {
+        if (hipDeviceSynchronize() != hipSuccess) {  // (see grow())
+            (void)hipFree(more);
+            return nullptr;
+        }
+        (void)hipFree(st.ws);
+    }
+    st.ws = static_cast<float *>(more);
+    st.ws_bytes = sz;
+    return st.ws;
 }
 
 void *scratch(size_t bytes) {
