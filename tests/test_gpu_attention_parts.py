@@ -102,3 +102,25 @@ def test_capture_with_a_small_workspace(gpu):
     code = "import sys; sys.path[:0] = [%r, %r]; import test_gpu_attention_parts as t; t.captured_in_a_small_workspace()" % (here, os.path.dirname(here))
     r = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=100)
     assert r.returncode == 0 and "captured" in r.stdout, r.stdout + r.stderr
+
+
+def large_step():
+    import __graft_entry__ as ge
+    pkg = ge.load_package()
+    gpu = pkg.load()
+    assert gpu.ptl_init(0) == 0
+    ws, sc = ctypes.c_size_t(0), ctypes.c_size_t(0)
+    for case in ((64, 256, 512, 512, 8), (64, 256, 1024, 1024, 16)):
+        test_against_64_bits(pkg, gpu, case)
+        gpu.ptl_reserved(ctypes.byref(ws), ctypes.byref(sc))
+        print(case, ws.value >> 20, "MiB", flush=True)
+        assert 0 < ws.value <= 160 << 20, ws.value
+    print("bounded", flush=True)
+
+
+def test_workspace_of_large_steps(gpu):
+    """Partial sums of at most 32 tiles of 16 KiB for each of the 512 places of a workgroup, and the quarter more that is allocated."""
+    here = os.path.dirname(os.path.abspath(__file__))
+    code = "import sys; sys.path[:0] = [%r, %r]; import test_gpu_attention_parts as t; t.large_step()" % (here, os.path.dirname(here))
+    r = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=100)
+    assert r.returncode == 0 and "bounded" in r.stdout, r.stdout + r.stderr
