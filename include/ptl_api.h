@@ -328,8 +328,8 @@ int ptl_sync(void);
  * ptl_last_gemm_tile() the output tile of the last product that ran a tile-per-workgroup kernel of the
  * look-up-free pipelined GEMM or of the kernel for any size and alignment (of several products in one launch, all of
  * them), as rows * 1000 + columns (256256 = 256 x 256, 128064 = 128 x 64);
- * ptl_last_gemm_form() how the last dense layer, matrix product or Conv2D call formed its sums: an fp32 product of it
- * from three bf16 pieces of each value (1), the contraction shared out over the waves of a 32 x 32 tile (2), the kernels
+ * ptl_last_gemm_form() how the last dense layer, matrix product, Conv2D or attention call formed its sums: an fp32 product of
+ * it (attention: the weight gradients) from three bf16 pieces of each value (1), the contraction shared out over the waves of a 32 x 32 tile (2), the kernels
  * for dense layers on a few samples (3), or otherwise (0). */
 void ptl_set_gemm_path(int path);
 int ptl_last_conv_direct(void);

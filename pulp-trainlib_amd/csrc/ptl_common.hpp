@@ -144,7 +144,7 @@ struct State {
     int last_conv_direct = 0;  // 1 if the last Conv2D forward / input-gradient call ran the direct kernel
     int last_gemm_tile = 0;    // rows * 1000 + columns of the tile of the last look-up-free pipelined product
     int staging_copies = 0;  // see ptl_staging_copies
-    int last_gemm_form = 0;    // of the last dense layer, matrix product or Conv2D: see ptl_last_gemm_form
+    int last_gemm_form = 0;    // of the last dense layer, matrix product, Conv2D or attention call: see ptl_last_gemm_form
 };
 
 State &state();

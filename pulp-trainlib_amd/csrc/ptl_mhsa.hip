@@ -1437,6 +1437,7 @@ static int mhsa_fw(const Mhsa_args *a, int ns, const char *fn) {
         set_error("%s: tensor larger than 2^31 elements", fn);
         return 1;
     }
+    state().last_gemm_form = 0;
     const int L = m.L, E = m.E, F = m.F;
     const size_t xe = (size_t)ns * E * L, fe = (size_t)ns * F * L, pe = (size_t)ns * m.heads * L * L;
     Stager sg;

@@ -176,3 +176,17 @@ def test_mhsa_rejects_bad_geometry(pkg, gpu):
     assert gpu.ptl_mhsa_fp32_fw_batched(ctypes.byref(a), 1) == 1
     assert b"geometry" in gpu.ptl_last_error()
     assert np.all(data["y"] == 0)
+
+
+def test_form_is_that_of_the_last_call(pkg, gpu):
+    """A dense layer in bf16 pieces, then an attention forward pass, which has none."""
+    g = torch.Generator(device="cuda").manual_seed(1)
+    x, w, y = (torch.rand(s, generator=g, device="cuda") for s in ((2048, 1000), (1001, 1000), (2048, 1001)))
+    a, keep = hp.linear_args(pkg, x, None, w, None, y, y, 1000, 1001)
+    pkg.call("ptl_linear_fp32_fw_batched", a, 2048)
+    assert gpu.ptl_sync() == 0 and gpu.ptl_last_gemm_form() == 1
+    L, E, F, heads = 33, 20, 64, 2
+    data = {n: torch.rand(s, generator=g, device="cuda") for n, s in hp.mhsa_shapes(2, L, E, F, heads).items()}
+    b, keep = hp.mhsa_args(pkg, data, {}, L, E, F, heads)
+    assert gpu.ptl_mhsa_fp32_fw_batched(ctypes.byref(b), 2) == 0, gpu.ptl_last_error().decode()
+    assert gpu.ptl_sync() == 0 and gpu.ptl_last_gemm_form() == 0
