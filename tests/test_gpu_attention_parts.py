@@ -124,3 +124,49 @@ def test_workspace_of_large_steps(gpu):
     code = "import sys; sys.path[:0] = [%r, %r]; import test_gpu_attention_parts as t; t.large_step()" % (here, os.path.dirname(here))
     r = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=100)
     assert r.returncode == 0 and "bounded" in r.stdout, r.stdout + r.stderr
+
+
+@pytest.mark.parametrize("what", ["infinity", "nan", "huge", "tiny"])
+@pytest.mark.parametrize("case", [(64, 130, 70, 96, 2), (32, 197, 192, 192, 3)])
+def test_values_outside_the_range_of_the_pieces(pkg, gpu, case, what):
+    """In the tokens and in the attention map, which only the weight gradients read: in pieces beside an input gradient that is not, which
+    keeps its bits.  Features without such a value keep theirs in the tiles that have none."""
+    ns, L, E, F, heads = case
+    sh = hp.mhsa_shapes(ns, L, E, F, heads)
+    g = torch.Generator().manual_seed(L)
+    data = {n: (torch.rand(s, generator=g) - 0.5).cuda() for n, s in sh.items()}
+    data["p"] /= L
+    dy = (torch.rand(sh["y"], generator=g) - 0.5).cuda()
+
+    def run():
+        diff = {n: torch.full(sh[n], 7.0, device="cuda") for n in ("q", "k", "v", "att", "p", "wo")}
+        diff.update({n: torch.full((F, E), 7.0, device="cuda") for n in ("wq", "wk", "wv")})
+        diff["x"], diff["y"] = torch.zeros(sh["x"], device="cuda"), dy
+        a, keep = hp.mhsa_args(pkg, data, diff, L, E, F, heads)
+        assert gpu.ptl_mhsa_fp32_bw_batched(ctypes.byref(a), ns) == 0, gpu.ptl_last_error().decode()
+        assert gpu.ptl_sync() == 0 and gpu.ptl_last_gemm_form() == 1
+        return diff
+
+    plain = run()
+    if what == "tiny":  # (the third piece of 1e-35 would lie below the smallest bf16)
+        data["x"].mul_(1e-35)
+        data["att"].mul_(1e-35)
+    else:  # (huge: rounds up to infinity as a bf16)
+        value = {"infinity": float("inf"), "nan": float("nan"), "huge": 3.4e38}[what]
+        data["x"][ns // 2, 66, 77] = value
+        data["att"][1, 67, 5] = -value
+    diff = run()
+    for n in ("x", "q", "k", "v", "att"):
+        assert torch.equal(diff[n], plain[n]), n
+    flat = lambda t: t.double().transpose(0, 1).reshape(t.shape[1], -1)
+    for w, left, right in (("wq", diff["q"], data["x"]), ("wk", diff["k"], data["x"]), ("wv", diff["v"], data["x"]), ("wo", dy, data["att"])):
+        if what in ("infinity", "nan"):
+            assert torch.equal(diff[w].reshape(left.shape[1], -1)[:, :64], plain[w].reshape(left.shape[1], -1)[:, :64]), w
+        ref, got = flat(left) @ flat(right).T.contiguous(), diff[w].reshape(left.shape[1], -1).double()
+        ref = torch.where(ref.abs() > torch.finfo(torch.float32).max, ref * float("inf"), ref)
+        assert torch.equal(got.isnan(), ref.isnan()), w
+        assert torch.equal(got.isinf(), ref.isinf()) and torch.equal(got[ref.isinf()], ref[ref.isinf()]), w
+        fin = ref.isfinite()
+        size = ref[fin].abs().max() if what == "huge" else (ref[fin] ** 2).mean().sqrt()
+        # up to 8320 products, 320 slabs: sqrt(320 / 3) roundings of 2^-25 and of 2^-24 in eight, six times that for the largest of 37 000
+        assert float((got[fin] - ref[fin]).abs().max()) <= 4e-6 * float(size), w
