@@ -285,7 +285,13 @@ void ptl_set_stream(void *hip_stream);
  * given sizes now (0 = leave); ptl_reserved reports their present sizes, so a caller can run its shapes once,
  * read the sizes and reserve them at start-up the next time.  A call that would have to grow a buffer while the
  * library's stream is being captured fails with status 2 and an error text that names ptl_reserve, and the
- * capture stays valid.  No counterpart in the reference (its callers own every buffer). */
+ * capture stays valid.  Two kinds of calls have another way when the workspace cannot grow, in a capture or for lack
+ * of memory, and take it without an error: sums of the columns of a matrix (the input gradient of a dense layer on
+ * one sample with 4096 outputs and more, on two to eight with 1536 and more, a product with a single row) walk their
+ * rows in one share, and the weight gradients of attention are added up in fewer parts (and as fp32 products or bf16
+ * pieces by the depth of those).  That takes longer, and their sums are rounded in another order than the same call's
+ * with the workspace that it asks for: reserve it, or run the step once before the capture, where either matters.
+ * No counterpart in the reference (its callers own every buffer). */
 int ptl_reserve(size_t workspace_bytes, size_t scratch_bytes);
 void ptl_reserved(size_t *workspace_bytes, size_t *scratch_bytes);
 int ptl_sync(void);
