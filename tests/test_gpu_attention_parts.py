@@ -119,7 +119,7 @@ def large_step():
 
 
 def test_workspace_of_large_steps(gpu):
-    """Partial sums of at most 32 tiles of 16 KiB for each of the 512 places of a workgroup, and the quarter more that is allocated."""
+    """52 and 64 MiB of partial sums (the latter 208 in parts of 40 slabs), and the quarter more that is allocated."""
     here = os.path.dirname(os.path.abspath(__file__))
     code = "import sys; sys.path[:0] = [%r, %r]; import test_gpu_attention_parts as t; t.large_step()" % (here, os.path.dirname(here))
     r = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=100)
